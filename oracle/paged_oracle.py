@@ -28,7 +28,7 @@ def build(force: bool = False) -> None:
     """Compile libpaged_oracle.so (and oracle/_ref when the reference checkout exists)."""
     if force or not os.path.exists(_LIB_PATH):
         subprocess.check_call(["make", "-C", _HERE, "-B" if force else "-s", "all"])
-    if os.path.isdir("/root/reference") and (force or not os.path.exists(_REF_LIB_PATH)
+    if os.path.isdir("/root/reference/compiler/runtime") and (force or not os.path.exists(_REF_LIB_PATH)
                                              or not os.path.exists(REF_ALLOC_DRIVER)):
         subprocess.check_call(["make", "-C", _HERE, "-B" if force else "-s", "_ref"])
 
