@@ -258,9 +258,9 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
  * where the caller keeps it:
  *   page_tables_flat_device  DEVICE pointer to n_page_tables_flat uint32 page ids (4-byte aligned)
  *   stream                   hipStream_t to launch on; NULL = the library's stream
- * Limits, refused with an error otherwise: batch <= 256; head_dim 64 or 128; GQA ratio 1, 2, 4, 8,
- * 16 or 32; page size a multiple of 64 (head_dim 64) or 32 (head_dim 128) tokens; q, o and the
- * pools 16-byte aligned.  mlc_hip_available() must have returned 1 before (set-up creates the
+ * Limits, refused with an error otherwise: batch <= 256; head_dim 64 or 128; GQA ratio 1 .. 16 or
+ * 32; page size 16, 32 or a multiple of 64 tokens (head_dim 64), 8, 16 or a multiple of 32 (head_dim
+ * 128); q, o and the pools 16-byte aligned.  mlc_hip_available() must have returned 1 before (set-up creates the
  * library's stream and looks up the scratch array's device address).  The call returns when the
  * kernel is enqueued (no synchronisation).  Every decode launch of this library on one GPU
  * uses the same scratch array, so they must follow each other: the library remembers the stream
@@ -296,7 +296,7 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
  * a call that would have to allocate, copy metadata or wait fails (and the capture with it): run
  * the pass once uncaptured first, which puts weights, norm vectors and tables on the device.  The
  * decode attention of a captured pass must be served by the tile-balanced kernel (head_dim 64 or
- * 128, page size a multiple of its tile, 16-byte aligned buffers).  mlc_hip_capture_end returns a
+ * 128, page sizes and GQA ratios as in the call above, 16-byte aligned buffers).  mlc_hip_capture_end returns a
  * handle > 0, or 0 (then nothing was kept; encode the pass uncaptured).  mlc_hip_captured_launches
  * counts the launches of the encode calls; the pass holds one more, the library's own first launch,
  * which moves a device word on by which the decode launches of one replay tell their split-K
@@ -406,7 +406,7 @@ long mlc_hip_decode_table_uploads(void);
  *                           KV head) pair this many; 0 = the same number of tiles; -1 (default) =
  *                           2 for GQA ratios of 4 and more (workgroups of four waves), 0 below
  *   "decode_mfma"           1 (default) = the tile-balanced decode kernel does a tile's arithmetic
- *                           on the matrix pipe where the shape allows it (4 to 16 query heads per
+ *                           on the matrix pipe where the shape allows it (up to 16 query heads per
  *                           KV head in 4 waves); 0 = on the vector pipe
  *   "prefill_stages"        2, 4, 6 or 8 K/V tiles staged in LDS by the prefill kernel (0 = automatic:
  *                           6); with 8 the kernel with 64 rows per wave lets its waves meet only

@@ -67,20 +67,18 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
 
     // ---- which kernel: the tile-balanced one wherever it applies
     int s_hpw = 0, s_nw = 0;
-    bool use_stream = !g.opt_force_generic && aligned &&
-                      (page_size_tokens % tile) == 0 && batch <= kStreamMaxBatch &&
-                      stream_variant(G, head_dim, &s_hpw, &s_nw);
     uint64_t total_tiles = 0;
-    if (use_stream) {
-        for (size_t r = 0; r < batch; ++r) {
-            uint64_t lim = seq_lens[r];
-            if (apply_causal && (uint64_t)q_positions[r] + 1 < lim) lim = (uint64_t)q_positions[r] + 1;  // :2286
-            total_tiles += (lim + tile - 1) / tile;
-        }
-        total_tiles *= kv_heads;
-        // (the kernel counts in units: tiles plus at most 64 per (request, KV head) pair)
-        if (total_tiles + 64ull * batch * kv_heads >= 0x7FFFFFFFull) use_stream = false;
+    for (size_t r = 0; r < batch; ++r) {
+        uint64_t lim = seq_lens[r];
+        if (apply_causal && (uint64_t)q_positions[r] + 1 < lim) lim = (uint64_t)q_positions[r] + 1;  // :2286
+        total_tiles += (lim + tile - 1) / tile;
     }
+    total_tiles *= kv_heads;
+    // (the kernel counts in units: tiles plus at most 64 per (request, KV head) pair)
+    const bool use_stream = !g.opt_force_generic && aligned && batch <= kStreamMaxBatch &&
+                            total_tiles + 64ull * batch * kv_heads < 0x7FFFFFFFull &&
+                            stream_variant(G, head_dim, page_size_tokens, total_tiles, &s_hpw, &s_nw) &&
+                            stream_page_ok(head_dim, page_size_tokens, s_hpw, s_nw);
     const DecodePlan* plan = nullptr;
     if (!use_stream) {
         if (!build_plan(page_tables_flat, n_flat, page_table_offsets, seq_lens, q_positions, batch,
@@ -127,11 +125,11 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
         if (!embed_table && !tables_upload(embed ? nullptr : meta3.data(), batch, &d_flat, &d_meta)) return 0;
         const size_t dyn_lds = batch <= 64 ? 0 : stream_dynamic_lds_bytes(batch);
         const int nbuf = stream_stages(batch);
-        const unsigned n_wg = stream_grid(G, head_dim, nbuf, dyn_lds);
+        const unsigned n_wg = stream_grid(s_hpw, s_nw, head_dim, nbuf, dyn_lds);
         StreamArgs a;
         stream_fill_common(a, q, k_pages, v_pages, o, batch, num_heads, kv_heads, head_dim, page_size_tokens,
                            apply_causal);
-        a.pair_cost = stream_pair_cost(s_nw, G, head_dim);
+        a.pair_cost = stream_pair_cost(s_nw);
         a.pt_flat = d_flat;
         {
             // pools this library allocated: the kernel clamps page ids below their size (the host
@@ -260,9 +258,10 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
     const size_t G = num_heads / kv_heads;
     const size_t tile = (head_dim == 64) ? 64 : 32;
     int hpw = 0, nw = 0;
-    if (!stream_variant(G, head_dim, &hpw, &nw) || (page_size_tokens % tile) != 0)
-        return fail("decode (no allocation): head_dim must be 64 or 128, the GQA ratio 1, 2, 4, 8, 16 or 32, "
-                    "the page size a multiple of 64 (head_dim 64) or 32 (head_dim 128) tokens");
+    if (!stream_variant(G, head_dim, page_size_tokens, 0, &hpw, &nw) || !stream_page_ok(head_dim, page_size_tokens, hpw, nw))
+        return fail("decode (no allocation): head_dim must be 64 or 128, the GQA ratio 1 .. 16 or 32, "
+                    "the page size 16, 32 or a multiple of 64 (head_dim 64), or 8, 16 or a multiple of 32 "
+                    "(head_dim 128) tokens");
     if (!aligned16(q) || !aligned16(k_pages) || !aligned16(v_pages) || !aligned16(o) ||
         (reinterpret_cast<uintptr_t>(page_tables_flat_device) & 3u))
         return fail("decode (no allocation): buffers must be 16-byte aligned");
@@ -275,6 +274,7 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
         total_tiles += (lim + tile - 1) / tile;
     }
     total_tiles *= kv_heads;
+    (void)stream_variant(G, head_dim, page_size_tokens, total_tiles, &hpw, &nw);   // (its choice, now that the tiles are known)
     if (total_tiles + 64ull * batch * kv_heads >= 0x7FFFFFFFull) return fail("decode (no allocation): too many KV tiles");
     {
         const size_t qo_bytes = batch * num_heads * head_dim * 4;
@@ -284,10 +284,10 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
     }
     const int nbuf = stream_stages(batch);
     const size_t dyn_lds = batch <= 64 ? 0 : stream_dynamic_lds_bytes(batch);
-    const unsigned n_wg = stream_grid(G, head_dim, nbuf, dyn_lds);
+    const unsigned n_wg = stream_grid(hpw, nw, head_dim, nbuf, dyn_lds);
     StreamArgs a;
     stream_fill_common(a, q, k_pages, v_pages, o, batch, num_heads, kv_heads, head_dim, page_size_tokens, apply_causal);
-    a.pair_cost = stream_pair_cost(nw, G, head_dim);
+    a.pair_cost = stream_pair_cost(nw);
     a.pt_flat = page_tables_flat_device;
     {
         // the page ids are on the device and cannot be checked here: pools this library allocated

@@ -158,9 +158,22 @@ int tables_upload(const uint32_t* meta3, size_t B, const uint32_t** d_flat, cons
 }
 
 // Shape of the tile-balanced launch for (G, D): query heads per wave, waves per workgroup;
-// false when the kernel does not cover the shape.
-bool stream_variant(size_t G, size_t D, int* hpw_out, int* nw_out) {
+// false when the kernel does not cover the shape.  On the matrix pipe every ratio up to 16 runs with
+// four waves, each with room for 1, 2 or 4 heads in the epilogue.  One or two query heads per KV head
+// stay on the vector pipe, in workgroups of one or two waves, where that is ahead: one head at head_dim
+// 64 (36.4 against 37.0 us at 32 requests of 8 / 8 heads), and calls of no more tiles than there are
+// workgroups (23.9 against 25.3 us per synchronous call at 512 tokens of 4 / 2 heads of 128: four waves
+// have to meet behind their one tile).  Elsewhere the matrix pipe is ahead by 10-20 % (50.9 against
+// 61.1 us at 8 requests of 32 / 32 heads of 128, 58.7 against 68.7 us at 32 of 16 / 8 heads of 64).
+bool stream_variant(size_t G, size_t D, size_t P, uint64_t total_tiles, int* hpw_out, int* nw_out) {
     if (D != 64 && D != 128) return false;
+    const bool whole_tiles = P % (D == 64 ? 64 : 32) == 0;
+    const bool vector_ahead = whole_tiles && G <= 2 && ((G == 1 && D == 64) || total_tiles <= 2ull * (uint64_t)g.n_cu);
+    if (g.opt_decode_mfma && g.opt_hpw_max == 0 && G >= 1 && G <= 16 && !vector_ahead) {
+        *hpw_out = G <= 4 ? 1 : G <= 8 ? 2 : 4;
+        *nw_out = 4;
+        return true;
+    }
     const long hpw_cap = g.opt_hpw_max > 0 ? g.opt_hpw_max : std::max<long>(1, (long)G / 4);
     int hpw = 8;
     while (hpw > 1 && (hpw > hpw_cap || (G % (size_t)hpw) != 0)) hpw >>= 1;
@@ -190,24 +203,32 @@ int stream_stages(size_t batch) {
 
 // Grid of the tile-balanced kernel: as many workgroups as stay resident (LDS decides), within
 // what the scratch array holds.
-unsigned stream_grid(size_t G, size_t D, int nbuf, size_t dyn_lds) {
-    const bool matrix_pipe = g.opt_decode_mfma && G >= 4 && G <= 16;
-    const size_t lds = stream_static_lds_bytes(nbuf, G, D, matrix_pipe) + dyn_lds;
+unsigned stream_grid(int hpw, int nw, size_t D, int nbuf, size_t dyn_lds) {
+    const size_t GP = (size_t)hpw * nw;
+    const bool matrix_pipe = g.opt_decode_mfma && nw == 4 && GP <= 16;
+    const size_t lds = stream_static_lds_bytes(nbuf, GP, D, matrix_pipe) + dyn_lds;
     size_t per_cu = std::max<size_t>(1, std::min<size_t>(160 * 1024 / lds, 2));
     if (g.opt_wgs_per_cu > 0) per_cu = (size_t)g.opt_wgs_per_cu;
     size_t W = (size_t)g.n_cu * per_cu;
     if (g.opt_grid_wgs > 0) W = (size_t)g.opt_grid_wgs;
     W = std::min<size_t>(W, kStreamMaxWgs);
-    int hpw = 1, nw = 1;
-    if (stream_variant(G, D, &hpw, &nw)) W = std::min<size_t>(W, kStreamPartBytes / stream_partial_bytes(G, D, (size_t)nw));
+    W = std::min<size_t>(W, kStreamPartBytes / stream_partial_bytes(GP, D, (size_t)nw));
     return (unsigned)std::max<size_t>(W, 1);
 }
 
-uint32_t stream_pair_cost(int nw, size_t G, size_t D) {
+uint32_t stream_pair_cost(int nw) {
     if (g.opt_pair_cost >= 0) return (uint32_t)g.opt_pair_cost;
-    (void)G;
-    (void)D;
     return nw == 4 ? 2u : 0u;
+}
+
+// Page sizes the tile-balanced kernel takes: pages of whole tiles (TT = 64 tokens at head_dim 64, 32 at
+// 128), and on the matrix pipe also pages that divide a tile into the slices of one or more of its four
+// waves (16 and 32 tokens at head_dim 64, 8 and 16 at 128).
+bool stream_page_ok(size_t D, size_t P, int hpw, int nw) {
+    const size_t tile = D == 64 ? 64 : 32;
+    if (P % tile == 0) return true;
+    const bool matrix_pipe = g.opt_decode_mfma && nw == 4 && hpw * nw <= 16;
+    return matrix_pipe && tile % P == 0 && P >= tile / 4;
 }
 
 // Arithmetic mode of the tile-balanced kernel: 0 fp32 softmax weights, 1 fp16 weights on the vector
@@ -280,6 +301,10 @@ void stream_fill_common(StreamArgs& a, const void* q, const void* k_pages, const
     a.num_heads = (uint32_t)H;
     a.kv_heads = (uint32_t)Hkv;
     a.page_size = (uint32_t)P;
+    a.group = (uint32_t)(H / Hkv);
+    const size_t tile = D == 64 ? 64 : 32;
+    a.pages_per_tile = P < tile ? (uint32_t)(tile / P) : 1u;
+    a.page_shift = (uint32_t)__builtin_ctzll(P);
     a.causal = causal ? 1u : 0u;
     a.capacity_pages = 0;
     a.meta = nullptr;

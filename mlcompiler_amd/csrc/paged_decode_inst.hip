@@ -31,12 +31,29 @@ void launch_stream_pv(int pvm, const StreamArgs& a, unsigned n_wg, size_t dyn_ld
     else
         hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, 0, SMALL, NBUF, SPLIT>), grid, block, dyn_lds, stream, a);
 }
+// The build for partly filled groups and pages smaller than a tile: two stages and fp32-grade softmax
+// weights, whatever the options ask for.
+template <int NW, bool SMALL, bool SPLIT>
+bool launch_stream_any(const StreamArgs& a, unsigned n_wg, size_t dyn_lds, hipStream_t stream) {
+    if constexpr (NW == 4 && MLC_HPW * NW <= 16) {
+        hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, 3, SMALL, 2, SPLIT, true>), dim3(n_wg), dim3(64 * NW),
+                           dyn_lds, stream, a);
+        return true;
+    }
+    return false;
+}
 template <int NW>
 bool launch_stream(int nbuf, int pvm, const StreamArgs& a, unsigned n_wg, size_t dyn_lds, hipStream_t stream) {
     // at most 64 requests: the variant that keeps the per-request figures in registers; larger
     // batches keep them in dynamic LDS, next to two or three stages
     // (the form that also splits its output for the matmul behind it: built for the default of
     // small batches only, two stages)
+    const bool any = a.group != MLC_HPW * NW || a.pages_per_tile > 1;
+    if (any) {
+        if (a.split_frag) return a.batch <= 64 && launch_stream_any<NW, true, true>(a, n_wg, 0, stream);
+        if (a.batch <= 64) return launch_stream_any<NW, true, false>(a, n_wg, 0, stream);
+        return launch_stream_any<NW, false, false>(a, n_wg, dyn_lds, stream);
+    }
     if (a.split_frag) {
         if (a.batch > 64 || nbuf != 2) return false;
         launch_stream_pv<NW, true, 2, true>(pvm, a, n_wg, 0, stream);

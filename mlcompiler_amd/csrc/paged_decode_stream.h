@@ -36,8 +36,9 @@ static constexpr uint32_t kStreamMaxBatch = 4096;   // 64-ary search over the ti
 static constexpr uint32_t kStreamMaxWgs = 2048;     // workgroups per launch, at most
 static constexpr size_t kStreamPartBytes = 8u << 20;  // the partial buffer
 static constexpr size_t kStreamProbeWord = kStreamPartBytes / 8;  // probe builds: time stamps behind the partials
-// Words per lane of a workgroup's partial (see the kernel): NW waves x (OPL + 1) words.
-constexpr size_t stream_partial_bytes(size_t G, size_t D, size_t NW) { return (G * D + 64 * NW) * 8; }
+// A workgroup's partial (see the kernel): NW waves x (OPL + 1) words per lane.  GP: query heads the
+// workgroup has room for (heads per wave x waves).
+constexpr size_t stream_partial_bytes(size_t GP, size_t D, size_t NW) { return (GP * D + 64 * NW) * 8; }
 
 struct StreamArgs {
     const float* q;             // [B][H][D]
@@ -56,6 +57,9 @@ struct StreamArgs {
     uint32_t num_heads;
     uint32_t kv_heads;
     uint32_t page_size;         // tokens per page
+    uint32_t group;             // query heads per KV head
+    uint32_t pages_per_tile;    // 1 where a page holds whole tiles; else pages in a tile (2, 4 or 8)
+    uint32_t page_shift;        // log2(page_size), used where pages_per_tile > 1
     uint32_t causal;
     uint32_t capacity_pages;    // page ids are clamped below this (0: not clamped)
     uint32_t meta_stride;
@@ -88,9 +92,9 @@ struct StreamArgs {
 static_assert(sizeof(StreamArgs) <= 4096, "kernel arguments are limited to 4 KiB");
 
 // LDS of one workgroup: NBUF stages of one K tile and one V tile (8 KiB each), and in matrix-pipe
-// mode (four waves, G query heads per KV head) the waves' results of a pair
-constexpr size_t stream_static_lds_bytes(int NBUF, size_t G, size_t D, bool matrix_pipe) {
-    return (size_t)NBUF * 2 * 8192 + (matrix_pipe ? (4 * G * D + 2 * 4 * G) * 4 : 24);
+// mode (four waves, room for GP query heads per KV head) the waves' results of a pair
+constexpr size_t stream_static_lds_bytes(int NBUF, size_t GP, size_t D, bool matrix_pipe) {
+    return (size_t)NBUF * 2 * 8192 + (matrix_pipe ? (4 * GP * D + 2 * 4 * GP) * 4 : 24);
 }
 // dynamic LDS: tile prefix [B + 1], visible lengths [B], page-table offsets [B]
 inline size_t stream_dynamic_lds_bytes(size_t batch) { return (4 * batch + 2) * 4; }
@@ -193,12 +197,16 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
 // through LDS where a pair of (request, KV head) ends.
 // SPLIT: the launch also writes its output as the split-fp16 activations of the Q4_0 matmul that
 // reads it (StreamArgs::split_frag).
-template <int D, int HPW, int NW, int PVM, bool SMALL, int NBUF, bool SPLIT = false>
+// ANY (matrix-pipe mode): the group may have fewer query heads than the workgroup has room for, and
+// pages may be smaller than a tile.  A build of its own because the extra uniform arithmetic costs the
+// kernel scalar registers, of which it has none left (2 % at 0.6 GB of KV when every launch had it).
+template <int D, int HPW, int NW, int PVM, bool SMALL, int NBUF, bool SPLIT = false, bool ANY = false>
 __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const StreamArgs a) {
     constexpr bool PV16 = PVM == 1;
     constexpr bool MF = PVM == 2 || PVM == 3;
     constexpr bool MF_SPLIT_P = PVM == 3;
     static_assert(!MF || (NW == 4 && HPW * NW <= 16), "matrix-pipe mode: 4 waves, at most 16 heads per KV head");
+    static_assert(!ANY || MF, "partly filled groups and small pages: matrix-pipe mode");
     static_assert(NBUF >= 2 && NBUF <= 4, "2 to 4 stages");
     static_assert(D == 64 || D == 128, "head_dim 64 and 128");
     static_assert(NW == 1 || NW == 2 || NW == 4, "waves per GQA group");
@@ -207,7 +215,11 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     constexpr int TT = 8 * RPI;        // tokens per tile
     constexpr int OPL = HPW * D / 64;  // outputs per lane in the epilogue
     constexpr int HPK = D / 64;        // epilogue registers per head
-    constexpr int G = HPW * NW;        // query heads per KV head
+    // Query heads per KV head.  With ANY any number up to GP: the heads are columns of the
+    // 16-wide MFMAs, whose unused ones cost nothing, and only the epilogue deals them out to the waves
+    // (wave hg has heads hg*HPW .. +HPW-1, as far as they exist).
+    constexpr int GP = HPW * NW;
+    const int G = ANY ? (int)a.group : GP;
     constexpr int TILE_BYTES = TT * D * 2;  // one tensor, one KV head: 8 KiB
     constexpr int LPW = 16 / NW;            // tile-load instructions per wave and tile (8 K + 8 V in all)
     constexpr int STAGE_BYTES = 2 * TILE_BYTES;
@@ -216,8 +228,8 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     constexpr int DB = D / 16;              // ... 16-row blocks of O^T
     __shared__ __attribute__((aligned(16))) unsigned char stages[NBUF * STAGE_BYTES];
     // matrix-pipe mode: the waves' (o, m, l) of a pair, combined where the pair ends
-    __shared__ __attribute__((aligned(16))) float comb_o[MF ? NW * G * D : 4];
-    __shared__ float comb_ml[MF ? 2 * NW * G : 2];
+    __shared__ __attribute__((aligned(16))) float comb_o[MF ? NW * GP * D : 4];
+    __shared__ float comb_ml[MF ? 2 * NW * GP : 2];
     extern __shared__ uint32_t s_meta[];
     const uint32_t B = a.batch;
     uint32_t* s_start = s_meta;            // [B + 1] tiles of the requests before r (one KV head)
@@ -444,7 +456,14 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         } while (req_tiles(cu.r) == 0);
         load_request(cu);
     };
-    const uint32_t tpp = a.page_size / TT;  // tiles per page (page size is a multiple of the tile)
+    // Pages and tiles: either a page holds `tpp` whole tiles, or (ANY) a tile spans `ppt`
+    // whole pages, each of which holds the token slices of one or more waves, so that a wave's loads
+    // of a tile stay in one page.  Page ids are kept by page unit: unit number t * ppt + page of the tile.
+    const uint32_t ppt = ANY ? a.pages_per_tile : 1u;
+    const uint32_t tpp = ppt > 1u ? 1u : a.page_size / TT;
+    auto page_units = [&](uint32_t tiles, uint32_t lim) {
+        return ppt > 1u ? (lim + a.page_size - 1u) >> a.page_shift : tiles;
+    };
 
     Cursor ci, cc;  // issue side (one tile ahead) and consume side
     if (PC == 0) {
@@ -478,10 +497,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     const uint32_t* emb_table = (const uint32_t*)(global_u32_ptr)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr() +
                                 offsetof(StreamArgs, emb) / 4 + 3u * (SMALL ? kStreamSmallStride : a.meta_stride);
     const uint32_t* pt_flat = a.pt_flat ? a.pt_flat : emb_table;
-    // Page ids of the issue side's request, 64 tiles at a time: lane i holds the page of tile
+    // Page ids of the issue side's request, 64 units at a time: lane i holds the page of unit
     // pv_win + i.  Refetched when the issue side enters another request or another window.
     uint32_t pv = 0, pv_win = 0, pv_req = 0xFFFFFFFFu;
-    // ... and of the first 64 tiles of the request behind it, requested when the issue side enters a
+    // ... and of the first 64 units of the request behind it, requested when the issue side enters a
     // request, so that the step into the next request finds them in a register
     uint32_t pv_nx = 0, pv_nx_req = 0xFFFFFFFFu;
     auto prefetch_next_pages = [&](uint32_t r) {
@@ -491,27 +510,27 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         } while (r < B && req_tiles(r) == 0);
         if (r >= B) return;
         pv_nx_req = r;
-        const uint32_t idx = min((uint32_t)lane, req_tiles(r) - 1u) / tpp;   // (lanes past the end repeat the last id)
+        const uint32_t idx = min((uint32_t)lane, page_units(req_tiles(r), req_lim(r)) - 1u) / tpp;   // (lanes past the end repeat the last id)
         pv_nx = pt_flat[req_off(r) + idx];
     };
     auto fetch_pages = [&](const Cursor& cu) {
-        if (pv_nx_req == cu.r && cu.t < 64u) {
+        if (pv_nx_req == cu.r && cu.t * ppt < 64u) {
             pv = pv_nx;
             pv_req = cu.r;
             pv_win = 0;
         } else {
             pv_req = cu.r;
-            pv_win = cu.t & ~63u;
+            pv_win = (cu.t * ppt) & ~63u;
             const uint32_t t = pv_win + (uint32_t)lane;
             pv = 0;
-            if (t < cu.tiles) pv = pt_flat[cu.off + t / tpp];
+            if (t < page_units(cu.tiles, cu.lim)) pv = pt_flat[cu.off + t / tpp];
         }
         // The ids are waited for here, inside whatever branch fetches them: left pending, the
         // compiler would wait at every later join of the control flow, and as it does not know
         // of the tile loads, that wait would be for all of them.
         asm volatile("" : "+v"(pv));
     };
-    auto pages_ready = [&](const Cursor& cu) { return pv_req == cu.r && (cu.t & ~63u) == pv_win; };
+    auto pages_ready = [&](const Cursor& cu) { return pv_req == cu.r && ((cu.t * ppt) & ~63u) == pv_win; };
     fetch_pages(ci);
     MLC_PROBE(2);
 
@@ -597,12 +616,16 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     // past the visible end are clamped onto the last visible row (in bounds, masked out later).
     const uint32_t stages_lds = sd_lds_addr(stages);
     auto issue_tile = [&](const Cursor& cu, uint32_t slot) {
-        uint32_t page_id = (uint32_t)__builtin_amdgcn_readlane((int)pv, (int)(cu.t & 63u));
-        if (a.capacity_pages && page_id >= a.capacity_pages) page_id = a.capacity_pages - 1u;
         const uint32_t tile_start = cu.t * TT;
-        const uint32_t slot0 = tile_start % a.page_size;
         const uint32_t last = cu.lim - 1u - tile_start;
-        const size_t row0 = ((size_t)page_id * a.page_size + slot0) * row_u4 + cu.kvh * CPR + c;
+        // (small pages: the page of this wave's slice, or of the last visible row where the slice lies
+        // behind it, and the tile row that is that page's slot 0)
+        uint32_t sub = 0, slot0 = 0;
+        if (ppt > 1u) sub = min((uint32_t)(hg * TW), last) >> a.page_shift;
+        else slot0 = tile_start % a.page_size;
+        uint32_t page_id = (uint32_t)__builtin_amdgcn_readlane((int)pv, (int)((cu.t * ppt + sub) & 63u));
+        if (a.capacity_pages && page_id >= a.capacity_pages) page_id = a.capacity_pages - 1u;
+        const size_t row0 = ((size_t)page_id * a.page_size + slot0 - ((size_t)sub << a.page_shift)) * row_u4 + cu.kvh * CPR + c;
         // (matrix-pipe mode: every wave loads exactly the rows it consumes, two loads of K and two
         // of V, so that no wave ever waits for another one's loads)
         constexpr int PARTS = (NW == 1 || MF) ? 2 : 1;
@@ -929,10 +952,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             if (n16 < G) {
 #pragma unroll
                 for (int b = 0; b < DB; ++b)
-                    *reinterpret_cast<sd_f4*>(&comb_o[((size_t)wave * G + n16) * D + b * 16 + 4 * g4]) = mf_o[b];
+                    *reinterpret_cast<sd_f4*>(&comb_o[((size_t)wave * GP + n16) * D + b * 16 + 4 * g4]) = mf_o[b];
                 if (g4 == 0) {
-                    comb_ml[wave * G + n16] = mf_m;
-                    comb_ml[NW * G + wave * G + n16] = lt;
+                    comb_ml[wave * GP + n16] = mf_m;
+                    comb_ml[NW * GP + wave * GP + n16] = lt;
                 }
             }
             sd_barrier();
@@ -942,7 +965,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                 float mw[NW], m = kNegBig;
 #pragma unroll
                 for (int w2 = 0; w2 < NW; ++w2) {
-                    mw[w2] = comb_ml[w2 * G + hh];
+                    mw[w2] = comb_ml[w2 * GP + hh];
                     m = max_nn(m, mw[w2]);
                 }
                 m_all[h] = m;
@@ -952,10 +975,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
 #pragma unroll
                 for (int w2 = 0; w2 < NW; ++w2) {
                     const float wgt = fast_exp2(mw[w2] - m);
-                    l += comb_ml[NW * G + w2 * G + hh] * wgt;
+                    l += comb_ml[NW * GP + w2 * GP + hh] * wgt;
 #pragma unroll
                     for (int kk = 0; kk < HPK; ++kk)
-                        o[kk] += comb_o[((size_t)w2 * G + hh) * D + c * 8 + r_l * HPK + kk] * wgt;
+                        o[kk] += comb_o[((size_t)w2 * GP + hh) * D + c * 8 + r_l * HPK + kk] * wgt;
                 }
                 l_all[h] = l;
 #pragma unroll
@@ -1003,6 +1026,8 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             }
         }
     };
+    // (a wave whose share of the heads the group does not have: nothing to publish, to wait for or to store)
+    const bool has_heads = !ANY || hg * HPW < G;
     // element (head k / HPK, dim) of output register k of this lane
     const int dim0 = c * 8 + r_l * HPK;
     // workgroup that holds unit u
@@ -1029,6 +1054,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             const float l = l_all[k / HPK];
             const float inv = l > 0.f ? 1.0f / l : 0.f;
             val[k] = o_un[k] * inv;
+            if (ANY && hg * HPW + k / HPK >= G) continue;   // (uniform: a head the group does not have)
             orow[(k / HPK) * D + dim0 + (k % HPK)] = val[k];
         }
         if constexpr (SPLIT) {
@@ -1043,6 +1069,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             const uint32_t t32 = req / 32, n32 = req % 32;
 #pragma unroll
             for (int h = 0; h < HPW; ++h) {
+                if (ANY && hg * HPW + h >= G) continue;
                 float amax = 0.f;
 #pragma unroll
                 for (int kk = 0; kk < HPK; ++kk) amax = fmaxf(amax, fabsf(val[h * HPK + kk]));
@@ -1315,12 +1342,12 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             } else {
 #ifndef MLC_NO_TAIL
                 // (the pair goes on in the next workgroup: the range ends here)
-                if (!(a.test_flags & 1u)) publish(o_un, m_all, l_all);
+                if (has_heads && !(a.test_flags & 1u)) publish(o_un, m_all, l_all);
 #endif
                 MLC_PROBE(26);
             }
 #ifndef MLC_NO_TAIL
-            if (range_done && (kept || cur)) {
+            if (range_done && (kept || cur) && has_heads) {
                 MLC_PROBE(28);
                 if (kept) merge_pair(kept_po, kept_o, kept_m, kept_l);
                 else merge_pair(cur_po, o_un, m_all, l_all);
