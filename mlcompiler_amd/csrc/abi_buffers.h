@@ -73,8 +73,7 @@ int mlc_hip_upload(void* buffer, const void* src, size_t bytes, size_t dst_offse
     if (known && dst_offset + bytes > known) return fail("upload: beyond the buffer");
     HIP_OK(hipMemcpyAsync(static_cast<char*>(buffer) + dst_offset, src, bytes,
                           hipMemcpyHostToDevice, g.stream));
-    HIP_OK(hipStreamSynchronize(g.stream));
-    return 1;
+    return wait_stream();
 }
 
 int mlc_hip_download(const void* buffer, void* dst, size_t bytes, size_t src_offset) {
@@ -87,8 +86,7 @@ int mlc_hip_download(const void* buffer, void* dst, size_t bytes, size_t src_off
     if (known && src_offset + bytes > known) return fail("download: beyond the buffer");
     HIP_OK(hipMemcpyAsync(dst, static_cast<const char*>(buffer) + src_offset, bytes,
                           hipMemcpyDeviceToHost, g.stream));
-    HIP_OK(hipStreamSynchronize(g.stream));
-    return 1;
+    return wait_stream();
 }
 
 int mlc_hip_zero(void* buffer, size_t bytes) {
@@ -114,8 +112,7 @@ int mlc_hip_flush(void) {
     if (!settle()) return 0;
     if (!g.pass_open) return 1;
     g.pass_open = false;
-    HIP_OK(hipStreamSynchronize(g.stream));
-    return check_fault();
+    return wait_stream() && check_fault();
 }
 
 int mlc_hip_has_open_pass(void) { return (g.inited && g.pass_open) ? 1 : 0; }

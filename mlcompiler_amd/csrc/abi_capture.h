@@ -19,6 +19,10 @@ int mlc_hip_capture_begin(void) {
         const uint32_t* d_meta = nullptr;
         if (!tables_upload(g.tables.last_meta.data(), g.tables.last_meta.size() / 3, &d_flat, &d_meta)) return 0;
     }
+    // ... and so do the page rows of the last KV write
+    if (!g.last_ids.empty() &&
+        !resident_page_rows(g.last_ids.data(), g.last_slots.data(), g.last_ids.size(), g.last_page_size))
+        return 0;
     g.cap = Ctx::Captured{};
     g_capture_failed = false;
     HIP_OK(hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal));
@@ -125,7 +129,7 @@ int mlc_hip_replay_update(int handle, const uint32_t* page_tables_flat, size_t n
             // the captured attention launch writes the step's K / V rows itself: they must still be
             // every request's newest visible position, on pages no two requests share
             if (!page_ids || !slots_in_page) return fail("replay: the captured pass writes K / V rows, page ids needed");
-            bool ok = g.tables.shared_pages == 0;
+            bool ok = !tables_share_pages();
             for (size_t r = 0; ok && r < batch; ++r) {
                 const uint64_t S = seq_lens[r];
                 const bool visible = !c.causal || (uint64_t)q_positions[r] + 1 >= S;
@@ -135,14 +139,14 @@ int mlc_hip_replay_update(int handle, const uint32_t* page_tables_flat, size_t n
             if (!ok) return fail("replay: the rows to write are not every request's newest position (run this step uncaptured)");
         }
     }
-    if (c.ids_dev) {
+    if (c.rows_dev) {
         if (!page_ids || !slots_in_page) return fail("replay: the captured pass writes K / V rows, page ids needed");
-        if (batch != c.ids_batch) return fail("replay: the batch size differs from the captured pass (capture again)");
+        if (batch != c.rows_batch) return fail("replay: the batch size differs from the captured pass (capture again)");
         for (size_t r = 0; r < batch; ++r)
-            if (c.P && slots_in_page[r] >= c.P) return fail("replay: slot >= page size");
-        const void* dev = resident_ids(page_ids, slots_in_page, batch, align_up(batch * 4, 16));
+            if (slots_in_page[r] >= c.rows_page_size) return fail("replay: slot >= page size");
+        const void* dev = resident_page_rows(page_ids, slots_in_page, batch, c.rows_page_size);
         if (!dev) return 0;
-        if (dev != c.ids_dev) return fail("replay: the device copy of the page ids had to move (capture again)");
+        if (dev != c.rows_dev) return fail("replay: the device copy of the page rows had to move (capture again)");
     }
     return 1;
 }

@@ -33,15 +33,16 @@ int fail(const std::string& msg) {
             return fail(std::string(#expr) + ": " + hipGetErrorString(e_));           \
     } while (0)
 
-// A host-pinned + device pair used to hand small metadata to kernels with one
-// stream-ordered copy.  `done` is recorded after the kernel that reads the
-// device copy, so waiting on it makes both halves safe to overwrite or grow.
+// A host-pinned + device pair used to hand small metadata to kernels.  What was enqueued with it
+// has run once the host has waited for the stream: `wait` is the number of such waits (Ctx::waits)
+// when the slot was last used, and a slot is written again only after another one.  (An event per
+// use said the same for one more call and one more packet on the queue each time.)
 struct MetaSlot {
     void* host = nullptr;
     void* dev = nullptr;
     size_t cap = 0;
-    hipEvent_t done = nullptr;
-    bool pending = false;
+    uint64_t wait = 0;
+    bool used = false;
 };
 
 // Scratch memory of the tile-balanced decode kernel: the split-K partials (one slot per
@@ -71,6 +72,8 @@ struct StreamTables {
     void* dev = nullptr;
     size_t cap = 0;
     bool filled = false;          // dev holds `flat` (version `uploaded`) and `meta`
+    MetaSlot stage[4];            // pinned copies that a launch reads while it fills dev (tables_stage)
+    int stage_next = 0;
     std::vector<uint32_t> flat;   // the caller's flat table as last seen
     uint64_t version = 0;         // counts the changes of `flat`
     uint64_t uploaded = ~0ull;    // version of `flat` that dev holds
@@ -78,9 +81,11 @@ struct StreamTables {
     size_t meta_off = 0;          // byte offset of the arrays in dev
     uint32_t max_page = 0;        // largest page id in flat
     // does some page id occur in two requests' tables (then a row written for one request may be
-    // read for another)?  -1: not computed for this content
+    // read for another)?  -1: not computed for this content (tables_share_pages)
     int shared_pages = -1;
-    std::vector<uint32_t> off;    // page_table_offsets the shared_pages answer was computed for
+    std::vector<uint32_t> off;    // the caller's page_table_offsets as last seen
+    std::vector<uint32_t> stamps; // by page id: the last question (stamp) in which the id was met
+    uint32_t stamp = 0;
     std::vector<uint32_t> last_meta;  // seq_lens | q_positions | offsets of the last decode call (host copy)
 };
 
@@ -129,6 +134,7 @@ struct Ctx {
     long opt_q4_ksplit = 0;  // 0 = automatic
     MetaSlot ring[8];
     int ring_next = 0;
+    uint64_t waits = 0;   // times the host has waited for everything on the library's stream (wait_stream)
     // Small host arrays that callers pass again and again with the same content (norm weights,
     // the page ids of a decode step across its layers): kept on the device, uploaded only when
     // the content changes.
@@ -163,8 +169,6 @@ struct Ctx {
         int n = 0;
         bool wide = false;                  // plain form: 16-byte units
         std::vector<uint32_t> ids, slots;   // of the scatter(s) that joined so far
-        const uint32_t* d_ids = nullptr;
-        const uint32_t* d_slots = nullptr;
         size_t batch = 0, row_elems = 0, page_size = 0;
     } kv;
     // A Q4_0 matmul of the open pass whose launch is held back for one call: when that call is
@@ -208,6 +212,8 @@ struct Ctx {
     long gemm_silu_fused = 0;        // ... with the gate/up split + SiLU * up as epilogue
     long gemm_rms_fused = 0;         // ... with the residual add, the RMSNorm's sums and the next matmul's fragments as epilogue
     long gemm_silu_split_fused = 0;  // ... of which also wrote the next matmul's activation fragments
+    std::vector<uint32_t> last_ids, last_slots;   // see place_page_rows
+    size_t last_page_size = 0;
     long kv_fused = 0;               // KV writes that went out fused with a neighbour (for tests)
     long kv_in_decode = 0;           // ... of which inside the attention launch
     long opt_fuse_rows = 1;          // 0 = every operator is launched when it is encoded
@@ -267,8 +273,8 @@ struct Ctx {
         bool carried_kv = false;             // ... and does the step's KV write
         size_t n_decode = 0;                 // tile-balanced decode launches of the pass
         uint64_t buffer_generation = 0;      // Ctx::buffer_generation when the pass was captured
-        const void* ids_dev = nullptr;       // device copy of the KV write's page ids and slots
-        size_t ids_batch = 0;
+        const void* rows_dev = nullptr;      // device copy of the KV write's page rows
+        size_t rows_batch = 0, rows_page_size = 0;
     };
     std::map<int, Captured> captures;
     // Counts the times a device buffer that the library owns (and a captured launch may have its
@@ -322,15 +328,19 @@ bool init_once() {
     return true;
 }
 
+// Waits for everything enqueued on the library's stream.
+int wait_stream() {
+    HIP_OK(hipStreamSynchronize(g.stream));
+    ++g.waits;
+    return 1;
+}
+
 int slot_reserve(MetaSlot& s, size_t bytes) {
     // (every copy of metadata to the device comes through here)
     NOT_WHILE_CAPTURING("copying metadata to the device (run the pass once uncaptured first; the planned and "
                         "generic decode kernels, one-request scatter / gather and prefill copy on every call)");
-    if (s.pending) {
-        HIP_OK(hipEventSynchronize(s.done));
-        s.pending = false;
-    }
-    if (!s.done) HIP_OK(hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+    if (s.used && s.wait == g.waits && !wait_stream()) return 0;
+    s.used = false;
     if (bytes > s.cap) {
         size_t cap = std::max<size_t>(4096, bytes * 2);
         if (s.host) HIP_OK(hipHostFree(s.host));
@@ -349,10 +359,11 @@ int slot_upload(MetaSlot& s, size_t bytes) {
     return 1;
 }
 
-int slot_mark(MetaSlot& s) {
-    HIP_OK(hipEventRecord(s.done, g.stream));
-    s.pending = true;
-    return 1;
+// (called when what reads the slot has been enqueued, or is held back and will be before the slot's
+// turn comes again)
+void slot_mark(MetaSlot& s) {
+    s.wait = g.waits;
+    s.used = true;
 }
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
@@ -365,7 +376,7 @@ const void* resident_blob(int kind, const void* key, const void* blob, size_t by
     // refers to one of the copies (their launches come later).
     if (g.resident.size() > 1024 && !g.rows.active && !g.kv.active && !g.gemm.active && !g.dec.active && !g_capturing &&
         g.captures.empty()) {   // (a captured pass keeps the addresses of the copies it read)
-        if (hipStreamSynchronize(g.stream) != hipSuccess) { fail("resident: synchronize failed"); return nullptr; }
+        if (!wait_stream()) return nullptr;
         for (auto& kv : g.resident)
             if (kv.second.dev) (void)hipFree(kv.second.dev);
         g.resident.clear();
@@ -391,7 +402,7 @@ const void* resident_blob(int kind, const void* key, const void* blob, size_t by
         fail("resident: upload failed");
         return nullptr;
     }
-    if (!slot_mark(s)) return nullptr;
+    slot_mark(s);
     r.content.assign(static_cast<const unsigned char*>(blob), static_cast<const unsigned char*>(blob) + bytes);
     return r.dev;
 }
@@ -408,13 +419,16 @@ constexpr size_t kRowMaxLen = 16384;  // row_program_kernel: 8 groups of 8 eleme
 bool row_len_ok(size_t len) { return len > 0 && len % 8 == 0 && len <= kRowMaxLen; }
 
 // The matrix-core Q4_0 kernel for nbt batch tiles of 32 and rt row tiles per workgroup; option
-// q4_int_operand picks the arithmetic (see q4_matmul_kernels.h).
-void launch_q4_mfma(int nbt, int rt, dim3 grid, const Q4Args& a) {
+// q4_int_operand picks the arithmetic (see q4_matmul_kernels.h).  With Q4RopeArgs: the split + RoPE + cast
+// of the output as epilogue.
+template <class Args>
+void launch_q4_mfma(int nbt, int rt, dim3 grid, const Args& a) {
+    constexpr bool ROPE = std::is_same_v<Args, Q4RopeArgs>;
 #define MLC_Q4(NBT, RT, WAVES)                                                                              \
     if (g.opt_q4_int_operand)                                                                               \
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, true>), grid, dim3(WAVES * 64), 0, g.stream, a); \
+        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, true, false, false, ROPE>), grid, dim3(WAVES * 64), 0, g.stream, a); \
     else                                                                                                    \
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, false>), grid, dim3(WAVES * 64), 0, g.stream, a)
+        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, false, false, false, ROPE>), grid, dim3(WAVES * 64), 0, g.stream, a)
     if (nbt == 1) {
         if (rt == 1) { MLC_Q4(1, 1, 16); } else { MLC_Q4(1, 2, 16); }
     } else {
@@ -428,9 +442,11 @@ void launch_q4_mfma(int nbt, int rt, dim3 grid, const Q4Args& a) {
 // a wave of 16 has do not hold the exponents as well), and not with two batch tiles (256 do not
 // either): q4_block_scales_fit() is what callers ask first.
 bool q4_block_scales_fit(size_t bpad, int row_tiles) { return !(bpad > 32 && row_tiles == 2); }
-void launch_q4_mfma_block_scales(int nbt, int rt, dim3 grid, const Q4Args& a) {
+template <class Args>
+void launch_q4_mfma_block_scales(int nbt, int rt, dim3 grid, const Args& a) {
+    constexpr bool ROPE = std::is_same_v<Args, Q4RopeArgs>;
 #define MLC_Q4(NBT, RT, WAVES) \
-    hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, true, true>), grid, dim3(WAVES * 64), 0, g.stream, a)
+    hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, true, true, false, ROPE>), grid, dim3(WAVES * 64), 0, g.stream, a)
     if (nbt == 1) {
         if (rt == 1) { MLC_Q4(1, 1, 16); } else { MLC_Q4(1, 2, 8); }
     } else {
@@ -458,13 +474,18 @@ int settle_gemm(const RopeArgs* rope = nullptr) {
     Ctx::GemmPending& m = g.gemm;
     if (!m.active) return 1;
     m.active = false;
-    Q4Args a = m.a;
-    if (rope) {
-        a.rope_on = 1;
-        a.rope = *rope;
-        ++g.gemm_rope_fused;
-    }
+    const Q4Args& a = m.a;
     const dim3 grid(m.grid_x, 1, m.grid_z);
+    if (rope) {
+        Q4RopeArgs ra{};
+        static_cast<Q4Args&>(ra) = a;
+        ra.rope = *rope;
+        ++g.gemm_rope_fused;
+        if (m.block_scales) launch_q4_mfma_block_scales(m.nbt, m.rt, grid, ra);
+        else launch_q4_mfma(m.nbt, m.rt, grid, ra);
+        HIP_OK(hipGetLastError());
+        return 1;
+    }
     if (m.silu) {
         m.silu = false;
         ++g.gemm_silu_fused;
@@ -504,13 +525,47 @@ int settle_decode() {
     return 1;
 }
 
+// The rows (page_id * page_size + slot) of one batched KV write on the device: what a captured pass and
+// batches too large for the kernel arguments read (the layers of a decode step all write to the same
+// rows, so only the first of them uploads).
+const uint64_t* resident_page_rows(const uint32_t* page_ids, const uint32_t* slots, size_t batch, size_t page_size) {
+    static thread_local std::vector<uint64_t> rows;
+    rows.resize(batch);
+    for (size_t r = 0; r < batch; ++r) rows[r] = (uint64_t)page_ids[r] * page_size + slots[r];
+    const void* dev = resident_blob(1, nullptr, rows.data(), batch * 8);
+    if (dev && g_capturing) {
+        g.cap.rows_dev = dev;
+        g.cap.rows_batch = batch;
+        g.cap.rows_page_size = page_size;
+    }
+    return static_cast<const uint64_t*>(dev);
+}
+
+// Sets where a KV write's launch finds its page rows: in the kernel arguments (emb, room for `most`), or on
+// the device.  What travelled in the arguments is remembered: mlc_hip_capture_begin sends it to the device,
+// so that a pass captured right after this one finds it there.
+bool place_page_rows(const uint32_t* page_ids, const uint32_t* slots, size_t batch, size_t page_size, uint64_t* emb, size_t most,
+                     const uint64_t** dev) {
+    *dev = nullptr;
+    if (batch > most || g_capturing) return (*dev = resident_page_rows(page_ids, slots, batch, page_size)) != nullptr;
+    for (size_t r = 0; r < batch; ++r) emb[r] = (uint64_t)page_ids[r] * page_size + slots[r];
+    g.last_ids.assign(page_ids, page_ids + batch);
+    g.last_slots.assign(slots, slots + batch);
+    g.last_page_size = page_size;
+    return true;
+}
+
 // Launches the pending KV write.
 int settle_kv() {
     Ctx::KvPending& kv = g.kv;
     if (!kv.active) return 1;
     kv.active = false;
     if (kv.rope) {
-        if (kv.a.k_pages || kv.a.v_pages) ++g.kv_fused;
+        if (kv.a.k_pages || kv.a.v_pages) {
+            ++g.kv_fused;
+            if (!place_page_rows(kv.ids.data(), kv.slots.data(), kv.batch, kv.page_size, kv.a.emb_rows, kRopeEmbBatch, &kv.a.page_rows))
+                return 0;
+        }
         if (kv.from_gemm) return settle_gemm(&kv.a);
         launch_qkv_split_rope_cast(kv.a, g.stream);
         HIP_OK(hipGetLastError());
@@ -521,16 +576,13 @@ int settle_kv() {
     const unsigned total = (unsigned)(kv.batch * row_units) * (unsigned)kv.n;
     const dim3 grid((total + block - 1) / block);
     if (kv.n == 2) ++g.kv_fused;
-    if (kv.wide)
-        hipLaunchKernelGGL(scatter_kv_pair_kernel<uint4>, grid, dim3(block), 0, g.stream,
-                           static_cast<const uint4*>(kv.src[0]), static_cast<uint4*>(kv.pages[0]),
-                           static_cast<const uint4*>(kv.src[1]), static_cast<uint4*>(kv.pages[1]), kv.d_ids,
-                           kv.d_slots, (uint32_t)kv.batch, row_units, (uint32_t)kv.page_size, (uint32_t)kv.n);
-    else
-        hipLaunchKernelGGL(scatter_kv_pair_kernel<uint16_t>, grid, dim3(block), 0, g.stream,
-                           static_cast<const uint16_t*>(kv.src[0]), static_cast<uint16_t*>(kv.pages[0]),
-                           static_cast<const uint16_t*>(kv.src[1]), static_cast<uint16_t*>(kv.pages[1]), kv.d_ids,
-                           kv.d_slots, (uint32_t)kv.batch, row_units, (uint32_t)kv.page_size, (uint32_t)kv.n);
+    ScatterPairArgs a{};
+    a.src[0] = kv.src[0]; a.src[1] = kv.src[1];
+    a.pages[0] = kv.pages[0]; a.pages[1] = kv.pages[1];
+    a.batch = (uint32_t)kv.batch; a.row_units = row_units; a.n_tensors = (uint32_t)kv.n;
+    if (!place_page_rows(kv.ids.data(), kv.slots.data(), kv.batch, kv.page_size, a.emb_rows, kScatterEmbBatch, &a.page_rows)) return 0;
+    if (kv.wide) hipLaunchKernelGGL(scatter_kv_pair_kernel<uint4>, grid, dim3(block), 0, g.stream, a);
+    else hipLaunchKernelGGL(scatter_kv_pair_kernel<uint16_t>, grid, dim3(block), 0, g.stream, a);
     HIP_OK(hipGetLastError());
     return 1;
 }
@@ -617,25 +669,9 @@ int finish(int sync) {
     if (sync) {
         NOT_WHILE_CAPTURING("a call with sync = 1");
         if (!settle()) return 0;
-        HIP_OK(hipStreamSynchronize(g.stream));
-        return check_fault();
+        return wait_stream() && check_fault();
     }
     return 1;
-}
-
-// Page ids and slots of one batched KV write, side by side in one resident blob: the layers of
-// a decode step all write to the same (page, slot) per request, so only the first of them uploads.
-const void* resident_ids(const uint32_t* page_ids, const uint32_t* slots, size_t batch, size_t ids_bytes) {
-    static thread_local std::vector<unsigned char> blob;
-    blob.assign(ids_bytes * 2, 0);
-    std::memcpy(blob.data(), page_ids, batch * 4);
-    std::memcpy(blob.data() + ids_bytes, slots, batch * 4);
-    const void* dev = resident_blob(1, nullptr, blob.data(), blob.size());
-    if (dev && g_capturing) {
-        g.cap.ids_dev = dev;
-        g.cap.ids_batch = batch;
-    }
-    return dev;
 }
 
 }  // namespace

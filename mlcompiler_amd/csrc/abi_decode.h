@@ -93,13 +93,14 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
         // That also needs every page to belong to one request (and to appear once in its
         // table): with a repeated page id another workgroup could read the row while it is
         // being written, and the separate launches are the ones that give the order of the calls.
-        carries_kv = use_stream && g.tables.shared_pages == 0;
+        carries_kv = use_stream;
         for (size_t r = 0; carries_kv && r < batch; ++r) {
             const uint64_t S = seq_lens[r];
             const bool visible = !apply_causal || (uint64_t)q_positions[r] + 1 >= S;
             carries_kv = S > 0 && visible && g.kv.slots[r] == (S - 1) % page_size_tokens &&
                          g.kv.ids[r] == page_tables_flat[page_table_offsets[r] + (S - 1) / page_size_tokens];
         }
+        carries_kv = carries_kv && !tables_share_pages();
         if (!carries_kv && !settle()) return 0;
     }
 
@@ -122,15 +123,19 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
         const bool embed_table = embed && 3 * emb_stride + n_flat <= kStreamEmbWords;
         const uint32_t* d_flat = nullptr;
         const uint32_t* d_meta = nullptr;
-        if (!embed_table && !tables_upload(embed ? nullptr : meta3.data(), batch, &d_flat, &d_meta)) return 0;
         const size_t dyn_lds = batch <= 64 ? 0 : stream_dynamic_lds_bytes(batch);
         const int nbuf = stream_stages(batch);
         const unsigned n_wg = stream_grid(s_hpw, s_nw, head_dim, nbuf, dyn_lds);
+        uint32_t* d_copy = nullptr;
+        if (embed && !embed_table && !tables_stage((size_t)n_wg * 64 * s_nw, &d_flat, &d_copy)) return 0;
+        if (!embed && !tables_upload(meta3.data(), batch, &d_flat, &d_meta)) return 0;
         StreamArgs a;
         stream_fill_common(a, q, k_pages, v_pages, o, batch, num_heads, kv_heads, head_dim, page_size_tokens,
                            apply_causal);
         a.pair_cost = stream_pair_cost(s_nw);
         a.pt_flat = d_flat;
+        a.pt_copy = d_copy;
+        a.pt_words = (uint32_t)n_flat;
         {
             // pools this library allocated: the kernel clamps page ids below their size (the host
             // checks above already refuse such tables; the clamp keeps a stale or overwritten
@@ -150,8 +155,6 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
         if (carries_kv) {
             a.new_k = static_cast<const uint4*>(g.kv.src[0]);
             a.new_v = static_cast<const uint4*>(g.kv.src[1]);
-            a.new_ids = g.kv.d_ids;
-            a.new_slots = g.kv.d_slots;
         }
         if (g_capturing && g.cap.n_decode > kReplayTagStep)
             return fail("capture: more decode launches in one pass than its tags can tell apart");
@@ -220,7 +223,7 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
         std::snprintf(g.last_kernel, sizeof g.last_kernel, "generic");
         ++g.last_launches;
     }
-    if (!slot_mark(slot)) return 0;
+    slot_mark(slot);
     return finish(sync);
 }
 

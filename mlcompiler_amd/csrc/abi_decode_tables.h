@@ -73,32 +73,60 @@ int check_pool_bounds(const void* pool, const uint32_t* flat, const uint32_t* of
 
 // ---------------------------------------------------------------- tile-balanced decode
 
-// Refreshes what is remembered about the caller's page tables: their content, the largest
-// page id and whether any page id occurs twice (in one table or in two requests' tables).
-// The device copy is brought up to date by tables_upload.
+// Refreshes what is remembered about the caller's page tables: their content and the largest
+// page id.  The device copy is brought up to date by tables_upload.
 void tables_refresh(const uint32_t* flat, size_t n_flat, const uint32_t* off, size_t B) {
     StreamTables& t = g.tables;
     const bool same_flat = t.flat.size() == n_flat && (n_flat == 0 || std::memcmp(t.flat.data(), flat, n_flat * 4) == 0);
-    const bool same_off = t.off.size() == B + 1 && std::memcmp(t.off.data(), off, (B + 1) * 4) == 0;
-    if (same_flat && same_off && t.shared_pages >= 0) return;
     if (!same_flat) {
         ++t.version;
         t.flat.assign(flat, flat + n_flat);
         t.max_page = 0;
         for (size_t i = 0; i < n_flat; ++i) t.max_page = std::max(t.max_page, flat[i]);
+        t.shared_pages = -1;
     }
-    t.off.assign(off, off + B + 1);
-    // duplicates among the entries the requests own ([off[r], off[r+1]), a superset of what a
-    // call dereferences): the owned ids, sorted.  (No table indexed by page id: an id may be any
-    // 32-bit number -- padding, or a corrupt entry that the bounds checks refuse afterwards.)
-    static thread_local std::vector<uint32_t> owned;
-    owned.clear();
-    for (size_t r = 0; r < B; ++r) {
-        const size_t b0 = std::min<size_t>(off[r], n_flat), e = std::min<size_t>(off[r + 1], n_flat);
-        if (e > b0) owned.insert(owned.end(), flat + b0, flat + e);
+    if (t.off.size() != B + 1 || std::memcmp(t.off.data(), off, (B + 1) * 4) != 0) {
+        t.off.assign(off, off + B + 1);
+        t.shared_pages = -1;
     }
-    std::sort(owned.begin(), owned.end());
-    t.shared_pages = std::adjacent_find(owned.begin(), owned.end()) != owned.end() ? 1 : 0;
+}
+
+// Does some page id occur twice among the entries the requests own ([off[r], off[r+1]), a superset
+// of what a call dereferences)?  Asked only by a call that would carry the step's KV write, and
+// answered once per content: one pass over a table of stamps indexed by page id (2 us for 2 100
+// pages, where sorting them took 60), or by sorting where the largest id makes that table too large
+// (an id may be any 32-bit number: padding, or a corrupt entry that the bounds checks refuse).
+bool tables_share_pages() {
+    StreamTables& t = g.tables;
+    if (t.shared_pages >= 0) return t.shared_pages != 0;
+    const size_t n_flat = t.flat.size(), B = t.off.size() - 1;
+    bool shared = false;
+    constexpr uint32_t kMostStamps = 1u << 22;
+    if (n_flat && t.max_page < kMostStamps) {
+        if (t.stamps.size() <= t.max_page) t.stamps.resize((size_t)t.max_page + 1, 0);
+        if (++t.stamp == 0) {
+            std::fill(t.stamps.begin(), t.stamps.end(), 0u);
+            t.stamp = 1;
+        }
+        for (size_t r = 0; r < B && !shared; ++r) {
+            const size_t e = std::min<size_t>(t.off[r + 1], n_flat);
+            for (size_t i = t.off[r]; i < e; ++i) {
+                uint32_t& st = t.stamps[t.flat[i]];
+                shared |= st == t.stamp;
+                st = t.stamp;
+            }
+        }
+    } else {
+        std::vector<uint32_t> owned;
+        for (size_t r = 0; r < B; ++r) {
+            const size_t b0 = std::min<size_t>(t.off[r], n_flat), e = std::min<size_t>(t.off[r + 1], n_flat);
+            if (e > b0) owned.insert(owned.end(), t.flat.begin() + b0, t.flat.begin() + e);
+        }
+        std::sort(owned.begin(), owned.end());
+        shared = std::adjacent_find(owned.begin(), owned.end()) != owned.end();
+    }
+    t.shared_pages = shared ? 1 : 0;
+    return shared;
 }
 
 // Makes the device copy of the flat table (and of the per-request arrays when `meta3` is
@@ -120,7 +148,7 @@ int tables_upload(const uint32_t* meta3, size_t B, const uint32_t** d_flat, cons
     if (upload) {
         NOT_WHILE_CAPTURING("copying the decode tables to the device (run the pass once uncaptured first)");
         if (total > t.cap) {
-            HIP_OK(hipStreamSynchronize(g.stream));
+            if (!wait_stream()) return 0;
             if (t.dev) HIP_OK(hipFree(t.dev));
             if (t.dev) ++g.buffer_generation;
             t.dev = nullptr;
@@ -145,7 +173,7 @@ int tables_upload(const uint32_t* meta3, size_t B, const uint32_t** d_flat, cons
             t.meta.clear();
             if (n_flat) HIP_OK(hipMemcpyAsync(t.dev, h, n_flat * 4, hipMemcpyHostToDevice, g.stream));
         }
-        if (!slot_mark(s)) return 0;
+        slot_mark(s);
         t.filled = true;
         t.uploaded = t.version;
         t.meta_off = flat_room;
@@ -154,6 +182,34 @@ int tables_upload(const uint32_t* meta3, size_t B, const uint32_t** d_flat, cons
     const char* dev = static_cast<const char*>(t.dev);
     *d_flat = reinterpret_cast<const uint32_t*>(dev);
     *d_meta = meta3 ? reinterpret_cast<const uint32_t*>(dev + t.meta_off) : nullptr;
+    return 1;
+}
+
+// The same for a launch whose per-request arrays travel in its arguments: a table that is already on
+// the device is read there (*d_copy null); a new one is put into pinned host memory, where the launch
+// reads the few ids each workgroup needs and from where it also fills the device copy for the launches
+// behind it (`threads` of it, one word each).  The reads across the bus cost the launch 1.4 us (28.0
+// against 26.6 us at 64 requests with 2 100 pages), where a copy in front of it cost 6 to 9 us per call.
+int tables_stage(size_t threads, const uint32_t** d_flat, uint32_t** d_copy) {
+    StreamTables& t = g.tables;
+    const size_t n_flat = t.flat.size();
+    *d_copy = nullptr;
+    const uint32_t* none = nullptr;
+    const bool current = t.uploaded == t.version && t.filled && n_flat * 4 <= t.meta_off;
+    // (no device copy to fill yet, or one that is too small: tables_upload makes it)
+    if (current || n_flat * 4 > t.meta_off || n_flat > threads) return tables_upload(nullptr, 0, d_flat, &none);
+    MetaSlot& s = t.stage[t.stage_next];
+    t.stage_next = (t.stage_next + 1) % 4;
+    if (!slot_reserve(s, n_flat * 4)) return 0;
+    std::memcpy(s.host, t.flat.data(), n_flat * 4);
+    slot_mark(s);
+    void* mapped = nullptr;
+    HIP_OK(hipHostGetDevicePointer(&mapped, s.host, 0));
+    *d_flat = static_cast<const uint32_t*>(mapped);
+    *d_copy = static_cast<uint32_t*>(t.dev);
+    t.meta.clear();
+    t.uploaded = t.version;
+    ++g.table_uploads;
     return 1;
 }
 
@@ -274,6 +330,7 @@ bool launch_stream_variant(size_t D, int hpw, int nw, int nbuf, const StreamArgs
     MLC_CASE(64, 1) MLC_CASE(64, 2) MLC_CASE(64, 4) MLC_CASE(64, 8)
     MLC_CASE(128, 1) MLC_CASE(128, 2) MLC_CASE(128, 4) MLC_CASE(128, 8)
 #undef MLC_CASE
+    if (!launched) g.tables.filled = false;   // (it may have been the launch that fills the tables' device copy)
     return launched && scratch_launched(stream);
 }
 
@@ -312,10 +369,11 @@ void stream_fill_common(StreamArgs& a, const void* q, const void* k_pages, const
     a.scale_log2e = (1.0f / std::sqrt(static_cast<float>(D))) * 1.44269504088896340736f;
     a.pair_cost = 0;  // (set by the caller once the workgroup shape is known: stream_pair_cost)
     a.new_k = a.new_v = nullptr;
-    a.new_ids = a.new_slots = nullptr;
     a.split_frag = nullptr;
     a.split_exp = nullptr;
     a.split_rows = 0;
+    a.pt_copy = nullptr;
+    a.pt_words = 0;
 }
 
 }  // namespace

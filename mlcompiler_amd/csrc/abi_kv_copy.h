@@ -44,11 +44,6 @@ int mlc_hip_scatter_kv_paged_batched_f16(void* page_storage, const uint32_t* pag
             const bool as_v = !as_k && src == kv.a.v_f16 && !kv.a.v_pages && kv.a.v_rows == row_bytes / 2;
             if ((as_k || as_v) && (reinterpret_cast<uintptr_t>(page_storage) & 3u) == 0) {
                 if (kv.ids.empty()) {
-                    const size_t ids_bytes = align_up(batch * 4, 16);
-                    const char* blob = static_cast<const char*>(resident_ids(page_ids, slots_in_page, batch, ids_bytes));
-                    if (!blob) return 0;
-                    kv.a.page_ids = reinterpret_cast<const uint32_t*>(blob);
-                    kv.a.slots = reinterpret_cast<const uint32_t*>(blob + ids_bytes);
                     kv.a.page_size = (uint32_t)page_size_tokens;
                     kv.page_size = page_size_tokens;
                     kv.ids.assign(page_ids, page_ids + batch);
@@ -67,9 +62,6 @@ int mlc_hip_scatter_kv_paged_batched_f16(void* page_storage, const uint32_t* pag
     }
     if (!settle()) return 0;
 
-    const size_t ids_bytes = align_up(batch * 4, 16);
-    const char* d_blob = static_cast<const char*>(resident_ids(page_ids, slots_in_page, batch, ids_bytes));
-    if (!d_blob) return 0;
     kv = Ctx::KvPending{};
     kv.active = true;
     kv.src[0] = src;
@@ -78,8 +70,6 @@ int mlc_hip_scatter_kv_paged_batched_f16(void* page_storage, const uint32_t* pag
     kv.wide = wide;
     kv.ids.assign(page_ids, page_ids + batch);
     kv.slots.assign(slots_in_page, slots_in_page + batch);
-    kv.d_ids = reinterpret_cast<const uint32_t*>(d_blob);
-    kv.d_slots = reinterpret_cast<const uint32_t*>(d_blob + ids_bytes);
     kv.batch = batch;
     kv.row_elems = row_bytes / 2;
     kv.page_size = page_size_tokens;
@@ -140,7 +130,7 @@ int mlc_hip_scatter_kv_paged(void* page_storage, const uint32_t* page_table, siz
                            (uint32_t)tokens, (uint32_t)head_dim, (uint32_t)page_size_tokens,
                            (uint32_t)start_slot);
     }
-    if (!slot_mark(s)) return 0;
+    slot_mark(s);
     return finish(1);
 }
 
@@ -193,7 +183,7 @@ int mlc_hip_gather_kv_pages(const void* page_storage, const uint32_t* page_table
                            static_cast<uint16_t*>(dst), d_pt, (uint32_t)n_kv_heads,
                            (uint32_t)num_tokens, (uint32_t)head_dim, (uint32_t)page_size_tokens);
     }
-    if (!slot_mark(s)) return 0;
+    slot_mark(s);
     return finish(1);
 }
 

@@ -81,7 +81,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         const Ctx::GemmPending& m = g.gemm;
         const RowProgram& p = g.rows.p;
         const size_t tiles = rows / 32, row_tiles = tiles > 256 ? 2 : 1;
-        feeds_rms = !m.silu && m.rt == 1 && m.a.rope_on == 0 && !g.kv.active && p.src == m.out && p.n_slices == 1 &&
+        feeds_rms = !m.silu && m.rt == 1 && !g.kv.active && p.src == m.out && p.n_slices == 1 &&
                     !p.src_store && !p.silu && p.addend && p.rms && !p.frag && g.rows.batch == batch &&
                     g.rows.len == cols && m.batch == batch && m.rows == cols && cols / 32 <= (batch <= 32 ? 128u : 64u) &&
                     batch * cols <= (tiles / row_tiles) * 1024;   // (every workgroup of the reader writes 1024 elements of the norm)
@@ -195,8 +195,6 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         a.out = ksplit > 1 ? slices : o;
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)nblocks;
         a.blocks_per_slice = (uint32_t)per_slice; a.ksplit = (uint32_t)ksplit;
-        a.rope_on = 0;
-        a.rope = RopeArgs{};
         // one batch tile of more than 16 requests on a grid that fills at most half of the CUs: two
         // workgroups per (row tile, K slice), each with half of the tile's requests
         const unsigned bsplit = (bpad == 32 && bn > 16 && wgs * ksplit <= (size_t)g.n_cu / 2) ? 2u : 1u;

@@ -71,7 +71,7 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
     a.scale_log2e = (1.0f / std::sqrt(static_cast<float>(head_dim))) * 1.44269504088896340736f;
     a.row_blocks = 0;  // set by the launcher
     launch_prefill(a, head_dim, (int)g.opt_prefill_stages, g.opt_prefill_rows64 != 0, g.stream);
-    if (!slot_mark(s)) return 0;
+    slot_mark(s);
     return finish(sync);
 }
 

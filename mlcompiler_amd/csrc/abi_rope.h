@@ -112,9 +112,6 @@ int mlc_hip_qkv_split_rope_scatter(const void* qkv, void* q, void* k_pages, void
         if ((known_k && end > known_k) || (known_v && end > known_v))
             return fail("qkv split: page id beyond the pool");
     }
-    const size_t ids_bytes = align_up(batch * 4, 16);
-    const char* d_blob = static_cast<const char*>(resident_ids(page_ids, slots_in_page, batch, ids_bytes));
-    if (!d_blob) return 0;
     RopeArgs a{};
     a.qkv = static_cast<const float*>(qkv);
     a.q = static_cast<float*>(q);
@@ -124,11 +121,10 @@ int mlc_hip_qkv_split_rope_scatter(const void* qkv, void* q, void* k_pages, void
     a.v_pages = static_cast<_Float16*>(v_pages);
     a.cos_table = static_cast<const float*>(cos_buf);
     a.sin_table = static_cast<const float*>(sin_buf);
-    a.page_ids = reinterpret_cast<const uint32_t*>(d_blob);
-    a.slots = reinterpret_cast<const uint32_t*>(d_blob + ids_bytes);
     a.batch = (uint32_t)batch; a.head_dim = (uint32_t)head_dim; a.qkv_rows = (uint32_t)qkv_rows;
     a.q_rows = (uint32_t)q_rows; a.k_rows = (uint32_t)k_rows; a.v_rows = (uint32_t)v_rows;
     a.rotary_dim = (uint32_t)rotary_dim; a.page_size = (uint32_t)page_size_tokens;
+    if (!place_page_rows(page_ids, slots_in_page, batch, page_size_tokens, a.emb_rows, kRopeEmbBatch, &a.page_rows)) return 0;
     if (from_gemm && g.gemm.active) {  // (still held back: the id upload above launches nothing)
         if (!settle_gemm(&a)) return 0;
     } else {

@@ -16,6 +16,7 @@
 #include <cstring>
 #include <map>
 #include <tuple>
+#include <type_traits>
 #include <string>
 #include <unordered_map>
 #include <vector>

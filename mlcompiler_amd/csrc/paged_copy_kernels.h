@@ -12,43 +12,34 @@ namespace mlc_hip {
 
 // MSL scatter_kv_paged_batched_f16 (compiler/runtime/metal_runtime.mm:405-424):
 //   page[page_ids[r]][slots[r]][kv][d] = src[r][kv][d].
-// src row r (n_kv_heads*head_dim halves) and its destination row are both
-// contiguous, so the copy runs in units of UNIT bytes (16 when everything is
-// 16-byte aligned, else 2).
-template <typename UnitT>
-__global__ void scatter_kv_paged_batched_kernel(const UnitT* __restrict__ src,
-                                                UnitT* __restrict__ page_storage,
-                                                const uint32_t* __restrict__ page_ids,
-                                                const uint32_t* __restrict__ slots,
-                                                uint32_t batch, uint32_t row_units,
-                                                uint32_t page_size) {
-    const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= batch * row_units) return;
-    const uint32_t req = gid / row_units;
-    const uint32_t u = gid - req * row_units;
-    const size_t dst_row = (size_t)page_ids[req] * page_size + slots[req];
-    page_storage[dst_row * row_units + u] = src[gid];
-}
-
+// src row r (n_kv_heads*head_dim halves) and its destination row are both contiguous, so the copy
+// runs in units of 16 bytes when everything is 16-byte aligned, else of 2.
 // The K row and the V row of a decode step in one launch: two scatter_kv_paged_batched copies
 // with the same (page id, slot) per request.  The batched step encodes them back to back
 // (compiler/runtime/batched_walker.cpp:304-307); each on its own costs a launch for 32 KiB.
+// The page row of every request travels inside the kernel arguments for up to kScatterEmbBatch
+// requests, so that a call copies nothing to the device.
+static constexpr size_t kScatterEmbBatch = 256;
+struct ScatterPairArgs {
+    const void* src[2];
+    void* pages[2];
+    const uint64_t* page_rows;  // [batch] page_id * page_size + slot on the device, or null: emb_rows
+    uint32_t batch, row_units, n_tensors;
+    uint64_t emb_rows[kScatterEmbBatch];
+};
 template <typename UnitT>
-__global__ void scatter_kv_pair_kernel(const UnitT* __restrict__ src0, UnitT* __restrict__ pages0,
-                                       const UnitT* __restrict__ src1, UnitT* __restrict__ pages1,
-                                       const uint32_t* __restrict__ page_ids,
-                                       const uint32_t* __restrict__ slots, uint32_t batch,
-                                       uint32_t row_units, uint32_t page_size, uint32_t n_tensors) {
-    // n_tensors = 1: only the first copy exists (src1 / pages1 are null and must not be touched)
+__global__ void scatter_kv_pair_kernel(const ScatterPairArgs a) {
+    // n_tensors = 1: only the first copy exists (src[1] / pages[1] are null and must not be touched)
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t per = batch * row_units;
-    if (gid >= n_tensors * per) return;
+    const uint32_t per = a.batch * a.row_units;
+    if (gid >= a.n_tensors * per) return;
     const uint32_t which = gid / per, e = gid - which * per;
-    const uint32_t req = e / row_units;
-    const uint32_t u = e - req * row_units;
-    const size_t dst_row = (size_t)page_ids[req] * page_size + slots[req];
-    if (which == 0) pages0[dst_row * row_units + u] = src0[e];
-    else pages1[dst_row * row_units + u] = src1[e];
+    const uint32_t req = e / a.row_units;
+    const uint32_t u = e - req * a.row_units;
+    const uint64_t dst_row = a.page_rows ? a.page_rows[req] : a.emb_rows[req];
+    const UnitT* src = static_cast<const UnitT*>(which ? a.src[1] : a.src[0]);
+    UnitT* pages = static_cast<UnitT*>(which ? a.pages[1] : a.pages[0]);
+    pages[dst_row * a.row_units + u] = src[e];
 }
 
 // MSL scatter_kv_paged_f16/f32 (metal_runtime.mm:468-512): src is

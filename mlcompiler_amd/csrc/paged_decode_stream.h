@@ -46,6 +46,8 @@ struct StreamArgs {
     const uint4* v_pages;
     float* o;                   // [B][H][D]
     const uint32_t* pt_flat;    // device copy of page_tables_flat; null: the table is in emb, behind the arrays
+    uint32_t* pt_copy;          // null, or where the launch leaves a copy of pt_flat (which then is pinned host
+    uint32_t pt_words;          // memory) for the launches behind it: one word per thread, pt_words in all
     const uint32_t* meta;       // device [3][meta_stride]: seq_lens, q_positions, page_table_offsets;
                                 // null: the arrays are in emb
     uint64_t* part;             // [n_wg][NW][OPL + 1][64] tagged words {value, launch tag}: one partial per
@@ -69,13 +71,11 @@ struct StreamArgs {
                                 // partials may still lie in `part`
     uint32_t spin_limit;        // rounds a merge polls for its partials before it gives up
     uint32_t test_flags;        // bit 0: partials are not published (tests of the give-up path)
-    // The step's KV write done by this launch (null: none), as in DecodeArgs: the workgroup
-    // that owns a pair's last tile writes that pair's slice of the new rows before it loads
-    // anything.
+    // The step's KV write done by this launch (null: none): every request's newest visible position
+    // gets its row of new_k / new_v ([batch][kv_heads][head_dim] fp16).  The workgroup that owns a
+    // pair's last tile writes that pair's slice of the new rows before it loads anything.
     const uint4* new_k;
     const uint4* new_v;
-    const uint32_t* new_ids;
-    const uint32_t* new_slots;
     // The split of the output for the Q4_0 matmul that reads it (null: none): whoever writes a row
     // of o also writes it as hi + lo fp16 fragments in that matmul's B-operand layout
     // (q4_matmul_kernels.h), scaled by one power of two per (request, block of 32 columns), and the
@@ -261,6 +261,14 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int lane = threadIdx.x % 64;
     const int hg = wave;  // head group of this wave
+    // The table copy for later launches: a word per thread is requested now and stored where the
+    // workgroup ends (uniform branches only; threads behind the last word repeat it).
+    uint32_t copy_word = 0;
+    auto copy_at = [&]() { return min((uint32_t)(threadIdx.x * gridDim.x + blockIdx.x), a.pt_words - 1u); };
+    if (a.pt_copy) copy_word = a.pt_flat[copy_at()];
+    auto leave_copy = [&]() {
+        if (a.pt_copy) a.pt_copy[copy_at()] = copy_word;
+    };
     uint32_t tag_add = 0;   // (needed where the range ends; requested now)
     if (a.tag_dev) tag_add = *a.tag_dev;
     const int c = lane % CPR;
@@ -390,7 +398,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     const uint32_t UT = T + PC * nz_head * Hkv;                // ... and this
     const uint32_t W = gridDim.x < UT ? gridDim.x : UT;
     const uint32_t w = blockIdx.x;
-    if (w >= W) return;
+    if (w >= W) {
+        leave_copy();
+        return;
+    }
     // UT = W * tq + trem: the first trem workgroups take tq + 1 units, the others tq
     const uint32_t tq = __builtin_amdgcn_readfirstlane(UT / W), trem = UT - tq * W;
     auto unit_start = [&](uint32_t wg) { return wg * tq + (wg < trem ? wg : trem); };
@@ -482,7 +493,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             cc.t = x;
             g0 = pair0 + x;
         } else {
-            if (u0 + (per - x) >= u1) return;  // nothing but units of a pair's end
+            if (u0 + (per - x) >= u1) {  // nothing but units of a pair's end
+                leave_copy();
+                return;
+            }
             g0 = pair0 + cc.tiles;
             cc.t = cc.tiles - 1u;
             advance(cc);
@@ -1232,7 +1246,11 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                     const uint32_t l2 = (uint32_t)lane % LPP;
                     const bool is_v = l2 >= (uint32_t)CPR;
                     const uint32_t cch = l2 % CPR;
-                    const size_t row = (size_t)a.new_ids[cw.r] * a.page_size + a.new_slots[cw.r];
+                    // (the newest position's page and slot)
+                    const uint32_t pos = cw.lim - 1u, page = pos / a.page_size;
+                    uint32_t page_id = pt_flat[cw.off + page];
+                    if (a.capacity_pages && page_id >= a.capacity_pages) page_id = a.capacity_pages - 1u;
+                    const size_t row = (size_t)page_id * a.page_size + (pos - page * a.page_size);
                     const uint4 val = (is_v ? a.new_v : a.new_k)[((size_t)cw.r * Hkv + cw.kvh) * CPR + cch];
                     uint4* dst = const_cast<uint4*>(is_v ? a.v_pages : a.k_pages);
                     dst[(row * Hkv + cw.kvh) * CPR + cch] = val;
@@ -1365,6 +1383,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         }
         slot = slot + 1u == (uint32_t)NBUF ? 0u : slot + 1u;
     }
+    leave_copy();
     MLC_PROBE(5);
 #ifdef MLC_STREAM_PROBE
     if (threadIdx.x == 0) {

@@ -15,9 +15,12 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace mlc_hip {
+
+static constexpr size_t kRopeEmbBatch = 64;   // requests whose page rows travel inside the kernel arguments
 
 struct RopeArgs {
     const float* qkv;        // [batch][qkv_rows]
@@ -30,10 +33,20 @@ struct RopeArgs {
     _Float16* v_pages;
     const float* cos_table;  // [batch][rotary_dim / 2]
     const float* sin_table;
-    const uint32_t* page_ids;  // [batch], needed when k_pages or v_pages is set
-    const uint32_t* slots;     // [batch]
+    // page_id * page_size + slot of every request's row of k_pages / v_pages: on the device, or null and
+    // inside the arguments (emb_rows)
+    const uint64_t* page_rows;
     uint32_t batch, head_dim, qkv_rows, q_rows, k_rows, v_rows, rotary_dim, page_size;
+    uint64_t emb_rows[kRopeEmbBatch];
 };
+
+// Where a kernel finds the page rows.  (As global memory, which the argument segment is: one load of
+// either, instead of a branch around two.)
+__device__ __forceinline__ const uint64_t* rope_page_rows(const RopeArgs& a, uint32_t args_offset) {
+    typedef const __attribute__((address_space(1))) char* global_char_ptr;
+    const char* args = (const char*)(global_char_ptr)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    return a.page_rows ? a.page_rows : reinterpret_cast<const uint64_t*>(args + args_offset + offsetof(RopeArgs, emb_rows));
+}
 
 // (x0, x1) -> (x0*c - x1*s, x0*s + x1*c): four products, one difference, one sum, each
 // rounded on its own -- contraction into v_fma is switched off for this function.
@@ -79,7 +92,7 @@ __global__ __launch_bounds__(256) void qkv_split_rope_cast_kernel(const RopeArgs
     if (pool) {
         // scatter_kv_paged_batched_f16 (metal_runtime.mm:418-422): a row of all KV heads is
         // contiguous at page_ids[r]*P*rows + slots[r]*rows
-        const size_t dst = ((size_t)a.page_ids[req] * a.page_size + a.slots[req]) * rows + local;
+        const size_t dst = (size_t)rope_page_rows(a, 0)[req] * rows + local;
         *reinterpret_cast<half2_t*>(pool + dst) = h;
     }
 }

@@ -30,6 +30,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "paged_decode_kernels.h"
 #include "paged_rope_kernels.h"
 
@@ -157,10 +159,6 @@ struct Q4Args {
     // grid would otherwise leave half of the CUs idle anyway (quarters of the batch on four
     // workgroups were measured as well and gain nothing more).  0 or 1: the whole tile.
     uint32_t bsplit;
-    // When rope_on is set (ksplit == 1, out is a fused qkv row of rope.qkv_rows = rows floats per
-    // request): the epilogue also does what qkv_split_rope_cast_kernel would do with that row.
-    uint32_t rope_on;
-    RopeArgs rope;
     // Kernels built with BS: the activations were split with one power-of-two scale per (request,
     // block of 32 columns) instead of one per request: x = (hi + lo) * 2^e.  blk_exp holds the
     // exponents e as [batch tile of 32][nblocks][32 bytes], request c of the tile at byte
@@ -203,6 +201,14 @@ struct Q4Args {
     const float* rms_src;
     float* rms_out;
 };
+// ... and for the kernels built with ROPE (ksplit == 1, out is a fused qkv row of rope.qkv_rows = rows
+// floats per request), whose epilogue also does what qkv_split_rope_cast_kernel would do with that row.
+// (A type of its own: the launches without it need not carry its page rows.)
+struct Q4RopeArgs : Q4Args {
+    RopeArgs rope;
+};
+static constexpr uint32_t kQ4RopeOffset = (sizeof(Q4Args) + alignof(RopeArgs) - 1) / alignof(RopeArgs) * alignof(RopeArgs);
+static_assert(sizeof(Q4RopeArgs) == kQ4RopeOffset + sizeof(RopeArgs), "where the kernel finds rope in its arguments");
 
 // Maximum / sum over the 32 lanes of a half wave, every lane gets the result.
 __device__ __forceinline__ float q4_half_wave_max(float v) {
@@ -251,11 +257,12 @@ __device__ __forceinline__ void q4_emit_block(float v, uint32_t b, uint32_t col,
 // matmul's main loop, so that the epilogue adds no memory round trip to the kernel's tail.
 struct Q4RopeFetch {
     float c, s;        // rotation of this element's pair (1, 0 where none applies)
-    uint32_t page_row; // page_ids[req] * page_size + slots[req]
+    uint64_t page_row; // page_id * page_size + slot
 };
 
-__device__ __forceinline__ Q4RopeFetch q4_rope_prefetch(const RopeArgs& p, uint32_t req, uint32_t feat) {
-    Q4RopeFetch f = {1.0f, 0.0f, 0u};
+__device__ __forceinline__ Q4RopeFetch q4_rope_prefetch(const RopeArgs& p, const uint64_t* page_rows, uint32_t req,
+                                                         uint32_t feat) {
+    Q4RopeFetch f = {1.0f, 0.0f, 0ull};
     if (req >= p.batch || feat >= p.q_rows + p.k_rows + p.v_rows) return f;
     const bool is_q = feat < p.q_rows;
     const bool is_k = !is_q && feat < p.q_rows + p.k_rows;
@@ -268,7 +275,7 @@ __device__ __forceinline__ Q4RopeFetch q4_rope_prefetch(const RopeArgs& p, uint3
             f.s = p.sin_table[ci];
         }
     }
-    if (!is_q && (is_k ? p.k_pages : p.v_pages)) f.page_row = p.page_ids[req] * p.page_size + p.slots[req];
+    if (!is_q && (is_k ? p.k_pages : p.v_pages)) f.page_row = page_rows[req];
     return f;
 }
 
@@ -332,8 +339,8 @@ __device__ __forceinline__ float q4_silu_times(float g, float u) {  // walker_ke
     return silu * u;
 }
 
-template <int NBT, int RT, int WAVES, bool IOP, bool BS = false, bool SILU = false>
-__global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const Q4Args a) {
+template <int NBT, int RT, int WAVES, bool IOP, bool BS = false, bool SILU = false, bool ROPE = false>
+__global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const std::conditional_t<ROPE, Q4RopeArgs, Q4Args> a) {
     static_assert(!BS || IOP, "per-block activation scales: integer-operand arithmetic only");
     static_assert(!SILU || (IOP && RT == 2), "SiLU epilogue: gate tile and up tile, integer-operand arithmetic");
     constexpr int PF = WAVES >= 16 ? 2 : 4;  // blocks in flight per wave
@@ -372,16 +379,16 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const Q4Ar
     const uint32_t row = threadIdx.x % ROWS, bsub = threadIdx.x / ROWS;
     // (fetched ahead only where a thread has one or two outputs: more would cost the loop registers)
     constexpr bool ROPE_AHEAD = PASSES <= 2;
-    Q4RopeFetch rope_pre[ROPE_AHEAD ? PASSES : 1];
-    if (ROPE_AHEAD && a.rope_on) {
+    [[maybe_unused]] Q4RopeFetch rope_pre[ROPE_AHEAD ? PASSES : 1];
+    if constexpr (ROPE && ROPE_AHEAD) {
 #pragma unroll
         for (uint32_t pass = 0; pass < PASSES; ++pass)
-            rope_pre[pass] = q4_rope_prefetch(a.rope, pass * COLS_PER_PASS + bsub, tile0 * 32 + row);
+            rope_pre[pass] = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4RopeOffset), pass * COLS_PER_PASS + bsub, tile0 * 32 + row);
     }
 
     // (the fused residual add: the residual and gamma of this thread's outputs, fetched ahead like the
     // RoPE operands)
-    constexpr bool ADD_AHEAD = IOP && RT == 1 && PASSES <= 2;
+    constexpr bool ADD_AHEAD = IOP && RT == 1 && PASSES <= 2 && !ROPE;
     float resid_pre[ADD_AHEAD ? PASSES : 1] = {};
     float gamma_pre = 1.0f;
     if constexpr (ADD_AHEAD) {
@@ -650,7 +657,7 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const Q4Ar
 #pragma unroll
     for (uint32_t pass = 0; pass < PASSES; ++pass) {
         const uint32_t b = pass * COLS_PER_PASS + bsub;
-        const bool fused_add = IOP && RT == 1 && a.add_resid;   // (uniform; then a half wave is one request's 32 columns)
+        const bool fused_add = IOP && RT == 1 && !ROPE && a.add_resid;   // (uniform; then a half wave is one request's 32 columns)
         if (b >= a.batch && !fused_add) continue;
         if (a.bsplit == 2 && (b % 32) / 16 != bz) continue;   // the other half's workgroup has these requests
         const bool live = b < a.batch;
@@ -665,9 +672,12 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const Q4Ar
         else val = live ? sum * a.inv_scale[b] : 0.f;
         const uint32_t col = tile0 * 32 + row;
         if (live) out[(size_t)b * a.rows + col] = val;
-        if (a.rope_on)  // (the lanes of a pair share b)
-            q4_rope_epilogue(a.rope, ROPE_AHEAD ? rope_pre[ROPE_AHEAD ? pass : 0] : q4_rope_prefetch(a.rope, b, col), b, col, val);
-        if constexpr (IOP && RT == 1) {
+        if constexpr (ROPE)  // (the lanes of a pair share b)
+            q4_rope_epilogue(a.rope,
+                             ROPE_AHEAD ? rope_pre[ROPE_AHEAD ? pass : 0]
+                                        : q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4RopeOffset), b, col),
+                             b, col, val);
+        if constexpr (IOP && RT == 1 && !ROPE) {
             if (fused_add) {
                 // residual add, this request's sum of squares over the 32 columns, and h * gamma as the
                 // next matmul's fragments (requests past the batch: zeros)
