@@ -4,6 +4,56 @@
 // A section of the one translation unit mlc_hip.hip, which includes it once, in order, after the
 // sections before it; not a header for anybody else.
 
+namespace {
+
+template <typename UnitT, bool TO_PAGES>
+void launch_kv_copy(const KvCopyArgs& a) {
+    const size_t total = (size_t)a.n_kv_heads * a.tokens * a.head_units;
+    const bool wide = total >= 256 * 8 * (size_t)g.n_cu;
+    const size_t per_wg = wide ? 1024 : 256;
+    const dim3 grid((unsigned)((total + per_wg - 1) / per_wg)), block(256);
+    if (total > 0x7FFF0000ull) hipLaunchKernelGGL((kv_copy_kernel<UnitT, TO_PAGES, 4, uint64_t>), grid, block, 0, g.stream, a);
+    else if (wide) hipLaunchKernelGGL((kv_copy_kernel<UnitT, TO_PAGES, 4, uint32_t>), grid, block, 0, g.stream, a);
+    else hipLaunchKernelGGL((kv_copy_kernel<UnitT, TO_PAGES, 1, uint32_t>), grid, block, 0, g.stream, a);
+}
+
+// The multi-token copies between contiguous rows and pages.
+template <bool TO_PAGES>
+int kv_copy(const void* src, void* dst, const uint32_t* page_table, size_t pages, size_t page_size, size_t n_kv_heads,
+            size_t head_dim, size_t tokens, size_t start_slot, size_t dtype_bytes) {
+    KvCopyArgs a;
+    a.src = src;
+    a.dst = dst;
+    a.page_table = nullptr;
+    a.n_kv_heads = (uint32_t)n_kv_heads;
+    a.tokens = (uint32_t)tokens;
+    a.page_size = (uint32_t)page_size;
+    a.start_slot = (uint32_t)start_slot;
+    if (pages <= kKvCopyEmbPages) {
+        std::memcpy(a.emb_table, page_table, pages * 4);
+    } else {
+        MetaSlot& s = g.ring[g.ring_next];
+        g.ring_next = (g.ring_next + 1) % 8;
+        if (!slot_reserve(s, pages * 4)) return 0;
+        std::memcpy(s.host, page_table, pages * 4);
+        if (!slot_upload(s, pages * 4)) return 0;
+        slot_mark(s);
+        a.page_table = static_cast<const uint32_t*>(s.dev);
+    }
+    const size_t head_bytes = head_dim * dtype_bytes;
+    if ((head_bytes % 16) == 0 && aligned16(src) && aligned16(dst)) {
+        a.head_units = (uint32_t)(head_bytes / 16);
+        launch_kv_copy<uint4, TO_PAGES>(a);
+    } else {
+        a.head_units = (uint32_t)head_dim;
+        if (dtype_bytes == 4) launch_kv_copy<uint32_t, TO_PAGES>(a);
+        else launch_kv_copy<uint16_t, TO_PAGES>(a);
+    }
+    return finish(1);
+}
+
+}  // namespace
+
 extern "C" {
 
 int mlc_hip_scatter_kv_paged_batched_f16(void* page_storage, const uint32_t* page_ids,
@@ -82,6 +132,7 @@ int mlc_hip_scatter_kv_paged(void* page_storage, const uint32_t* page_table, siz
                              size_t tokens, size_t start_slot, const void* src,
                              size_t dtype_bytes) {
     if (!init_once()) return fail("GPU unavailable");
+    NOT_WHILE_CAPTURING("one-request scatter (it waits)");
     if (!settle()) return 0;
     // metal_runtime.mm:7839-7845
     if (!page_storage || !src) return fail("scatter_paged: null buffer");
@@ -100,44 +151,14 @@ int mlc_hip_scatter_kv_paged(void* page_storage, const uint32_t* page_table, siz
     const size_t known_src = known_bytes(src);
     if (known_src && tokens * row_bytes > known_src) return fail("scatter_paged: src too small");
 
-    MetaSlot& s = g.ring[g.ring_next];
-    g.ring_next = (g.ring_next + 1) % 8;
-    if (!slot_reserve(s, needed * 4)) return 0;
-    std::memcpy(s.host, page_table, needed * 4);
-    if (!slot_upload(s, needed * 4)) return 0;
-    const uint32_t* d_pt = static_cast<const uint32_t*>(s.dev);
-    const size_t head_bytes = head_dim * dtype_bytes;
-    const unsigned block = 256;
-    if ((head_bytes % 16) == 0 && aligned16(page_storage) && aligned16(src)) {
-        const uint32_t hu = (uint32_t)(head_bytes / 16);
-        const size_t total = n_kv_heads * tokens * hu;
-        hipLaunchKernelGGL(scatter_kv_paged_kernel<uint4>, dim3((unsigned)((total + block - 1) / block)),
-                           dim3(block), 0, g.stream, static_cast<const uint4*>(src),
-                           static_cast<uint4*>(page_storage), d_pt, (uint32_t)n_kv_heads,
-                           (uint32_t)tokens, hu, (uint32_t)page_size_tokens, (uint32_t)start_slot);
-    } else if (dtype_bytes == 4) {
-        const size_t total = n_kv_heads * tokens * head_dim;
-        hipLaunchKernelGGL(scatter_kv_paged_kernel<uint32_t>, dim3((unsigned)((total + block - 1) / block)),
-                           dim3(block), 0, g.stream, static_cast<const uint32_t*>(src),
-                           static_cast<uint32_t*>(page_storage), d_pt, (uint32_t)n_kv_heads,
-                           (uint32_t)tokens, (uint32_t)head_dim, (uint32_t)page_size_tokens,
-                           (uint32_t)start_slot);
-    } else {
-        const size_t total = n_kv_heads * tokens * head_dim;
-        hipLaunchKernelGGL(scatter_kv_paged_kernel<uint16_t>, dim3((unsigned)((total + block - 1) / block)),
-                           dim3(block), 0, g.stream, static_cast<const uint16_t*>(src),
-                           static_cast<uint16_t*>(page_storage), d_pt, (uint32_t)n_kv_heads,
-                           (uint32_t)tokens, (uint32_t)head_dim, (uint32_t)page_size_tokens,
-                           (uint32_t)start_slot);
-    }
-    slot_mark(s);
-    return finish(1);
+    return kv_copy<true>(src, page_storage, page_table, needed, page_size_tokens, n_kv_heads, head_dim, tokens, start_slot, dtype_bytes);
 }
 
 int mlc_hip_gather_kv_pages(const void* page_storage, const uint32_t* page_table,
                             size_t n_page_table, size_t page_size_tokens, size_t n_kv_heads,
                             size_t head_dim, size_t num_tokens, void* dst, size_t dtype_bytes) {
     if (!init_once()) return fail("GPU unavailable");
+    NOT_WHILE_CAPTURING("gather (it waits)");
     if (!settle()) return 0;
     // metal_runtime.mm:7657-7662
     if (!page_storage || !dst) return fail("gather: null buffer");
@@ -155,36 +176,7 @@ int mlc_hip_gather_kv_pages(const void* page_storage, const uint32_t* page_table
     const size_t known_dst = known_bytes(dst);
     if (known_dst && num_tokens * row_bytes > known_dst) return fail("gather: dst too small");
 
-    MetaSlot& s = g.ring[g.ring_next];
-    g.ring_next = (g.ring_next + 1) % 8;
-    if (!slot_reserve(s, needed * 4)) return 0;
-    std::memcpy(s.host, page_table, needed * 4);
-    if (!slot_upload(s, needed * 4)) return 0;
-    const uint32_t* d_pt = static_cast<const uint32_t*>(s.dev);
-    const size_t head_bytes = head_dim * dtype_bytes;
-    const unsigned block = 256;
-    if ((head_bytes % 16) == 0 && aligned16(page_storage) && aligned16(dst)) {
-        const uint32_t hu = (uint32_t)(head_bytes / 16);
-        const size_t total = n_kv_heads * num_tokens * hu;
-        hipLaunchKernelGGL(gather_kv_pages_kernel<uint4>, dim3((unsigned)((total + block - 1) / block)),
-                           dim3(block), 0, g.stream, static_cast<const uint4*>(page_storage),
-                           static_cast<uint4*>(dst), d_pt, (uint32_t)n_kv_heads,
-                           (uint32_t)num_tokens, hu, (uint32_t)page_size_tokens);
-    } else if (dtype_bytes == 4) {
-        const size_t total = n_kv_heads * num_tokens * head_dim;
-        hipLaunchKernelGGL(gather_kv_pages_kernel<uint32_t>, dim3((unsigned)((total + block - 1) / block)),
-                           dim3(block), 0, g.stream, static_cast<const uint32_t*>(page_storage),
-                           static_cast<uint32_t*>(dst), d_pt, (uint32_t)n_kv_heads,
-                           (uint32_t)num_tokens, (uint32_t)head_dim, (uint32_t)page_size_tokens);
-    } else {
-        const size_t total = n_kv_heads * num_tokens * head_dim;
-        hipLaunchKernelGGL(gather_kv_pages_kernel<uint16_t>, dim3((unsigned)((total + block - 1) / block)),
-                           dim3(block), 0, g.stream, static_cast<const uint16_t*>(page_storage),
-                           static_cast<uint16_t*>(dst), d_pt, (uint32_t)n_kv_heads,
-                           (uint32_t)num_tokens, (uint32_t)head_dim, (uint32_t)page_size_tokens);
-    }
-    slot_mark(s);
-    return finish(1);
+    return kv_copy<false>(page_storage, dst, page_table, needed, page_size_tokens, n_kv_heads, head_dim, num_tokens, 0, dtype_bytes);
 }
 
 }  // extern "C"

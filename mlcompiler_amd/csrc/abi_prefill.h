@@ -41,28 +41,32 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
         !aligned16(k_pages) || !aligned16(v_pages) || !aligned16(o))
         return fail("prefill: unsupported shape (head_dim 64 or 128, page size a multiple of 32, heads/kv_heads in {1,2,4,8}, 16-byte aligned buffers)");
 
-    MetaSlot& s = g.ring[g.ring_next];
-    g.ring_next = (g.ring_next + 1) % 8;
-    const size_t flat_bytes = align_up(std::max<size_t>(n_flat, 1) * 4, 16);
-    const size_t vec_bytes = align_up(batch * 4, 16);
-    const size_t total = flat_bytes + 3 * vec_bytes;
-    if (!slot_reserve(s, total)) return 0;
-    char* h = static_cast<char*>(s.host);
-    if (n_flat) std::memcpy(h, page_tables_flat, n_flat * 4);
-    std::memcpy(h + flat_bytes, page_table_offsets, batch * 4);
-    std::memcpy(h + flat_bytes + vec_bytes, seq_lens, batch * 4);
-    std::memcpy(h + flat_bytes + 2 * vec_bytes, q_start, batch * 4);
-    if (!slot_upload(s, total)) return 0;
-    const char* dev = static_cast<const char*>(s.dev);
+    // The tables travel inside the kernel arguments, or, where they are too large for those, are read from
+    // pinned host memory: a workgroup takes 64 page ids at a time, which is nothing against the tiles
+    // behind them, while a copy to the device is 6 us in front of every call.
+    NOT_WHILE_CAPTURING("prefill (its tables change with every call)");
     PrefillArgs a;
+    a.tables = nullptr;
+    uint32_t* t = a.emb;
+    const size_t words = 3 * batch + n_flat;
+    if (words > kPrefillEmbWords) {
+        MetaSlot& s = g.ring[g.ring_next];
+        g.ring_next = (g.ring_next + 1) % 8;
+        if (!slot_reserve(s, words * 4)) return 0;
+        t = static_cast<uint32_t*>(s.host);
+        void* mapped = nullptr;
+        HIP_OK(hipHostGetDevicePointer(&mapped, s.host, 0));
+        a.tables = static_cast<const uint32_t*>(mapped);
+        slot_mark(s);
+    }
+    std::memcpy(t, page_table_offsets, batch * 4);
+    std::memcpy(t + batch, seq_lens, batch * 4);
+    std::memcpy(t + 2 * batch, q_start, batch * 4);
+    if (n_flat) std::memcpy(t + 3 * batch, page_tables_flat, n_flat * 4);
     a.q = static_cast<const _Float16*>(q_f16);
     a.k_pages = static_cast<const _Float16*>(k_pages);
     a.v_pages = static_cast<const _Float16*>(v_pages);
     a.o = static_cast<float*>(o);
-    a.pt_flat = reinterpret_cast<const uint32_t*>(dev);
-    a.pt_off = reinterpret_cast<const uint32_t*>(dev + flat_bytes);
-    a.seq_lens = reinterpret_cast<const uint32_t*>(dev + flat_bytes + vec_bytes);
-    a.q_start = reinterpret_cast<const uint32_t*>(dev + flat_bytes + 2 * vec_bytes);
     a.batch = (uint32_t)batch;
     a.chunk = (uint32_t)chunk;
     a.num_heads = (uint32_t)num_heads;
@@ -71,7 +75,6 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
     a.scale_log2e = (1.0f / std::sqrt(static_cast<float>(head_dim))) * 1.44269504088896340736f;
     a.row_blocks = 0;  // set by the launcher
     launch_prefill(a, head_dim, (int)g.opt_prefill_stages, g.opt_prefill_rows64 != 0, g.stream);
-    slot_mark(s);
     return finish(sync);
 }
 

@@ -42,50 +42,49 @@ __global__ void scatter_kv_pair_kernel(const ScatterPairArgs a) {
     pages[dst_row * a.row_units + u] = src[e];
 }
 
-// MSL scatter_kv_paged_f16/f32 (metal_runtime.mm:468-512): src is
-// [kv][token][dim]; token t goes to absolute slot start_slot + t of the page
-// table.  One thread per UNIT of a (kv, token) row of head_dim elements.
-template <typename UnitT>
-__global__ void scatter_kv_paged_kernel(const UnitT* __restrict__ src,
-                                        UnitT* __restrict__ page_storage,
-                                        const uint32_t* __restrict__ page_table,
-                                        uint32_t n_kv_heads, uint32_t tokens, uint32_t head_units,
-                                        uint32_t page_size, uint32_t start_slot) {
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t total = (size_t)n_kv_heads * tokens * head_units;
-    if (gid >= total) return;
-    const uint32_t u = (uint32_t)(gid % head_units);
-    const size_t tmp = gid / head_units;
-    const uint32_t token = (uint32_t)(tmp % tokens);
-    const uint32_t kv = (uint32_t)(tmp / tokens);
-    const uint32_t abs_slot = start_slot + token;
-    const uint32_t page_idx = abs_slot / page_size;
-    const uint32_t slot = abs_slot - page_idx * page_size;
-    const size_t dst = (((size_t)page_table[page_idx] * page_size + slot) * n_kv_heads + kv) *
-                           head_units + u;
-    page_storage[dst] = src[gid];
-}
+// A prompt's rows between contiguous [kv][token][dim] (MSL scatter_kv_paged_f16/f32,
+// metal_runtime.mm:468-512, and its inverse gather_kv_pages_f16/f32, :328-370) and its pages: token t
+// sits at absolute slot start_slot + t of the page table.  Units are taken in page order (token, KV
+// head, unit of the head's row), so one side is one contiguous stream and the other pieces of a head's
+// row.  The page table travels inside the kernel arguments where it fits: a call of 1 500 tokens is
+// then one launch of 3 us instead of a copy of 3 us and the launch behind it.
+static constexpr size_t kKvCopyEmbPages = 960;
+struct KvCopyArgs {
+    const void* src;
+    void* dst;
+    const uint32_t* page_table;   // on the device, or null: emb_table
+    uint32_t n_kv_heads, tokens, head_units, page_size, start_slot;
+    uint32_t emb_table[kKvCopyEmbPages];
+};
 
-// MSL gather_kv_pages_f16/f32 (metal_runtime.mm:328-370): the inverse, into
-// dst [kv][token][dim].
-template <typename UnitT>
-__global__ void gather_kv_pages_kernel(const UnitT* __restrict__ page_storage,
-                                       UnitT* __restrict__ dst,
-                                       const uint32_t* __restrict__ page_table,
-                                       uint32_t n_kv_heads, uint32_t num_tokens,
-                                       uint32_t head_units, uint32_t page_size) {
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t total = (size_t)n_kv_heads * num_tokens * head_units;
-    if (gid >= total) return;
-    const uint32_t u = (uint32_t)(gid % head_units);
-    const size_t tmp = gid / head_units;
-    const uint32_t tok = (uint32_t)(tmp % num_tokens);
-    const uint32_t kv = (uint32_t)(tmp / num_tokens);
-    const uint32_t page_idx = tok / page_size;
-    const uint32_t slot = tok - page_idx * page_size;
-    const size_t s = (((size_t)page_table[page_idx] * page_size + slot) * n_kv_heads + kv) *
-                         head_units + u;
-    dst[gid] = page_storage[s];
+// UNITS per thread, all in flight together: 1 where the copy is too small to give every CU several
+// workgroups otherwise, 4 above (16-byte units: 4 KiB per wave in flight).  Index: 32 bits wherever the
+// unit count allows it (a 64-bit division is a hundred instructions).
+template <typename UnitT, bool TO_PAGES, int UNITS, typename Index>
+__global__ __launch_bounds__(256) void kv_copy_kernel(const KvCopyArgs a) {
+    const Index row_units = (Index)a.n_kv_heads * a.head_units;
+    const Index total = row_units * a.tokens;
+    const UnitT* src = static_cast<const UnitT*>(a.src);
+    UnitT* dst = static_cast<UnitT*>(a.dst);
+    const Index first = (Index)blockIdx.x * (256 * UNITS) + threadIdx.x;
+    UnitT v[UNITS];
+    size_t to[UNITS];
+#pragma unroll
+    for (int i = 0; i < UNITS; ++i) {
+        const Index unit = first + (Index)(i * 256) < total ? first + (Index)(i * 256) : total - 1;
+        const uint32_t token = (uint32_t)(unit / row_units);
+        const uint32_t in_row = (uint32_t)(unit - token * row_units);
+        const uint32_t kv = in_row / a.head_units, u = in_row - kv * a.head_units;
+        const uint32_t abs_slot = a.start_slot + token, page = abs_slot / a.page_size, slot = abs_slot - page * a.page_size;
+        const uint32_t page_id = a.page_table ? a.page_table[page] : a.emb_table[page];
+        const size_t paged = ((size_t)page_id * a.page_size + slot) * row_units + in_row;
+        const size_t flat = ((size_t)kv * a.tokens + token) * a.head_units + u;
+        v[i] = src[TO_PAGES ? flat : paged];
+        to[i] = TO_PAGES ? paged : flat;
+    }
+#pragma unroll
+    for (int i = 0; i < UNITS; ++i)
+        if (first + (Index)(i * 256) < total) dst[to[i]] = v[i];
 }
 
 }  // namespace mlc_hip

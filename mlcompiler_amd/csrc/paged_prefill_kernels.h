@@ -29,25 +29,34 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include <type_traits>
 
 namespace mlc_hip {
 
+static constexpr size_t kPrefillEmbWords = 960;   // words of tables that travel inside the kernel arguments
+
 struct PrefillArgs {
     const _Float16* q;
     const _Float16* k_pages;
     const _Float16* v_pages;
     float* o;
-    const uint32_t* pt_flat;
-    const uint32_t* pt_off;
-    const uint32_t* seq_lens;
-    const uint32_t* q_start;
+    // page_table_offsets [batch] | seq_lens [batch] | q_start [batch] | flat page table: in pinned host
+    // memory, or null and inside the arguments (emb)
+    const uint32_t* tables;
     uint32_t batch, chunk, num_heads, kv_heads, page_size;
     uint32_t row_blocks;  // workgroups along the chunk
     float scale_log2e;
+    uint32_t emb[kPrefillEmbWords];
 };
+// (the argument segment is global memory, too: one kind of load for either place)
+__device__ __forceinline__ const uint32_t* pf_tables(const PrefillArgs& a) {
+    typedef const __attribute__((address_space(1))) char* global_char_ptr;
+    const char* args = (const char*)(global_char_ptr)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    return a.tables ? a.tables : reinterpret_cast<const uint32_t*>(args + offsetof(PrefillArgs, emb));
+}
 
 typedef _Float16 pf_half8 __attribute__((ext_vector_type(8)));
 typedef float pf_float16 __attribute__((ext_vector_type(16)));
@@ -138,9 +147,10 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
     const uint32_t head = kvh * G + (wave % G);
     const uint32_t row0 = row0_wg + (wave / G) * kPfRows;  // first chunk row of this wave
 
-    const uint32_t seq_len = a.seq_lens[req];
-    const uint32_t qs = a.q_start[req];
-    const uint32_t pt_base = a.pt_off[req];
+    const uint32_t* tables = pf_tables(a);
+    const uint32_t seq_len = __builtin_amdgcn_readfirstlane(tables[a.batch + req]);
+    const uint32_t qs = __builtin_amdgcn_readfirstlane(tables[2 * a.batch + req]);
+    const uint32_t* pt = tables + 3 * a.batch + __builtin_amdgcn_readfirstlane(tables[req]);   // this request's page ids
     // keys any row of this workgroup may see
     const uint32_t last_row = min(row0_wg + kPfRows * RB, a.chunk) - 1u;
     const uint64_t lim64 = (uint64_t)qs + last_row + 1u;
@@ -190,7 +200,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
     uint32_t page_vec = 0;
     auto fetch_pages = [&](uint32_t group) {
         const uint32_t idx = group * 64u + (uint32_t)lane;
-        page_vec = n_pages ? a.pt_flat[pt_base + (idx < n_pages ? idx : n_pages - 1u)] : 0u;
+        page_vec = n_pages ? pt[idx < n_pages ? idx : n_pages - 1u] : 0u;
         pf_wait_vmcnt<0>();  // here, so that the paths that skip the refill carry no pending load
     };
     auto issue = [&](uint32_t tile, unsigned char* st) {
@@ -497,9 +507,10 @@ __global__ __launch_bounds__(256) void paged_prefill_mfma64_kernel(const Prefill
     const uint32_t head = kvh * G + (wave % G);
     const uint32_t row0 = row0_wg + (wave / G) * (kPfRows * HALVES);  // first chunk row of this wave
 
-    const uint32_t seq_len = a.seq_lens[req];
-    const uint32_t qs = a.q_start[req];
-    const uint32_t pt_base = a.pt_off[req];
+    const uint32_t* tables = pf_tables(a);
+    const uint32_t seq_len = __builtin_amdgcn_readfirstlane(tables[a.batch + req]);
+    const uint32_t qs = __builtin_amdgcn_readfirstlane(tables[2 * a.batch + req]);
+    const uint32_t* pt = tables + 3 * a.batch + __builtin_amdgcn_readfirstlane(tables[req]);   // this request's page ids
     const uint32_t last_row = min(row0_wg + ROWS_WG, a.chunk) - 1u;
     const uint64_t lim64 = (uint64_t)qs + last_row + 1u;
     const uint32_t wg_limit = (uint32_t)(lim64 < seq_len ? lim64 : seq_len);
@@ -550,7 +561,7 @@ __global__ __launch_bounds__(256) void paged_prefill_mfma64_kernel(const Prefill
     // it wait for every load in flight, the tile loads included, wherever page_vec is read)
     auto fetch_pages = [&](uint32_t group) PF_INLINE {
         const uint32_t idx = group * 64u + (uint32_t)lane;
-        const uint32_t* src = a.pt_flat + pt_base + (idx < n_pages ? idx : (n_pages ? n_pages - 1u : 0u));
+        const uint32_t* src = pt + (idx < n_pages ? idx : (n_pages ? n_pages - 1u : 0u));
         if (n_pages)
             asm volatile("global_load_dword %0, %1, off\n\ts_waitcnt vmcnt(0)" : "=v"(page_vec) : "v"(src) : "memory");
     };
