@@ -3,6 +3,7 @@
   libmlc_hip.so       HIP kernels + the C ABI declared in include/mlc_hip.h
   libhip_executor.so  the C++ HipExecutor class (mirror of the reference's
                       MetalExecutor paged-path methods) on top of that ABI
+  _call.so            HipExecutor's inner-loop calls into the ABI as a Python module
   libmlc_bench.so     native benchmark loops that call the ABI, plus a plain copy kernel
                       used to calibrate the HBM traffic counters
 """
@@ -17,6 +18,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(CSRC, "libmlc_hip.so")
 EXECUTOR_LIB_PATH = os.path.join(CSRC, "libhip_executor.so")
+CALL_MODULE_PATH = os.path.join(PKG_DIR, "_call.so")
 BENCH_LIB_PATH = os.path.join(CSRC, "libmlc_bench.so")
 STAMP_PATH = os.path.join(CSRC, "libmlc_hip.stamp")   # hash of the sources the libraries were built from
 
@@ -49,7 +51,7 @@ def source_hash() -> str:
 
 def built_from_current_sources() -> bool:
     """True when the libraries exist and were built from the sources as they are now."""
-    if not all(os.path.exists(p) for p in (LIB_PATH, EXECUTOR_LIB_PATH, BENCH_LIB_PATH, STAMP_PATH)):
+    if not all(os.path.exists(p) for p in (LIB_PATH, EXECUTOR_LIB_PATH, BENCH_LIB_PATH, CALL_MODULE_PATH, STAMP_PATH)):
         return False
     with open(STAMP_PATH) as fh:
         return fh.read().strip() == source_hash()
@@ -66,6 +68,15 @@ def _run(cmd: list[str]) -> None:
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise RuntimeError("build failed: " + " ".join(cmd) + "\n" + proc.stdout)
+
+
+def build_call_module() -> None:
+    import sysconfig
+
+    import numpy
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I" + sysconfig.get_paths()["include"],
+          "-I" + numpy.get_include(), os.path.join(CSRC, "py_call.cpp"), "-o", CALL_MODULE_PATH,
+          "-L" + CSRC, "-lmlc_hip", "-Wl,-rpath,$ORIGIN/csrc"])
 
 
 def build_all(verbose: bool = False) -> None:
@@ -92,10 +103,11 @@ def build_all(verbose: bool = False) -> None:
           "-o", EXECUTOR_LIB_PATH, "-L" + CSRC, "-lmlc_hip", "-Wl,-rpath,$ORIGIN"])
     _run([cc, *HIPCC_FLAGS, "-shared", "-x", "hip", os.path.join(CSRC, "bench_loop.cpp"),
           "-o", BENCH_LIB_PATH, "-L" + CSRC, "-lmlc_hip", "-Wl,-rpath,$ORIGIN"])
+    build_call_module()
     with open(STAMP_PATH, "w") as fh:
         fh.write(source_hash() + "\n")
     if verbose:
-        print("built", LIB_PATH, EXECUTOR_LIB_PATH, BENCH_LIB_PATH)
+        print("built", LIB_PATH, EXECUTOR_LIB_PATH, BENCH_LIB_PATH, CALL_MODULE_PATH)
 
 
 if __name__ == "__main__":

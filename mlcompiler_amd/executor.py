@@ -4,7 +4,8 @@ order and bool-return conventions of the reference's MetalExecutor paged path
 read like tests/test_paged_flash.cpp and tests/test_paged_kv.cpp.
 
 Buffers are opaque device pointers (ints), metadata are sequences of uint32.
-Nothing here computes: every method is one call into csrc/libmlc_hip.so.
+Nothing here computes: every method is one call into csrc/libmlc_hip.so, the ones of a program's
+inner loop through the module _call (csrc/py_call.cpp), the others through ctypes.
 """
 from __future__ import annotations
 
@@ -38,6 +39,8 @@ class HipExecutor:
 
     def __init__(self):
         self._lib = load()
+        from . import _call    # (built next to the library that load() has just checked)
+        self._call = _call
 
     # -- availability / errors
     def isAvailable(self) -> bool:
@@ -77,93 +80,60 @@ class HipExecutor:
 
     # -- forward pass (metal_runtime.hpp:181-183)
     def beginForwardPassCB(self) -> bool:
-        return bool(self._lib.mlc_hip_begin())
+        return self._call.begin()
 
     def flushForwardPassCB(self) -> bool:
-        return bool(self._lib.mlc_hip_flush())
+        return self._call.flush()
 
     def hasForwardPassCB(self) -> bool:
         return bool(self._lib.mlc_hip_has_open_pass())
 
     # -- paged flash attention (metal_runtime.hpp:510-523, 645-658)
-    def _attn(self, q, k_pages, v_pages, o, page_tables_flat, page_table_offsets, seq_lens,
-              q_positions, batch, num_heads, kv_heads, head_dim, page_size_tokens, apply_causal,
-              sync) -> bool:
-        flat = _u32(page_tables_flat)
-        off = _u32(page_table_offsets)
-        sl = _u32(seq_lens)
-        qp = _u32(q_positions)
-        # the reference rejects vectors of the wrong length (metal_runtime.mm:7747-7748)
-        if off.size != batch + 1 or sl.size != batch or qp.size != batch:
-            return False
-        flat_arg = flat if flat.size else np.zeros(1, np.uint32)
-        return bool(self._lib.mlc_hip_paged_attn_decode(
-            q, k_pages, v_pages, o, _ptr(flat_arg), flat.size, _ptr(off), _ptr(sl), _ptr(qp),
-            batch, num_heads, kv_heads, head_dim, page_size_tokens, int(bool(apply_causal)), sync))
-
     def runPagedFlashAttention(self, q_buffer, k_pages_buffer, v_pages_buffer, o_buffer,
                                page_tables_flat, page_table_offsets, seq_lens, q_positions,
                                batch, num_heads, kv_heads, head_dim, page_size_tokens,
                                apply_causal) -> bool:
-        return self._attn(q_buffer, k_pages_buffer, v_pages_buffer, o_buffer, page_tables_flat,
-                          page_table_offsets, seq_lens, q_positions, batch, num_heads, kv_heads,
-                          head_dim, page_size_tokens, apply_causal, 1)
+        return self._call.attention(q_buffer, k_pages_buffer, v_pages_buffer, o_buffer, page_tables_flat,
+                                    page_table_offsets, seq_lens, q_positions, batch, num_heads, kv_heads,
+                                    head_dim, page_size_tokens, apply_causal, True)
 
     def encodePagedFlashAttention(self, q_buf, k_pages_buf, v_pages_buf, o_buf, page_tables_flat,
                                   page_table_offsets, seq_lens, q_positions, batch, num_heads,
                                   kv_heads, head_dim, page_size_tokens, apply_causal) -> bool:
-        return self._attn(q_buf, k_pages_buf, v_pages_buf, o_buf, page_tables_flat,
-                          page_table_offsets, seq_lens, q_positions, batch, num_heads, kv_heads,
-                          head_dim, page_size_tokens, apply_causal, 0)
+        return self._call.attention(q_buf, k_pages_buf, v_pages_buf, o_buf, page_tables_flat, page_table_offsets,
+                                    seq_lens, q_positions, batch, num_heads, kv_heads, head_dim, page_size_tokens,
+                                    apply_causal, False)
 
     # -- batched paged KV write (metal_runtime.hpp:526-533, 680-687)
-    def _scatter_batched(self, page_storage, page_ids, slots_in_page, page_size_tokens,
-                         n_kv_heads, head_dim, batch, src, sync) -> bool:
-        pid = _u32(page_ids)
-        sl = _u32(slots_in_page)
-        if sync and (pid.size != batch or sl.size != batch):  # metal_runtime.mm:7243
-            return False
-        if pid.size < batch or sl.size < batch:
-            return False
-        return bool(self._lib.mlc_hip_scatter_kv_paged_batched_f16(
-            page_storage, _ptr(pid), _ptr(sl), page_size_tokens, n_kv_heads, head_dim, batch, src,
-            sync))
-
     def scatterKVPagedBatched(self, page_storage_buffer, page_ids, slots_in_page,
                               page_size_tokens, n_kv_heads, head_dim, batch, src_buffer) -> bool:
-        return self._scatter_batched(page_storage_buffer, page_ids, slots_in_page,
-                                     page_size_tokens, n_kv_heads, head_dim, batch, src_buffer, 1)
+        return self._call.scatter_batched(page_storage_buffer, page_ids, slots_in_page, page_size_tokens,
+                                          n_kv_heads, head_dim, batch, src_buffer, True)
 
     def encodeScatterKVPagedBatched(self, page_storage_buffer, page_ids, slots_in_page,
                                     page_size_tokens, n_kv_heads, head_dim, batch,
                                     src_buffer) -> bool:
-        return self._scatter_batched(page_storage_buffer, page_ids, slots_in_page,
-                                     page_size_tokens, n_kv_heads, head_dim, batch, src_buffer, 0)
+        return self._call.scatter_batched(page_storage_buffer, page_ids, slots_in_page, page_size_tokens,
+                                          n_kv_heads, head_dim, batch, src_buffer, False)
 
     # -- single-request scatter / gather (metal_runtime.hpp:619-626, 666-674)
     def scatterKVPaged(self, page_storage_buffer, page_table, page_size_tokens, n_kv_heads,
                        head_dim, tokens, start_slot, src_buffer, dtype_bytes) -> bool:
-        pt = _u32(page_table)
-        pt_arg = pt if pt.size else np.zeros(1, np.uint32)
-        return bool(self._lib.mlc_hip_scatter_kv_paged(
-            page_storage_buffer, _ptr(pt_arg), pt.size, page_size_tokens, n_kv_heads, head_dim,
-            tokens, start_slot, src_buffer, dtype_bytes))
+        return self._call.scatter(page_storage_buffer, page_table, page_size_tokens, n_kv_heads, head_dim, tokens,
+                                  start_slot, src_buffer, dtype_bytes)
 
     def gatherKVPages(self, page_storage_buffer, page_table, page_size_tokens, n_kv_heads,
                       head_dim, num_tokens, dst_buffer, dtype_bytes) -> bool:
-        pt = _u32(page_table)
-        pt_arg = pt if pt.size else np.zeros(1, np.uint32)
-        return bool(self._lib.mlc_hip_gather_kv_pages(
-            page_storage_buffer, _ptr(pt_arg), pt.size, page_size_tokens, n_kv_heads, head_dim,
-            num_tokens, dst_buffer, dtype_bytes))
+        return self._call.gather(page_storage_buffer, page_table, page_size_tokens, n_kv_heads, head_dim, num_tokens,
+                                 dst_buffer, dtype_bytes)
 
     # -- the step before the KV write (metal_runtime.hpp:540-547, metal_runtime.mm:7915-8025)
     def encodeQkvSplitRopeCast(self, qkv_buf, q_buf, k_buf, v_buf, k_f16_buf, v_f16_buf, cos_buf,
                                sin_buf, batch, num_heads, kv_heads, head_dim, qkv_rows, q_rows,
                                k_rows, v_rows, rotary_dim, sync: bool = False) -> bool:
-        return bool(self._lib.mlc_hip_qkv_split_rope_cast(
+        return self._call.rope_cast(
             qkv_buf, q_buf, k_buf, v_buf, k_f16_buf, v_f16_buf, cos_buf, sin_buf, batch, num_heads,
-            kv_heads, head_dim, qkv_rows, q_rows, k_rows, v_rows, rotary_dim, int(bool(sync))))
+            kv_heads, head_dim, qkv_rows, q_rows, k_rows, v_rows, rotary_dim, sync)
 
     # the same step fused with the two batched scatters that follow it in the walker
     # (batched_walker.cpp:287-331); no single reference method
@@ -184,14 +154,10 @@ class HipExecutor:
     # -- the other per-layer operators of the batched decode step
     def encodeRmsNormBatched(self, in_buf, weight, epsilon, batch, length, out_buf,
                              sync: bool = False) -> bool:  # metal_runtime.hpp:474-479
-        w = np.ascontiguousarray(weight, np.float32)
-        return bool(self._lib.mlc_hip_rms_norm_batched(
-            in_buf, w.ctypes.data if w.size else None, w.size, float(epsilon), batch, length, out_buf,
-            int(bool(sync))))
+        return self._call.rms_norm(in_buf, weight, epsilon, batch, length, out_buf, sync)
 
     def encodeAddBatched(self, a_buf, b_buf, out_buf, total_elements, sync: bool = False) -> bool:
-        return bool(self._lib.mlc_hip_add_batched(a_buf, b_buf, out_buf, total_elements,
-                                                  int(bool(sync))))  # metal_runtime.hpp:501-502
+        return self._call.add(a_buf, b_buf, out_buf, total_elements, sync)  # metal_runtime.hpp:501-502
 
     def encodeSiluMulBatched(self, gate_buf, up_buf, out_buf, total_elements,
                              sync: bool = False) -> bool:  # metal_runtime.hpp:505-506
@@ -200,43 +166,28 @@ class HipExecutor:
 
     def encodeGateUpSplitSiluMul(self, gate_up_buf, gate_buf, up_buf, out_buf, batch, ffn_inner,
                                  ffn_gate_up_rows, sync: bool = False) -> bool:  # :549-552
-        return bool(self._lib.mlc_hip_gate_up_split_silu_mul(
-            gate_up_buf, gate_buf, up_buf, out_buf, batch, ffn_inner, ffn_gate_up_rows,
-            int(bool(sync))))
+        return self._call.gate_up(gate_up_buf, gate_buf, up_buf, out_buf, batch, ffn_inner, ffn_gate_up_rows, sync)
 
     def encodeMatMulQ4_0Batched(self, weight_name, weights, in_buf, batch, rows, cols, row_stride,
                                 quant_version, out_buf, sync: bool = False) -> bool:
         """metal_runtime.hpp:481-489; `weights` is the host byte array of the Q4_0 rows."""
-        w = np.ascontiguousarray(weights, np.uint8)
-        return bool(self._lib.mlc_hip_matmul_q4_0_batched(
-            weight_name.encode(), w.ctypes.data, w.size, in_buf, batch, rows, cols, row_stride,
-            quant_version, out_buf, int(bool(sync))))
-
-    # -- chunked prefill (no reference method; see include/mlc_hip.h)
+        return self._call.matmul_q4_0(weight_name, weights, in_buf, batch, rows, cols, row_stride, quant_version,
+                                      out_buf, sync)
 
     def encodeMatMulQ6KBatched(self, weight_name, weights, in_buf, batch, rows, cols, row_stride,
                                out_buf, sync: bool = False) -> bool:
         """metal_runtime.hpp:491-498 (sync=True: runMatMulQ6KBatched, :452-459); `weights` is the
         host byte array of the Q6_K rows."""
-        w = np.ascontiguousarray(weights, np.uint8)
-        return bool(self._lib.mlc_hip_matmul_q6_k_batched(
-            weight_name.encode(), w.ctypes.data, w.size, in_buf, batch, rows, cols, row_stride,
-            out_buf, int(bool(sync))))
+        return self._call.matmul_q6_k(weight_name, weights, in_buf, batch, rows, cols, row_stride, out_buf, sync)
+
+    # -- chunked prefill (no reference method; see include/mlc_hip.h)
     def runPagedPrefillAttention(self, q_f16_buffer, k_pages_buffer, v_pages_buffer, o_buffer,
                                  page_tables_flat, page_table_offsets, seq_lens, q_start, batch,
                                  chunk, num_heads, kv_heads, head_dim, page_size_tokens,
                                  sync: bool = True) -> bool:
-        flat = _u32(page_tables_flat)
-        off = _u32(page_table_offsets)
-        sl = _u32(seq_lens)
-        qs = _u32(q_start)
-        if off.size != batch + 1 or sl.size != batch or qs.size != batch:
-            return False
-        flat_arg = flat if flat.size else np.zeros(1, np.uint32)
-        return bool(self._lib.mlc_hip_paged_attn_prefill(
-            q_f16_buffer, k_pages_buffer, v_pages_buffer, o_buffer, _ptr(flat_arg), flat.size,
-            _ptr(off), _ptr(sl), _ptr(qs), batch, chunk, num_heads, kv_heads, head_dim,
-            page_size_tokens, int(bool(sync))))
+        return self._call.prefill(q_f16_buffer, k_pages_buffer, v_pages_buffer, o_buffer, page_tables_flat,
+                                  page_table_offsets, seq_lens, q_start, batch, chunk, num_heads, kv_heads, head_dim,
+                                  page_size_tokens, sync)
 
     # -- a pass replayed from a HIP graph
     def captureBegin(self) -> bool:
@@ -251,15 +202,11 @@ class HipExecutor:
 
     def replayUpdate(self, handle, page_tables_flat, page_table_offsets, seq_lens, q_positions,
                      page_ids=None, slots_in_page=None) -> bool:
-        flat, off, seq, pos = (_u32(x) for x in (page_tables_flat, page_table_offsets, seq_lens, q_positions))
-        ids = _u32(page_ids) if page_ids is not None else None
-        slots = _u32(slots_in_page) if slots_in_page is not None else None
-        return bool(self._lib.mlc_hip_replay_update(handle, _ptr(flat), flat.size, _ptr(off), _ptr(seq), _ptr(pos),
-                                                    _ptr(ids) if ids is not None else None,
-                                                    _ptr(slots) if slots is not None else None, seq.size))
+        return self._call.replay_update(handle, page_tables_flat, page_table_offsets, seq_lens, q_positions, page_ids,
+                                        slots_in_page)
 
     def replay(self, handle: int) -> bool:
-        return bool(self._lib.mlc_hip_replay(handle))
+        return self._call.replay(handle)
 
     def captureRelease(self, handle: int) -> None:
         self._lib.mlc_hip_capture_release(handle)
