@@ -30,6 +30,7 @@
 #include "walker_kernels.h"
 #include "q4_matmul_kernels.h"
 #include "q6k_matmul_kernels.h"
+#include "matmul_tokens_kernels.h"
 
 namespace mlc_hip {
 // Defined in paged_decode_inst.hip, one object per (head_dim, heads-per-wave).
@@ -47,6 +48,7 @@ MLC_DECL(128, 1) MLC_DECL(128, 2) MLC_DECL(128, 4) MLC_DECL(128, 8)
 #include "abi_kv_copy.h"
 #include "abi_rope.h"
 #include "abi_row_ops.h"
+#include "abi_matmul_tokens.h"
 #include "abi_matmul.h"
 #include "abi_prefill.h"
 #include "abi_capture.h"
