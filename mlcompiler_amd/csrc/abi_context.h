@@ -154,7 +154,7 @@ struct Ctx {
         size_t n_flat = 0;
         size_t len = 0;              // current row length
         const void* cur = nullptr;   // buffer that will hold the chain's current values
-        size_t grid_rows = 0;        // rows launched (padded to a multiple of 32 for the split stage)
+        size_t grid_rows = 0;        // rows launched
     } rows;
     // The KV write of a decode step that has been encoded but not launched: either the split +
     // RoPE + cast (whose fp16 K / V rows the batched scatters that follow it consume: they join

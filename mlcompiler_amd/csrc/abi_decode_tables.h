@@ -371,7 +371,6 @@ void stream_fill_common(StreamArgs& a, const void* q, const void* k_pages, const
     a.new_k = a.new_v = nullptr;
     a.split_frag = nullptr;
     a.split_exp = nullptr;
-    a.split_rows = 0;
     a.pt_copy = nullptr;
     a.pt_words = 0;
 }

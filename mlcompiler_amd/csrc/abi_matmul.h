@@ -161,7 +161,6 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         } else if (feeds_attn) {
             g.dec.a.split_frag = frag;
             g.dec.a.split_exp = blk_exp;
-            g.dec.a.split_rows = (uint32_t)bpad;
             if (!settle()) return 0;
         } else if (feeds_rms) {
             Ctx::GemmPending& m = g.gemm;
@@ -187,10 +186,10 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         } else if (feeds) {  // the chain that produces the input also splits it (batch <= 64: one round)
             g.rows.p.frag = frag;
             g.rows.p.inv_scale = inv;
-            g.rows.grid_rows = bpad;
+            g.rows.grid_rows = bn;
             if (!settle()) return 0;
         } else {
-            hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bpad), dim3(256), 0, g.stream, xin, frag,
+            hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bn), dim3(256), 0, g.stream, xin, frag,
                                inv, (uint32_t)bn, (uint32_t)cols);
         }
         // (the chain has been launched: its K-slice source may be replaced now)
@@ -367,10 +366,10 @@ int mlc_hip_matmul_q6_k_batched(const char* weight_name, const void* weights, si
         if (feeds) {
             g.rows.p.frag = frag;
             g.rows.p.inv_scale = inv;
-            g.rows.grid_rows = bpad;
+            g.rows.grid_rows = bn;
             if (!settle()) return 0;
         } else {
-            hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bpad), dim3(256), 0, g.stream, xin, frag,
+            hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bn), dim3(256), 0, g.stream, xin, frag,
                                inv, (uint32_t)bn, (uint32_t)cols);
         }
         Q6KArgs a;

@@ -79,11 +79,10 @@ struct StreamArgs {
     // The split of the output for the Q4_0 matmul that reads it (null: none): whoever writes a row
     // of o also writes it as hi + lo fp16 fragments in that matmul's B-operand layout
     // (q4_matmul_kernels.h), scaled by one power of two per (request, block of 32 columns), and the
-    // exponents where the matmul's block-scale form looks for them.  Requests batch .. split_rows-1
-    // are the padding of the last tile of 32 requests and are written as zeros.
+    // exponents where the matmul's block-scale form looks for them.  Requests
+    // without visible tokens are written as zeros.
     _Float16* split_frag;
     int8_t* split_exp;
-    uint32_t split_rows;
     // seq_lens | q_positions | page_table_offsets (at a stride of 64 words for up to 64 requests,
     // of meta_stride words above) and, where it fits as well, the flat page table behind them: a
     // call whose tables travel here copies nothing to the device
@@ -371,10 +370,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             for (uint32_t i = threadIdx.x; i < a.num_heads * D; i += 64 * NW) orow[i] = 0.f;
         }
     }
-    if constexpr (SPLIT) {  // ... and so are their fragments, and those of the padding requests
+    if constexpr (SPLIT) {  // ... and so are their fragments
         const uint32_t cols = a.num_heads * D;
-        for (uint32_t rr = blockIdx.x; rr < a.split_rows; rr += gridDim.x) {
-            if (rr < B && req_lim(rr) != 0) continue;
+        for (uint32_t rr = blockIdx.x; rr < B; rr += gridDim.x) {
+            if (req_lim(rr) != 0) continue;
             const uint32_t t32 = rr / 32, n32 = rr % 32;
             for (uint32_t k8 = threadIdx.x; k8 < cols / 8; k8 += 64 * NW) {
                 const size_t base = ((size_t)t32 * (cols / 16) + k8 / 2) * 2;

@@ -67,12 +67,13 @@ __global__ __launch_bounds__(256) void q4_0_matmul_generic_kernel(
     if (lane == 0) out[(size_t)b * rows + r] = acc;
 }
 
-// ---- activations -> B-operand fragments.  One workgroup per (padded) request row:
+// ---- activations -> B-operand fragments.  One workgroup per request row:
 // s = 2^(14 - exponent(max|x|)), then hi = fp16(x*s), lo = fp16(x*s - hi).  Element (n, k) of
 // the padded batch goes to
 //   frag[((n/32 * ksteps + k/16) * 2 + part) * 64 + ((k%16)/8)*32 + n%32][k%8],  part 0 hi, 1 lo
 // so that lane l of a wave finds the 8 halves the MFMA wants from it (column n = l%32 of the
-// batch tile, k group l/32) in 16 contiguous bytes.  Rows past `batch` are written as zeros.
+// batch tile, k group l/32) in 16 contiguous bytes.  Rows past `batch` of the last tile are neither
+// written nor read.
 __global__ __launch_bounds__(256) void q4_split_activations_kernel(
     const float* __restrict__ x, _Float16* __restrict__ frag, float* __restrict__ inv_scale,
     uint32_t batch, uint32_t cols) {
@@ -360,7 +361,15 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const std:
     const uint32_t tile_step = SILU ? a.tile_stride : 1u;   // row tile r of the workgroup: tile0 + r * tile_step
     const uint32_t slice = blockIdx.y;
     const uint32_t bz = blockIdx.z;   // (batch half, with bsplit == 2)
-    const uint32_t lane_x = (a.bsplit < 2 || (lane % 32) / 16 == bz) ? lane : (lane ^ 16u);
+    // the request whose fragments a lane fetches: its own, and in lanes past the last request (and in
+    // the other half's lanes, with bsplit) one that another lane fetches as well; their results are dropped.
+    // (The fragments of 32 requests are the largest stream of a workgroup, whatever the batch: one request
+    // of the 1 B shape, per kernel: qkv 8.3 -> 7.0 us, gate/up 12.4 -> 11.2, a whole step 1 231 -> 1 144; and
+    // nobody has to write zeros for the missing requests.)
+    uint32_t lane_x[NBT];
+#pragma unroll
+    for (int t = 0; t < NBT; ++t)
+        lane_x[t] = lane / 32 * 32 + min(a.bsplit < 2 ? l32 : bz * 16 + l32 % 16, a.batch - 1u - t * 32);
     const uint32_t b0 = slice * a.blocks_per_slice;
     const uint32_t b1 = min(b0 + a.blocks_per_slice, a.nblocks);
     const uint32_t ksteps = a.nblocks * 2;
@@ -440,7 +449,7 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const std:
 #pragma unroll
                 for (int p = 0; p < 2; ++p)
                     k.x[t][ks][p] = *reinterpret_cast<const q4_half8*>(
-                        a.xfrag + ((((size_t)t * ksteps + blk * 2 + ks) * 2 + p) * 64 + lane_x) * 8);
+                        a.xfrag + ((((size_t)t * ksteps + blk * 2 + ks) * 2 + p) * 64 + lane_x[t]) * 8);
         if constexpr (BS) {
             // register i of the accumulator is batch column (i/4)*8 + (lane/32)*4 + i%4
 #pragma unroll
@@ -588,13 +597,16 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const std:
     // ---- the waves' sums meet in LDS.  Accumulator layout: lane holds batch column l32 of the
     // tile and, in register i, weight row (i/4)*8 + (lane/32)*4 + i%4 of the 32-row tile (IOP:
     // the other way round, lane holds the weight row and the register the batch column).
+    auto put = [&](int i0, int i1) __attribute__((always_inline)) {
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
+        for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int t = 0; t < NBT; ++t)
+            for (int t = 0; t < NBT; ++t)
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                red[(((wave * RT + r) * NBT + t) * 16 + i) * PITCH + lane] = acc[r][t][i];
+                for (int i = i0; i < i1; ++i) red[(((wave * RT + r) * NBT + t) * 16 + i) * PITCH + lane] = acc[r][t][i];
+    };
+    put(0, 4);
+    if (!IOP || NBT > 1 || a.batch > 8) put(4, 16);   // (IOP: registers 0 .. 3 hold requests 0 .. 7)
     __syncthreads();
     if constexpr (BS) {
         if (a.ssq_in) {

@@ -117,7 +117,7 @@ struct RowProgram {
     float* rms_out;
     _Float16* frag;          // nullptr = no split
     float* inv_scale;
-    uint32_t batch;          // rows that exist; the grid may be padded to a multiple of 32 for split
+    uint32_t batch;          // rows that exist
 };
 
 typedef _Float16 row_half8 __attribute__((ext_vector_type(8)));
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(kRowThreads) void row_program_kernel(const RowProgr
     }
     if (!p.frag) return;
 
-    // ---- split (the whole workgroup takes part, padding rows write zeros)
+    // ---- split (the whole workgroup takes part)
     float amax = 0.f;
     if (live) {
 #pragma unroll
