@@ -39,6 +39,8 @@ namespace mlc_hip {
 static constexpr size_t kPrefillEmbWords = 960;   // words of tables that travel inside the kernel arguments
 
 struct PrefillArgs {
+    float* part_o;       // keys split over workgroups: the parts' sums [part][row][head_dim] and their
+    float2* part_ml;     // (reference, sum of weights), row = (request, chunk row, query head)
     const _Float16* q;
     const _Float16* k_pages;
     const _Float16* v_pages;
@@ -155,7 +157,11 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
     const uint32_t last_row = min(row0_wg + kPfRows * RB, a.chunk) - 1u;
     const uint64_t lim64 = (uint64_t)qs + last_row + 1u;
     const uint32_t wg_limit = (uint32_t)(lim64 < seq_len ? lim64 : seq_len);
-    const uint32_t n_tiles = (wg_limit + kPfKeys - 1) / kPfKeys;
+    const uint32_t all_tiles = (wg_limit + kPfKeys - 1) / kPfKeys;
+    // this workgroup's share of the keys (all of them, or part blockIdx.y of gridDim.y)
+    const uint32_t per_split = (all_tiles + gridDim.y - 1) / gridDim.y;
+    const uint32_t tile0 = min(blockIdx.y * per_split, all_tiles);
+    const uint32_t n_tiles = min(per_split, all_tiles - tile0);
 
     // this lane's query row and its absolute position
     const uint32_t my_row = row0 + l32;
@@ -204,7 +210,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
         pf_wait_vmcnt<0>();  // here, so that the paths that skip the refill carry no pending load
     };
     auto issue = [&](uint32_t tile, unsigned char* st) {
-        tile = tile < n_tiles ? tile : n_tiles - 1u;  // past the end: refetch, never used
+        tile = tile0 + (tile < n_tiles ? tile : n_tiles - 1u);  // past the end: refetch, never used
         const uint32_t key0 = tile * kPfKeys;
         const uint32_t page = key0 / a.page_size;
         if (page % 64u == 0 && key0 % a.page_size == 0) fetch_pages(page / 64u);
@@ -244,7 +250,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
     float m_run = -1.0e30f, l_run = 0.f;  // m_run is identical in lanes l and l^32
 
     auto compute_tile = [&](uint32_t tile, const unsigned char* kbuf, const unsigned char* vbuf) {
-        const uint32_t key0 = tile * kPfKeys;
+        const uint32_t key0 = (tile0 + tile) * kPfKeys;
         // ---- S^T = K . Q^T.  All operand reads of a phase are issued before its first MFMA,
         // and the V^T reads before the softmax, so LDS latency is paid once per phase and
         // mostly behind other work instead of once per MFMA.
@@ -326,6 +332,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
     };
 
     if (n_tiles > 0) {
+        if (tile0) fetch_pages(tile0 * kPfKeys / a.page_size / 64u);
         issue(0, st0);
         if (AHEAD > 1) issue(1, st1);
         if (AHEAD > 2) issue(2, st2);
@@ -366,8 +373,14 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
     // ---- write O: lane owns row my_row; register i of block mb is dim mb*32 + (i/4)*8 + half*4 + i%4
     if (row_ok) {
         l_run += __shfl_xor(l_run, 32);
-        const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+        float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
         float* orow = a.o + out_row;
+        if (gridDim.y > 1) {   // a part's sums, on the part's own reference, for prefill_combine_kernel
+            const size_t rows = (size_t)a.batch * a.chunk * a.num_heads, row = blockIdx.y * rows + out_row / D;
+            inv = 1.0f;
+            orow = a.part_o + row * D;
+            if (half == 0) a.part_ml[row] = make_float2(m_run, l_run);
+        }
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
@@ -378,6 +391,29 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
             }
         }
     }
+}
+
+// Adds the parts of a prefill whose keys were split over workgroups: o = sum_s 2^(m_s - m) O_s / sum_s
+// 2^(m_s - m) l_s.  One thread per four dims of a row; rows without visible keys become zero.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs a, uint32_t splits) {
+    const size_t rows = (size_t)a.batch * a.chunk * a.num_heads;
+    const size_t row = ((size_t)blockIdx.x * 256 + threadIdx.x) / (D / 4);
+    const uint32_t d = threadIdx.x % (D / 4) * 4;
+    if (row >= rows) return;
+    float m = -1.0e30f;
+    for (uint32_t s = 0; s < splits; ++s) m = fmaxf(m, a.part_ml[s * rows + row].x);
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    float l = 0.f;
+    for (uint32_t s = 0; s < splits; ++s) {
+        const float2 ml = a.part_ml[s * rows + row];
+        const float w = ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - m) : 0.f;
+        const float4 v = *reinterpret_cast<const float4*>(a.part_o + (s * rows + row) * D + d);
+        l = fmaf(w, ml.y, l);
+        o.x = fmaf(w, v.x, o.x); o.y = fmaf(w, v.y, o.y); o.z = fmaf(w, v.z, o.z); o.w = fmaf(w, v.w, o.w);
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    *reinterpret_cast<float4*>(a.o + row * D + d) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
 }
 
 // ---- the same computation with 64 chunk rows per wave (GQA ratios 1, 2 and 4).  One workgroup
@@ -933,9 +969,9 @@ inline bool prefill_shape_supported(size_t head_dim, size_t page_size, size_t nu
 }
 
 template <int D, int G>
-inline void launch_prefill_dg(PrefillArgs a, int stages, bool rows64, hipStream_t stream) {
+inline void launch_prefill_dg(PrefillArgs a, int stages, bool rows64, uint32_t splits, hipStream_t stream) {
     if constexpr (G <= 4) {
-        if (rows64) {
+        if (rows64 && splits == 1) {
             const uint32_t rows_per_wg = kPfRows * 2 * (4 / G);
             a.row_blocks = (a.chunk + rows_per_wg - 1) / rows_per_wg;
             const dim3 grid(a.row_blocks * a.kv_heads * a.batch), block(256);
@@ -950,29 +986,51 @@ inline void launch_prefill_dg(PrefillArgs a, int stages, bool rows64, hipStream_
     }
     const uint32_t rows_per_wg = kPfRows * (kPfWaves / G);
     a.row_blocks = (a.chunk + rows_per_wg - 1) / rows_per_wg;
-    const dim3 grid(a.row_blocks * a.kv_heads * a.batch), block(64 * kPfWaves);
+    const dim3 grid(a.row_blocks * a.kv_heads * a.batch, splits), block(64 * kPfWaves);
     switch (stages) {
         case 2: hipLaunchKernelGGL((paged_prefill_mfma_kernel<D, G, 2>), grid, block, 0, stream, a); break;
         case 4: hipLaunchKernelGGL((paged_prefill_mfma_kernel<D, G, 4>), grid, block, 0, stream, a); break;
         case 8: hipLaunchKernelGGL((paged_prefill_mfma_kernel<D, G, 8>), grid, block, 0, stream, a); break;
         default: hipLaunchKernelGGL((paged_prefill_mfma_kernel<D, G, 6>), grid, block, 0, stream, a); break;
     }
-}
-
-template <int D>
-inline void launch_prefill_d(const PrefillArgs& a, int stages, bool rows64, hipStream_t stream) {
-    switch (a.num_heads / a.kv_heads) {
-        case 8: launch_prefill_dg<D, 8>(a, stages, rows64, stream); break;
-        case 4: launch_prefill_dg<D, 4>(a, stages, rows64, stream); break;
-        case 2: launch_prefill_dg<D, 2>(a, stages, rows64, stream); break;
-        default: launch_prefill_dg<D, 1>(a, stages, rows64, stream); break;
+    if (splits > 1) {
+        const size_t threads = (size_t)a.batch * a.chunk * a.num_heads * (D / 4);
+        hipLaunchKernelGGL((prefill_combine_kernel<D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a, splits);
     }
 }
 
+template <int D>
+inline void launch_prefill_d(const PrefillArgs& a, int stages, bool rows64, uint32_t splits, hipStream_t stream) {
+    switch (a.num_heads / a.kv_heads) {
+        case 8: launch_prefill_dg<D, 8>(a, stages, rows64, splits, stream); break;
+        case 4: launch_prefill_dg<D, 4>(a, stages, rows64, splits, stream); break;
+        case 2: launch_prefill_dg<D, 2>(a, stages, rows64, splits, stream); break;
+        default: launch_prefill_dg<D, 1>(a, stages, rows64, splits, stream); break;
+    }
+}
+
+// A prefill of few rows leaves most of the chip idle while each workgroup walks all of the keys, about 1 us
+// per 32-key tile; its keys are then cut into parts of at least 4 tiles, as many as there are CUs for.
+// max_tiles: key tiles of the longest row block.  Whole calls, before -> after: 3 x 77 rows behind up to 900 keys
+// (36 workgroups) 40 -> 32 us, 256 rows behind 3 840 at 32 / 8 heads of 128 (32) 162 -> 57, 64 rows behind
+// 8 000 218 -> 55, 700 rows from scratch at 16 / 4 heads of 64 41 -> 32; two parts (4 x 256 rows behind up to
+// 2 000, 128 workgroups) still 87 -> 76.  Under 16 tiles the second launch (4 us) costs what the parts save.
+inline uint32_t prefill_splits(size_t batch, size_t chunk, size_t num_heads, size_t kv_heads, size_t head_dim,
+                               size_t max_tiles, size_t n_cu, size_t part_bytes) {
+    const size_t rows_per_wg = kPfRows * kPfWaves / (num_heads / kv_heads);
+    const size_t wgs = (chunk + rows_per_wg - 1) / rows_per_wg * kv_heads * batch;
+    if (max_tiles < 16) return 1;
+    const size_t one = batch * chunk * num_heads * (head_dim + 2) * 4;
+    const size_t splits = std::min({n_cu / wgs, max_tiles / 4, part_bytes / one, (size_t)64});
+    return splits < 2 ? 1u : (uint32_t)splits;
+}
+
 // stages: LDS pipeline depth (2, 4, 6 or 8; anything else selects 6).  rows64: 64 chunk rows per
-// wave (GQA ratios up to 4), else 32.
-inline void launch_prefill(const PrefillArgs& a, size_t head_dim, int stages, bool rows64, hipStream_t stream) {
-    if (head_dim == 64) launch_prefill_d<64>(a, stages, rows64, stream); else launch_prefill_d<128>(a, stages, rows64, stream);
+// wave (GQA ratios up to 4), else 32.  splits: parts into which every workgroup's keys are cut (more than
+// one: 32 rows per wave, partial sums in a.part_o / part_ml, prefill_splits() says how many).
+inline void launch_prefill(const PrefillArgs& a, size_t head_dim, int stages, bool rows64, uint32_t splits, hipStream_t stream) {
+    if (head_dim == 64) launch_prefill_d<64>(a, stages, rows64, splits, stream);
+    else launch_prefill_d<128>(a, stages, rows64, splits, stream);
 }
 
 }  // namespace mlc_hip
