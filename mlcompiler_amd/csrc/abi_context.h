@@ -418,6 +418,14 @@ constexpr size_t kRowMaxLen = 16384;  // row_program_kernel: 8 groups of 8 eleme
 
 bool row_len_ok(size_t len) { return len > 0 && len % 8 == 0 && len <= kRowMaxLen; }
 
+// One batch tile, two row tiles: a workgroup of 16 waves has a CU to itself (133 KB of LDS for its sums), so
+// where there are more of them than CUs two workgroups of 8 waves share one: the first loads of one overlap
+// the last sums of the other, and the last round is no longer a whole one.  28672 x 4096 (448 workgroups),
+// one to 32 requests: 46.5 .. 49.8 -> 40.0 .. 44.1 us a call, its kernel with SiLU 32.8 -> 29.9; at 176
+// workgroups (11264 x 2048, with block-wise scales) 16 waves are ahead (13.0 us, with 8 14.2).  Up to 128 blocks
+// of K: beyond, half as many waves would add up more blocks each in a row than 16 partial sums make up for.
+bool q4_pair_on_cu(dim3 grid, const Q4Args& a) { return grid.x > (unsigned)g.n_cu && a.nblocks <= 128; }
+
 // The matrix-core Q4_0 kernel for nbt batch tiles of 32 and rt row tiles per workgroup; option
 // q4_int_operand picks the arithmetic (see q4_matmul_kernels.h).  With Q4RopeArgs: the split + RoPE + cast
 // of the output as epilogue.
@@ -430,7 +438,7 @@ void launch_q4_mfma(int nbt, int rt, dim3 grid, const Args& a) {
     else                                                                                                    \
         hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, false, false, false, ROPE>), grid, dim3(WAVES * 64), 0, g.stream, a)
     if (nbt == 1) {
-        if (rt == 1) { MLC_Q4(1, 1, 16); } else { MLC_Q4(1, 2, 16); }
+        if (rt == 1) { MLC_Q4(1, 1, 16); } else if (!q4_pair_on_cu(grid, a)) { MLC_Q4(1, 2, 16); } else { MLC_Q4(1, 2, 8); }
     } else {
         if (rt == 1) { MLC_Q4(2, 1, 8); } else { MLC_Q4(2, 2, 8); }
     }
@@ -462,6 +470,8 @@ void launch_q4_mfma_block_scales(int nbt, int rt, dim3 grid, const Args& a) {
 void launch_q4_mfma_silu(int nbt, bool block_scales, dim3 grid, const Q4Args& a) {
     if (nbt == 1 && block_scales)
         hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<1, 2, 16, true, true, true>), grid, dim3(16 * 64), 0, g.stream, a);
+    else if (nbt == 1 && q4_pair_on_cu(grid, a))
+        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<1, 2, 8, true, false, true>), grid, dim3(8 * 64), 0, g.stream, a);
     else if (nbt == 1)
         hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<1, 2, 16, true, false, true>), grid, dim3(16 * 64), 0, g.stream, a);
     else

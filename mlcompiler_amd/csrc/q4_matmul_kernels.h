@@ -340,11 +340,15 @@ __device__ __forceinline__ float q4_silu_times(float g, float u) {  // walker_ke
     return silu * u;
 }
 
+// One batch tile, two row tiles, 8 waves: built for two workgroups per CU (128 registers, 67 KB of LDS).
+constexpr bool q4_two_per_cu(int nbt, int rt, int waves, bool bs) { return nbt == 1 && rt == 2 && waves == 8 && !bs; }
+
 template <int NBT, int RT, int WAVES, bool IOP, bool BS = false, bool SILU = false, bool ROPE = false>
-__global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const std::conditional_t<ROPE, Q4RopeArgs, Q4Args> a) {
+__global__ __launch_bounds__(WAVES * 64, q4_two_per_cu(NBT, RT, WAVES, BS) ? 4 : 1) void q4_0_matmul_mfma_kernel(const std::conditional_t<ROPE, Q4RopeArgs, Q4Args> a) {
     static_assert(!BS || IOP, "per-block activation scales: integer-operand arithmetic only");
     static_assert(!SILU || (IOP && RT == 2), "SiLU epilogue: gate tile and up tile, integer-operand arithmetic");
-    constexpr int PF = WAVES >= 16 ? 2 : 4;  // blocks in flight per wave
+    constexpr bool TIGHT = WAVES >= 16 || q4_two_per_cu(NBT, RT, WAVES, BS);   // 128 registers per wave
+    constexpr int PF = TIGHT ? 2 : 4;        // blocks in flight per wave
     constexpr int PITCH = 65;                // floats per accumulator register in LDS (bank spread)
     __shared__ float red[WAVES * RT * NBT * 16 * PITCH];
     __shared__ float rms_scale[BS ? 32 * NBT : 1];   // BS with ssq_in: every request's RMSNorm factor
@@ -415,7 +419,7 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const std:
     // from the L2) are fetched separately: the weights further ahead, PFW blocks, where the registers
     // allow it.  A wave of the TinyLlama shapes has four blocks in all, so all of its weights are on
     // the way from the start instead of in two rounds of a memory latency each.
-    constexpr int PFW = (IOP && WAVES >= 16 && (RT == 1 || (SILU && !BS))) ? 4 : PF;
+    constexpr int PFW = (IOP && TIGHT && (RT == 1 || (SILU && !BS))) ? 4 : PF;
     static_assert(PFW % PF == 0, "a block's activations sit in slot (block number) % PF");
     struct BlockW {
         uint2 q[RT];
@@ -463,7 +467,7 @@ __global__ __launch_bounds__(WAVES * 64) void q4_0_matmul_mfma_kernel(const std:
             for (int r = 0; r < RT; ++r) {
                 // (SILU: one row tile's products after the other, or the scheduler keeps three
                 // sets of 16 in flight and the loop no longer fits the 128 registers a wave has)
-                if constexpr (SILU && WAVES == 16) { if (r) __builtin_amdgcn_sched_barrier(0); }
+                if constexpr (SILU && TIGHT) { if (r) __builtin_amdgcn_sched_barrier(0); }
                 const float d = k.real ? (float)k.d[r] : 0.0f;
                 q4_half8 w[2];
 #pragma unroll
