@@ -12,15 +12,27 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (gfx950) device")
 
 
+# The programs linked with the reference's own sources (a test file or a test -> its program), and one of the
+# sources they are compiled from where the reference is checked out.
+REFERENCE_PROGRAMS = {"test_walker_end_to_end_gpu.py": "walker_end_to_end",
+                      "test_reference_paged_kv_storage_runs_on_the_hip_library": "paged_kv_roundtrip"}
+REFERENCE_SOURCE = "/root/reference/compiler/runtime/paged_kv.cpp"
+
+
+def why_skipped(file_name, test_name, root=ROOT, source=REFERENCE_SOURCE):
+    """Tests of those programs are skipped where the program is missing because there is nothing to build it from;
+    where the sources are at hand a missing program is a failed build, and its tests run and fail."""
+    program = REFERENCE_PROGRAMS.get(file_name) or REFERENCE_PROGRAMS.get(test_name)
+    if not program or os.path.exists(source) or os.path.exists(os.path.join(root, "oracle", "_ref", "integration", program)):
+        return None
+    return f"{program} is not built and there is no reference checkout to build it from"
+
+
 def pytest_collection_modifyitems(items):
-    """The tests that run programs linked with the reference's own sources are skipped where those were
-    never built (__graft_entry__.build() makes them only where the reference checkout exists)."""
-    programs = {"test_walker_end_to_end_gpu.py": "walker_end_to_end",
-                "test_reference_paged_kv_storage_runs_on_the_hip_library": "paged_kv_roundtrip"}
     for item in items:
-        name = programs.get(item.path.name) or programs.get(item.name)
-        if name and not os.path.exists(os.path.join(ROOT, "oracle", "_ref", "integration", name)):
-            item.add_marker(pytest.mark.skip(reason=f"{name} is not built (no reference checkout at build time)"))
+        reason = why_skipped(item.path.name, item.name)
+        if reason:
+            item.add_marker(pytest.mark.skip(reason=reason))
 
 
 @pytest.fixture(scope="session")
