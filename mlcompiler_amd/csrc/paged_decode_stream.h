@@ -183,14 +183,16 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
     return x;
 }
 
+static constexpr float kLowPart = 2048.0f;   // matrix-pipe mode: by how much the second part of q is larger than it counts
+
 // SMALL: at most 64 requests; lane r of every wave holds request r's figures in registers and
 // nothing goes through LDS.  Otherwise they are kept in (dynamic) LDS.
 // NBUF: tiles staged in LDS per workgroup; tile k + NBUF - 1 is requested while tile k is consumed.
 // PVM: how a tile's arithmetic is done.  0: on the vector pipe with fp32 softmax weights; 1: on the
 // vector pipe, weights rounded to fp16 for P.V (v_dot2); 2 and 3: on the matrix pipe (4 waves, at most
 // 16 query heads per KV head): every wave takes a quarter of the tile's tokens for all heads of
-// the group, S^T = K.q^T with v_mfma_f32_16x16x32_f16 (q as the sum of two fp16 numbers, so that
-// the products are as exact as with fp32 q), O^T += V^T.P^T with v_mfma_f32_16x16x16_f16 (fp16
+// the group, S^T = K.q^T with v_mfma_f32_16x16x32_f16 (q, scaled by a power of two per head, as the
+// sum of two fp16 numbers: 23 bits of it, see split_q), O^T += V^T.P^T with v_mfma_f32_16x16x16_f16 (fp16
 // weights as in mode 1; mode 3: the weight as the sum of two fp16 numbers, two MFMAs per V block,
 // fp32-grade like mode 0), V^T through the transposing LDS read; the waves' results are combined
 // through LDS where a pair of (request, KV head) ends.
@@ -557,6 +559,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     typedef _Float16 sd_half4 __attribute__((ext_vector_type(4)));
     typedef float sd_f4 __attribute__((ext_vector_type(4)));
     half8_t qh[MF ? KST : 1], ql[MF ? KST : 1];
+    float q_unscale = 1.f;   // of column n16: the score (in log2 units) per unit of the products
     uint32_t mf_k_off[MF ? KST : 1], mf_v_off[MF ? DB : 1];
     if constexpr (MF) {
         constexpr int RPB = 128 / D;   // rows per 256 bytes
@@ -591,19 +594,45 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             q_raw[2 * ks + 1] = *reinterpret_cast<const float4*>(qb + 32 * ks + 4);
         }
     };
+    // The head's row enters the products multiplied by one power of two, which brings its largest
+    // element to [2^14, 2^15) and is taken back where the scores are formed: any finite q fits, and the
+    // multiplication is exact, so the two parts belong to the same number.  (Split behind a rounded
+    // product, with the softmax scale, the compiler rounds the first part's two uses differently, and now
+    // and then a score was off by the first part's last place.)  The second part is 2^11 times larger
+    // than it counts and its products are summed apart: 23 bits of an element down to 2^-25 of the
+    // row's largest, and what is smaller to within 2^-50 of it.
+    // (A third part, which holds all 24 bits, was no closer to float64 in the output by more than a tenth
+    // and 1 to 3 % slower; scale and second sum cost 0.2 to 0.9 us a call: 23.0 -> 23.5 at 32 requests of
+    // 32 / 4 heads of 64.)
     auto split_q = [&]() {
-        const float q_factor = n16 < G ? a.scale_log2e : 0.f;
+        float amax = 0.f;
+#pragma unroll
+        for (int i = 0; i < (MF ? 2 * KST : 0); ++i)
+            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(q_raw[i].x), fabsf(q_raw[i].y)), fmaxf(fabsf(q_raw[i].z), fabsf(q_raw[i].w))));
+        const auto sw16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
+        amax = fmaxf(__uint_as_float(sw16[0]), __uint_as_float(sw16[1]));
+        const auto sw32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
+        amax = fmaxf(__uint_as_float(sw32[0]), __uint_as_float(sw32[1]));
+        const bool finite = amax < INFINITY;
+        const int se = min(15 - (finite ? __builtin_amdgcn_frexp_expf(amax) : 128), 100);   // (a row below 2^-85: its scores are zero)
+        const float up = n16 < G ? __builtin_ldexpf(1.0f, se) : 0.f, up_low = up * kLowPart;
+        q_unscale = __builtin_ldexpf(a.scale_log2e, -se);
 #pragma unroll
         for (int ks = 0; ks < (MF ? KST : 0); ++ks) {
             const float4 x0 = q_raw[2 * ks], x1 = q_raw[2 * ks + 1];
             const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float v = x[i] * q_factor;
-                const _Float16 hi = (_Float16)v;
+                const _Float16 hi = (_Float16)(x[i] * up);
                 qh[ks][i] = hi;
-                ql[ks][i] = (_Float16)(v - (float)hi);
+                ql[ks][i] = (_Float16)fmaf((float)hi, -kLowPart, x[i] * up_low);
             }
+        }
+        if (__any(!finite)) {   // an infinite element: the first part alone, or its difference with itself would be added
+#pragma unroll
+            for (int ks = 0; ks < (MF ? KST : 0); ++ks)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ql[ks][i] = finite ? ql[ks][i] : (_Float16)0.f;
         }
     };
     auto load_q = [&](const Cursor& cu) {
@@ -719,22 +748,26 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             for (int b = 0; b < DB; ++b)
                 va[b] = __builtin_bit_cast(sd_half4, __builtin_amdgcn_ds_read_tr16_b64_v4f16(
                     (sd_fp16x4 __attribute__((address_space(3)))*)(cur + mf_v_off[b])));
-            sd_f4 s4 = {0.f, 0.f, 0.f, 0.f};
+            sd_f4 s4 = {0.f, 0.f, 0.f, 0.f}, s4_low = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < KST; ++ks) {
                 s4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], s4, 0, 0, 0);
-                s4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], s4, 0, 0, 0);
+                s4_low = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], s4_low, 0, 0, 0);
             }
-            // lane (n16, g4) holds the scores of head n16 for the wave's keys 4*g4 .. 4*g4+3
+            // lane (n16, g4) holds the scores of head n16 for the wave's keys 4*g4 .. 4*g4+3, once they are
+            // scaled (rounded once, here: the largest one and its reference must cancel)
+            const float low_unscale = q_unscale * (1.0f / kLowPart);
             const uint32_t key0 = tile_start + (uint32_t)(wave * TW + 4 * g4);
             float mloc = -INFINITY;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const bool visible = (4 * g4 + i < TW) && key0 + (uint32_t)i < lim;
-                s4[i] = visible ? s4[i] : -INFINITY;
+                s4[i] = visible ? fmaf(s4_low[i], low_unscale, s4[i] * q_unscale) : -INFINITY;
                 mloc = max_nn(mloc, s4[i]);
             }
-            if (__any(mloc > mf_m + kLazyTau)) {
+            // (as a difference, which is exact where it matters: a sum would be rounded, for large scores to
+            // more than the weight's 16 bits of range allow)
+            if (__any(mloc - mf_m > kLazyTau)) {
                 float mcol = max_nn(mloc, __shfl_xor(mloc, 16));
                 mcol = max_nn(mcol, __shfl_xor(mcol, 32));
                 const float m_new = max_nn(mf_m, mcol);
@@ -1275,7 +1308,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     }
     uint32_t issued = 1;
     issue_tile(ci, 0);
-    load_q(cc);   // (behind the tile's request: q is a memory round trip of its own)
+    // (q behind the tile's request, a memory round trip of its own; matrix-pipe mode splits it as late as
+    // possible: the split waits for it, and the lane exchanges in it keep the compiler from moving it down)
+    if constexpr (MF) fetch_q(cc);
+    else load_q(cc);
     if (pv_win == 0) prefetch_next_pages(ci.r);
     if (!kv_first) {
         g1 = tiles_before(u1);
@@ -1285,6 +1321,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         write_new_rows();
         kv_unsettled = true;
     }
+    if constexpr (MF) split_q();
     uint32_t seg_first = g0;  // first tile consumed for the pair under cc
     bool drain = false;       // stores are in flight: they do not complete in order with loads
     uint32_t slot = 0;        // stage of tile k
