@@ -183,6 +183,12 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
     return x;
 }
 
+// Matrix-pipe mode: the reference lies this far (in log2) below the largest score, so that a weight that
+// is split into two fp16 numbers has their range to itself: up to 2^15 before the reference is raised, and
+// 23 bits of every weight down to 2^-9 of the largest, to within 2^-32 of the largest below.  (With the reference at
+// the maximum that was 2^-25: weights 12 powers of two below the largest were wrong by 1e-4 of themselves,
+// 20 powers below by half.)  The shift cancels where the sums are divided.
+static constexpr float kWeightShift = 7.0f;
 static constexpr float kLowPart = 2048.0f;   // matrix-pipe mode: by how much the second part of q is larger than it counts
 
 // SMALL: at most 64 requests; lane r of every wave holds request r's figures in registers and
@@ -194,7 +200,7 @@ static constexpr float kLowPart = 2048.0f;   // matrix-pipe mode: by how much th
 // the group, S^T = K.q^T with v_mfma_f32_16x16x32_f16 (q, scaled by a power of two per head, as the
 // sum of two fp16 numbers: 23 bits of it, see split_q), O^T += V^T.P^T with v_mfma_f32_16x16x16_f16 (fp16
 // weights as in mode 1; mode 3: the weight as the sum of two fp16 numbers, two MFMAs per V block,
-// fp32-grade like mode 0), V^T through the transposing LDS read; the waves' results are combined
+// fp32-grade, see kWeightShift), V^T through the transposing LDS read; the waves' results are combined
 // through LDS where a pair of (request, KV head) ends.
 // SPLIT: the launch also writes its output as the split-fp16 activations of the Q4_0 matmul that
 // reads it (StreamArgs::split_frag).
@@ -767,10 +773,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             }
             // (as a difference, which is exact where it matters: a sum would be rounded, for large scores to
             // more than the weight's 16 bits of range allow)
-            if (__any(mloc - mf_m > kLazyTau)) {
+            if (__any(mloc - mf_m > kLazyTau + kWeightShift)) {
                 float mcol = max_nn(mloc, __shfl_xor(mloc, 16));
                 mcol = max_nn(mcol, __shfl_xor(mcol, 32));
-                const float m_new = max_nn(mf_m, mcol);
+                const float m_new = max_nn(mf_m, mcol - kWeightShift);
                 const float alpha = fast_exp2(mf_m - m_new);
                 mf_m = m_new;
                 mf_l *= alpha;
@@ -782,13 +788,15 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                 // the weight enters as the sum of two fp16 numbers, like q: the products with the
                 // fp16 V are exact, only the order of the fp32 additions differs from the vector pipe
                 sd_half4 pl;
+                float w4[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float pf = fast_exp2(s4[i] - mf_m);
-                    mf_l += pf;
+                    w4[i] = pf;
                     pb[i] = (_Float16)pf;
                     pl[i] = (_Float16)(pf - (float)pb[i]);
                 }
+                mf_l += (w4[0] + w4[1]) + (w4[2] + w4[3]);
                 if constexpr (TW == 8) {
                     // A wave has 8 tokens of the tile, the product sums over 16: the upper 8 places
                     // (lanes 32 .. 63, whose own weights are masked to zero and whose V^T operand
