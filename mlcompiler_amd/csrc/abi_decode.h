@@ -77,7 +77,7 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
     // (the kernel counts in units: tiles plus at most 64 per (request, KV head) pair)
     const bool use_stream = !g.opt_force_generic && aligned && batch <= kStreamMaxBatch &&
                             total_tiles + 64ull * batch * kv_heads < 0x7FFFFFFFull &&
-                            stream_variant(G, head_dim, page_size_tokens, total_tiles, &s_hpw, &s_nw) &&
+                            stream_variant(G, head_dim, page_size_tokens, &s_hpw, &s_nw) &&
                             stream_page_ok(head_dim, page_size_tokens, s_hpw, s_nw);
     const DecodePlan* plan = nullptr;
     if (!use_stream) {
@@ -261,7 +261,7 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
     const size_t G = num_heads / kv_heads;
     const size_t tile = (head_dim == 64) ? 64 : 32;
     int hpw = 0, nw = 0;
-    if (!stream_variant(G, head_dim, page_size_tokens, 0, &hpw, &nw) || !stream_page_ok(head_dim, page_size_tokens, hpw, nw))
+    if (!stream_variant(G, head_dim, page_size_tokens, &hpw, &nw) || !stream_page_ok(head_dim, page_size_tokens, hpw, nw))
         return fail("decode (no allocation): head_dim must be 64 or 128, the GQA ratio 1 .. 16 or 32, "
                     "the page size 16, 32 or a multiple of 64 (head_dim 64), or 8, 16 or a multiple of 32 "
                     "(head_dim 128) tokens");
@@ -277,7 +277,6 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
         total_tiles += (lim + tile - 1) / tile;
     }
     total_tiles *= kv_heads;
-    (void)stream_variant(G, head_dim, page_size_tokens, total_tiles, &hpw, &nw);   // (its choice, now that the tiles are known)
     if (total_tiles + 64ull * batch * kv_heads >= 0x7FFFFFFFull) return fail("decode (no allocation): too many KV tiles");
     {
         const size_t qo_bytes = batch * num_heads * head_dim * 4;

@@ -216,16 +216,17 @@ int tables_stage(size_t threads, const uint32_t** d_flat, uint32_t** d_copy) {
 // Shape of the tile-balanced launch for (G, D): query heads per wave, waves per workgroup;
 // false when the kernel does not cover the shape.  On the matrix pipe every ratio up to 16 runs with
 // four waves, each with room for 1, 2 or 4 heads in the epilogue.  One or two query heads per KV head
-// stay on the vector pipe, in workgroups of one or two waves, where that is ahead: one head at head_dim
-// 64 (36.4 against 37.0 us at 32 requests of 8 / 8 heads), and calls of no more tiles than there are
-// workgroups (23.9 against 25.3 us per synchronous call at 512 tokens of 4 / 2 heads of 128: four waves
-// have to meet behind their one tile).  Elsewhere the matrix pipe is ahead by 10-20 % (50.9 against
-// 61.1 us at 8 requests of 32 / 32 heads of 128, 58.7 against 68.7 us at 32 of 16 / 8 heads of 64).
-bool stream_variant(size_t G, size_t D, size_t P, uint64_t total_tiles, int* hpw_out, int* nw_out) {
+// over pages of whole tiles run on the vector pipe, in workgroups of one or two waves: it multiplies the
+// fp32 numbers themselves and comes closer to float64 (2.3e-7 .. 4.4e-7 against 2.8e-7 .. 5.1e-7 of the
+// output at 6 000 to 8 000 tokens), although the matrix pipe is faster (31.2 against 28.5 us a call at 32
+// requests of 16 / 8 heads of 64, 44.8 against 44.1 at 8 of 32 / 16 of 128, 84.8 against 69.5 at 8 of
+// 32 / 32 of 128).
+// The choice depends on the shape alone: a captured pass keeps its kernel while the contexts grow, and gives
+// what the same step gives when it is encoded call by call.
+bool stream_variant(size_t G, size_t D, size_t P, int* hpw_out, int* nw_out) {
     if (D != 64 && D != 128) return false;
-    const bool whole_tiles = P % (D == 64 ? 64 : 32) == 0;
-    const bool vector_ahead = whole_tiles && G <= 2 && ((G == 1 && D == 64) || total_tiles <= 2ull * (uint64_t)g.n_cu);
-    if (g.opt_decode_mfma && g.opt_hpw_max == 0 && G >= 1 && G <= 16 && !vector_ahead) {
+    const bool vector_pipe = G <= 2 && P % (D == 64 ? 64 : 32) == 0;
+    if (g.opt_decode_mfma && g.opt_hpw_max == 0 && G >= 1 && G <= 16 && !vector_pipe) {
         *hpw_out = G <= 4 ? 1 : G <= 8 ? 2 : 4;
         *nw_out = 4;
         return true;
