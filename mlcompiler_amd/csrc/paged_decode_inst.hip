@@ -14,33 +14,26 @@ namespace mlc_hip {
 
 namespace {
 template <int NW, bool SMALL, int NBUF, bool SPLIT>
-void launch_stream_pv(int pvm, const StreamArgs& a, unsigned n_wg, size_t dyn_lds, hipStream_t stream) {
+bool launch_stream_pv(int pvm, const StreamArgs& a, unsigned n_wg, size_t dyn_lds, hipStream_t stream) {
     const dim3 grid(n_wg), block(64 * NW);
+    // groups that do not fill the workgroup's places, and pages smaller than a tile: a build of their own
+    const bool any = a.group != MLC_HPW * NW || a.pages_per_tile > 1;
+#define MLC_LAUNCH(PVM, ANY) \
+    hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, PVM, SMALL, NBUF, SPLIT, ANY>), grid, block, dyn_lds, stream, a)
     if constexpr (NW == 4 && MLC_HPW * NW <= 16) {
-        if (pvm == 2) {
-            hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, 2, SMALL, NBUF, SPLIT>), grid, block, dyn_lds, stream, a);
-            return;
-        }
-        if (pvm == 3) {
-            hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, 3, SMALL, NBUF, SPLIT>), grid, block, dyn_lds, stream, a);
-            return;
+        if (pvm == 2 || pvm == 3) {
+            if (pvm == 2 && any) MLC_LAUNCH(2, true);
+            else if (pvm == 2) MLC_LAUNCH(2, false);
+            else if (any) MLC_LAUNCH(3, true);
+            else MLC_LAUNCH(3, false);
+            return true;
         }
     }
-    if (pvm == 1 || pvm == 2)
-        hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, 1, SMALL, NBUF, SPLIT>), grid, block, dyn_lds, stream, a);
-    else
-        hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, 0, SMALL, NBUF, SPLIT>), grid, block, dyn_lds, stream, a);
-}
-// The build for partly filled groups and pages smaller than a tile: two stages and fp32-grade softmax
-// weights, whatever the options ask for.
-template <int NW, bool SMALL, bool SPLIT>
-bool launch_stream_any(const StreamArgs& a, unsigned n_wg, size_t dyn_lds, hipStream_t stream) {
-    if constexpr (NW == 4 && MLC_HPW * NW <= 16) {
-        hipLaunchKernelGGL((paged_decode_stream_kernel<MLC_D, MLC_HPW, NW, 3, SMALL, 2, SPLIT, true>), dim3(n_wg), dim3(64 * NW),
-                           dyn_lds, stream, a);
-        return true;
-    }
-    return false;
+    if (any) return false;
+    if (pvm == 1 || pvm == 2) MLC_LAUNCH(1, false);
+    else MLC_LAUNCH(0, false);
+#undef MLC_LAUNCH
+    return true;
 }
 template <int NW>
 bool launch_stream(int nbuf, int pvm, const StreamArgs& a, unsigned n_wg, size_t dyn_lds, hipStream_t stream) {
@@ -48,26 +41,17 @@ bool launch_stream(int nbuf, int pvm, const StreamArgs& a, unsigned n_wg, size_t
     // batches keep them in dynamic LDS, next to two or three stages
     // (the form that also splits its output for the matmul behind it: built for the default of
     // small batches only, two stages)
-    const bool any = a.group != MLC_HPW * NW || a.pages_per_tile > 1;
-    if (any) {
-        if (a.split_frag) return a.batch <= 64 && launch_stream_any<NW, true, true>(a, n_wg, 0, stream);
-        if (a.batch <= 64) return launch_stream_any<NW, true, false>(a, n_wg, 0, stream);
-        return launch_stream_any<NW, false, false>(a, n_wg, dyn_lds, stream);
-    }
     if (a.split_frag) {
         if (a.batch > 64 || nbuf != 2) return false;
-        launch_stream_pv<NW, true, 2, true>(pvm, a, n_wg, 0, stream);
-        return true;
+        return launch_stream_pv<NW, true, 2, true>(pvm, a, n_wg, 0, stream);
     }
     if (a.batch <= 64) {
-        if (nbuf == 2) launch_stream_pv<NW, true, 2, false>(pvm, a, n_wg, 0, stream);
-        else if (nbuf == 3) launch_stream_pv<NW, true, 3, false>(pvm, a, n_wg, 0, stream);
-        else launch_stream_pv<NW, true, 4, false>(pvm, a, n_wg, 0, stream);
-    } else {
-        if (nbuf == 2) launch_stream_pv<NW, false, 2, false>(pvm, a, n_wg, dyn_lds, stream);
-        else launch_stream_pv<NW, false, 3, false>(pvm, a, n_wg, dyn_lds, stream);
+        if (nbuf == 2) return launch_stream_pv<NW, true, 2, false>(pvm, a, n_wg, 0, stream);
+        if (nbuf == 3) return launch_stream_pv<NW, true, 3, false>(pvm, a, n_wg, 0, stream);
+        return launch_stream_pv<NW, true, 4, false>(pvm, a, n_wg, 0, stream);
     }
-    return true;
+    if (nbuf == 2) return launch_stream_pv<NW, false, 2, false>(pvm, a, n_wg, dyn_lds, stream);
+    return launch_stream_pv<NW, false, 3, false>(pvm, a, n_wg, dyn_lds, stream);
 }
 }  // namespace
 
