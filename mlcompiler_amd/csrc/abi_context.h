@@ -552,16 +552,18 @@ const uint64_t* resident_page_rows(const uint32_t* page_ids, const uint32_t* slo
 }
 
 // Sets where a KV write's launch finds its page rows: in the kernel arguments (emb, room for `most`), or on
-// the device.  What travelled in the arguments is remembered: mlc_hip_capture_begin sends it to the device,
-// so that a pass captured right after this one finds it there.
+// the device.  They are remembered either way: mlc_hip_capture_begin brings the device copy to the rows of the
+// last uncaptured KV write, so that a pass captured right after it finds them there.
 bool place_page_rows(const uint32_t* page_ids, const uint32_t* slots, size_t batch, size_t page_size, uint64_t* emb, size_t most,
                      const uint64_t** dev) {
     *dev = nullptr;
+    if (!g_capturing) {
+        g.last_ids.assign(page_ids, page_ids + batch);
+        g.last_slots.assign(slots, slots + batch);
+        g.last_page_size = page_size;
+    }
     if (batch > most || g_capturing) return (*dev = resident_page_rows(page_ids, slots, batch, page_size)) != nullptr;
     for (size_t r = 0; r < batch; ++r) emb[r] = (uint64_t)page_ids[r] * page_size + slots[r];
-    g.last_ids.assign(page_ids, page_ids + batch);
-    g.last_slots.assign(slots, slots + batch);
-    g.last_page_size = page_size;
     return true;
 }
 
