@@ -33,16 +33,14 @@ int fail(const std::string& msg) {
             return fail(std::string(#expr) + ": " + hipGetErrorString(e_));           \
     } while (0)
 
-// A host-pinned + device pair used to hand small metadata to kernels.  What was enqueued with it
-// has run once the host has waited for the stream: `wait` is the number of such waits (Ctx::waits)
-// when the slot was last used, and a slot is written again only after another one.  (An event per
-// use said the same for one more call and one more packet on the queue each time.)
+// A host-pinned + device pair used to hand small metadata to kernels.  `use` is the number of the slot's
+// last use (Ctx::slot_uses, counted over all slots); it is written again once that use has run, which the
+// host knows from a wait for the whole stream or for a marker (slot_reserve).
 struct MetaSlot {
     void* host = nullptr;
     void* dev = nullptr;
     size_t cap = 0;
-    uint64_t wait = 0;
-    bool used = false;
+    uint64_t use = 0;
 };
 
 // Scratch memory of the tile-balanced decode kernel: the split-K partials (one slot per
@@ -134,7 +132,17 @@ struct Ctx {
     long opt_q4_ksplit = 0;  // 0 = automatic
     MetaSlot ring[8];
     int ring_next = 0;
-    uint64_t waits = 0;   // times the host has waited for everything on the library's stream (wait_stream)
+    uint64_t slot_uses = 0;    // uses of metadata slots so far
+    uint64_t slots_done = 0;   // ... of which are known to have run
+    // Markers: events on the library's stream, each behind the first `uses` uses.  One is recorded for every
+    // second use that no wait has covered (the smallest rings have four slots), so that a caller that encodes
+    // many calls without a wait waits for the oldest of them only, and one that waits now and then records none.
+    struct SlotMarker {
+        hipEvent_t ev = nullptr;
+        uint64_t uses = 0;
+    } markers[4];
+    int marker_next = 0;
+    uint64_t slots_marked = 0;   // uses that have a marker behind them, or have run
     // Small host arrays that callers pass again and again with the same content (norm weights,
     // the page ids of a decode step across its layers): kept on the device, uploaded only when
     // the content changes.
@@ -324,6 +332,8 @@ bool init_once() {
     if (hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking) != hipSuccess) return false;
     if (hipEventCreate(&g.ev0) != hipSuccess || hipEventCreate(&g.ev1) != hipSuccess) return false;
     if (hipEventCreateWithFlags(&g.scratch_ev, hipEventDisableTiming) != hipSuccess) return false;
+    for (Ctx::SlotMarker& m : g.markers)
+        if (hipEventCreateWithFlags(&m.ev, hipEventDisableTiming) != hipSuccess) return false;
     g.available = true;
     return true;
 }
@@ -331,7 +341,8 @@ bool init_once() {
 // Waits for everything enqueued on the library's stream.
 int wait_stream() {
     HIP_OK(hipStreamSynchronize(g.stream));
-    ++g.waits;
+    // (a held-back attention launch, whose tables may lie in a slot, is not on the stream yet)
+    if (!g.dec.active) g.slots_done = g.slots_marked = g.slot_uses;
     return 1;
 }
 
@@ -339,8 +350,25 @@ int slot_reserve(MetaSlot& s, size_t bytes) {
     // (every copy of metadata to the device comes through here)
     NOT_WHILE_CAPTURING("copying metadata to the device (run the pass once uncaptured first; the planned and "
                         "generic decode kernels, one-request scatter / gather and prefill copy on every call)");
-    if (s.used && s.wait == g.waits && !wait_stream()) return 0;
-    s.used = false;
+    // (everything that reads a slot is on the stream by now, unless an attention launch is held back)
+    if (g.slot_uses - g.slots_marked >= 2 && !g.dec.active) {
+        Ctx::SlotMarker& m = g.markers[g.marker_next];
+        g.marker_next = (g.marker_next + 1) % 4;
+        m.uses = 0;
+        HIP_OK(hipEventRecord(m.ev, g.stream));
+        m.uses = g.slots_marked = g.slot_uses;
+    }
+    if (s.use > g.slots_done) {
+        Ctx::SlotMarker* oldest = nullptr;   // that lies behind this slot's use
+        for (Ctx::SlotMarker& m : g.markers)
+            if (m.uses >= s.use && (!oldest || m.uses < oldest->uses)) oldest = &m;
+        if (oldest) {
+            HIP_OK(hipEventSynchronize(oldest->ev));
+            g.slots_done = oldest->uses;
+        } else if (!wait_stream()) {
+            return 0;
+        }
+    }
     if (bytes > s.cap) {
         size_t cap = std::max<size_t>(4096, bytes * 2);
         if (s.host) HIP_OK(hipHostFree(s.host));
@@ -361,10 +389,7 @@ int slot_upload(MetaSlot& s, size_t bytes) {
 
 // (called when what reads the slot has been enqueued, or is held back and will be before the slot's
 // turn comes again)
-void slot_mark(MetaSlot& s) {
-    s.wait = g.waits;
-    s.used = true;
-}
+void slot_mark(MetaSlot& s) { s.use = ++g.slot_uses; }
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
