@@ -2,7 +2,9 @@
 // the C ABI.  A call through ctypes with numpy metadata spends 5 to 8 us on conversions (an array's
 // data_as alone is more than 1 us), as much as a small kernel takes; here it is 0.3 to 0.5 us.
 // Metadata may be anything numpy turns into an array of its type; what already is a contiguous array of
-// that type is used where it lies.  The interpreter is released around calls that wait for the GPU.
+// that type is used where it lies.  The interpreter is released around every call: those that only encode
+// may wait as well (a weight's first use, tables that wait for a slot), and what they are given is held
+// by the caller's arguments.
 #define PY_SSIZE_T_CLEAN
 #define NPY_NO_DEPRECATED_API NPY_1_7_API_VERSION
 #include <Python.h>
@@ -109,18 +111,14 @@ private:
     int n_held_ = 0;
 };
 
-// The result of an ABI call as a bool; `waits`: without the interpreter's lock.
+// The result of an ABI call, made without the interpreter's lock, as a bool.
 template <class F>
-PyObject* answer(const Args& a, bool waits, F&& call) {
+PyObject* answer(const Args& a, F&& call) {
     if (!a.ok()) return nullptr;
     int done = 0;
-    if (waits) {
-        Py_BEGIN_ALLOW_THREADS
-        done = call();
-        Py_END_ALLOW_THREADS
-    } else {
-        done = call();
-    }
+    Py_BEGIN_ALLOW_THREADS
+    done = call();
+    Py_END_ALLOW_THREADS
     return PyBool_FromLong(done);
 }
 
@@ -128,11 +126,11 @@ PyObject* answer(const Args& a, bool waits, F&& call) {
 
 MLC_CALL(begin) {
     const Args a(args, n, 0);
-    return answer(a, false, [] { return mlc_hip_begin(); });
+    return answer(a, [] { return mlc_hip_begin(); });
 }
 MLC_CALL(flush) {
     const Args a(args, n, 0);
-    return answer(a, true, [] { return mlc_hip_flush(); });
+    return answer(a, [] { return mlc_hip_flush(); });
 }
 // q, k_pages, v_pages, o, flat table, offsets, seq_lens, q_positions, batch, heads, kv_heads, head_dim, page size, causal, sync
 MLC_CALL(attention) {
@@ -144,7 +142,7 @@ MLC_CALL(attention) {
     const int causal = a.truth(), sync = a.truth();
     // the reference rejects vectors of the wrong length (metal_runtime.mm:7747-7748)
     if (a.ok() && (n_off != batch + 1 || n_seq != batch || n_pos != batch)) Py_RETURN_FALSE;
-    return answer(a, sync, [=] { return mlc_hip_paged_attn_decode(q, k, v, o, flat, n_flat, off, seq, pos, batch, heads, kv, dim, page, causal, sync); });
+    return answer(a, [=] { return mlc_hip_paged_attn_decode(q, k, v, o, flat, n_flat, off, seq, pos, batch, heads, kv, dim, page, causal, sync); });
 }
 // q, k_pages, v_pages, o, flat table, offsets, seq_lens, q_start, batch, chunk, heads, kv_heads, head_dim, page size, sync
 MLC_CALL(prefill) {
@@ -155,7 +153,7 @@ MLC_CALL(prefill) {
     const size_t batch = a.size(), chunk = a.size(), heads = a.size(), kv = a.size(), dim = a.size(), page = a.size();
     const int sync = a.truth();
     if (a.ok() && (n_off != batch + 1 || n_seq != batch || n_start != batch)) Py_RETURN_FALSE;
-    return answer(a, sync, [=] { return mlc_hip_paged_attn_prefill(q, k, v, o, flat, n_flat, off, seq, start, batch, chunk, heads, kv, dim, page, sync); });
+    return answer(a, [=] { return mlc_hip_paged_attn_prefill(q, k, v, o, flat, n_flat, off, seq, start, batch, chunk, heads, kv, dim, page, sync); });
 }
 // page storage, page ids, slots, page size, kv_heads, head_dim, batch, src, sync
 MLC_CALL(scatter_batched) {
@@ -167,7 +165,7 @@ MLC_CALL(scatter_batched) {
     void* src = a.ptr();
     const int sync = a.truth();
     if (a.ok() && (n_ids < batch || n_slots < batch || (sync && (n_ids != batch || n_slots != batch)))) Py_RETURN_FALSE;  // metal_runtime.mm:7243
-    return answer(a, sync, [=] { return mlc_hip_scatter_kv_paged_batched_f16(pages, ids, slots, page, kv, dim, batch, src, sync); });
+    return answer(a, [=] { return mlc_hip_scatter_kv_paged_batched_f16(pages, ids, slots, page, kv, dim, batch, src, sync); });
 }
 // page storage, page table, page size, kv_heads, head_dim, tokens, start slot, src, dtype bytes
 MLC_CALL(scatter) {
@@ -178,7 +176,7 @@ MLC_CALL(scatter) {
     const size_t page = a.size(), kv = a.size(), dim = a.size(), tokens = a.size(), start = a.size();
     void* src = a.ptr();
     const size_t bytes = a.size();
-    return answer(a, true, [=] { return mlc_hip_scatter_kv_paged(pages, table, n_table, page, kv, dim, tokens, start, src, bytes); });
+    return answer(a, [=] { return mlc_hip_scatter_kv_paged(pages, table, n_table, page, kv, dim, tokens, start, src, bytes); });
 }
 // page storage, page table, page size, kv_heads, head_dim, tokens, dst, dtype bytes
 MLC_CALL(gather) {
@@ -189,7 +187,7 @@ MLC_CALL(gather) {
     const size_t page = a.size(), kv = a.size(), dim = a.size(), tokens = a.size();
     void* dst = a.ptr();
     const size_t bytes = a.size();
-    return answer(a, true, [=] { return mlc_hip_gather_kv_pages(pages, table, n_table, page, kv, dim, tokens, dst, bytes); });
+    return answer(a, [=] { return mlc_hip_gather_kv_pages(pages, table, n_table, page, kv, dim, tokens, dst, bytes); });
 }
 // qkv, q, k, v, k_f16, v_f16, cos, sin, batch, heads, kv_heads, head_dim, qkv_rows, q_rows, k_rows, v_rows, rotary_dim, sync
 MLC_CALL(rope_cast) {
@@ -199,7 +197,7 @@ MLC_CALL(rope_cast) {
     for (void*& x : p) x = a.ptr();
     for (size_t& x : d) x = a.size();
     const int sync = a.truth();
-    return answer(a, sync, [&] {
+    return answer(a, [&] {
         return mlc_hip_qkv_split_rope_cast(p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], d[0], d[1], d[2], d[3], d[4], d[5], d[6], d[7], d[8], sync);
     });
 }
@@ -213,7 +211,7 @@ MLC_CALL(rms_norm) {
     const size_t batch = a.size(), length = a.size();
     void* out = a.ptr();
     const int sync = a.truth();
-    return answer(a, sync, [=] { return mlc_hip_rms_norm_batched(in, n_weight ? weight : nullptr, n_weight, eps, batch, length, out, sync); });
+    return answer(a, [=] { return mlc_hip_rms_norm_batched(in, n_weight ? weight : nullptr, n_weight, eps, batch, length, out, sync); });
 }
 // a, b, out, elements, sync
 MLC_CALL(add) {
@@ -221,7 +219,7 @@ MLC_CALL(add) {
     void *x = a.ptr(), *y = a.ptr(), *out = a.ptr();
     const size_t count = a.size();
     const int sync = a.truth();
-    return answer(a, sync, [=] { return mlc_hip_add_batched(x, y, out, count, sync); });
+    return answer(a, [=] { return mlc_hip_add_batched(x, y, out, count, sync); });
 }
 // gate_up, gate, up, out, batch, ffn_inner, gate_up rows, sync
 MLC_CALL(gate_up) {
@@ -229,7 +227,7 @@ MLC_CALL(gate_up) {
     void *gu = a.ptr(), *gate = a.ptr(), *up = a.ptr(), *out = a.ptr();
     const size_t batch = a.size(), inner = a.size(), rows = a.size();
     const int sync = a.truth();
-    return answer(a, sync, [=] { return mlc_hip_gate_up_split_silu_mul(gu, gate, up, out, batch, inner, rows, sync); });
+    return answer(a, [=] { return mlc_hip_gate_up_split_silu_mul(gu, gate, up, out, batch, inner, rows, sync); });
 }
 // name, weights, in, batch, rows, cols, row stride, quant version, out, sync
 MLC_CALL(matmul_q4_0) {
@@ -241,7 +239,7 @@ MLC_CALL(matmul_q4_0) {
     const size_t batch = a.size(), rows = a.size(), cols = a.size(), stride = a.size(), version = a.size();
     void* out = a.ptr();
     const int sync = a.truth();
-    return answer(a, sync, [=] { return mlc_hip_matmul_q4_0_batched(name, w, n_bytes, in, batch, rows, cols, stride, (uint32_t)version, out, sync); });
+    return answer(a, [=] { return mlc_hip_matmul_q4_0_batched(name, w, n_bytes, in, batch, rows, cols, stride, (uint32_t)version, out, sync); });
 }
 // name, weights, in, batch, rows, cols, row stride, out, sync
 MLC_CALL(matmul_q6_k) {
@@ -253,7 +251,7 @@ MLC_CALL(matmul_q6_k) {
     const size_t batch = a.size(), rows = a.size(), cols = a.size(), stride = a.size();
     void* out = a.ptr();
     const int sync = a.truth();
-    return answer(a, sync, [=] { return mlc_hip_matmul_q6_k_batched(name, w, n_bytes, in, batch, rows, cols, stride, out, sync); });
+    return answer(a, [=] { return mlc_hip_matmul_q6_k_batched(name, w, n_bytes, in, batch, rows, cols, stride, out, sync); });
 }
 // handle, flat table, offsets, seq_lens, q_positions, page ids or None, slots or None
 MLC_CALL(replay_update) {
@@ -262,12 +260,12 @@ MLC_CALL(replay_update) {
     size_t n_flat = 0, batch = 0, unused = 0;
     const uint32_t *flat = a.u32(&n_flat), *off = a.u32(&unused), *seq = a.u32(&batch), *pos = a.u32(&unused);
     const uint32_t *ids = a.u32_or_none(&unused), *slots = a.u32_or_none(&unused);
-    return answer(a, false, [=] { return mlc_hip_replay_update((int)handle, flat, n_flat, off, seq, pos, ids, slots, batch); });
+    return answer(a, [=] { return mlc_hip_replay_update((int)handle, flat, n_flat, off, seq, pos, ids, slots, batch); });
 }
 MLC_CALL(replay) {
     Args a(args, n, 1);
     const size_t handle = a.size();
-    return answer(a, false, [=] { return mlc_hip_replay((int)handle); });
+    return answer(a, [=] { return mlc_hip_replay((int)handle); });
 }
 #undef MLC_CALL
 
