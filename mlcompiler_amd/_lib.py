@@ -4,7 +4,8 @@ from __future__ import annotations
 import ctypes as C
 import os
 
-from .build import LIB_PATH, build_all, built_from_current_sources
+from .build import (CALL_MODULE_PATH, LIB_PATH, build_all, build_call_module, built_from_current_sources,
+                    call_module_is_current)
 
 
 class NativeLibraryError(RuntimeError):
@@ -86,6 +87,11 @@ def load(build_if_missing: bool = True) -> C.CDLL:
             raise NativeLibraryError(f"{LIB_PATH} is missing or older than its sources; "
                                      "run mlcompiler_amd/build.py")
         build_all()
+    if not call_module_is_current():   # built by another interpreter or for another numpy
+        if not build_if_missing:
+            raise NativeLibraryError(f"{CALL_MODULE_PATH} is missing or was built for another numpy or from other "
+                                     "sources; run mlcompiler_amd/build.py")
+        build_call_module()
     try:
         lib = C.CDLL(LIB_PATH)
     except OSError as exc:  # pragma: no cover

@@ -3,7 +3,8 @@
   libmlc_hip.so       HIP kernels + the C ABI declared in include/mlc_hip.h
   libhip_executor.so  the C++ HipExecutor class (mirror of the reference's
                       MetalExecutor paged-path methods) on top of that ABI
-  _call.so            HipExecutor's inner-loop calls into the ABI as a Python module
+  _call.<abi>.so      HipExecutor's inner-loop calls into the ABI as a Python module, for the interpreter
+                      and the numpy that build it
   libmlc_bench.so     native benchmark loops that call the ABI, plus a plain copy kernel
                       used to calibrate the HBM traffic counters
 """
@@ -13,12 +14,14 @@ import hashlib
 import os
 import shutil
 import subprocess
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(CSRC, "libmlc_hip.so")
 EXECUTOR_LIB_PATH = os.path.join(CSRC, "libhip_executor.so")
-CALL_MODULE_PATH = os.path.join(PKG_DIR, "_call.so")
+CALL_MODULE_PATH = os.path.join(PKG_DIR, "_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+CALL_STAMP_PATH = CALL_MODULE_PATH + ".stamp"         # what that module was built from and for
 BENCH_LIB_PATH = os.path.join(CSRC, "libmlc_bench.so")
 STAMP_PATH = os.path.join(CSRC, "libmlc_hip.stamp")   # hash of the sources the libraries were built from
 
@@ -51,10 +54,28 @@ def source_hash() -> str:
 
 def built_from_current_sources() -> bool:
     """True when the libraries exist and were built from the sources as they are now."""
-    if not all(os.path.exists(p) for p in (LIB_PATH, EXECUTOR_LIB_PATH, BENCH_LIB_PATH, CALL_MODULE_PATH, STAMP_PATH)):
+    if not all(os.path.exists(p) for p in (LIB_PATH, EXECUTOR_LIB_PATH, BENCH_LIB_PATH, STAMP_PATH)):
         return False
     with open(STAMP_PATH) as fh:
         return fh.read().strip() == source_hash()
+
+
+def call_module_identity() -> str:
+    """What the call module is built from and for: its sources and numpy (the interpreter is in its name)."""
+    import numpy
+    h = hashlib.sha256()
+    for f in (os.path.join(CSRC, "py_call.cpp"), os.path.join(os.path.dirname(PKG_DIR), "include", "mlc_hip.h")):
+        with open(f, "rb") as fh:
+            h.update(fh.read())
+    return f"{h.hexdigest()} numpy {numpy.__version__}"
+
+
+def call_module_is_current() -> bool:
+    """True when the call module exists for this interpreter, from the sources and for the numpy of now."""
+    if not all(os.path.exists(p) for p in (CALL_MODULE_PATH, CALL_STAMP_PATH)):
+        return False
+    with open(CALL_STAMP_PATH) as fh:
+        return fh.read().strip() == call_module_identity()
 
 
 def hipcc() -> str:
@@ -71,12 +92,14 @@ def _run(cmd: list[str]) -> None:
 
 
 def build_call_module() -> None:
-    import sysconfig
-
     import numpy
+    if os.path.exists(CALL_STAMP_PATH):
+        os.remove(CALL_STAMP_PATH)
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I" + sysconfig.get_paths()["include"],
           "-I" + numpy.get_include(), os.path.join(CSRC, "py_call.cpp"), "-o", CALL_MODULE_PATH,
           "-L" + CSRC, "-lmlc_hip", "-Wl,-rpath,$ORIGIN/csrc"])
+    with open(CALL_STAMP_PATH, "w") as fh:
+        fh.write(call_module_identity() + "\n")
 
 
 def build_all(verbose: bool = False) -> None:

@@ -73,3 +73,36 @@ def test_other_threads_run_during_every_call(tmp_path):
                            "-L" + str(tmp_path), "-lmlc_hip", "-Wl,-rpath," + str(tmp_path)])
     done = subprocess.run([sys.executable, str(tmp_path / "program.py"), str(tmp_path)], capture_output=True, text=True, timeout=120)
     assert done.returncode == 0, done.stdout + done.stderr
+
+
+def test_the_built_module_names_its_interpreter_and_is_current():
+    assert build.CALL_MODULE_PATH.endswith("_call" + sysconfig.get_config_var("EXT_SUFFIX"))
+    assert sysconfig.get_config_var("SOABI") in os.path.basename(build.CALL_MODULE_PATH)
+    assert build.call_module_is_current()
+
+
+def test_another_numpy_or_other_sources_make_it_stale(tmp_path, monkeypatch):
+    with monkeypatch.context() as m:
+        m.setattr(numpy, "__version__", "1.0.0")
+        assert not build.call_module_is_current()
+    (tmp_path / "py_call.cpp").write_text("// other\n")
+    with monkeypatch.context() as m:
+        m.setattr(build, "CSRC", str(tmp_path))
+        assert not build.call_module_is_current()
+    with monkeypatch.context() as m:      # an interpreter that nothing was built for yet
+        m.setattr(build, "CALL_MODULE_PATH", str(tmp_path / "_call.other.so"))
+        assert not build.call_module_is_current()
+    assert build.call_module_is_current()
+
+
+def test_a_stale_module_alone_does_not_rebuild_the_libraries(monkeypatch):
+    from mlcompiler_amd import _lib
+    asked = []
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "call_module_is_current", lambda: False)
+    monkeypatch.setattr(_lib, "build_call_module", lambda: asked.append("module"))
+    monkeypatch.setattr(_lib, "build_all", lambda: asked.append("all"))
+    with pytest.raises(_lib.NativeLibraryError):
+        _lib.load(build_if_missing=False)
+    _lib.load()
+    assert asked == ["module"]
