@@ -189,7 +189,6 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
 // the maximum that was 2^-25: weights 12 powers of two below the largest were wrong by 1e-4 of themselves,
 // 20 powers below by half.)  The shift cancels where the sums are divided.
 static constexpr float kWeightShift = 7.0f;
-static constexpr float kLowPart = 2048.0f;   // matrix-pipe mode: by how much the second part of q is larger than it counts
 
 // SMALL: at most 64 requests; lane r of every wave holds request r's figures in registers and
 // nothing goes through LDS.  Otherwise they are kept in (dynamic) LDS.
@@ -604,12 +603,13 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     // element to [2^14, 2^15) and is taken back where the scores are formed: any finite q fits, and the
     // multiplication is exact, so the two parts belong to the same number.  (Split behind a rounded
     // product, with the softmax scale, the compiler rounds the first part's two uses differently, and now
-    // and then a score was off by the first part's last place.)  The second part is 2^11 times larger
-    // than it counts and its products are summed apart: 23 bits of an element down to 2^-25 of the
-    // row's largest, and what is smaller to within 2^-50 of it.
-    // (A third part, which holds all 24 bits, was no closer to float64 in the output by more than a tenth
-    // and 1 to 3 % slower; scale and second sum cost 0.2 to 0.9 us a call: 23.0 -> 23.5 at 32 requests of
-    // 32 / 4 heads of 64.)
+    // and then a score was off by the first part's last place.)  The two hold 23 bits of an element down
+    // to 2^-16 of the row's largest, and what is smaller to within 2^-39 of it.  The products of the second
+    // part are summed first: the sum is small while they come, and nothing of them is rounded away.
+    // (A second part with a sum and a scale of its own, which reaches down to 2^-50, was no closer to
+    // float64 and 0.2 us slower; a third part, which holds all 24 bits, no closer by more than a tenth and
+    // 1 to 3 % slower.  Scaling costs 0.1 to 0.4 us a call: 23.3 -> 23.7 at 32 requests of 32 / 4 heads
+    // of 64.)
     auto split_q = [&]() {
         float amax = 0.f;
 #pragma unroll
@@ -621,7 +621,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         amax = fmaxf(__uint_as_float(sw32[0]), __uint_as_float(sw32[1]));
         const bool finite = amax < INFINITY;
         const int se = min(15 - (finite ? __builtin_amdgcn_frexp_expf(amax) : 128), 100);   // (a row below 2^-85: its scores are zero)
-        const float up = n16 < G ? __builtin_ldexpf(1.0f, se) : 0.f, up_low = up * kLowPart;
+        const float up = n16 < G ? __builtin_ldexpf(1.0f, se) : 0.f;
         q_unscale = __builtin_ldexpf(a.scale_log2e, -se);
 #pragma unroll
         for (int ks = 0; ks < (MF ? KST : 0); ++ks) {
@@ -629,9 +629,10 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const _Float16 hi = (_Float16)(x[i] * up);
+                const float t = x[i] * up;
+                const _Float16 hi = (_Float16)t;
                 qh[ks][i] = hi;
-                ql[ks][i] = (_Float16)fmaf((float)hi, -kLowPart, x[i] * up_low);
+                ql[ks][i] = (_Float16)(t - (float)hi);
             }
         }
         if (__any(!finite)) {   // an infinite element: the first part alone, or its difference with itself would be added
@@ -754,21 +755,19 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             for (int b = 0; b < DB; ++b)
                 va[b] = __builtin_bit_cast(sd_half4, __builtin_amdgcn_ds_read_tr16_b64_v4f16(
                     (sd_fp16x4 __attribute__((address_space(3)))*)(cur + mf_v_off[b])));
-            sd_f4 s4 = {0.f, 0.f, 0.f, 0.f}, s4_low = {0.f, 0.f, 0.f, 0.f};
+            sd_f4 s4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int ks = 0; ks < KST; ++ks) {
-                s4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], s4, 0, 0, 0);
-                s4_low = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], s4_low, 0, 0, 0);
-            }
+            for (int ks = 0; ks < KST; ++ks) s4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], ql[ks], s4, 0, 0, 0);
+#pragma unroll
+            for (int ks = 0; ks < KST; ++ks) s4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[ks], qh[ks], s4, 0, 0, 0);
             // lane (n16, g4) holds the scores of head n16 for the wave's keys 4*g4 .. 4*g4+3, once they are
             // scaled (rounded once, here: the largest one and its reference must cancel)
-            const float low_unscale = q_unscale * (1.0f / kLowPart);
             const uint32_t key0 = tile_start + (uint32_t)(wave * TW + 4 * g4);
             float mloc = -INFINITY;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const bool visible = (4 * g4 + i < TW) && key0 + (uint32_t)i < lim;
-                s4[i] = visible ? fmaf(s4_low[i], low_unscale, s4[i] * q_unscale) : -INFINITY;
+                s4[i] = visible ? s4[i] * q_unscale : -INFINITY;
                 mloc = max_nn(mloc, s4[i]);
             }
             // (as a difference, which is exact where it matters: a sum would be rounded, for large scores to
