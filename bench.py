@@ -969,8 +969,8 @@ def main() -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32 (fp16 K/V storage, fp32 q, accumulate and output; fp32-grade products, no operand rounded: on "
-                 "the f16 MFMA q and the softmax weights enter as sums of two fp16 numbers; option decode_pv_fp16 = 1 "
+        "dtype": "f32 (fp16 K/V storage, fp32 q, accumulate and output; fp32-grade products: on the f16 MFMA q and "
+                 "the softmax weights enter as scaled sums of two fp16 numbers, 23 bits of each; option decode_pv_fp16 = 1 "
                  "rounds the weights to fp16, us_per_layer_pv_fp16 is its time; option decode_mfma = 0: every product "
                  "on the vector pipe, us_per_layer_vector_pipe is its time)",
         "data": "synthetic",

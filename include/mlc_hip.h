@@ -83,7 +83,12 @@ int mlc_hip_has_open_pass(void);
  *   page_tables_flat  all requests' page ids, concatenated (n_page_tables_flat)
  *   page_table_offsets [batch+1]; seq_lens [batch]; q_positions [batch]
  * Softmax scale is 1/sqrt(head_dim), derived inside as the reference does
- * (metal_runtime.mm:7133).  Query head h reads KV head h*kv_heads/num_heads. */
+ * (metal_runtime.mm:7133).  Query head h reads KV head h*kv_heads/num_heads.
+ * Precision: sums in fp32.  GQA ratios 3 to 16 (1 and 2 over pages smaller than 64 tokens at head_dim 64,
+ * 32 at 128), head_dim 64 and 128, page sizes as listed at mlc_hip_paged_attn_decode_noalloc: q and the
+ * softmax weights enter the products as two fp16 numbers each.
+ * Of an element of q that is 23 bits, or its value to within 2^-39 of the largest of its row (any finite q
+ * fits); of a weight 23 bits, or to within 2^-32 of the row's largest.  Elsewhere both are fp32 numbers. */
 int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_pages, void* o,
                               const uint32_t* page_tables_flat, size_t n_page_tables_flat,
                               const uint32_t* page_table_offsets,
@@ -404,10 +409,10 @@ long mlc_hip_decode_table_uploads(void);
  *   "decode_pair_cost"      0..64: the tile-balanced decode kernel gives every workgroup the same
  *                           number of units, a KV tile counting one and the end of a (request,
  *                           KV head) pair this many; 0 = the same number of tiles; -1 (default) =
- *                           2 for GQA ratios of 4 and more (workgroups of four waves), 0 below
+ *                           2 in workgroups of four waves, 0 in smaller ones
  *   "decode_mfma"           1 (default) = the tile-balanced decode kernel does a tile's arithmetic
- *                           on the matrix pipe where the shape allows it (up to 16 query heads per
- *                           KV head in 4 waves); 0 = on the vector pipe
+ *                           on the matrix pipe where the shape allows it (3 to 16 query heads per KV
+ *                           head, 1 and 2 over pages smaller than a tile); 0 = on the vector pipe
  *   "prefill_stages"        2, 4, 6 or 8 K/V tiles staged in LDS by the prefill kernel (0 = automatic:
  *                           6); with 8 the kernel with 64 rows per wave lets its waves meet only
  *                           after every second tile;

@@ -72,8 +72,8 @@ __global__ __launch_bounds__(256) void q4_0_matmul_generic_kernel(
 // the padded batch goes to
 //   frag[((n/32 * ksteps + k/16) * 2 + part) * 64 + ((k%16)/8)*32 + n%32][k%8],  part 0 hi, 1 lo
 // so that lane l of a wave finds the 8 halves the MFMA wants from it (column n = l%32 of the
-// batch tile, k group l/32) in 16 contiguous bytes.  Rows past `batch` of the last tile are neither
-// written nor read.
+// batch tile, k group l/32) in 16 contiguous bytes.  Rows past `batch` of the last tile are not written
+// here, and nobody reads them.
 __global__ __launch_bounds__(256) void q4_split_activations_kernel(
     const float* __restrict__ x, _Float16* __restrict__ frag, float* __restrict__ inv_scale,
     uint32_t batch, uint32_t cols) {
@@ -368,8 +368,8 @@ __global__ __launch_bounds__(WAVES * 64, q4_two_per_cu(NBT, RT, WAVES, BS) ? 4 :
     // the request whose fragments a lane fetches: its own, and in lanes past the last request (and in
     // the other half's lanes, with bsplit) one that another lane fetches as well; their results are dropped.
     // (The fragments of 32 requests are the largest stream of a workgroup, whatever the batch: one request
-    // of the 1 B shape, per kernel: qkv 8.3 -> 7.0 us, gate/up 12.4 -> 11.2, a whole step 1 231 -> 1 144; and
-    // nobody has to write zeros for the missing requests.)
+    // of the 1 B shape, per kernel: qkv 8.3 -> 7.0 us, gate/up 12.4 -> 11.2, a whole step 1 231 -> 1 144.  The
+    // fragments of missing requests are read by nobody; the epilogues below write zeros there all the same.)
     uint32_t lane_x[NBT];
 #pragma unroll
     for (int t = 0; t < NBT; ++t)
@@ -610,7 +610,9 @@ __global__ __launch_bounds__(WAVES * 64, q4_two_per_cu(NBT, RT, WAVES, BS) ? 4 :
                 for (int i = i0; i < i1; ++i) red[(((wave * RT + r) * NBT + t) * 16 + i) * PITCH + lane] = acc[r][t][i];
     };
     put(0, 4);
-    if (!IOP || NBT > 1 || a.batch > 8) put(4, 16);   // (IOP: registers 0 .. 3 hold requests 0 .. 7)
+    // (IOP: registers 0 .. 3 hold requests 0 .. 7; the epilogues add up words of the others all the same and
+    // drop the sums)
+    if (!IOP || NBT > 1 || a.batch > 8) put(4, 16);
     __syncthreads();
     if constexpr (BS) {
         if (a.ssq_in) {
