@@ -94,7 +94,7 @@ __global__ __launch_bounds__(256) void gate_up_split_silu_mul_kernel(
 //   add      row = row + addend[row] -> add_out
 //   rms      row = row * 1/sqrt(mean(row^2) + eps) * weight -> rms_out
 //   split    row * 2^e = hi + lo (fp16 each) in the matmul's B-operand layout -> frag, 2^-e ->
-//            inv_scale  (q4_split_activations_kernel's arithmetic; rows >= batch are zero padding)
+//            inv_scale  (q4_split_activations_kernel's arithmetic)
 // One workgroup of 1024 threads per row (there are only as many rows as requests, so the row
 // is spread as wide as a workgroup goes).  A thread keeps its part of the row in registers from
 // the first stage to the last: groups of 8 consecutive elements, group number j * 1024 + thread.

@@ -46,11 +46,12 @@ def _errors(got, want):
 @pytest.mark.parametrize("D,P", [(64, 64), (64, 16), (128, 64), (128, 8)])
 @pytest.mark.parametrize("ratio", [3, 4, 6, 8, 16])
 def test_q_of_any_finite_size(exe, D, P, ratio):
-    """Heads of 1e6 and of 1e-6 side by side over keys of 2e4, one head with an infinite element."""
+    """Heads of 1e6 and of 1e-6 side by side over keys of 2e4, a head of zeros, one with an infinite element."""
     c = make_case(f"q_{ratio}_{D}_{P}", 3, 2 * ratio, 2, D, P, [40, 300, 777], seed=ratio + D + P)
     k = c.k_pages.view(np.float16)
     k *= np.float16(2e4 / 6)                    # (the largest of these normal values is below 6)
     c.q *= np.where(np.arange(2 * ratio) % 2, 1e-6, 1e6).astype(np.float32)[None, :, None]
+    c.q[0, 1] = 0.0
     want = _exact(c)
     c.q[1, 0, 5] = np.inf
     got, kernel = _run(exe, c)
