@@ -608,7 +608,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     // part are summed first: the sum is small while they come, and nothing of them is rounded away.
     // (A second part with a sum and a scale of its own, which reaches down to 2^-50, was no closer to
     // float64 and 0.2 us slower; a third part, which holds all 24 bits, no closer by more than a tenth and
-    // 1 to 3 % slower.  Scaling costs 0.1 to 0.4 us a call: 23.3 -> 23.7 at 32 requests of 32 / 4 heads
+    // 1 to 3 % slower.  Scaling costs 0.1 to 0.3 us a call: 23.3 -> 23.5 at 32 requests of 32 / 4 heads
     // of 64.)
     auto split_q = [&]() {
         float amax = 0.f;
@@ -1010,6 +1010,11 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                     comb_ml[wave * GP + n16] = mf_m;
                     comb_ml[NW * GP + wave * GP + n16] = lt;
                 }
+            }
+            // (the next pair's q, which came with that pair's first tile, is split while the waves meet:
+            // 0.15 us less per call at the benchmark shape than behind the meeting)
+            if constexpr (Q_AHEAD) {
+                if (!last_of_range) split_q();
             }
             sd_barrier();
 #pragma unroll
@@ -1419,9 +1424,8 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         }
         if (!range_done) {
             advance(cc);
-            if (pair_done) {
-                if constexpr (Q_AHEAD) split_q();
-                else load_q(cc);
+            if constexpr (!Q_AHEAD) {   // (else split where the pair's figures were put together)
+                if (pair_done) load_q(cc);
             }
         }
         slot = slot + 1u == (uint32_t)NBUF ? 0u : slot + 1u;
