@@ -117,6 +117,11 @@ def build_all(verbose: bool = False) -> None:
             obj = os.path.join(obj_dir, f"decode_d{d}_h{h}.o")
             jobs.append(([cc, *HIPCC_FLAGS, f"-DMLC_D={d}", f"-DMLC_HPW={h}", "-c",
                           os.path.join(CSRC, "paged_decode_inst.hip"), "-o", obj], obj))
+    tok_obj = os.path.join(obj_dir, "matmul_tokens.o")
+    jobs.append(([cc, *HIPCC_FLAGS, "-c", os.path.join(CSRC, "matmul_tokens_inst.hip"), "-o", tok_obj], tok_obj))
+    for ni in (1, 2, 4):
+        obj = os.path.join(obj_dir, f"q4_matmul_ni{ni}.o")
+        jobs.append(([cc, *HIPCC_FLAGS, f"-DMLC_Q4_NI={ni}", "-c", os.path.join(CSRC, "q4_matmul_inst.hip"), "-o", obj], obj))
     rt_obj = os.path.join(obj_dir, "mlc_hip.o")
     jobs.append(([cc, *HIPCC_FLAGS, "-c", os.path.join(CSRC, "mlc_hip.hip"), "-o", rt_obj], rt_obj))
     with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:

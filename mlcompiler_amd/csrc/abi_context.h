@@ -115,7 +115,7 @@ struct Ctx {
     struct Q4Weight {
         size_t bytes = 0, rows = 0, cols = 0, stride = 0;
         void* raw = nullptr;
-        void* qs = nullptr;
+        void* q = nullptr;
         void* d = nullptr;
     };
     std::unordered_map<std::string, Q4Weight> q4_weights;
@@ -191,8 +191,6 @@ struct Ctx {
     struct GemmPending {
         bool active = false;
         Q4Args a{};
-        unsigned grid_x = 0, grid_z = 1;
-        int nbt = 1, rt = 1;
         const void* out = nullptr;
         size_t batch = 0, rows = 0;
         bool block_scales = false;       // the activations carry one scale per (request, block)
@@ -443,64 +441,27 @@ constexpr size_t kRowMaxLen = 16384;  // row_program_kernel: 8 groups of 8 eleme
 
 bool row_len_ok(size_t len) { return len > 0 && len % 8 == 0 && len <= kRowMaxLen; }
 
-// One batch tile, two row tiles: a workgroup of 16 waves has a CU to itself (133 KB of LDS for its sums), so
-// where there are more of them than CUs two workgroups of 8 waves share one: the first loads of one overlap
-// the last sums of the other, and the last round is no longer a whole one.  28672 x 4096 (448 workgroups),
-// one to 32 requests: 46.5 .. 49.8 -> 40.0 .. 44.1 us a call, its kernel with SiLU 32.8 -> 29.9; at 176
-// workgroups (11264 x 2048, with block-wise scales) 16 waves are ahead (13.0 us, with 8 14.2).  Up to 128 blocks
-// of K: beyond, half as many waves would add up more blocks each in a row than 16 partial sums make up for.
-bool q4_pair_on_cu(dim3 grid, const Q4Args& a) { return grid.x > (unsigned)g.n_cu && a.nblocks <= 128; }
+// Rows of a Q4_0 matmul that come as 64 per workgroup, in tiles of 16.
+bool q4_wide(size_t rows) { return rows > 8192; }
 
-// The matrix-core Q4_0 kernel for nbt batch tiles of 32 and rt row tiles per workgroup; option
-// q4_int_operand picks the arithmetic (see q4_matmul_kernels.h).  With Q4RopeArgs: the split + RoPE + cast
-// of the output as epilogue.
-template <class Args>
-void launch_q4_mfma(int nbt, int rt, dim3 grid, const Args& a) {
-    constexpr bool ROPE = std::is_same_v<Args, Q4RopeArgs>;
-#define MLC_Q4(NBT, RT, WAVES)                                                                              \
-    if (g.opt_q4_int_operand)                                                                               \
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, true, false, false, ROPE>), grid, dim3(WAVES * 64), 0, g.stream, a); \
-    else                                                                                                    \
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, false, false, false, ROPE>), grid, dim3(WAVES * 64), 0, g.stream, a)
-    if (nbt == 1) {
-        if (rt == 1) { MLC_Q4(1, 1, 16); } else if (!q4_pair_on_cu(grid, a)) { MLC_Q4(1, 2, 16); } else { MLC_Q4(1, 2, 8); }
-    } else {
-        if (rt == 1) { MLC_Q4(2, 1, 8); } else { MLC_Q4(2, 2, 8); }
-    }
-#undef MLC_Q4
-}
-
-// The same with activations that were split with one scale per (request, block): a.blk_exp.
-// Integer-operand arithmetic only.  Two row tiles per workgroup run with 8 waves (the 128 registers
-// a wave of 16 has do not hold the exponents as well), and not with two batch tiles (256 do not
-// either): q4_block_scales_fit() is what callers ask first.
-bool q4_block_scales_fit(size_t bpad, int row_tiles) { return !(bpad > 32 && row_tiles == 2); }
-template <class Args>
-void launch_q4_mfma_block_scales(int nbt, int rt, dim3 grid, const Args& a) {
-    constexpr bool ROPE = std::is_same_v<Args, Q4RopeArgs>;
-#define MLC_Q4(NBT, RT, WAVES) \
-    hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<NBT, RT, WAVES, true, true, false, ROPE>), grid, dim3(WAVES * 64), 0, g.stream, a)
-    if (nbt == 1) {
-        if (rt == 1) { MLC_Q4(1, 1, 16); } else { MLC_Q4(1, 2, 8); }
-    } else {
-        MLC_Q4(2, 1, 8);
-    }
-#undef MLC_Q4
-}
-
-// The gate/up projection with the gate/up split + SiLU * up (and, when a.split_frag is set, the
-// split of the products for the matmul that reads them) as epilogue: two row tiles per workgroup.
-// (with block-wise activation scales: one batch tile only, see launch_q4_mfma_block_scales; its 16
-// waves fit their 128 registers because the epilogue's kernel schedules the scaling in groups of four)
-void launch_q4_mfma_silu(int nbt, bool block_scales, dim3 grid, const Q4Args& a) {
-    if (nbt == 1 && block_scales)
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<1, 2, 16, true, true, true>), grid, dim3(16 * 64), 0, g.stream, a);
-    else if (nbt == 1 && q4_pair_on_cu(grid, a))
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<1, 2, 8, true, false, true>), grid, dim3(8 * 64), 0, g.stream, a);
-    else if (nbt == 1)
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<1, 2, 16, true, false, true>), grid, dim3(16 * 64), 0, g.stream, a);
-    else
-        hipLaunchKernelGGL((q4_0_matmul_mfma_kernel<2, 2, 8, true, false, true>), grid, dim3(8 * 64), 0, g.stream, a);
+// Launches q4_matmul_kernel in one of its forms.  Tiles per workgroup: 4 for matrices of more than 8192 rows
+// and for the SiLU epilogue, 2 for the residual add's, else 1 where that leaves no more workgroups than CUs
+// (a workgroup of 16 waves has a CU to itself) and 2 where it does not.  RoPE: at most 2.
+int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a, size_t ksplit = 1) {
+    const uint32_t tiles = a.rows / 16;
+    a.z_groups = (a.batch + 15) / 16;
+    int rt = (size_t)tiles * a.z_groups * ksplit <= (size_t)g.n_cu ? 1 : 2;
+    if (form == kQ4Silu || (form == kQ4Plain && q4_wide(a.rows))) rt = 4;
+    else if (form == kQ4Add) rt = 2;
+    a.row_groups = tiles / rt;
+    // Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; a wide matrix with more
+    // row groups than CUs runs with 8, two workgroups to a CU, so that one's first loads overlap the other's products.
+    const int waves = q4_wide(a.rows) && (size_t)(tiles / 4) * a.z_groups * ksplit > (size_t)g.n_cu ? 8 : 16;
+    const dim3 grid((a.row_groups + 7) / 8 * 8 * a.z_groups, (unsigned)ksplit);
+    const auto launch = a.batch <= 4 ? launch_q4_matmul_1 : a.batch <= 8 ? launch_q4_matmul_2 : launch_q4_matmul_4;
+    if (!launch(form, rt, waves, block_scales, grid, a, g.stream)) return fail("q4 matmul: kernel variant not built");
+    HIP_OK(hipGetLastError());
+    return 1;
 }
 
 // Launches the held-back matmul, with the split + RoPE + cast of its output as epilogue when
@@ -509,32 +470,22 @@ int settle_gemm(const RopeArgs* rope = nullptr) {
     Ctx::GemmPending& m = g.gemm;
     if (!m.active) return 1;
     m.active = false;
-    const Q4Args& a = m.a;
-    const dim3 grid(m.grid_x, 1, m.grid_z);
+    Q4RopeArgs a;
+    static_cast<Q4Args&>(a) = m.a;
+    Q4Form form = kQ4Plain;
     if (rope) {
-        Q4RopeArgs ra{};
-        static_cast<Q4Args&>(ra) = a;
-        ra.rope = *rope;
+        a.rope = *rope;
+        form = kQ4Rope;
         ++g.gemm_rope_fused;
-        if (m.block_scales) launch_q4_mfma_block_scales(m.nbt, m.rt, grid, ra);
-        else launch_q4_mfma(m.nbt, m.rt, grid, ra);
-        HIP_OK(hipGetLastError());
-        return 1;
-    }
-    if (m.silu) {
+    } else if (m.silu) {
         m.silu = false;
+        form = kQ4Silu;
         ++g.gemm_silu_fused;
         if (a.split_frag) ++g.gemm_silu_split_fused;
-        launch_q4_mfma_silu(m.nbt, m.block_scales, grid, a);
-        HIP_OK(hipGetLastError());
-        return 1;
+    } else if (a.add_resid) {
+        form = kQ4Add;
     }
-    if (m.block_scales)
-        launch_q4_mfma_block_scales(m.nbt, m.rt, grid, a);
-    else
-        launch_q4_mfma(m.nbt, m.rt, grid, a);
-    HIP_OK(hipGetLastError());
-    return 1;
+    return launch_q4(form, m.block_scales, a);
 }
 
 // True when the held-back matmul's output is exactly the fused qkv rows a split + RoPE + cast

@@ -10,7 +10,14 @@ extern "C" {
 namespace {
 
 bool q4_fast_shape(size_t rows, size_t cols, size_t row_stride) {
-    return rows % 64 == 0 && cols % 32 == 0 && row_stride >= cols / 32 * 18;
+    // (the kernels address a tile's weights and a row's fragments with 32 bits)
+    return rows % 64 == 0 && cols % 32 == 0 && cols <= (1u << 24) && row_stride >= cols / 32 * 18;
+}
+
+// Copies weights to the device in the order of the library's stream (a plain hipMemcpy may return before the data is
+// there, and the library's stream does not wait for it), and waits.
+bool upload_weights(void* dst, const void* host, size_t bytes) {
+    return hipMemcpyAsync(dst, host, bytes, hipMemcpyHostToDevice, g.stream) == hipSuccess && hipStreamSynchronize(g.stream) == hipSuccess;
 }
 
 // Uploads the weight matrix on first use of its name (or when its size changed).
@@ -20,32 +27,24 @@ Ctx::Q4Weight* q4_weight(const char* name, const uint8_t* host, size_t bytes, si
     if (w.raw && w.bytes == bytes && w.rows == rows && w.cols == cols && w.stride == stride) return &w;
     if (g_capturing) { fail("q4 matmul: the weights are not on the device yet (run the pass once uncaptured first)"); return nullptr; }
     (void)hipStreamSynchronize(g.stream);
-    for (void** p : {&w.raw, &w.qs, &w.d})
+    for (void** p : {&w.raw, &w.q, &w.d})
         if (*p) { (void)hipFree(*p); *p = nullptr; ++g.buffer_generation; }
     w = Ctx::Q4Weight{};
     void* raw = nullptr;
     if (hipMalloc(&raw, bytes) != hipSuccess) { (void)hipGetLastError(); fail("q4 matmul: hipMalloc failed"); return nullptr; }
-    if (hipMemcpy(raw, host, bytes, hipMemcpyHostToDevice) != hipSuccess) { (void)hipFree(raw); fail("q4 matmul: upload failed"); return nullptr; }
+    if (!upload_weights(raw, host, bytes)) { (void)hipFree(raw); fail("q4 matmul: upload failed"); return nullptr; }
     w.raw = raw; w.bytes = bytes; w.rows = rows; w.cols = cols; w.stride = stride;
     if (q4_fast_shape(rows, cols, stride)) {
-        const size_t nb = cols / 32, tiles = rows / 32;
-        std::vector<uint8_t> qs(tiles * nb * 64 * 8);
-        std::vector<uint16_t> d(tiles * nb * 32);
-        for (size_t t = 0; t < tiles; ++t)
-            for (size_t b = 0; b < nb; ++b)
-                for (size_t m = 0; m < 32; ++m) {
-                    const uint8_t* blk = host + (t * 32 + m) * stride + b * 18;
-                    std::memcpy(&d[(t * nb + b) * 32 + m], blk, 2);
-                    for (size_t h = 0; h < 2; ++h)
-                        std::memcpy(&qs[((t * nb + b) * 64 + h * 32 + m) * 8], blk + 2 + h * 8, 8);
-                }
-        if (hipMalloc(&w.qs, qs.size()) != hipSuccess || hipMalloc(&w.d, d.size() * 2) != hipSuccess ||
-            hipMemcpy(w.qs, qs.data(), qs.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(w.d, d.data(), d.size() * 2, hipMemcpyHostToDevice) != hipSuccess) {
+        const size_t nb = cols / 32, quads = (nb + 3) / 4, tiles = rows / 16, units = tiles * quads * 64;
+        if (hipMalloc(&w.q, units * 16) != hipSuccess || hipMalloc(&w.d, tiles * quads * 16 * 8) != hipSuccess) {
             (void)hipGetLastError();
-            fail("q4 matmul: repacked upload failed");
+            fail("q4 matmul: hipMalloc failed");
             return nullptr;
         }
+        hipLaunchKernelGGL(q4_repack_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, g.stream,
+                           static_cast<const uint8_t*>(w.raw), static_cast<uint4*>(w.q), static_cast<uint16_t*>(w.d),
+                           (uint32_t)tiles, (uint32_t)nb, (uint32_t)quads, stride);
+        if (hipGetLastError() != hipSuccess) { fail("q4 matmul: repacking failed"); return nullptr; }
     }
     return &w;
 }
@@ -74,17 +73,18 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     // ... and is that chain  held-back matmul -> + residual -> RMSNorm?  Then the held-back matmul's
     // epilogue adds, leaves the sums of squares and writes (sum * gamma) as this matmul's fragments,
     // block-wise scaled, and this matmul finishes the norm: no launch in between.
-    // (block-wise scaled activations: not every shape of workgroup is built for them)
-    const bool scales_fit = q4_block_scales_fit((batch + 31) / 32 * 32, rows / 32 > 256 ? 2 : 1);
+    // (Wide matrices read block-wise scaled activations for up to 32 requests only: which launches are fused
+    // beyond is pinned by tests of the launch counts.)
+    const bool scales_fit = batch <= 32 || !q4_wide(rows);
     bool feeds_rms = false;
     if (feeds && scales_fit && g.gemm.active && g.opt_q4_int_operand) {
         const Ctx::GemmPending& m = g.gemm;
         const RowProgram& p = g.rows.p;
-        const size_t tiles = rows / 32, row_tiles = tiles > 256 ? 2 : 1;
-        feeds_rms = !m.silu && m.rt == 1 && !g.kv.active && p.src == m.out && p.n_slices == 1 &&
+        feeds_rms = !m.silu && !q4_wide(m.rows) && !g.kv.active && p.src == m.out && p.n_slices == 1 &&
                     !p.src_store && !p.silu && p.addend && p.rms && !p.frag && g.rows.batch == batch &&
-                    g.rows.len == cols && m.batch == batch && m.rows == cols && cols / 32 <= (batch <= 32 ? 128u : 64u) &&
-                    batch * cols <= (tiles / row_tiles) * 1024;   // (every workgroup of the reader writes 1024 elements of the norm)
+                    g.rows.len == cols && m.batch == batch && m.rows == cols && cols / 32 <= 128 &&
+                    batch * cols <= rows / (q4_wide(rows) ? 64 : 32) * 1024;   // (every thread of the reader writes at most one
+                                                                              // element of its z group's part of the norm)
     }
     // ... or is the input the SiLU * up product that the held-back gate/up projection's epilogue
     // will write?  Then that epilogue also splits it, per (request, block of 32 columns).
@@ -102,7 +102,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     Ctx::Q4Weight* w = q4_weight(weight_name, static_cast<const uint8_t*>(weights), weight_bytes, rows, cols, row_stride);
     if (!w) return 0;
 
-    if (!w->qs || g.opt_q4_force_generic || (reinterpret_cast<uintptr_t>(out) & 15u)) {
+    if (!w->q || g.opt_q4_force_generic || (reinterpret_cast<uintptr_t>(out) & 15u)) {
         if (!settle()) return 0;
         const size_t waves = batch * rows;
         hipLaunchKernelGGL(q4_0_matmul_generic_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, g.stream,
@@ -117,26 +117,23 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     // at 28672 x 4096.)
     if (batch > 64 && g.opt_q4_int_operand && g.opt_q4_ksplit == 0) {
         TokensArgs t{};
-        t.q = static_cast<const uint2*>(w->qs);
+        t.q = static_cast<const uint2*>(w->q);
         t.d = static_cast<const _Float16*>(w->d);
         t.nblocks = (uint32_t)(cols / 32);
-        if (matmul_tokens<TokensQ4>(t, static_cast<const float*>(in), static_cast<float*>(out), batch, rows, cols))
+        if (matmul_tokens(false, t, static_cast<const float*>(in), static_cast<float*>(out), batch, rows, cols))
             return finish(sync);
     }
 
-    // MFMA path, one pass over at most 64 requests at a time.  A workgroup takes one or two
-    // 32-row tiles and, unless K is split, all of K; two tiles when one would give more
-    // workgroups than CUs.  K is split only to fill CUs that would otherwise idle, and only as
-    // far as a workgroup keeps about 64 blocks of work.
-    const size_t nblocks = cols / 32, tiles = rows / 32;
-    const int row_tiles = tiles > 256 ? 2 : 1;
-    const size_t wgs = tiles / row_tiles;
+    // MFMA path, one pass over at most 64 requests at a time.  K is split over workgroups (of 32 rows) only where there
+    // are too few of them for the CUs and K is long: from 96 quads of blocks (K = 12288) on, so that each of a slice's
+    // 16 waves keeps three.
+    const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
     size_t ksplit = (size_t)g.opt_q4_ksplit;
-    if (ksplit == 0)
-        ksplit = std::max<size_t>(1, std::min<size_t>(256 / std::max<size_t>(wgs, 1), (nblocks * row_tiles + 63) / 64));
+    if (ksplit == 0) ksplit = std::max<size_t>(1, std::min<size_t>((size_t)g.n_cu / (rows / 32), quads / 48));
     ksplit = std::min(ksplit, std::max<size_t>(1, nblocks / 16));
-    const size_t per_slice = (nblocks + ksplit - 1) / ksplit;
-    ksplit = (nblocks + per_slice - 1) / per_slice;
+    if (!g.opt_q4_int_operand) ksplit = 1;
+    const size_t per_slice = (quads + ksplit - 1) / ksplit;
+    ksplit = (quads + per_slice - 1) / per_slice;
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;
@@ -145,41 +142,41 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             feeds_silu ? "q4_x_fragments_silu" : feeds_attn ? "q4_x_fragments_attention" : feeds_rms ? "q4_x_fragments_norm" : "q4_x_fragments",
             bpad * cols * 4));
         float* inv = static_cast<float*>(cached_buffer("q4_x_inv_scale", 64 * 4));
-        int8_t* blk_exp = !block_scales ? nullptr : static_cast<int8_t*>(cached_buffer(
-            feeds_silu ? "q4_x_block_exponents_silu" : feeds_attn ? "q4_x_block_exponents_attention" : "q4_x_block_exponents_norm",
-            bpad * nblocks));
+        float* blk_scale = !block_scales ? nullptr : static_cast<float*>(cached_buffer(
+            feeds_silu ? "q4_x_block_scales_silu" : feeds_attn ? "q4_x_block_scales_attention" : "q4_x_block_scales_norm",
+            bpad * nblocks * 4));
         float* ssq = feeds_rms ? static_cast<float*>(cached_buffer("q4_norm_partial_sums", nblocks * 64 * 4)) : nullptr;
         if (feeds_rms && !ssq) return fail("q4 matmul: scratch allocation failed");
         Q4Args norm{};   // (what this matmul needs to finish the norm)
-        if (!frag || !inv || (block_scales && !blk_exp)) return fail("q4 matmul: scratch allocation failed");
+        if (!frag || !inv || (block_scales && !blk_scale)) return fail("q4 matmul: scratch allocation failed");
         const float* xin = static_cast<const float*>(in) + bo * cols;
         float* o = static_cast<float*>(out) + bo * rows;
         if (feeds_silu) {
             g.gemm.a.split_frag = frag;
-            g.gemm.a.split_blk_exp = blk_exp;
+            g.gemm.a.split_blk_scale = blk_scale;
             if (!settle()) return 0;
         } else if (feeds_attn) {
             g.dec.a.split_frag = frag;
-            g.dec.a.split_exp = blk_exp;
+            g.dec.a.split_scale = blk_scale;
             if (!settle()) return 0;
         } else if (feeds_rms) {
             Ctx::GemmPending& m = g.gemm;
             const RowProgram& p = g.rows.p;
             m.a.add_resid = p.addend;
             m.a.add_out = p.add_out;
-            m.a.gamma = p.rms_weight;
-            m.a.n_gamma = p.n_weight;
+            m.a.add_gamma = p.rms_weight;
+            m.a.add_n_gamma = p.n_weight;
             m.a.ssq_out = ssq;
             m.a.split_frag = frag;
-            m.a.split_blk_exp = blk_exp;
+            m.a.split_blk_scale = blk_scale;
             norm.ssq_in = ssq;
             norm.ssq_tiles = (uint32_t)nblocks;   // one partial per 32 columns of the norm's row
             norm.rms_len = (uint32_t)cols;
             norm.rms_eps = p.epsilon;
             norm.rms_src = p.add_out;
             norm.rms_out = p.rms_out;
-            norm.gamma = p.rms_weight;
-            norm.n_gamma = p.n_weight;
+            norm.rms_gamma = p.rms_weight;
+            norm.rms_n_gamma = p.n_weight;
             g.rows.active = false;   // the two matmuls do the chain's work
             ++g.gemm_rms_fused;
             if (!settle()) return 0;
@@ -195,21 +192,21 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         // (the chain has been launched: its K-slice source may be replaced now)
         float* slices = ksplit > 1 ? static_cast<float*>(cached_buffer("q4_k_slices", ksplit * bn * rows * 4)) : nullptr;
         if (ksplit > 1 && !slices) return fail("q4 matmul: scratch allocation failed");
-        Q4Args a{};
-        a.qs = static_cast<const uint2*>(w->qs);
-        a.blk_exp = blk_exp;
-        a.ssq_in = norm.ssq_in; a.ssq_tiles = norm.ssq_tiles; a.rms_len = norm.rms_len; a.rms_eps = norm.rms_eps;
-        a.rms_src = norm.rms_src; a.rms_out = norm.rms_out; a.gamma = norm.gamma; a.n_gamma = norm.n_gamma;
-        a.d = static_cast<const _Float16*>(w->d);
+        Q4RopeArgs ra;
+        Q4Args& a = ra;
+        a = norm;
+        a.q = static_cast<const uint4*>(w->q);
+        a.d = static_cast<const uint2*>(w->d);
         a.xfrag = frag;
+        a.blk_scale = blk_scale;
         a.inv_scale = inv;
         a.out = ksplit > 1 ? slices : o;
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)nblocks;
-        a.blocks_per_slice = (uint32_t)per_slice; a.ksplit = (uint32_t)ksplit;
-        // one batch tile of more than 16 requests on a grid that fills at most half of the CUs: two
-        // workgroups per (row tile, K slice), each with half of the tile's requests
-        const unsigned bsplit = (bpad == 32 && bn > 16 && wgs * ksplit <= (size_t)g.n_cu / 2) ? 2u : 1u;
-        a.bsplit = bsplit;
+        a.nquads = (uint32_t)quads; a.quads_per_slice = (uint32_t)per_slice;
+        if (!g.opt_q4_int_operand) {
+            hipLaunchKernelGGL(q4_pairs_kernel, dim3((unsigned)(rows / 16), (unsigned)((bn + 15) / 16)), dim3(512), 0, g.stream, a);
+            continue;
+        }
         if (g.opt_fuse_rows && !sync && ksplit == 1 && batch <= 64) {
             // held back for one call: a split + RoPE + cast of this output becomes the epilogue
             Ctx::GemmPending& m = g.gemm;
@@ -217,20 +214,12 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             m.silu = false;
             m.block_scales = block_scales;
             m.a = a;
-            m.grid_x = (unsigned)wgs;
-            m.grid_z = bsplit;
-            m.nbt = bpad == 32 ? 1 : 2;
-            m.rt = row_tiles;
             m.out = out;
             m.batch = batch;
             m.rows = rows;
             return finish(sync);
         }
-        const dim3 grid((unsigned)wgs, (unsigned)ksplit, bsplit);
-        if (block_scales)
-            launch_q4_mfma_block_scales(bpad == 32 ? 1 : 2, row_tiles, grid, a);
-        else
-            launch_q4_mfma(bpad == 32 ? 1 : 2, row_tiles, grid, a);
+        if (!launch_q4(kQ4Plain, block_scales, ra, ksplit)) return 0;
         if (ksplit > 1) {
             const uint32_t n = (uint32_t)(bn * rows);
             if (g.opt_fuse_rows && batch <= 64 && rows <= 2 * kRowMaxLen) {
@@ -271,7 +260,7 @@ Ctx::Q6KWeight* q6k_weight(const char* name, const uint8_t* host, size_t bytes, 
     w = Ctx::Q6KWeight{};
     void* raw = nullptr;
     if (hipMalloc(&raw, bytes) != hipSuccess) { (void)hipGetLastError(); fail("q6_k matmul: hipMalloc failed"); return nullptr; }
-    if (hipMemcpy(raw, host, bytes, hipMemcpyHostToDevice) != hipSuccess) { (void)hipFree(raw); fail("q6_k matmul: upload failed"); return nullptr; }
+    if (!upload_weights(raw, host, bytes)) { (void)hipFree(raw); fail("q6_k matmul: upload failed"); return nullptr; }
     w.raw = raw; w.bytes = bytes; w.rows = rows; w.cols = cols; w.stride = stride;
     if (q6k_fast_shape(rows, cols, stride)) {
         const size_t nb = cols / 256, tiles = rows / 32, groups = nb * 4;
@@ -299,9 +288,8 @@ Ctx::Q6KWeight* q6k_weight(const char* name, const uint8_t* host, size_t bytes, 
             }
         if (hipMalloc(&w.qa, qa.size()) != hipSuccess || hipMalloc(&w.sc, sc.size()) != hipSuccess ||
             hipMalloc(&w.d, d.size() * 2) != hipSuccess ||
-            hipMemcpy(w.qa, qa.data(), qa.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(w.sc, sc.data(), sc.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(w.d, d.data(), d.size() * 2, hipMemcpyHostToDevice) != hipSuccess) {
+            !upload_weights(w.qa, qa.data(), qa.size()) || !upload_weights(w.sc, sc.data(), sc.size()) ||
+            !upload_weights(w.d, d.data(), d.size() * 2)) {
             (void)hipGetLastError();
             fail("q6_k matmul: repacked upload failed");
             return nullptr;
@@ -349,7 +337,7 @@ int mlc_hip_matmul_q6_k_batched(const char* weight_name, const void* weights, si
         t.sc = static_cast<const uint32_t*>(w->sc);
         t.d = static_cast<const _Float16*>(w->d);
         t.nblocks = (uint32_t)(cols / 256);
-        if (matmul_tokens<TokensQ6>(t, static_cast<const float*>(in), static_cast<float*>(out), batch, rows, cols))
+        if (matmul_tokens(true, t, static_cast<const float*>(in), static_cast<float*>(out), batch, rows, cols))
             return finish(sync);
     }
 

@@ -23,8 +23,7 @@ TokensPlan tokens_plan(size_t wgs, size_t slots, size_t stages, size_t out_bytes
 
 // All tokens of a call with more than 64 in one launch per piece (matmul_tokens_kernels.h).
 // Returns 0 where the call has to go 64 requests at a time instead: workspaces not at hand.
-template <class W>
-int matmul_tokens(TokensArgs a, const float* in, float* out, size_t batch, size_t rows, size_t cols) {
+int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t batch, size_t rows, size_t cols) {
     const size_t piece = kTokensFragBytes / (4 * cols) / 64 * 64;
     if (piece == 0) return 0;
     for (const char* name : {"tokens_x_fragments", "tokens_x_inv_scale", "tokens_k_slices"})
@@ -44,15 +43,14 @@ int matmul_tokens(TokensArgs a, const float* in, float* out, size_t batch, size_
         float* o = out + bo * rows;
         a.tokens = (uint32_t)bn;
         a.token_blocks = (uint32_t)((bn + 63) / 64);
-        hipLaunchKernelGGL(tokens_split_kernel, dim3(a.token_blocks * 16), dim3(256), 0, g.stream,
-                           in + bo * cols, frag, inv, (uint32_t)bn, (uint32_t)cols);
+        launch_tokens_split(in + bo * cols, frag, inv, (uint32_t)bn, (uint32_t)cols, a.token_blocks * 16, g.stream);
         const size_t wgs = (size_t)a.token_blocks * a.row_blocks;
         const TokensPlan plan = tokens_plan(wgs, 2 * (size_t)g.n_cu, a.stages, bn * rows * 4);
         a.stages_per_slice = plan.stages_per_slice;
         // (first-level sums of 4, 8 or 16 stages: about as many as there are of them)
         a.flush_mask = a.stages_per_slice <= 48 ? 0 : a.stages_per_slice <= 512 ? 1 : 3;
         a.out = plan.ksplit > 1 ? slices : o;
-        hipLaunchKernelGGL((matmul_tokens_kernel<W>), dim3((unsigned)(wgs * plan.ksplit)), dim3(256), 0, g.stream, a);
+        launch_matmul_tokens(q6, a, (unsigned)(wgs * plan.ksplit), g.stream);
         if (plan.ksplit > 1) {
             const uint32_t n = (uint32_t)(bn * rows);
             hipLaunchKernelGGL(q4_sum_slices_kernel, dim3((n + 255) / 256), dim3(256), 0, g.stream, slices, o, n,

@@ -69,7 +69,7 @@ int mlc_hip_add_batched(const void* a, const void* b, void* out, size_t total_el
     // else comes the matmul and the chain are launched one after the other, as always.
     const Ctx::GemmPending& m = g.gemm;
     const bool on_gemm = fusable && !sync && !joins && !r.active && !g.kv.active && !g.dec.active && m.active && !m.silu &&
-                         m.rt == 1 && g.opt_q4_int_operand && (m.out == a || m.out == b) &&
+                         !q4_wide(m.rows) && g.opt_q4_int_operand && (m.out == a || m.out == b) &&
                          m.batch * m.rows == total_elements && row_len_ok(m.rows);
     if (!joins && !on_gemm && !settle()) return 0;
     if (fusable) {
@@ -77,8 +77,7 @@ int mlc_hip_add_batched(const void* a, const void* b, void* out, size_t total_el
         if (joins) {
             other = r.cur == a ? b : a;
         } else if (on_gemm) {
-            rows_begin(m.out, 0, 0);
-            r.n_flat = total_elements;
+            rows_begin(m.out, m.batch, m.rows);
             other = m.out == a ? b : a;
         } else {
             rows_begin(a, 0, 0);
@@ -121,21 +120,20 @@ int mlc_hip_gate_up_split_silu_mul(const void* gate_up, void* gate, void* up, vo
     if (kg && batch * ffn_gate_up_rows * 4 > kg) return fail("gate/up split: gate_up buffer too small");
     {
         // The gate/up projection itself is still held back: the operator becomes its epilogue
-        // (workgroup j takes row tile j of the gate half and row tile j of the up half).
+        // (workgroup j takes columns 32 j .. 32 j + 31 of the gate half and of the up half).
         Ctx::GemmPending& m = g.gemm;
         if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && m.active && !m.silu && !g.rows.active && !g.kv.active &&
-            m.rt == 2 && m.grid_z == 1 && !(m.block_scales && m.nbt != 1) && m.out == gate_up && m.batch == batch && m.rows == ffn_gate_up_rows &&
+            q4_wide(m.rows) && m.out == gate_up && m.batch == batch && m.rows == ffn_gate_up_rows &&
             ffn_gate_up_rows == 2 * ffn_inner && ffn_inner % 32 == 0 && aligned16(gate) && aligned16(up) && aligned16(out)) {
             m.silu = true;
             m.silu_out = out;
             m.ffn_inner = ffn_inner;
-            m.a.tile_stride = (uint32_t)(ffn_inner / 32);
             m.a.ffn_inner = (uint32_t)ffn_inner;
             m.a.gate = static_cast<float*>(gate);
             m.a.up = static_cast<float*>(up);
             m.a.silu_out = static_cast<float*>(out);
             m.a.split_frag = nullptr;
-            m.a.split_blk_exp = nullptr;
+            m.a.split_blk_scale = nullptr;
             return finish(sync);
         }
         Ctx::RowPending& r = g.rows;

@@ -1,7 +1,7 @@
 // Q4_0 and Q6_K matmul over many tokens (a prompt chunk, a batch of more than 64) for gfx950:
 // out[t][r] = sum_c W[r][c] * x[t][c], all tokens in one launch.
 //
-// The arithmetic is that of the integer-operand kernels in q4_matmul_kernels.h and
+// The arithmetic is that of the integer-operand kernels in q4_matmul_mfma.h and
 // q6k_matmul_kernels.h: exact small integers times activations split into fp16 pairs on the matrix
 // cores, every block's (Q4_0) or 16-column group's (Q6_K) sum multiplied with its scale in fp32.
 // Those kernels take 64 requests at a time and stream everything through registers, which suits a
@@ -13,7 +13,8 @@
 //     double buffered (from memory each wave would read 64 bytes a clock, all that a CU's L1 gives);
 //   * weights go straight into registers, two stages ahead;
 //   * while the matrix pipe works on one block's products, the vector pipe scales and adds the sums of the
-//     block before;
+//     block before (Q4_0 in the compiler's order: with its order prescribed, as for Q6_K, 70.2 us instead of 66.7 at
+//     11264 x 2048 and 512 tokens);
 //   * fp32 sums are kept in two levels (4 stages = 256 columns or more, then those sums), so that an
 //     element is rounded no more often than in the waves' partial sums of the other kernels;
 //   * workgroups of one XCD share row blocks and groups of 8 token blocks.
@@ -31,15 +32,16 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "q4_matmul_kernels.h"
-#include "q6k_matmul_kernels.h"
+#include "matmul_tokens_args.h"
+#include "q4_matmul_mfma.h"
+#include "q6k_unpack.h"
 
 namespace mlc_hip {
 
 // What q4_split_activations_kernel does (q4_matmul_kernels.h), four tokens per workgroup: neighbouring
 // lanes hold neighbouring tokens, so that a store of 16 bytes per lane fills 64-byte pieces of the
 // fragments instead of leaving every piece to another workgroup.
-__global__ __launch_bounds__(256) void tokens_split_kernel(const float* __restrict__ x, _Float16* __restrict__ frag,
+static __global__ __launch_bounds__(256) void tokens_split_kernel(const float* __restrict__ x, _Float16* __restrict__ frag,
                                                            float* __restrict__ inv_scale, uint32_t tokens, uint32_t cols) {
     constexpr int MAXV = 8;   // groups of 8 columns a thread keeps in registers: cols <= 4096
     __shared__ float red[4][4];
@@ -99,48 +101,29 @@ __global__ __launch_bounds__(256) void tokens_split_kernel(const float* __restri
     }
 }
 
-struct TokensArgs {
-    const uint2* q;          // repacked weights: Q4Args::qs / Q6KArgs::qa
-    const uint32_t* sc;      // Q6KArgs::sc (Q4_0: not read)
-    const _Float16* d;       // Q4Args::d / Q6KArgs::d
-    const _Float16* xfrag;   // split activations of token_blocks * 64 rows (q4_split_activations_kernel)
-    const float* inv_scale;  // [tokens]
-    float* out;              // [tokens][rows], or the slice buffer [ksplit][tokens][rows]
-    uint32_t tokens, rows;
-    uint32_t ksteps;         // cols / 16
-    uint32_t nblocks;        // cols / 32 (Q4_0) or cols / 256 (Q6_K)
-    uint32_t stages, stages_per_slice;   // stages of 64 columns
-    uint32_t token_blocks, row_blocks;   // blocks of 64 tokens / 128 rows
-    uint32_t flush_mask;                 // a first-level sum ends where (stage group number & mask) == mask, groups of 4
-};
-
 // One stage's weights of one row tile: 4 k steps of 16 columns.
 struct TokensQ4 {
-    static constexpr int KSTEPS_PER_SCALE = 2, UNPACK = 8, VALU_PER_PRODUCT = 6;
-    uint2 q[2];
-    _Float16 d[2];
-    bool real[2];
+    static constexpr int KSTEPS_PER_SCALE = 2, UNPACK = 0, VALU_PER_PRODUCT = 0;   // (the compiler's order)
+    // (the layout is that of 16-row tiles and quads of blocks: a stage is half a quad, and k step s of its blocks
+    // takes the column groups 2 s and 2 s + 1)
+    uint2 q[2];     // [k step of a block]: a word per block
+    q4_half2 d;     // a scale per block
+    bool real;
     __device__ __forceinline__ void load(const TokensArgs& a, uint32_t tile, uint32_t stage, uint32_t end, uint32_t lane) {
+        const uint32_t st = min(stage, a.stages - 1u);   // past the end: the last stage again, with scale 0
+        real = stage < end;
+        const size_t tq = (size_t)(tile * 2 + lane % 32 / 16) * ((a.nblocks + 3) / 4) + st / 2;
 #pragma unroll
-        for (uint32_t j = 0; j < 2; ++j) {   // past the end: the last block again, with scale 0
-            const uint32_t raw = stage * 2 + j, blk = min(raw, a.nblocks - 1u);
-            real[j] = stage < end && raw < a.nblocks;
-            const size_t tb = (size_t)tile * a.nblocks + blk;
-            q[j] = a.q[tb * 64 + lane];
-            d[j] = a.d[tb * 32 + lane % 32];
-        }
+        for (uint32_t s = 0; s < 2; ++s) q[s] = a.q[(tq * 64 + (s * 2 + lane / 32) * 16 + lane % 16) * 2 + st % 2];
+        d = reinterpret_cast<const q4_half2*>(a.d)[(tq * 16 + lane % 16) * 2 + st % 2];
     }
     static __device__ __forceinline__ uint32_t kstep(const TokensArgs& a, uint32_t stage, uint32_t k) {
         return min(stage * 2 + k / 2, a.nblocks - 1u) * 2 + (k & 1u);
     }
     __device__ __forceinline__ q4_half8 operand(int k) const {
-        const uint32_t w0 = ((k & 1) ? (q[k / 2].x >> 4) : q[k / 2].x) & 0x0F0F0F0Fu;
-        const uint32_t w1 = ((k & 1) ? (q[k / 2].y >> 4) : q[k / 2].y) & 0x0F0F0F0Fu;
-        const q4_half2 n0 = q4_pair(w0, 0x04010400u), n1 = q4_pair(w0, 0x04030402u);
-        const q4_half2 n2 = q4_pair(w1, 0x04010400u), n3 = q4_pair(w1, 0x04030402u);
-        return q4_half8{n0[0], n0[1], n1[0], n1[1], n2[0], n2[1], n3[0], n3[1]};
+        return q4_unpack(k < 2 ? q[k & 1].x : q[k & 1].y, 0x64006400u);
     }
-    __device__ __forceinline__ float scale(int k) const { return real[k / 2] ? (float)d[k / 2] : 0.0f; }
+    __device__ __forceinline__ float scale(int k) const { return real ? (float)d[k / 2] : 0.0f; }
 };
 
 struct TokensQ6 {   // a stage is one group (see Q6KArgs): k step = quarter
@@ -278,12 +261,14 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
                             s[n][x] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xa[k][p][x], wk[k], s[n][x], 0, 0, 0);
                 if (i + step > 0) add(1 - n);
                 // the scheduler's order: fragments, then the products with the vector work between them
-                __builtin_amdgcn_sched_group_barrier(0x100, 4 * KS, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, W::UNPACK, 0);
+                if constexpr (W::VALU_PER_PRODUCT > 0) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 4 * KS, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, W::UNPACK, 0);
 #pragma unroll
-                for (int m = 0; m < 4 * KS; ++m) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, W::VALU_PER_PRODUCT, 0);
+                    for (int m = 0; m < 4 * KS; ++m) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, W::VALU_PER_PRODUCT, 0);
+                    }
                 }
             }
             w[i % 2].load(a, tile_in, base + i + 2, s1, lane);

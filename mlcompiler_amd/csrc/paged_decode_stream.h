@@ -78,11 +78,11 @@ struct StreamArgs {
     const uint4* new_v;
     // The split of the output for the Q4_0 matmul that reads it (null: none): whoever writes a row
     // of o also writes it as hi + lo fp16 fragments in that matmul's B-operand layout
-    // (q4_matmul_kernels.h), scaled by one power of two per (request, block of 32 columns), and the
-    // exponents where the matmul's block-scale form looks for them.  Requests
+    // (q4_matmul_mfma.h), scaled by one power of two per (request, block of 32 columns), and the
+    // scales where the matmul's block-scale form looks for them.  Requests
     // without visible tokens are written as zeros.
     _Float16* split_frag;
-    int8_t* split_exp;
+    float* split_scale;
     // seq_lens | q_positions | page_table_offsets (at a stride of 64 words for up to 64 requests,
     // of meta_stride words above) and, where it fits as well, the flat page table behind them: a
     // call whose tables travel here copies nothing to the device
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                 *reinterpret_cast<uint4*>(a.split_frag + ((base + 1) * 64 + fl) * 8) = z;
             }
             for (uint32_t blk = threadIdx.x; blk < cols / 32; blk += 64 * NW)
-                a.split_exp[((size_t)t32 * (cols / 32) + blk) * 32 + ((n32 % 8) / 4) * 16 + (n32 / 8) * 4 + n32 % 4] = 0;
+                a.split_scale[((size_t)t32 * (cols / 32) + blk) * 32 + n32] = 1.0f;
         }
     }
 
@@ -1167,8 +1167,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                     f_lo[0] = lo[0];
                 }
                 if (c % 4 == 0 && r_l == 0)
-                    a.split_exp[((size_t)t32 * (cols / 32) + col / 32) * 32 + ((n32 % 8) / 4) * 16 + (n32 / 8) * 4 + n32 % 4] =
-                        (int8_t)(-se);
+                    a.split_scale[((size_t)t32 * (cols / 32) + col / 32) * 32 + n32] = __builtin_ldexpf(1.0f, -se);
             }
         }
     };

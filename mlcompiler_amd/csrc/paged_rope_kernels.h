@@ -59,7 +59,7 @@ __device__ __forceinline__ float2 rope_rotate(float2 x, float c, float s) {
 // One thread per pair.  Pair index pi of a request counts pairs of the q, then k, then v
 // segment (every segment length is even on this path).  Which of the k / v outputs exist
 // (fp32 copy, fp16 staging copy, paged write) is decided per launch by the pointers.
-__global__ __launch_bounds__(256) void qkv_split_rope_cast_kernel(const RopeArgs a) {
+static __global__ __launch_bounds__(256) void qkv_split_rope_cast_kernel(const RopeArgs a) {
     const uint32_t pairs_row = (a.q_rows + a.k_rows + a.v_rows) / 2;
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= a.batch * pairs_row) return;

@@ -1,0 +1,537 @@
+// Batched Q4_0 matmul for gfx950: out[b][r] = sum_c W[r][c] * x[b][c], W in Q4_0 blocks
+// (32 weights: fp16 scale d, 16 bytes of nibbles; weight j in the low nibble of byte j,
+// weight j+16 in the high nibble, value d * (nibble - 8)), x and out fp32.
+//
+// Reference: MSL q4_0_matmul_v3_batched (compiler/runtime/metal_runtime.mm:710-785), one
+// simdgroup per (4 rows, request), fp32 scalar arithmetic.  With a decode batch of up to 64
+// requests this is a GEMM (M = rows, N = batch, K = cols) that should be bound by reading the
+// weights once, so here it runs on the matrix cores (fp32 accumulate) with fp32-grade accuracy:
+//   * an activation is split x*s = x_hi + x_lo (fp16 each, relative error 2^-22), s a power of
+//     two per request that places the row's largest magnitude at 2^13..2^14;
+//   * q4_matmul_kernel takes the integers q - 8 as operand, exact in fp16, and adds every block's sum
+//     (q-8).x_hi + (q-8).x_lo to the result as d * sum: nothing is dropped.  There the activations may
+//     also come with one power-of-two scale per (request, block of 32 columns) (BS), which a kernel
+//     that produces 32 neighbouring columns of a request can compute on its own: the epilogues
+//     (gate/up split + SiLU * up; residual add + RMSNorm) and the decode attention write the next
+//     matmul's fragments that way;
+//   * option q4_int_operand = 0 (q4_pairs_kernel): a weight d*(q-8) has at most 15 significant bits, so
+//     it is EXACTLY w_hi + w_lo with w_hi = fp16(d*(q-8)) and w_lo = fma(d, q-8, -w_hi), and
+//     out = (W_hi.X_hi + W_hi.X_lo + W_lo.X_hi) / s; the dropped W_lo.X_lo is below 2^-22 of the products.
+// The weights are repacked once, on the device, when they enter the library's weight cache
+// (q4_repack_kernel); the activations are split by a small kernel, or by whoever produces them, into
+// matrix operand fragments, so that a fragment is one 16-byte load per lane.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "paged_decode_kernels.h"
+#include "paged_rope_kernels.h"
+
+namespace mlc_hip {
+
+typedef _Float16 q4_half2 __attribute__((ext_vector_type(2)));
+typedef _Float16 q4_half8 __attribute__((ext_vector_type(8)));
+typedef float q4_float4 __attribute__((ext_vector_type(4)));
+typedef float q4_float16 __attribute__((ext_vector_type(16)));
+
+// ---- activations as operand fragments, for whoever makes them.  Element (n, k) of the padded batch, x*s = hi + lo with
+// hi = fp16(x*s), lo = fp16(x*s - hi), goes to
+//   frag[((n/32 * ksteps + k/16) * 2 + part) * 64 + ((k%16)/8)*32 + n%32][k%8],  part 0 hi, 1 lo, ksteps = K / 16
+// (two 16-column steps of it are the 32 columns of a block).
+
+// ---- repacked weights: tiles of 16 rows, quads of 4 blocks (128 columns), for
+// v_mfma_f32_16x16x32_f16, whose K is one block.
+//   q  [rows/16][nquads][64 lanes] x 4 words: lane kg * 16 + row % 16, word b: the 8 weights kg*8 .. +7 of
+//      block quad * 4 + b, weight e in nibble e / 2 + (e % 2) * 4 (q4_unpack)
+//   d  [rows/16][nquads][16 rows] x 4 halves
+// One 16-byte load brings a lane the weights of four blocks, 1 KB per wave in a row.  Blocks past the last one
+// have scale 0.
+struct Q4Args {
+    const uint4* q;             // repacked weights (q4_repack_kernel)
+    const uint2* d;
+    const _Float16* xfrag;      // split activations, layout above
+    const float* inv_scale;     // [batch]
+    float* out;                 // [batch][rows], or the slice buffer [ksplit][batch][rows]
+    uint32_t batch, rows, nblocks, nquads, quads_per_slice;
+    // The grid's x dimension: row groups (of RT tiles) times z groups of 16 requests, see q4_matmul_kernel.
+    uint32_t row_groups, z_groups;
+    // Kernels built with BS: the activations were split with one power-of-two scale per (request,
+    // block of 32 columns) instead of one per request: x = (hi + lo) * scale.  The scales are
+    // [batch tile of 32][nblocks][32 requests]; inv_scale is not read.
+    const float* blk_scale;
+    // SILU (ksplit == 1, rows = 2 * ffn_inner): the output is a fused gate/up row; row group j takes columns
+    // 32 j .. 32 j + 31 of the gate half and of the up half and its epilogue also does the gate/up split and
+    // SiLU(gate) * up -> gate, up, silu_out ([batch][ffn_inner] each).  With split_frag set it goes on
+    // to split the 32 products of every request into the fragments of the matmul that consumes
+    // them (K = ffn_inner), scaled per (request, block): block j of that matmul is exactly this
+    // row group's 32 columns.
+    uint32_t ffn_inner;
+    float* gate;
+    float* up;
+    float* silu_out;
+    _Float16* split_frag;
+    float* split_blk_scale;
+    // ADD (32 rows per workgroup, ksplit == 1): the epilogue also does the residual add that follows
+    // the matmul (add_out = out + add_resid, [batch][rows]), leaves every request's sum of squares over
+    // the workgroup's 32 columns in ssq_out[request][rows / 32] (the RMSNorm that follows is
+    // finished by the matmul that reads it, see ssq_in) and writes add_out * add_gamma as the
+    // split-fp16 fragments of that matmul (split_frag / split_blk_scale, K = rows).  add_gamma[c] for
+    // c < add_n_gamma, 1 beyond.
+    const float* add_resid;
+    float* add_out;
+    const float* add_gamma;
+    uint32_t add_n_gamma;
+    float* ssq_out;
+    // ssq_in set (BS kernels): the activations are h * rms_gamma of an RMSNorm whose per-request factor
+    // 1 / sqrt(mean(h^2) + eps) is still missing: it is computed here from the ssq_tiles partial
+    // sums of squares per request (ssq_in[request][ssq_tiles], summed in a fixed order) and multiplied into
+    // the result, and the workgroups also write the RMSNorm's own output rms_out = h * factor * rms_gamma
+    // ([batch][rms_len], h = rms_src), every thread of the grid one element of its z group's requests.
+    const float* ssq_in;
+    uint32_t ssq_tiles, rms_len;
+    float rms_eps;
+    const float* rms_src;
+    float* rms_out;
+    const float* rms_gamma;     // as add_gamma
+    uint32_t rms_n_gamma;
+};
+// ... and for the kernels built for ROPE (ksplit == 1, out is a fused qkv row of rope.qkv_rows = rows
+// floats per request), whose epilogue also does what qkv_split_rope_cast_kernel would do with that row.
+// (A type of its own: the launches without it need not carry its page rows.)
+struct Q4RopeArgs : Q4Args {
+    RopeArgs rope;
+};
+static constexpr uint32_t kQ4RopeOffset = (sizeof(Q4Args) + alignof(RopeArgs) - 1) / alignof(RopeArgs) * alignof(RopeArgs);
+static_assert(sizeof(Q4RopeArgs) == kQ4RopeOffset + sizeof(RopeArgs), "where the kernel finds rope in its arguments");
+
+// Maximum / sum over the 32 lanes of a half wave, every lane gets the result.
+__device__ __forceinline__ float q4_half_wave_max(float v) {
+    v = fmaxf(v, dpp_f<kDppQuadXor1>(v));
+    v = fmaxf(v, dpp_f<kDppQuadXor2>(v));
+    v = fmaxf(v, dpp_f<kDppHalfMirror>(v));
+    v = fmaxf(v, dpp_f<kDppRowRor8>(v));
+    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+}
+__device__ __forceinline__ float q4_half_wave_sum(float v) {
+    v += dpp_f<kDppQuadXor1>(v);
+    v += dpp_f<kDppQuadXor2>(v);
+    v += dpp_f<kDppHalfMirror>(v);
+    v += dpp_f<kDppRowRor8>(v);
+    const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+}
+
+// One value per lane, the 32 lanes of a half wave holding columns col0 .. col0+31 (one Q4_0 block)
+// of request b: writes them as hi + lo fp16 fragments of a matmul with K = k_cols, scaled by the
+// block's own power of two, and the scale that undoes it (q4_split_activations_kernel's scale, per block).
+__device__ __forceinline__ void q4_emit_block(float v, uint32_t b, uint32_t col, uint32_t k_cols, _Float16* frag,
+                                              float* blk_scale) {
+    const float amax = q4_half_wave_max(fabsf(v));
+    int e = 0;
+    if (amax > 0.f && amax < INFINITY) (void)frexpf(amax, &e);
+    int se = 14 - e;
+    se = se > 100 ? 100 : (se < -100 ? -100 : se);
+    const float tv = __builtin_ldexpf(v, se);
+    const _Float16 hi = (_Float16)tv;
+    const _Float16 lo = (_Float16)(tv - (float)hi);
+    const uint32_t t = b / 32, c = b % 32;
+    const size_t base = ((size_t)t * (k_cols / 16) + col / 16) * 2;
+    const uint32_t fl = ((col % 16) / 8) * 32 + c;
+    frag[((base + 0) * 64 + fl) * 8 + col % 8] = hi;
+    frag[((base + 1) * 64 + fl) * 8 + col % 8] = lo;
+    if (col % 32 == 0) blk_scale[((size_t)t * (k_cols / 32) + col / 32) * 32 + c] = __builtin_ldexpf(1.0f, -se);
+}
+
+// The split + RoPE + cast (+ paged write) of one element of a request's fused qkv row, by the
+// thread that just produced it; the partner of its (even, odd) pair sits in the neighbouring
+// lane.  Same arithmetic, element for element, as qkv_split_rope_cast_kernel.  What the thread
+// needs from memory for it (its cos / sin pair, its request's page row) is fetched before the
+// matmul's main loop, so that the epilogue adds no memory round trip to the kernel's tail.
+struct Q4RopeFetch {
+    float c, s;        // rotation of this element's pair (1, 0 where none applies)
+    uint64_t page_row; // page_id * page_size + slot
+};
+
+__device__ __forceinline__ Q4RopeFetch q4_rope_prefetch(const RopeArgs& p, const uint64_t* page_rows, uint32_t req,
+                                                         uint32_t feat) {
+    Q4RopeFetch f = {1.0f, 0.0f, 0ull};
+    if (req >= p.batch || feat >= p.q_rows + p.k_rows + p.v_rows) return f;
+    const bool is_q = feat < p.q_rows;
+    const bool is_k = !is_q && feat < p.q_rows + p.k_rows;
+    const uint32_t local = is_q ? feat : (is_k ? feat - p.q_rows : feat - p.q_rows - p.k_rows);
+    if (is_q || is_k) {
+        const uint32_t d = (local & ~1u) % p.head_dim;
+        if (d < p.rotary_dim) {
+            const uint32_t ci = req * (p.rotary_dim / 2) + d / 2;
+            f.c = p.cos_table[ci];
+            f.s = p.sin_table[ci];
+        }
+    }
+    if (!is_q && (is_k ? p.k_pages : p.v_pages)) f.page_row = page_rows[req];
+    return f;
+}
+
+__device__ __forceinline__ void q4_rope_epilogue(const RopeArgs& p, const Q4RopeFetch& f, uint32_t req,
+                                                 uint32_t feat, float val) {
+    const float other = __shfl_xor(val, 1);
+    const bool odd = (feat & 1u) != 0;
+    const float2 x = odd ? make_float2(other, val) : make_float2(val, other);
+    if (feat >= p.q_rows + p.k_rows + p.v_rows) return;
+    const bool is_q = feat < p.q_rows;
+    const bool is_k = !is_q && feat < p.q_rows + p.k_rows;
+    const uint32_t local = is_q ? feat : (is_k ? feat - p.q_rows : feat - p.q_rows - p.k_rows);
+    float2 y = x;
+    if ((is_q || is_k) && (local & ~1u) % p.head_dim < p.rotary_dim) y = rope_rotate(x, f.c, f.s);
+    const float mine = odd ? y.y : y.x;
+    if (is_q) {
+        p.q[(size_t)req * p.q_rows + local] = mine;
+        return;
+    }
+    float* f32 = is_k ? p.k : p.v;
+    const uint32_t rows = is_k ? p.k_rows : p.v_rows;
+    if (f32) f32[(size_t)req * rows + local] = mine;
+    const _Float16 h = (_Float16)mine;
+    _Float16* f16 = is_k ? p.k_f16 : p.v_f16;
+    if (f16) f16[(size_t)req * rows + local] = h;
+    _Float16* pool = is_k ? p.k_pages : p.v_pages;
+    if (pool) pool[(size_t)f.page_row * rows + local] = h;
+}
+
+// 8- and 16-byte non-temporal loads (data that is read once and need not displace anything in the L2).
+typedef uint32_t q4_u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t q4_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 q4_stream_u2(const uint2* p) {
+    const q4_u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const q4_u32x2*>(p));
+    return make_uint2(v[0], v[1]);
+}
+
+// A buffer descriptor of `bytes` bytes: loads behind its end return zero and move no data.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t q4_buffer(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00027000);
+}
+
+// 0x64006400 in a register the compiler does not see into: (w & mask) | ones is then one instruction (with two
+// constants it takes two, an instruction of three operands having room for one).
+__device__ __forceinline__ uint32_t q4_ones() {
+    uint32_t ones = 0x64006400u;
+    asm("" : "+v"(ones));
+    return ones;
+}
+// The 8 weights of a word of the repacked layout as halves q - 8, exactly: (0x6400 | n) is the half
+// 1024 + n, (0x6400 | n << 4) is 1024 + 16 n.  Nine instructions.
+__device__ __forceinline__ q4_half8 q4_unpack(uint32_t w, uint32_t ones) {
+    const q4_half2 k1032 = {(_Float16)1032.0f, (_Float16)1032.0f}, k72 = {(_Float16)72.0f, (_Float16)72.0f};
+    const q4_half2 k16th = {(_Float16)0.0625f, (_Float16)0.0625f};
+    const uint32_t v = w >> 8;
+    const q4_half2 n0 = __builtin_bit_cast(q4_half2, (w & 0x000F000Fu) | ones) - k1032;
+    const q4_half2 n1 = __builtin_elementwise_fma(__builtin_bit_cast(q4_half2, (w & 0x00F000F0u) | ones), k16th, -k72);
+    const q4_half2 n2 = __builtin_bit_cast(q4_half2, (v & 0x000F000Fu) | ones) - k1032;
+    const q4_half2 n3 = __builtin_elementwise_fma(__builtin_bit_cast(q4_half2, (v & 0x00F000F0u) | ones), k16th, -k72);
+    return q4_half8{n0[0], n0[1], n1[0], n1[1], n2[0], n2[1], n3[0], n3[1]};
+}
+
+__device__ __forceinline__ float q4_silu_times(float g, float u) {  // walker_kernels.h: silu_times
+    const float silu = g / (1.0f + expf(-g));
+    return silu * u;
+}
+
+// What the epilogue of q4_matmul_kernel does besides storing the result.
+enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
+
+// One workgroup of 16 (or 8) waves: RT tiles of 16 weight rows x up to 16 requests x one K slice.  The slice's
+// quads of blocks are dealt out to the waves; a wave streams its quads' nibbles and scales (one quad ahead) and
+// activation fragments (XD blocks ahead) straight from memory into registers, unpacks and multiplies; there is
+// no staging memory and no barrier until the waves' sums meet in LDS at the end.
+//
+// The matrix product runs over the exact integers q - 8 and the block scale d is applied to each block's sum
+// in fp32, acc += d * ((q-8).x_hi + (q-8).x_lo): per 16 rows and block two MFMAs, 9 instructions to unpack and
+// one (with block scales two) per accumulator register.  The weights are the B operand (a lane holds weight
+// row lane % 16, so d is one number per lane), the activations the A operand.  No product is rounded and no
+// term is dropped: what remains is the fp32 rounding of the additions and of one multiply per block.
+//
+// These kernels are bound by the vector pipe of the CUs they run on as soon as the weights are there: one
+// of them takes 1.7 us until its first loads are back, whatever it loads.  Hence 16 x 16 products:
+// of a 32 x 32 product's 16 accumulator registers a batch of up to 16 requests uses half, and each costs
+// one to three instructions per block.  NI: accumulator registers per product that are used: request r sits
+// in row (r / NI) * 4 + r % NI of the A operand, so that 4 NI requests leave the registers NI .. 3 empty.
+//
+// More than 16 requests: z groups of 16, workgroups of their own that read the same weights at the same
+// time on the same XCD (workgroup x: row group x / (8 Z) * 8 + x % 8, z group x / 8 % Z).  Each fetches its
+// own activations only, 4 bytes per request and column through one CU's memory path, which would be the
+// longest stream of a workgroup that had them all.
+//
+// Measured, kernel times in us, before (32 x 32 products, one workgroup per 32 rows, branches or clamps around the loads of
+// a wave's last blocks) -> now.  One request of the 1 B shape: qkv (2560 x 2048) 7.0 -> 5.1, out-projection with the
+// residual add 8.4 -> 5.0, gate/up with SiLU (11264 x 2048) 11.2 -> 7.4, down (2048 x 5632) 8.1 and 5.0 for the sum of
+// its K slices -> 8.7 with the residual add and no slices; a step of 22 layers 1 145 -> 853.  32 requests: qkv 7.5 -> 6.9,
+// gate/up 13.3 -> 14.0, a step 1 330 -> 1 207.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
+// a layer 141 -> 114.  2-norm error against float64: 0.95e-7 .. 1.15e-7, before 1.03e-7 .. 1.34e-7.
+template <int NI, int RT, int WAVES, bool BS, int FORM>
+__global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
+    const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
+    static_assert(FORM != kQ4Silu || RT == 4, "SiLU epilogue: 32 rows of gate and 32 of up");
+    static_assert(FORM != kQ4Add || RT == 2, "residual add: 32 rows, one block of the next matmul's K");
+    constexpr int XD = RT == 4 ? 2 : 4;              // blocks of activations in flight
+    constexpr int QR = 4 * NI;                       // requests of the workgroup
+    constexpr int TILE_PITCH = NI * 64 + 16;         // floats per tile in LDS (16: bank spread)
+    __shared__ float red[WAVES * RT * TILE_PITCH];
+    // BS: a quad's scales, [block][request]: fetched by a load of 4 bytes per lane, handed out from here.  (A load of
+    // every lane's own scales per block would take as long as one of the block's two fragments: what bounds these
+    // kernels next to the vector pipe is the 64 bytes a clock that a CU's loads return.)
+    __shared__ __attribute__((aligned(16))) float scales[BS ? WAVES : 1][64];
+    __shared__ float rms_scale[BS ? QR : 1];         // BS with ssq_in: every request's RMSNorm factor
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t lane = threadIdx.x % 64, l16 = lane % 16, kg = lane / 16;
+    const uint32_t z8 = 8 * a.z_groups;
+    const uint32_t row_group = blockIdx.x / z8 * 8 + blockIdx.x % 8, zg = blockIdx.x / 8 % a.z_groups;
+    if (row_group >= a.row_groups) return;           // (the grid is a multiple of 8 row groups)
+    const uint32_t slice = blockIdx.y;
+    const uint32_t req0 = zg * 16, live = min((uint32_t)QR, a.batch - req0);   // (the last group may be smaller)
+    // tile r of the workgroup
+    const uint32_t tile0 = FORM == kQ4Silu ? row_group * 2 : row_group * RT;
+    auto tile_of = [&](int r) __attribute__((always_inline)) {
+        return FORM == kQ4Silu && r >= 2 ? a.ffn_inner / 16 + tile0 + (uint32_t)r - 2u : tile0 + (uint32_t)r;
+    };
+
+    // ---- thread -> output: row `row` of the workgroup's (SiLU: column of its 32), request req0 + q
+    constexpr uint32_t ROWS = FORM == kQ4Silu ? 32 : 16 * RT, PER_PASS = WAVES * 64 / ROWS;
+    constexpr int PASSES = (QR + PER_PASS - 1) / PER_PASS;   // outputs per thread
+    static_assert(PASSES == 1 || FORM == kQ4Plain, "the other epilogues: one output per thread");
+    const uint32_t row = threadIdx.x % ROWS, qi = threadIdx.x / ROWS;
+    // (which request: so that the 64 lanes of a wave read 64 different banks)
+    constexpr uint32_t SB = 2 * NI;
+    const uint32_t q = ROWS == 16   ? (qi % 4) * NI + qi / 4
+                       : ROWS == 32 ? (qi & ~(1u | SB)) | ((qi & 1u) ? SB : 0u) | ((qi & SB) ? 1u : 0u)
+                                    : qi;
+    const bool has_out = qi < QR && q < live;
+    const uint32_t b = req0 + q, col = tile0 * 16 + row;
+
+    // ---- what the epilogue reads besides the sums is fetched before the main loop, so that it adds no memory
+    // round trip to the kernel's tail
+    [[maybe_unused]] Q4RopeFetch rope_pre = {1.0f, 0.0f, 0ull};
+    if constexpr (FORM == kQ4Rope)
+        if (has_out) rope_pre = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4RopeOffset), b, col);
+    [[maybe_unused]] float resid_pre = 0.f, gamma_pre = 1.0f, inv_pre[PASSES] = {};
+    if constexpr (FORM == kQ4Add) {
+        if (has_out) resid_pre = a.add_resid[(size_t)b * a.rows + col];
+        if (col < a.add_n_gamma) gamma_pre = a.add_gamma[col];
+    }
+    if constexpr (!BS) {
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p)
+            if (q + p * PER_PASS < live) inv_pre[p] = a.inv_scale[b + p * PER_PASS];
+    }
+    // The RMSNorm that the producer of the activations left unfinished (ssq_in): a wave sums up the partials of
+    // one or two requests, and the row group writes 1024 elements of the norm's own output at the end.
+    constexpr int RMS_N = 16 / WAVES;   // requests per wave, and elements per thread
+    constexpr int SSQ_NL = 2;           // partials per lane: up to 128 tiles, rows of 4096 (the host checks)
+    [[maybe_unused]] float ssq_part[RMS_N][SSQ_NL] = {}, rms_h[RMS_N] = {}, rms_gamma[RMS_N];
+    const uint32_t rms_el = row_group * 1024 + threadIdx.x;
+    if constexpr (BS) {
+        if (a.ssq_in) {
+#pragma unroll
+            for (int n = 0; n < RMS_N; ++n) {
+                const uint32_t sq = wave + n * WAVES, el = rms_el + n * WAVES * 64;
+#pragma unroll
+                for (int j = 0; j < SSQ_NL; ++j) {
+                    const uint32_t tl = lane + j * 64;
+                    if (sq < live && tl < a.ssq_tiles) ssq_part[n][j] = a.ssq_in[(size_t)(req0 + sq) * a.ssq_tiles + tl];
+                }
+                rms_gamma[n] = 1.0f;
+                if (el < live * a.rms_len) {
+                    const uint32_t rc = el % a.rms_len;
+                    rms_h[n] = a.rms_src[(size_t)req0 * a.rms_len + el];
+                    if (rc < a.rms_n_gamma) rms_gamma[n] = a.rms_gamma[rc];
+                }
+            }
+        }
+    }
+    asm volatile("" ::: "memory");
+
+    // ---- main loop
+    struct QuadW {
+        q4_u32x4 q[RT];
+        q4_u32x2 d[RT];
+        float sc;   // BS: the scale of request l16 in block kg of the quad
+    };
+    struct BlockX {
+        q4_half8 hi, lo;
+    };
+    // Everything is fetched with buffer loads: a descriptor per stream in scalar registers and 32 bits per lane.  Their
+    // descriptors end where the data does; what lies behind (the last blocks of an incomplete quad, the weights
+    // behind a wave's last quad) reads as zero.
+    const uint32_t first = slice * a.quads_per_slice + wave, end = min((slice + 1) * a.quads_per_slice, a.nquads);
+    __amdgpu_buffer_rsrc_t q_desc[RT], d_desc[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        const size_t tile = (size_t)tile_of(r) * a.nquads;
+        q_desc[r] = q4_buffer(a.q + tile * 64, end * 1024);
+        d_desc[r] = q4_buffer(a.d + tile * 16, end * 128);
+    }
+    const __amdgpu_buffer_rsrc_t x_desc = q4_buffer(a.xfrag + (size_t)(req0 / 32) * a.nblocks * 2048, a.nblocks * 4096);
+    const __amdgpu_buffer_rsrc_t s_desc = q4_buffer(BS ? a.blk_scale + (size_t)(req0 / 32) * a.nblocks * 32 : nullptr, a.nblocks * 128);
+    // (request of this lane's row of the A operand; rows without one fetch another's again)
+    const uint32_t xreq = min(l16 / 4 * NI + min(l16 % 4, (uint32_t)NI - 1u), live - 1u) + req0 % 32;
+    const uint32_t x_lane = (kg / 2 * 128 + kg % 2 * 32 + xreq) * 16;   // (fragment layout: two 16-column steps)
+    const uint32_t s_lane = kg * 128 + (req0 % 32 + l16) * 4;
+    auto load_w = [&](uint32_t quad, QuadW& k) __attribute__((always_inline)) {
+        constexpr int NT = 2;   // (non-temporal: a weight is read once per launch and need not stay in the L2)
+        if constexpr (BS) k.sc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s_desc, quad * 512 + s_lane, 0, 0));
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            k.q[r] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_desc[r], quad * 1024 + lane * 16, 0, NT));
+            k.d[r] = __builtin_bit_cast(q4_u32x2, __builtin_amdgcn_raw_buffer_load_b64(d_desc[r], quad * 128 + l16 * 8, 0, NT));
+        }
+        asm volatile("" ::: "memory");
+    };
+    auto load_x = [&](uint32_t blk, BlockX& k) __attribute__((always_inline)) {
+        k.hi = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc, blk * 4096 + x_lane, 0, 0));
+        k.lo = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc, blk * 4096 + x_lane + 1024, 0, 0));
+        asm volatile("" ::: "memory");
+    };
+    const uint32_t ones = q4_ones();
+    q4_float4 zero;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) zero[i] = 0.f;
+    float acc[RT][NI];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) acc[r][i] = 0.f;
+    auto multiply = [&](const QuadW& w, int j, const BlockX& x) __attribute__((always_inline)) {
+        // (the scales of this lane's requests in block j, see `turn`)
+        [[maybe_unused]] float sc[NI];
+        if constexpr (BS) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) sc[i] = scales[wave][j * 16 + kg * NI + i];
+        }
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const q4_half2 dd = __builtin_bit_cast(q4_half2, (uint32_t)w.d[r][j / 2]);
+            const float d = (float)dd[j % 2];
+            const q4_half8 wk = q4_unpack(w.q[r][j], ones);
+            q4_float4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.hi, wk, zero, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.lo, wk, s, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i) acc[r][i] = fmaf(BS ? d * sc[i] : d, s[i], acc[r][i]);
+            // (here, and not further down, where the compiler would move it: a quad's products do not fit
+            // the 128 registers a wave has)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(acc[r][i]));
+        }
+    };
+    // A wave's quads are first, first + WAVES, ...  While one is multiplied the next one's weights are on the way, and
+    // activations XD blocks ahead.  The last one is a copy of the code that fetches nothing: a load costs its share
+    // of the return path even where it reads nothing, and behind a branch around loads the compiler waits as if
+    // they had not been issued, and so for all of them.  (The empty asm statements pin every group of
+    // loads where it is written: without them they move down to just before their use.)
+    QuadW w, next;
+    BlockX x[XD];
+    auto turn = [&](uint32_t quad, auto more) __attribute__((always_inline)) {
+        if constexpr (BS) scales[wave][lane] = w.sc;   // (a wave's own: LDS operations of a wave are in order)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            multiply(w, j, x[j % XD]);
+            if (j + XD < 4) load_x(quad * 4 + j + XD, x[j % XD]);
+            else if constexpr (decltype(more)::value) load_x((quad + WAVES) * 4 + j + XD - 4, x[j % XD]);
+        }
+    };
+    if (first < end) {
+        load_w(first, w);
+#pragma unroll
+        for (int i = 0; i < XD; ++i) load_x(first * 4 + i, x[i]);
+        if (first + WAVES < end) load_w(first + WAVES, next);
+    }
+    if constexpr (BS) {
+        if (a.ssq_in) {
+#pragma unroll
+            for (int m = 0; m < RMS_N; ++m) {
+                float part = q4_half_wave_sum(ssq_part[m][0] + ssq_part[m][1]);
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(part), __float_as_uint(part), false, false);
+                part = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+                const uint32_t sq = wave + m * WAVES;
+                if (lane == 0 && sq < live) rms_scale[sq] = 1.0f / sqrtf(part / (float)a.rms_len + a.rms_eps);
+            }
+        }
+    }
+    if (first < end) {
+        uint32_t quad = first;
+        for (; quad + WAVES < end; quad += WAVES) {
+            turn(quad, std::true_type());
+            // (not before this point: the copy waits for the loads)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) asm volatile("" : "+v"(next.q[r]), "+v"(next.d[r]));
+            w = next;
+            load_w(quad + 2 * WAVES, next);
+        }
+        turn(quad, std::false_type());
+    }
+
+    // ---- the waves' sums meet in LDS.  A lane holds weight row l16 of the tile and, in register i, request
+    // kg * NI + i.
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) red[(wave * RT + r) * TILE_PITCH + i * 64 + lane] = acc[r][i];
+    __syncthreads();
+    if constexpr (BS) {
+        // the norm's own output: h * factor * gamma, the arithmetic of rms_norm_batched_kernel
+        if (a.ssq_in) {
+#pragma unroll
+            for (int m = 0; m < RMS_N; ++m) {
+                const uint32_t el = rms_el + m * WAVES * 64;
+                if (el < live * a.rms_len)
+                    a.rms_out[(size_t)req0 * a.rms_len + el] = rms_h[m] * rms_scale[el / a.rms_len] * rms_gamma[m];
+            }
+        }
+    }
+    if (!has_out) return;   // (whole half waves where the epilogue works across lanes: 32 rows share q)
+    auto sum_of = [&](uint32_t tile_row, uint32_t sq, float inv) __attribute__((always_inline)) {
+        const float* p = red + tile_row / 16 * TILE_PITCH + (sq % NI) * 64 + sq / NI * 16 + tile_row % 16;
+        float sum[WAVES];   // (added up in pairs: fewer roundings on the way of each)
+#pragma unroll
+        for (int k = 0; k < WAVES; ++k) sum[k] = p[k * RT * TILE_PITCH];
+#pragma unroll
+        for (int step = 1; step < WAVES; step *= 2)
+#pragma unroll
+            for (int k = 0; k < WAVES; k += 2 * step) sum[k] += sum[k + step];
+        if constexpr (BS) return a.ssq_in ? sum[0] * rms_scale[sq] : sum[0];
+        else return sum[0] * inv;
+    };
+    if constexpr (FORM == kQ4Silu) {
+        // the 32 lanes of a half wave hold one request's 32 columns, one block of the consuming matmul's K
+        const float gv = sum_of(row, q, inv_pre[0]), uv = sum_of(32 + row, q, inv_pre[0]);
+        const float prod = q4_silu_times(gv, uv);
+        a.out[(size_t)b * a.rows + col] = gv;
+        a.out[(size_t)b * a.rows + a.ffn_inner + col] = uv;
+        a.gate[(size_t)b * a.ffn_inner + col] = gv;
+        a.up[(size_t)b * a.ffn_inner + col] = uv;
+        a.silu_out[(size_t)b * a.ffn_inner + col] = prod;
+        if (a.split_frag) q4_emit_block(prod, b, col, a.ffn_inner, a.split_frag, a.split_blk_scale);
+        return;
+    }
+    float* out = a.out + (size_t)slice * a.batch * a.rows;
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+        const uint32_t qp = q + p * PER_PASS, bp = b + p * PER_PASS;
+        if (qp >= live) break;
+        const float val = sum_of(row, qp, inv_pre[p]);
+        out[(size_t)bp * a.rows + col] = val;
+        if constexpr (FORM == kQ4Rope) q4_rope_epilogue(a.rope, rope_pre, bp, col, val);   // (the lanes of a pair share b)
+        if constexpr (FORM == kQ4Add) {
+            // residual add, this request's sum of squares over the 32 columns, and h * gamma as the next
+            // matmul's fragments
+            const float hv = val + resid_pre;
+            a.add_out[(size_t)bp * a.rows + col] = hv;
+            const float ssq = q4_half_wave_sum(hv * hv);
+            if (row == 0) a.ssq_out[(size_t)bp * (a.rows / 32) + row_group] = ssq;
+            q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale);
+        }
+    }
+}
+
+}  // namespace mlc_hip

@@ -18,7 +18,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "q4_matmul_kernels.h"
+#include "q6k_unpack.h"
 
 namespace mlc_hip {
 
@@ -72,13 +72,6 @@ struct Q6KArgs {
     float* out;              // [batch][rows]
     uint32_t batch, rows, nblocks;
 };
-
-// (0x6400 | v) is the half 1024 + v: two bytes -> half2 (v0 - 32, v1 - 32), exactly.
-__device__ __forceinline__ q4_half2 q6_pair(uint32_t bytes, uint32_t sel) {
-    const uint32_t m = __builtin_amdgcn_perm(0x64646464u, bytes, sel);
-    const q4_half2 k1056 = {(_Float16)1056.0f, (_Float16)1056.0f};
-    return __builtin_bit_cast(q4_half2, m) - k1056;
-}
 
 // One workgroup: RT tiles of 32 weight rows x NBT batch tiles of 32 x all of K; its 8 waves
 // deal the groups out among themselves (group wave, wave + 8, ...), stream their pieces, scales

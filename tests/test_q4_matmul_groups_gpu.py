@@ -1,0 +1,61 @@
+"""Q4_0 matmuls of up to 64 requests at the edges of the kernel's division: 1, 2 or 4 accumulator registers per
+product (batches 4 | 5, 8 | 9), groups of 16 requests, incomplete quads of blocks, waves without a quad and with one or
+two, 1, 2 or 4 tiles of 16 rows per workgroup, 8 or 16 waves; and a matmul that both finishes one RMSNorm and
+carries the residual add of the next (its two norms have weights of their own)."""
+import numpy as np
+import pytest
+
+import test_q4_matmul_gpu as q4
+from oracle import paged_oracle as po
+from test_matmul_norm_fusion_gpu import EPS, _pool, _read
+from test_matmul_tokens_gpu import check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch", [1, 4, 5, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("rows,cols", [
+    (64, 64),        # half a quad of blocks, most waves without one
+    (4160, 160),     # a quad and one block; two tiles per workgroup (one of 65 row groups)
+    (192, 2080),     # 17 quads, the last incomplete: one wave has two
+    (8256, 1184),    # wide: four tiles per workgroup, 16 waves (8 from 17 requests on), 10 quads
+])
+def test_divisions(exe, rows, cols, batch):
+    q, x, stride = q4.make(rows, cols, batch, rows + cols + batch)
+    got = q4.run(exe, f"groups_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride)
+    check(got, q4.dequant(q, cols), x)
+    assert np.array_equal(got, q4.run(exe, f"groups_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride, sync=False))
+
+
+@pytest.mark.parametrize("batch", [1, 6, 16, 21, 40])
+def test_a_chain_of_norms(exe, batch):
+    """matmul, add, norm, matmul, add, norm, matmul: the one in the middle finishes the first norm and starts the second."""
+    rng = np.random.default_rng(batch)
+    n = 512
+    w = [po.quantize_q4_0((rng.standard_normal((r, n)) * 0.05).astype(np.float32)) for r in (n, n, 2 * n)]
+    gamma = [(1.0 + 0.3 * rng.standard_normal(n)).astype(np.float32) for _ in range(2)]
+    x, r0, r1 = (rng.standard_normal((batch, n)).astype(np.float32) for _ in range(3))
+    like = {m: np.empty((batch, 2 * n if m == "y" else n), np.float32) for m in ("p0", "h0", "n0", "p1", "h1", "n1", "y")}
+    dev = {m: _pool(exe, np.full_like(a, np.nan)) for m, a in like.items()}
+    src = [_pool(exe, a) for a in (x, r0, r1)]
+    before = exe.fusedMatmulNormLaunches()
+    try:
+        assert exe.beginForwardPassCB()
+        for i, (a, p, r, h, norm) in enumerate(((src[0], "p0", src[1], "h0", "n0"), (dev["n0"], "p1", src[2], "h1", "n1"))):
+            assert exe.encodeMatMulQ4_0Batched(f"norms{batch}.{i}", w[i], a, batch, n, n, w[i].shape[1], 1, dev[p])
+            assert exe.encodeAddBatched(dev[p], r, dev[h], batch * n)
+            assert exe.encodeRmsNormBatched(dev[h], gamma[i], EPS, batch, n, dev[norm])
+        assert exe.encodeMatMulQ4_0Batched(f"norms{batch}.2", w[2], dev["n1"], batch, 2 * n, n, w[2].shape[1], 1, dev["y"])
+        assert exe.flushForwardPassCB(), exe.lastError()
+        got = {m: _read(exe, dev[m], like[m]) for m in like}
+    finally:
+        for buf in list(dev.values()) + src:
+            exe.releaseScratchBuffer(buf)
+    assert exe.fusedMatmulNormLaunches() - before == (1 if batch <= 32 else 0) + 1   # (40: the norm has more elements than the reader's threads)
+    for a, m, i in ((x, "p0", 0), (got["n0"], "p1", 1), (got["n1"], "y", 2)):
+        check(got[m], q4.dequant(w[i], n), a)
+    for i, r in enumerate((r0, r1)):
+        assert np.array_equal(got[f"h{i}"], r + got[f"p{i}"])
+        want = po.rms_norm_batched(got[f"h{i}"], gamma[i], EPS, batch, n)
+        # (as in test_matmul_norm_fusion_gpu.py: a sum of n squares and one rounding per factor)
+        assert (np.abs(got[f"n{i}"] - want) <= 2e-6 * np.abs(want).max(axis=1, keepdims=True)).all()
