@@ -399,10 +399,21 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     // workgroup whose range crosses from one pair into the next gets fewer tiles.  Unit numbering:
     // [request][kv head][the pair's tiles, then PC units that stand for its end].
     const uint32_t T = tiles_head * Hkv;                       // the host keeps this below 2^31
+    // A workgroup gets at least 1 << `least` tiles.  A pair that is spread over more workgroups reads its tiles
+    // sooner, but is summed up from more partials, eight per memory round trip: with n tiles per pair the sum of
+    // the two is least at about sqrt(n) / 2 tiles (by 3 the pairs' ends rarely fall on a range's end: powers of
+    // two), and two tiles go to one workgroup, which then sums up nothing.
+    // (Whole calls, one tile per workgroup where there were places -> now, us; 32 query and 4 KV heads of 64, one
+    // request of 128, 1024, 2048, 4096, 8192 tokens: 16.7 -> 15.8, 19.7 -> 18.9, 23.7 -> 20.7, 31.8 -> 22.4,
+    // 51.8 -> 26.4; 8 KV heads of 128, one request of 2048: 34.3 -> 23.4, four of 512: 23.6 -> 20.1.)
+    const uint32_t twice = (uint32_t)(tiles_head * 4u > nz_head * 7u && tiles_head * 4u < nz_head * 9u);
+    const uint32_t least = twice + (uint32_t)(tiles_head > nz_head * 8u) + (uint32_t)(tiles_head >= nz_head * 48u) +
+                           (uint32_t)(tiles_head >= nz_head * 160u);
+    const uint32_t places = min((uint32_t)gridDim.x, (T + (1u << least) - 1u) >> least);
     // (nothing to balance where every tile gets a workgroup of its own)
-    const uint32_t PC = T > gridDim.x ? a.pair_cost : 0u;
+    const uint32_t PC = T > places ? a.pair_cost : 0u;
     const uint32_t UT = T + PC * nz_head * Hkv;                // ... and this
-    const uint32_t W = gridDim.x < UT ? gridDim.x : UT;
+    const uint32_t W = places < UT ? places : UT;
     const uint32_t w = blockIdx.x;
     if (w >= W) {
         leave_copy();
