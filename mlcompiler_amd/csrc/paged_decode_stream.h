@@ -25,6 +25,7 @@
 
 #include <cstddef>
 
+#include "fragments.h"
 #include "paged_decode_kernels.h"
 
 namespace mlc_hip {
@@ -77,8 +78,7 @@ struct StreamArgs {
     const uint4* new_k;
     const uint4* new_v;
     // The split of the output for the Q4_0 matmul that reads it (null: none): whoever writes a row
-    // of o also writes it as hi + lo fp16 fragments in that matmul's B-operand layout
-    // (q4_matmul_mfma.h), scaled by one power of two per (request, block of 32 columns), and the
+    // of o also writes it as hi + lo fp16 fragments (fragments.h), scaled by one power of two per (request, block of 32 columns), and the
     // scales where the matmul's block-scale form looks for them.  Requests
     // without visible tokens are written as zeros.
     _Float16* split_frag;
@@ -383,11 +383,9 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             if (req_lim(rr) != 0) continue;
             const uint32_t t32 = rr / 32, n32 = rr % 32;
             for (uint32_t k8 = threadIdx.x; k8 < cols / 8; k8 += 64 * NW) {
-                const size_t base = ((size_t)t32 * (cols / 16) + k8 / 2) * 2;
-                const uint32_t fl = (k8 % 2) * 32 + n32;
                 const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-                *reinterpret_cast<uint4*>(a.split_frag + ((base + 0) * 64 + fl) * 8) = z;
-                *reinterpret_cast<uint4*>(a.split_frag + ((base + 1) * 64 + fl) * 8) = z;
+                *reinterpret_cast<uint4*>(a.split_frag + frag_piece(rr, k8, 0, cols, frag_width(B))) = z;
+                *reinterpret_cast<uint4*>(a.split_frag + frag_piece(rr, k8, 1, cols, frag_width(B))) = z;
             }
             for (uint32_t blk = threadIdx.x; blk < cols / 32; blk += 64 * NW)
                 a.split_scale[((size_t)t32 * (cols / 32) + blk) * 32 + n32] = 1.0f;
@@ -1158,10 +1156,8 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                 int se = 14 - e;
                 se = se > 100 ? 100 : (se < -100 ? -100 : se);
                 const uint32_t col = (head0 + (uint32_t)h) * D + (uint32_t)dim0;   // this lane's first column
-                const size_t base = ((size_t)t32 * (cols / 16) + col / 16) * 2;
-                const uint32_t fl = ((col % 16) / 8) * 32 + n32;
-                _Float16* f_hi = a.split_frag + ((base + 0) * 64 + fl) * 8 + col % 8;
-                _Float16* f_lo = a.split_frag + ((base + 1) * 64 + fl) * 8 + col % 8;
+                _Float16* f_hi = a.split_frag + frag_piece(req, col / 8, 0, cols, frag_width(B)) + col % 8;
+                _Float16* f_lo = a.split_frag + frag_piece(req, col / 8, 1, cols, frag_width(B)) + col % 8;
                 _Float16 hi[HPK], lo[HPK];
 #pragma unroll
                 for (int kk = 0; kk < HPK; ++kk) {

@@ -35,7 +35,7 @@ __global__ __launch_bounds__(256) void q4_0_matmul_generic_kernel(
     if (lane == 0) out[(size_t)b * rows + r] = acc;
 }
 
-// ---- activations -> operand fragments (layout: q4_matmul_mfma.h).  One workgroup per request row:
+// ---- activations -> operand fragments (fragments.h).  One workgroup per request row:
 // s = 2^(14 - exponent(max|x|)).  Rows past `batch` of the last tile are not written here, and nobody reads them.
 __global__ __launch_bounds__(256) void q4_split_activations_kernel(
     const float* __restrict__ x, _Float16* __restrict__ frag, float* __restrict__ inv_scale,
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(256) void q4_split_activations_kernel(
     __shared__ float red[4];
     constexpr int MAXV = 4;  // register-resident groups of 8 columns per thread: cols <= 8192
     const uint32_t n = blockIdx.x;
-    const uint32_t ksteps = cols / 16;
+    const uint32_t width = frag_width(batch);
     const uint32_t groups = cols / 8;
     const bool live = n < batch;
     const float4* xr = reinterpret_cast<const float4*>(x + (size_t)(live ? n : 0) * cols);
@@ -88,11 +88,8 @@ __global__ __launch_bounds__(256) void q4_split_activations_kernel(
             hi[i] = (_Float16)t;
             lo[i] = (_Float16)(t - (float)hi[i]);
         }
-        const uint32_t k = k8 * 8;
-        const size_t base = ((size_t)(n / 32) * ksteps + k / 16) * 2;
-        const uint32_t lane = ((k % 16) / 8) * 32 + n % 32;
-        *reinterpret_cast<q4_half8*>(frag + ((base + 0) * 64 + lane) * 8) = hi;
-        *reinterpret_cast<q4_half8*>(frag + ((base + 1) * 64 + lane) * 8) = lo;
+        *reinterpret_cast<q4_half8*>(frag + frag_piece(n, k8, 0, cols, width)) = hi;
+        *reinterpret_cast<q4_half8*>(frag + frag_piece(n, k8, 1, cols, width)) = lo;
     };
     if (in_regs) {
 #pragma unroll
@@ -140,8 +137,7 @@ __global__ __launch_bounds__(512) void q4_pairs_kernel(const Q4Args a) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t lane = threadIdx.x % 64, l16 = lane % 16, kg = lane / 16;
     const uint32_t tile = blockIdx.x, req0 = blockIdx.y * 16, live = min(16u, a.batch - req0);
-    const uint32_t x_lane = (kg / 2 * 128 + kg % 2 * 32 + min(l16, live - 1u) + req0 % 32) * 8;
-    const _Float16* xbase = a.xfrag + (size_t)(req0 / 32) * a.nblocks * 2048;
+    const uint32_t width = frag_width(a.batch), req = req0 + min(l16, live - 1u);
     q4_float4 acc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] = 0.f;
@@ -151,8 +147,8 @@ __global__ __launch_bounds__(512) void q4_pairs_kernel(const Q4Args a) {
         const _Float16 d = reinterpret_cast<const _Float16*>(a.d)[(tq * 16 + l16) * 4 + blk % 4];
         const q4_half8 n = q4_unpack(word, 0x64006400u), d8 = {d, d, d, d, d, d, d, d};
         const q4_half8 whi = d8 * n, wlo = __builtin_elementwise_fma(d8, n, -whi);
-        const q4_half8 hi = *reinterpret_cast<const q4_half8*>(xbase + (size_t)blk * 2048 + x_lane);
-        const q4_half8 lo = *reinterpret_cast<const q4_half8*>(xbase + (size_t)blk * 2048 + x_lane + 512);
+        const q4_half8 hi = *reinterpret_cast<const q4_half8*>(a.xfrag + frag_piece(req, blk * 4 + kg, 0, a.nblocks * 32, width));
+        const q4_half8 lo = *reinterpret_cast<const q4_half8*>(a.xfrag + frag_piece(req, blk * 4 + kg, 1, a.nblocks * 32, width));
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, whi, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, whi, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, wlo, acc, 0, 0, 0);

@@ -27,6 +27,7 @@
 
 #include <type_traits>
 
+#include "fragments.h"
 #include "paged_decode_kernels.h"
 #include "paged_rope_kernels.h"
 
@@ -36,11 +37,6 @@ typedef _Float16 q4_half2 __attribute__((ext_vector_type(2)));
 typedef _Float16 q4_half8 __attribute__((ext_vector_type(8)));
 typedef float q4_float4 __attribute__((ext_vector_type(4)));
 typedef float q4_float16 __attribute__((ext_vector_type(16)));
-
-// ---- activations as operand fragments, for whoever makes them.  Element (n, k) of the padded batch, x*s = hi + lo with
-// hi = fp16(x*s), lo = fp16(x*s - hi), goes to
-//   frag[((n/32 * ksteps + k/16) * 2 + part) * 64 + ((k%16)/8)*32 + n%32][k%8],  part 0 hi, 1 lo, ksteps = K / 16
-// (two 16-column steps of it are the 32 columns of a block).
 
 // ---- repacked weights: tiles of 16 rows, quads of 4 blocks (128 columns), for
 // v_mfma_f32_16x16x32_f16, whose K is one block.
@@ -52,7 +48,7 @@ typedef float q4_float16 __attribute__((ext_vector_type(16)));
 struct Q4Args {
     const uint4* q;             // repacked weights (q4_repack_kernel)
     const uint2* d;
-    const _Float16* xfrag;      // split activations, layout above
+    const _Float16* xfrag;      // split activations (fragments.h)
     const float* inv_scale;     // [batch]
     float* out;                 // [batch][rows], or the slice buffer [ksplit][batch][rows]
     uint32_t batch, rows, nblocks, nquads, quads_per_slice;
@@ -129,7 +125,7 @@ __device__ __forceinline__ float q4_half_wave_sum(float v) {
 // of request b: writes them as hi + lo fp16 fragments of a matmul with K = k_cols, scaled by the
 // block's own power of two, and the scale that undoes it (q4_split_activations_kernel's scale, per block).
 __device__ __forceinline__ void q4_emit_block(float v, uint32_t b, uint32_t col, uint32_t k_cols, _Float16* frag,
-                                              float* blk_scale) {
+                                              float* blk_scale, uint32_t width) {
     const float amax = q4_half_wave_max(fabsf(v));
     int e = 0;
     if (amax > 0.f && amax < INFINITY) (void)frexpf(amax, &e);
@@ -138,12 +134,9 @@ __device__ __forceinline__ void q4_emit_block(float v, uint32_t b, uint32_t col,
     const float tv = __builtin_ldexpf(v, se);
     const _Float16 hi = (_Float16)tv;
     const _Float16 lo = (_Float16)(tv - (float)hi);
-    const uint32_t t = b / 32, c = b % 32;
-    const size_t base = ((size_t)t * (k_cols / 16) + col / 16) * 2;
-    const uint32_t fl = ((col % 16) / 8) * 32 + c;
-    frag[((base + 0) * 64 + fl) * 8 + col % 8] = hi;
-    frag[((base + 1) * 64 + fl) * 8 + col % 8] = lo;
-    if (col % 32 == 0) blk_scale[((size_t)t * (k_cols / 32) + col / 32) * 32 + c] = __builtin_ldexpf(1.0f, -se);
+    frag[frag_piece(b, col / 8, 0, k_cols, width) + col % 8] = hi;
+    frag[frag_piece(b, col / 8, 1, k_cols, width) + col % 8] = lo;
+    if (col % 32 == 0) blk_scale[((size_t)(b / 32) * (k_cols / 32) + col / 32) * 32 + b % 32] = __builtin_ldexpf(1.0f, -se);
 }
 
 // The split + RoPE + cast (+ paged write) of one element of a request's fused qkv row, by the
@@ -265,9 +258,10 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // longest stream of a workgroup that had them all.
 //
 // Measured, kernel times in us, before (32 x 32 products, one workgroup per 32 rows, branches or clamps around the loads of
-// a wave's last blocks) -> now.  One request of the 1 B shape: qkv (2560 x 2048) 7.0 -> 5.1, out-projection with the
-// residual add 8.4 -> 5.0, gate/up with SiLU (11264 x 2048) 11.2 -> 7.4, down (2048 x 5632) 8.1 and 5.0 for the sum of
-// its K slices -> 8.7 with the residual add and no slices; a step of 22 layers 1 145 -> 853.  32 requests: qkv 7.5 -> 6.9,
+// a wave's last blocks) -> now.  One request of the 1 B shape: qkv (2560 x 2048) 7.0 -> 4.5, out-projection with the
+// residual add 8.4 -> 4.6, gate/up with SiLU (11264 x 2048) 11.2 -> 7.0, down (2048 x 5632) 8.1 and 5.0 for the sum of
+// its K slices -> 8 with the residual add and no slices; a step of 22 layers 1 145 -> 801 (845 with the
+// fragments of 32 requests as they are for larger batches).  32 requests: qkv 7.5 -> 6.9,
 // gate/up 13.3 -> 14.0, a step 1 330 -> 1 207.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
 // a layer 141 -> 114.  2-norm error against float64: 0.95e-7 .. 1.15e-7, before 1.03e-7 .. 1.34e-7.
 template <int NI, int RT, int WAVES, bool BS, int FORM>
@@ -275,7 +269,14 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
     static_assert(FORM != kQ4Silu || RT == 4, "SiLU epilogue: 32 rows of gate and 32 of up");
     static_assert(FORM != kQ4Add || RT == 2, "residual add: 32 rows, one block of the next matmul's K");
-    constexpr int XD = RT == 4 ? 2 : 4;              // blocks of activations in flight
+    // Up to 8 requests: a quad's activations come 1 KB per load, without the places of requests that do not
+    // exist, and each lane's operand from LDS.  (16-byte loads of 64 lanes cost 16 clocks of the return path, however
+    // many of them ask for the same bytes or for none.)
+    constexpr bool PACKED = NI < 4;
+    constexpr uint32_t WIDTH = PACKED ? 4 * NI : 32;
+    constexpr int XQ = PACKED ? 2 * NI : 1;          // loads per quad
+    // blocks of activations in registers: as far as 128 registers per wave go
+    constexpr int XD = PACKED ? (RT == 4 ? 1 : 2) : RT == 4 ? 2 : 4;
     constexpr int QR = 4 * NI;                       // requests of the workgroup
     constexpr int TILE_PITCH = NI * 64 + 16;         // floats per tile in LDS (16: bank spread)
     __shared__ float red[WAVES * RT * TILE_PITCH];
@@ -283,6 +284,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     // every lane's own scales per block would take as long as one of the block's two fragments: what bounds these
     // kernels next to the vector pipe is the 64 bytes a clock that a CU's loads return.)
     __shared__ __attribute__((aligned(16))) float scales[BS ? WAVES : 1][64];
+    __shared__ q4_u32x4 packed[PACKED ? WAVES : 1][XQ * 64];
     __shared__ float rms_scale[BS ? QR : 1];         // BS with ssq_in: every request's RMSNorm factor
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t lane = threadIdx.x % 64, l16 = lane % 16, kg = lane / 16;
@@ -357,6 +359,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         q4_u32x4 q[RT];
         q4_u32x2 d[RT];
         float sc;   // BS: the scale of request l16 in block kg of the quad
+        q4_u32x4 x[XQ];   // PACKED: the quad's activations
     };
     struct BlockX {
         q4_half8 hi, lo;
@@ -372,11 +375,11 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         q_desc[r] = q4_buffer(a.q + tile * 64, end * 1024);
         d_desc[r] = q4_buffer(a.d + tile * 16, end * 128);
     }
-    const __amdgpu_buffer_rsrc_t x_desc = q4_buffer(a.xfrag + (size_t)(req0 / 32) * a.nblocks * 2048, a.nblocks * 4096);
+    const __amdgpu_buffer_rsrc_t x_desc = q4_buffer(a.xfrag + (size_t)(req0 / 32) * a.nblocks * 2048, a.nblocks * WIDTH * 128);
     const __amdgpu_buffer_rsrc_t s_desc = q4_buffer(BS ? a.blk_scale + (size_t)(req0 / 32) * a.nblocks * 32 : nullptr, a.nblocks * 128);
-    // (request of this lane's row of the A operand; rows without one fetch another's again)
+    // (request of this lane's row of the A operand; rows without one repeat another's)
     const uint32_t xreq = min(l16 / 4 * NI + min(l16 % 4, (uint32_t)NI - 1u), live - 1u) + req0 % 32;
-    const uint32_t x_lane = (kg / 2 * 128 + kg % 2 * 32 + xreq) * 16;   // (fragment layout: two 16-column steps)
+    const uint32_t x_lane = (kg / 2 * 4 * WIDTH + kg % 2 * WIDTH + xreq) * 16;   // (two 16-column steps, hi and lo of each)
     const uint32_t s_lane = kg * 128 + (req0 % 32 + l16) * 4;
     auto load_w = [&](uint32_t quad, QuadW& k) __attribute__((always_inline)) {
         constexpr int NT = 2;   // (non-temporal: a weight is read once per launch and need not stay in the L2)
@@ -386,11 +389,23 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
             k.q[r] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_desc[r], quad * 1024 + lane * 16, 0, NT));
             k.d[r] = __builtin_bit_cast(q4_u32x2, __builtin_amdgcn_raw_buffer_load_b64(d_desc[r], quad * 128 + l16 * 8, 0, NT));
         }
+        if constexpr (PACKED) {
+#pragma unroll
+            for (int i = 0; i < XQ; ++i)
+                k.x[i] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_desc, quad * (XQ * 1024) + i * 1024 + lane * 16, 0, 0));
+        }
         asm volatile("" ::: "memory");
     };
     auto load_x = [&](uint32_t blk, BlockX& k) __attribute__((always_inline)) {
+        if constexpr (PACKED) return;
         k.hi = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc, blk * 4096 + x_lane, 0, 0));
         k.lo = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc, blk * 4096 + x_lane + 1024, 0, 0));
+        asm volatile("" ::: "memory");
+    };
+    auto read_x = [&](int j, BlockX& k) __attribute__((always_inline)) {
+        const uint32_t piece = j * 8 * WIDTH + x_lane / 16;
+        k.hi = __builtin_bit_cast(q4_half8, packed[wave][piece]);
+        k.lo = __builtin_bit_cast(q4_half8, packed[wave][piece + 2 * WIDTH]);
         asm volatile("" ::: "memory");
     };
     const uint32_t ones = q4_ones();
@@ -423,6 +438,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
 #pragma unroll
             for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(acc[r][i]));
         }
+        if constexpr (PACKED && RT == 4 && (WAVES == 16 || !BS)) __builtin_amdgcn_sched_barrier(0);   // (for the same reason)
     };
     // A wave's quads are first, first + WAVES, ...  While one is multiplied the next one's weights are on the way, and
     // activations XD blocks ahead.  The last one is a copy of the code that fetches nothing: a load costs its share
@@ -433,8 +449,15 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     BlockX x[XD];
     auto turn = [&](uint32_t quad, auto more) __attribute__((always_inline)) {
         if constexpr (BS) scales[wave][lane] = w.sc;   // (a wave's own: LDS operations of a wave are in order)
+        if constexpr (PACKED) {
+#pragma unroll
+            for (int i = 0; i < XQ; ++i) packed[wave][i * 64 + lane] = w.x[i];
+            if constexpr (XD > 1) read_x(0, x[0]);
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+            if constexpr (PACKED)
+                if (j + XD - 1 < 4) read_x(j + XD - 1, x[(j + XD - 1) % XD]);
             multiply(w, j, x[j % XD]);
             if (j + XD < 4) load_x(quad * 4 + j + XD, x[j % XD]);
             else if constexpr (decltype(more)::value) load_x((quad + WAVES) * 4 + j + XD - 4, x[j % XD]);
@@ -511,7 +534,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         a.gate[(size_t)b * a.ffn_inner + col] = gv;
         a.up[(size_t)b * a.ffn_inner + col] = uv;
         a.silu_out[(size_t)b * a.ffn_inner + col] = prod;
-        if (a.split_frag) q4_emit_block(prod, b, col, a.ffn_inner, a.split_frag, a.split_blk_scale);
+        if (a.split_frag) q4_emit_block(prod, b, col, a.ffn_inner, a.split_frag, a.split_blk_scale, WIDTH);
         return;
     }
     float* out = a.out + (size_t)slice * a.batch * a.rows;
@@ -529,7 +552,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
             a.add_out[(size_t)bp * a.rows + col] = hv;
             const float ssq = q4_half_wave_sum(hv * hv);
             if (row == 0) a.ssq_out[(size_t)bp * (a.rows / 32) + row_group] = ssq;
-            q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale);
+            q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale, WIDTH);
         }
     }
 }

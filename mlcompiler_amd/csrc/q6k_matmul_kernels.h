@@ -67,7 +67,7 @@ struct Q6KArgs {
     const uint2* qa;
     const uint32_t* sc;
     const _Float16* d;
-    const _Float16* xfrag;   // split activations, layout of q4_split_activations_kernel
+    const _Float16* xfrag;   // split activations (fragments.h)
     const float* inv_scale;  // [batch]
     float* out;              // [batch][rows]
     uint32_t batch, rows, nblocks;
@@ -87,9 +87,10 @@ __global__ __launch_bounds__(512) void q6_k_matmul_mfma_kernel(const Q6KArgs a) 
     const uint32_t groups = a.nblocks * 4;
     const uint32_t ksteps = a.nblocks * 16;
     // (lanes past the last request fetch that one's fragments again; their results are dropped)
+    const uint32_t width = frag_width(a.batch);
     uint32_t lane_x[NBT];
 #pragma unroll
-    for (int t = 0; t < NBT; ++t) lane_x[t] = half * 32 + min(l32, a.batch - 1u - t * 32);
+    for (int t = 0; t < NBT; ++t) lane_x[t] = half * width + min(l32, a.batch - 1u - t * 32);
 
     q4_float16 acc[RT][NBT];
 #pragma unroll
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(512) void q6_k_matmul_mfma_kernel(const Q6KArgs a) 
 #pragma unroll
                 for (int pt = 0; pt < 2; ++pt)
                     k.x[t][q][pt] = *reinterpret_cast<const q4_half8*>(
-                        a.xfrag + ((((size_t)t * ksteps + kstep) * 2 + pt) * 64 + lane_x[t]) * 8);
+                        a.xfrag + ((((size_t)t * ksteps + kstep) * 2 + pt) * 2 * width + lane_x[t]) * 8);
             }
     };
     auto multiply = [&](const Group& k) __attribute__((always_inline)) {

@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fragments.h"
+
 namespace mlc_hip {
 
 // MSL rms_norm_kernel_v2_batched (compiler/runtime/metal_runtime.mm:166-208), CPU rmsNorm
@@ -252,7 +254,7 @@ __global__ __launch_bounds__(kRowThreads) void row_program_kernel(const RowProgr
     se = se > 100 ? 100 : (se < -100 ? -100 : se);
     const float s = ldexpf(1.0f, se);
     if (tid == 0 && live) p.inv_scale[row] = ldexpf(1.0f, -se);
-    const uint32_t ksteps = len / 16;
+    const uint32_t width = frag_width(p.batch);
 #pragma unroll
     for (int j = 0; j < NG; ++j) {
         const uint32_t k = (j * kRowThreads + tid) * 8;
@@ -264,10 +266,8 @@ __global__ __launch_bounds__(kRowThreads) void row_program_kernel(const RowProgr
             hi[e] = (_Float16)t;
             lo[e] = (_Float16)(t - (float)hi[e]);
         }
-        const size_t base = ((size_t)(row / 32) * ksteps + k / 16) * 2;
-        const uint32_t lane = ((k % 16) / 8) * 32 + row % 32;
-        *reinterpret_cast<row_half8*>(p.frag + ((base + 0) * 64 + lane) * 8) = hi;
-        *reinterpret_cast<row_half8*>(p.frag + ((base + 1) * 64 + lane) * 8) = lo;
+        *reinterpret_cast<row_half8*>(p.frag + frag_piece(row, k / 8, 0, len, width)) = hi;
+        *reinterpret_cast<row_half8*>(p.frag + frag_piece(row, k / 8, 1, len, width)) = lo;
     }
 }
 

@@ -5,8 +5,11 @@ carries the residual add of the next (its two norms have weights of their own)."
 import numpy as np
 import pytest
 
+import test_decode_split_fusion_gpu as split
+import test_matmul_silu_fusion_gpu as silu
 import test_q4_matmul_gpu as q4
 from oracle import paged_oracle as po
+from paged_cases import make_case
 from test_matmul_norm_fusion_gpu import EPS, _pool, _read
 from test_matmul_tokens_gpu import check
 
@@ -59,3 +62,22 @@ def test_a_chain_of_norms(exe, batch):
         want = po.rms_norm_batched(got[f"h{i}"], gamma[i], EPS, batch, n)
         # (as in test_matmul_norm_fusion_gpu.py: a sum of n squares and one rounding per factor)
         assert (np.abs(got[f"n{i}"] - want) <= 2e-6 * np.abs(want).max(axis=1, keepdims=True)).all()
+
+
+@pytest.mark.parametrize("batch", [1, 3, 4, 5, 7, 8, 9])
+def test_few_requests_behind_every_producer(exe, batch):
+    """The fragments of up to 4, up to 8 and more requests lie differently: written by the decode attention (with a
+    request without tokens) and by the SiLU epilogue, behind a matmul whose input the split kernel wrote."""
+    rng = np.random.default_rng(batch)
+    lens = rng.integers(1, 300, batch)
+    lens[batch // 2] = 0
+    case = make_case(f"few.{batch}", batch, 16, 2, 64, 64, lens, seed=batch)
+    w = po.quantize_q4_0((rng.standard_normal((192, 1024)) * 0.05).astype(np.float32))
+    o, out, _, n, _ = split._run(exe, case, w, 192, "proj", fuse=1)
+    assert n == 1
+    check(out, q4.dequant(w, 1024), o.reshape(batch, 1024))
+    c = silu.Case(batch, 160, 4128, 192, seed=batch)
+    got, n = silu._run(exe, c, "down", fuse=1)
+    assert n == (1, 1)
+    check(got["gate_up"], q4.dequant(c.w_gu, 160), c.x)
+    check(got["down"], q4.dequant(c.w_down, 4128), got["prod"])
