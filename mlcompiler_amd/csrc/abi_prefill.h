@@ -77,11 +77,13 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
     size_t max_tiles = 0;
     for (size_t r = 0; r < batch; ++r)
         max_tiles = std::max(max_tiles, (std::min<size_t>(seq_lens[r], q_start[r] + chunk) + kPfKeys - 1) / kPfKeys);
-    constexpr size_t kPartBytes = 32u << 20;   // (one size for good: a buffer that grows ends captured passes)
-    uint32_t splits = prefill_splits(batch, chunk, num_heads, kv_heads, head_dim, max_tiles, g.n_cu, kPartBytes);
-    a.part_o = splits > 1 ? static_cast<float*>(cached_buffer("prefill_parts", kPartBytes)) : nullptr;
+    // (one size for good: a buffer that grows ends captured passes.  A workgroup of 256 rows per CU fits, 34 MB)
+    constexpr size_t kPartBytes = 36u << 20;
+    const size_t wgs = prefill_wgs(batch, chunk, num_heads, kv_heads);
+    uint32_t splits = prefill_splits(wgs, head_dim, max_tiles, g.n_cu, kPartBytes);
+    a.part_o = splits > 1 ? static_cast<float4*>(cached_buffer("prefill_parts", kPartBytes)) : nullptr;
     if (!a.part_o) splits = 1;
-    a.part_ml = reinterpret_cast<float2*>(a.part_o + (splits > 1 ? splits * batch * chunk * num_heads * head_dim : 0));
+    a.part_ml = reinterpret_cast<float2*>(a.part_o + (splits > 1 ? splits * wgs * kPfWaves * kPfRows * head_dim / 4 : 0));
     launch_prefill(a, head_dim, (int)g.opt_prefill_stages, g.opt_prefill_rows64 != 0, splits, g.stream);
     return finish(sync);
 }

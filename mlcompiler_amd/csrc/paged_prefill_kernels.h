@@ -34,13 +34,15 @@
 
 #include <type_traits>
 
+#include "store_through.h"
+
 namespace mlc_hip {
 
 static constexpr size_t kPrefillEmbWords = 960;   // words of tables that travel inside the kernel arguments
 
 struct PrefillArgs {
-    float* part_o;       // keys split over workgroups: the parts' sums [part][row][head_dim] and their
-    float2* part_ml;     // (reference, sum of weights), row = (request, chunk row, query head)
+    float4* part_o;      // keys split over workgroups: the parts' sums [part][wave of the grid][head_dim / 8][lane], as the
+    float2* part_ml;     // lanes hold them, and their (reference, sum of weights) [part][wave of the grid][32 rows]
     const _Float16* q;
     const _Float16* k_pages;
     const _Float16* v_pages;
@@ -373,14 +375,18 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
     // ---- write O: lane owns row my_row; register i of block mb is dim mb*32 + (i/4)*8 + half*4 + i%4
     if (row_ok) {
         l_run += __shfl_xor(l_run, 32);
-        float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
-        float* orow = a.o + out_row;
         if (gridDim.y > 1) {   // a part's sums, on the part's own reference, for prefill_combine_kernel
-            const size_t rows = (size_t)a.batch * a.chunk * a.num_heads, row = blockIdx.y * rows + out_row / D;
-            inv = 1.0f;
-            orow = a.part_o + row * D;
-            if (half == 0) a.part_ml[row] = make_float2(m_run, l_run);
+            const uint32_t part_wave = (blockIdx.y * gridDim.x + wg) * kPfWaves + wave;
+            if (half == 0) store_through(&a.part_ml[part_wave * kPfRows + l32], make_float2(m_run, l_run));
+#pragma unroll
+            for (int i = 0; i < MB * 4; ++i)
+                store_through16(a.part_o, ((part_wave * (MB * 4) + i) * 64 + lane) * 16,
+                                make_float4(oacc[i / 4][i % 4 * 4 + 0], oacc[i / 4][i % 4 * 4 + 1],
+                                            oacc[i / 4][i % 4 * 4 + 2], oacc[i / 4][i % 4 * 4 + 3]));
+            return;
         }
+        const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
+        float* orow = a.o + out_row;
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
@@ -394,26 +400,62 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
 }
 
 // Adds the parts of a prefill whose keys were split over workgroups: o = sum_s 2^(m_s - m) O_s / sum_s
-// 2^(m_s - m) l_s.  One thread per four dims of a row; rows without visible keys become zero.
+// 2^(m_s - m) l_s.  One thread per four dims of a row, workgroup = a 32 x 32 block of a wave of the grid that made
+// the parts (`waves` of them); rows without visible keys become zero.
+// What it takes is the way to memory and back, so eight parts' loads go out together, in whole KB, and before anything
+// else (seven parts of 3 x 77 rows at 32 heads of 64, 16 MB: 5.6 -> 3.7 us, of which 2 are the launch's own).
 template <int D>
-__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs a, uint32_t splits) {
-    const size_t rows = (size_t)a.batch * a.chunk * a.num_heads;
-    const size_t row = ((size_t)blockIdx.x * 256 + threadIdx.x) / (D / 4);
-    const uint32_t d = threadIdx.x % (D / 4) * 4;
-    if (row >= rows) return;
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs a, uint32_t splits, uint32_t waves) {
+    constexpr int AT_ONCE = 8, MB = D / 32;
+    const uint32_t w = blockIdx.x / MB, block = blockIdx.x % MB * 4 + threadIdx.x / 64, lane = threadIdx.x % 64;
+    float2 ml[AT_ONCE];
+    float4 v[AT_ONCE];
+    auto load_ml = [&](uint32_t s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i)
+            ml[i] = s0 + i < splits ? a.part_ml[((s0 + i) * waves + w) * kPfRows + lane % 32] : make_float2(-1.0e30f, 0.f);
+    };
+    auto load_v = [&](uint32_t s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i)
+            if (s0 + i < splits) v[i] = a.part_o[(((s0 + i) * waves + w) * (MB * 4) + block) * 64 + lane];
+    };
+    load_ml(0);
+    load_v(0);
+    asm volatile("" ::: "memory");   // (the loads first: the divisions are a hundred instructions)
+    const uint32_t G = a.num_heads / a.kv_heads, wave = w % kPfWaves, wg = w / kPfWaves;
+    const uint32_t kvh = wg / a.row_blocks % a.kv_heads, req = wg / (a.row_blocks * a.kv_heads);
+    const uint32_t row = (wg % a.row_blocks * (kPfWaves / G) + wave / G) * kPfRows + lane % 32;
+    if (row >= a.chunk) return;
     float m = -1.0e30f;
-    for (uint32_t s = 0; s < splits; ++s) m = fmaxf(m, a.part_ml[s * rows + row].x);
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i) m = fmaxf(m, ml[i].x);
+    if (splits > AT_ONCE) {
+        for (uint32_t s0 = AT_ONCE; s0 < splits; s0 += AT_ONCE) {
+            load_ml(s0);
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i) m = fmaxf(m, ml[i].x);
+        }
+        load_ml(0);
+    }
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
     float l = 0.f;
-    for (uint32_t s = 0; s < splits; ++s) {
-        const float2 ml = a.part_ml[s * rows + row];
-        const float w = ml.y > 0.f ? __builtin_amdgcn_exp2f(ml.x - m) : 0.f;
-        const float4 v = *reinterpret_cast<const float4*>(a.part_o + (s * rows + row) * D + d);
-        l = fmaf(w, ml.y, l);
-        o.x = fmaf(w, v.x, o.x); o.y = fmaf(w, v.y, o.y); o.z = fmaf(w, v.z, o.z); o.w = fmaf(w, v.w, o.w);
+    for (uint32_t s0 = 0;;) {
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) {
+            if (s0 + i >= splits) break;
+            const float f = ml[i].y > 0.f ? __builtin_amdgcn_exp2f(ml[i].x - m) : 0.f;
+            l = fmaf(f, ml[i].y, l);
+            o.x = fmaf(f, v[i].x, o.x); o.y = fmaf(f, v[i].y, o.y); o.z = fmaf(f, v[i].z, o.z); o.w = fmaf(f, v[i].w, o.w);
+        }
+        s0 += AT_ONCE;
+        if (s0 >= splits) break;
+        load_ml(s0);
+        load_v(s0);
     }
     const float inv = l > 0.f ? 1.0f / l : 0.f;
-    *reinterpret_cast<float4*>(a.o + row * D + d) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+    float* orow = a.o + (((size_t)req * a.chunk + row) * a.num_heads + kvh * G + wave % G) * D;
+    *reinterpret_cast<float4*>(orow + block * 8 + lane / 32 * 4) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
 }
 
 // ---- the same computation with 64 chunk rows per wave (GQA ratios 1, 2 and 4).  One workgroup
@@ -994,8 +1036,8 @@ inline void launch_prefill_dg(PrefillArgs a, int stages, bool rows64, uint32_t s
         default: hipLaunchKernelGGL((paged_prefill_mfma_kernel<D, G, 6>), grid, block, 0, stream, a); break;
     }
     if (splits > 1) {
-        const size_t threads = (size_t)a.batch * a.chunk * a.num_heads * (D / 4);
-        hipLaunchKernelGGL((prefill_combine_kernel<D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a, splits);
+        const uint32_t waves = grid.x * kPfWaves;
+        hipLaunchKernelGGL((prefill_combine_kernel<D>), dim3(waves * (D / 32)), dim3(256), 0, stream, a, splits, waves);
     }
 }
 
@@ -1009,20 +1051,31 @@ inline void launch_prefill_d(const PrefillArgs& a, int stages, bool rows64, uint
     }
 }
 
-// A prefill of few rows leaves most of the chip idle while each workgroup walks all of the keys, about 1 us
-// per 32-key tile; its keys are then cut into parts of at least 4 tiles, as many as there are CUs for.
-// max_tiles: key tiles of the longest row block.  Whole calls, before -> after: 3 x 77 rows behind up to 900 keys
-// (36 workgroups) 40 -> 32 us, 256 rows behind 3 840 at 32 / 8 heads of 128 (32) 162 -> 57, 64 rows behind
-// 8 000 218 -> 55, 700 rows from scratch at 16 / 4 heads of 64 41 -> 32; two parts (4 x 256 rows behind up to
-// 2 000, 128 workgroups) still 87 -> 76.  Under 16 tiles the second launch (4 us) costs what the parts save.
-inline uint32_t prefill_splits(size_t batch, size_t chunk, size_t num_heads, size_t kv_heads, size_t head_dim,
-                               size_t max_tiles, size_t n_cu, size_t part_bytes) {
+// A prefill of few rows leaves most of the chip idle while each workgroup walks all of the keys, 0.77 us (head_dim
+// 64) or 0.97 us (128) per 32-key tile; its keys are then cut into parts, at most as many as there are CUs for,
+// of at least two tiles.  Writing the parts and adding them up takes 2 us and 0.36 us per MB of them (measured:
+// 1.4 to 2.9 us where they are 1 to 4 MB, 3.2 to 4.5 for 5 to 8 MB, 7.7 for 15 and 16): the number of parts is the one
+// with the least sum, and one where that saves less than 1 us.
+// max_tiles: key tiles of the longest row block.  Whole calls in us, one part (or, in brackets, the parts of a
+// rule that asked for 16 tiles and four per part, laid out by rows) -> now: 32 rows at 32 / 4 heads of 64 behind 224,
+// 320, 416 keys 23.0, 25.2, 27.5 -> 20.8, 21.1, 21.0; of 128 behind 416 33.3 -> 23.3, four requests of that
+// 33.9 -> 27.6; 3 x 77 rows behind up to 900 keys (36 workgroups) 39.9 (32.1) -> 26.4, 256 rows behind 3 840 at 32 / 8
+// heads of 128 (32) 117 (50.6) -> 46.4, 64 rows behind 8 000 (53) -> 40, 700 rows from scratch at 16 / 4 heads
+// of 64 (31.4) -> 25.6; two parts (4 x 256 rows behind up to 2 000, 128 workgroups) 77 -> 67.  Where both are equal:
+// 2 x 256 rows behind 400 at 32 / 8 heads of 128, 39.8 with one part, 39.3 with three (37.8).
+inline size_t prefill_wgs(size_t batch, size_t chunk, size_t num_heads, size_t kv_heads) {
     const size_t rows_per_wg = kPfRows * kPfWaves / (num_heads / kv_heads);
-    const size_t wgs = (chunk + rows_per_wg - 1) / rows_per_wg * kv_heads * batch;
-    if (max_tiles < 16) return 1;
-    const size_t one = batch * chunk * num_heads * (head_dim + 2) * 4;
-    const size_t splits = std::min({n_cu / wgs, max_tiles / 4, part_bytes / one, (size_t)64});
-    return splits < 2 ? 1u : (uint32_t)splits;
+    return (chunk + rows_per_wg - 1) / rows_per_wg * kv_heads * batch;
+}
+inline uint32_t prefill_splits(size_t wgs, size_t head_dim, size_t max_tiles, size_t n_cu, size_t part_bytes) {
+    const size_t one = wgs * kPfWaves * kPfRows * (head_dim + 2) * 4, tile_ns = head_dim == 64 ? 770 : 970;
+    const size_t most = std::min({n_cu / wgs, max_tiles / 2, part_bytes / one, (size_t)64});
+    size_t best = 1, best_ns = max_tiles * tile_ns - std::min<size_t>(max_tiles * tile_ns, 1000);
+    for (size_t p = 2; p <= most; ++p) {
+        const size_t ns = (max_tiles + p - 1) / p * tile_ns + 2000 + p * one / 2800;
+        if (ns < best_ns) best = p, best_ns = ns;
+    }
+    return (uint32_t)best;
 }
 
 // stages: LDS pipeline depth (2, 4, 6 or 8; anything else selects 6).  rows64: 64 chunk rows per
