@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "fragments.h"
+#include "store_through.h"
 #include "paged_decode_kernels.h"
 #include "paged_rope_kernels.h"
 
@@ -134,9 +135,9 @@ __device__ __forceinline__ void q4_emit_block(float v, uint32_t b, uint32_t col,
     const float tv = __builtin_ldexpf(v, se);
     const _Float16 hi = (_Float16)tv;
     const _Float16 lo = (_Float16)(tv - (float)hi);
-    frag[frag_piece(b, col / 8, 0, k_cols, width) + col % 8] = hi;
-    frag[frag_piece(b, col / 8, 1, k_cols, width) + col % 8] = lo;
-    if (col % 32 == 0) blk_scale[((size_t)(b / 32) * (k_cols / 32) + col / 32) * 32 + b % 32] = __builtin_ldexpf(1.0f, -se);
+    store_through(&frag[frag_piece(b, col / 8, 0, k_cols, width) + col % 8], hi);
+    store_through(&frag[frag_piece(b, col / 8, 1, k_cols, width) + col % 8], lo);
+    if (col % 32 == 0) store_through(&blk_scale[((size_t)(b / 32) * (k_cols / 32) + col / 32) * 32 + b % 32], __builtin_ldexpf(1.0f, -se));
 }
 
 // The split + RoPE + cast (+ paged write) of one element of a request's fused qkv row, by the
@@ -181,17 +182,17 @@ __device__ __forceinline__ void q4_rope_epilogue(const RopeArgs& p, const Q4Rope
     if ((is_q || is_k) && (local & ~1u) % p.head_dim < p.rotary_dim) y = rope_rotate(x, f.c, f.s);
     const float mine = odd ? y.y : y.x;
     if (is_q) {
-        p.q[(size_t)req * p.q_rows + local] = mine;
+        store_through(&p.q[(size_t)req * p.q_rows + local], mine);
         return;
     }
     float* f32 = is_k ? p.k : p.v;
     const uint32_t rows = is_k ? p.k_rows : p.v_rows;
-    if (f32) f32[(size_t)req * rows + local] = mine;
+    if (f32) store_through(&f32[(size_t)req * rows + local], mine);
     const _Float16 h = (_Float16)mine;
     _Float16* f16 = is_k ? p.k_f16 : p.v_f16;
-    if (f16) f16[(size_t)req * rows + local] = h;
+    if (f16) store_through(&f16[(size_t)req * rows + local], h);
     _Float16* pool = is_k ? p.k_pages : p.v_pages;
-    if (pool) pool[(size_t)f.page_row * rows + local] = h;
+    if (pool) store_through(&pool[(size_t)f.page_row * rows + local], h);
 }
 
 // 8- and 16-byte non-temporal loads (data that is read once and need not displace anything in the L2).
@@ -508,7 +509,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
             for (int m = 0; m < RMS_N; ++m) {
                 const uint32_t el = rms_el + m * WAVES * 64;
                 if (el < live * a.rms_len)
-                    a.rms_out[(size_t)req0 * a.rms_len + el] = rms_h[m] * rms_scale[el / a.rms_len] * rms_gamma[m];
+                    store_through(&a.rms_out[(size_t)req0 * a.rms_len + el], rms_h[m] * rms_scale[el / a.rms_len] * rms_gamma[m]);
             }
         }
     }
@@ -529,11 +530,11 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         // the 32 lanes of a half wave hold one request's 32 columns, one block of the consuming matmul's K
         const float gv = sum_of(row, q, inv_pre[0]), uv = sum_of(32 + row, q, inv_pre[0]);
         const float prod = q4_silu_times(gv, uv);
-        a.out[(size_t)b * a.rows + col] = gv;
-        a.out[(size_t)b * a.rows + a.ffn_inner + col] = uv;
-        a.gate[(size_t)b * a.ffn_inner + col] = gv;
-        a.up[(size_t)b * a.ffn_inner + col] = uv;
-        a.silu_out[(size_t)b * a.ffn_inner + col] = prod;
+        store_through(&a.out[(size_t)b * a.rows + col], gv);
+        store_through(&a.out[(size_t)b * a.rows + a.ffn_inner + col], uv);
+        store_through(&a.gate[(size_t)b * a.ffn_inner + col], gv);
+        store_through(&a.up[(size_t)b * a.ffn_inner + col], uv);
+        store_through(&a.silu_out[(size_t)b * a.ffn_inner + col], prod);
         if (a.split_frag) q4_emit_block(prod, b, col, a.ffn_inner, a.split_frag, a.split_blk_scale, WIDTH);
         return;
     }
@@ -543,15 +544,15 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         const uint32_t qp = q + p * PER_PASS, bp = b + p * PER_PASS;
         if (qp >= live) break;
         const float val = sum_of(row, qp, inv_pre[p]);
-        out[(size_t)bp * a.rows + col] = val;
+        store_through(&out[(size_t)bp * a.rows + col], val);
         if constexpr (FORM == kQ4Rope) q4_rope_epilogue(a.rope, rope_pre, bp, col, val);   // (the lanes of a pair share b)
         if constexpr (FORM == kQ4Add) {
             // residual add, this request's sum of squares over the 32 columns, and h * gamma as the next
             // matmul's fragments
             const float hv = val + resid_pre;
-            a.add_out[(size_t)bp * a.rows + col] = hv;
+            store_through(&a.add_out[(size_t)bp * a.rows + col], hv);
             const float ssq = q4_half_wave_sum(hv * hv);
-            if (row == 0) a.ssq_out[(size_t)bp * (a.rows / 32) + row_group] = ssq;
+            if (row == 0) store_through(&a.ssq_out[(size_t)bp * (a.rows / 32) + row_group], ssq);
             q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale, WIDTH);
         }
     }

@@ -4,6 +4,7 @@
 // to see them.  Nothing else runs meanwhile.  Stores of device scope write through as they are made and leave nothing
 // to write back.  That pays where a short kernel stores everything at its end, whole lines at a time: a prefill's
 // partial sums (16 MB in a kernel of 16 us) 28.6 -> 26.9 us a call, 4 to 8 % of a call in the ranges of that path.
+// The outputs of the Q4_0 matmuls of 32 requests: a step of 22 layers 1 217 -> 1 196 us, of one request 796 -> 794.
 // It does not where a kernel stores all along and the L2 does its writing behind other work: the output of a long
 // prefill 143 -> 154 us, of an 11264 x 2048 matmul over 512 tokens 80.6 -> 86.6; decode attention and row programs,
 // whose outputs are small, did not change.
