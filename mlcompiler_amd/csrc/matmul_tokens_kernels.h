@@ -40,14 +40,18 @@ namespace mlc_hip {
 
 // What q4_split_activations_kernel does (q4_matmul_kernels.h), four tokens per workgroup: neighbouring
 // lanes hold neighbouring tokens, so that a store of 16 bytes per lane fills 64-byte pieces of the
-// fragments instead of leaving every piece to another workgroup.
-static __global__ __launch_bounds__(256) void tokens_split_kernel(const float* __restrict__ x, _Float16* __restrict__ frag,
+// fragments instead of leaving every piece to another workgroup.  256 threads up to 4096 columns (64 per token), else
+// 1024: there are few workgroups, and rows that do not fit the registers are read twice (whole calls of 2048 x 5632 at
+// 512 tokens 62.5 -> 57.6 us, 4096 x 14336 at 200 tokens 106 -> 101; at 2048 columns both take 7 us).
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void tokens_split_kernel(const float* __restrict__ x, _Float16* __restrict__ frag,
                                                            float* __restrict__ inv_scale, uint32_t tokens, uint32_t cols) {
-    constexpr int MAXV = 8;   // groups of 8 columns a thread keeps in registers: cols <= 4096
-    __shared__ float red[4][4];
+    constexpr int PER = THREADS / 4, WAVES = THREADS / 64;   // threads per token, waves
+    constexpr int MAXV = THREADS == 256 ? 8 : 4;   // groups of 8 columns a thread keeps in registers: cols <= 4096 / 8192
+    __shared__ float red[WAVES][4];
     const uint32_t n4 = threadIdx.x % 4, n = blockIdx.x * 4 + n4, g0 = threadIdx.x / 4;
     const uint32_t groups = cols / 8, ksteps = cols / 16;
-    const bool live = n < tokens, in_regs = groups <= 64 * MAXV;
+    const bool live = n < tokens, in_regs = groups <= PER * MAXV;
     const float4* xr = reinterpret_cast<const float4*>(x + (size_t)(live ? n : 0) * cols);
     auto max8 = [](float m, const float4& a, const float4& b) __attribute__((always_inline)) {
         m = fmaxf(m, fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(a.w))));
@@ -58,20 +62,22 @@ static __global__ __launch_bounds__(256) void tokens_split_kernel(const float* _
     if (in_regs) {
 #pragma unroll
         for (int j = 0; j < MAXV; ++j) {
-            const uint32_t k8 = j * 64 + g0;
+            const uint32_t k8 = j * PER + g0;
             v[j][0] = v[j][1] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (live && k8 < groups) { v[j][0] = xr[k8 * 2]; v[j][1] = xr[k8 * 2 + 1]; }
         }
 #pragma unroll
         for (int j = 0; j < MAXV; ++j) amax = max8(amax, v[j][0], v[j][1]);
     } else if (live) {
-        for (uint32_t k8 = g0; k8 < groups; k8 += 64) amax = max8(amax, xr[k8 * 2], xr[k8 * 2 + 1]);
+        for (uint32_t k8 = g0; k8 < groups; k8 += PER) amax = max8(amax, xr[k8 * 2], xr[k8 * 2 + 1]);
     }
 #pragma unroll
     for (int off = 32; off >= 4; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
     if (threadIdx.x % 64 < 4) red[threadIdx.x / 64][n4] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(red[0][n4], red[1][n4]), fmaxf(red[2][n4], red[3][n4]));
+    amax = red[0][n4];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) amax = fmaxf(amax, red[w][n4]);
     int e = 0;
     if (amax > 0.f && amax < INFINITY) (void)frexpf(amax, &e);  // amax = m * 2^e, m in [0.5, 1)
     int se = 14 - e;
@@ -95,9 +101,9 @@ static __global__ __launch_bounds__(256) void tokens_split_kernel(const float* _
     if (in_regs) {
 #pragma unroll
         for (int j = 0; j < MAXV; ++j)
-            if (const uint32_t k8 = j * 64 + g0; k8 < groups) emit(k8, v[j][0], v[j][1]);
+            if (const uint32_t k8 = j * PER + g0; k8 < groups) emit(k8, v[j][0], v[j][1]);
     } else {
-        for (uint32_t k8 = g0; k8 < groups; k8 += 64) emit(k8, xr[k8 * 2], xr[k8 * 2 + 1]);
+        for (uint32_t k8 = g0; k8 < groups; k8 += PER) emit(k8, xr[k8 * 2], xr[k8 * 2 + 1]);
     }
 }
 
