@@ -164,14 +164,23 @@ __global__ __launch_bounds__(512) void q4_pairs_kernel(const Q4Args a) {
     a.out[(size_t)(req0 + q) * a.rows + tile * 16 + l16] = sum * a.inv_scale[req0 + q];
 }
 
-// out[i] = slice 0 + slice 1 + ... in that order.
+// out[i] = slice 0 + slice 1 + ... in that order, eight loads at a time: what this takes is the way to memory and back
+// (whole calls, one load at a time -> now: 512 x 4096 at 300 tokens, 25 slices, 37.8 -> 35.6 us; 2048 x 2048 at 512, four,
+// 43.9 -> 43.6).
 __global__ __launch_bounds__(256) void q4_sum_slices_kernel(const float* __restrict__ slices,
                                                             float* __restrict__ out, uint32_t n,
                                                             uint32_t ksplit) {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
     float s = slices[i];
-    for (uint32_t k = 1; k < ksplit; ++k) s += slices[(size_t)k * n + i];
+    for (uint32_t k0 = 1; k0 < ksplit; k0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = k0 + j < ksplit ? slices[(size_t)(k0 + j) * n + i] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (k0 + j < ksplit) s += v[j];
+    }
     out[i] = s;
 }
 
