@@ -263,8 +263,8 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // residual add 8.4 -> 4.6, gate/up with SiLU (11264 x 2048) 11.2 -> 7.0, down (2048 x 5632) 8.1 and 5.0 for the sum of
 // its K slices -> 8 with the residual add and no slices; a step of 22 layers 1 145 -> 801 (845 with the
 // fragments of 32 requests as they are for larger batches).  32 requests: qkv 7.5 -> 6.9,
-// gate/up 13.3 -> 14.0, a step 1 330 -> 1 207.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
-// a layer 141 -> 114.  2-norm error against float64: 0.95e-7 .. 1.15e-7, before 1.03e-7 .. 1.34e-7.
+// gate/up 13.3 -> 13.3, a step 1 330 -> 1 199.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
+// a layer 140 -> 112.  2-norm error against float64: 0.95e-7 .. 1.15e-7, before 1.03e-7 .. 1.34e-7.
 template <int NI, int RT, int WAVES, bool BS, int FORM>
 __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
