@@ -179,6 +179,9 @@ struct Ctx {
         std::vector<uint32_t> ids, slots;   // of the scatter(s) that joined so far
         size_t batch = 0, row_elems = 0, page_size = 0;
     } kv;
+    // Who writes a Q4_0 matmul's activation fragments: the split kernel or a row chain, or the epilogue of the
+    // launch in front (each with buffers of its own: the held-back matmul may still read another's).
+    enum Q4Input { kXSplit, kXSilu, kXAttention, kXNorm };
     // A Q4_0 matmul of the open pass whose launch is held back for one call: when that call is
     // the split + RoPE + cast of the matmul's output (the qkv projection of a layer), the
     // matmul's epilogue does it and the two -- with the KV scatters that join -- are one launch.
@@ -194,6 +197,8 @@ struct Ctx {
         const void* out = nullptr;
         size_t batch = 0, rows = 0;
         bool block_scales = false;       // the activations carry one scale per (request, block)
+        Q4Input x_from = kXSplit;        // who writes its activation fragments,
+        int x_set = 0;                   // and in which of that producer's buffers they lie
         bool silu = false;               // the gate/up split + SiLU * up has joined
         const void* silu_out = nullptr;
         size_t ffn_inner = 0;

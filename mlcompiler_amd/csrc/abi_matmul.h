@@ -98,6 +98,11 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
                             q4_fast_shape(rows, cols, row_stride) && g.dec.active && g.dec.o == in &&
                             g.dec.batch == batch && g.dec.cols == cols;
     const bool block_scales = feeds_silu || feeds_attn || feeds_rms;
+    const Ctx::Q4Input x_from = feeds_silu ? Ctx::kXSilu : feeds_attn ? Ctx::kXAttention : feeds_rms ? Ctx::kXNorm : Ctx::kXSplit;
+    // The held-back matmul writes this one's input.  Where its own came the same way (a matmul that both finishes a
+    // norm and starts the next one) the two inputs take turns between two sets of buffers: some of its workgroups
+    // still read the one when others are done and write the other.
+    const int x_set = (feeds_silu || feeds_rms) && g.gemm.x_from == x_from ? 1 - g.gemm.x_set : 0;
     if (!feeds && !block_scales && !settle()) return 0;
     Ctx::Q4Weight* w = q4_weight(weight_name, static_cast<const uint8_t*>(weights), weight_bytes, rows, cols, row_stride);
     if (!w) return 0;
@@ -137,15 +142,15 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;
-        // (the held-back projection still reads "q4_x_fragments": its products go to a buffer of their own)
-        _Float16* frag = static_cast<_Float16*>(cached_buffer(
-            feeds_silu ? "q4_x_fragments_silu" : feeds_attn ? "q4_x_fragments_attention" : feeds_rms ? "q4_x_fragments_norm" : "q4_x_fragments",
-            bpad * cols * 4));
+        static const char* const frag_names[][2] = {{"q4_x_fragments", nullptr}, {"q4_x_fragments_silu", "q4_x_fragments_silu_2"},
+                                                    {"q4_x_fragments_attention", nullptr}, {"q4_x_fragments_norm", "q4_x_fragments_norm_2"}};
+        static const char* const scale_names[][2] = {{nullptr, nullptr}, {"q4_x_block_scales_silu", "q4_x_block_scales_silu_2"},
+                                                     {"q4_x_block_scales_attention", nullptr}, {"q4_x_block_scales_norm", "q4_x_block_scales_norm_2"}};
+        static const char* const ssq_names[] = {"q4_norm_partial_sums", "q4_norm_partial_sums_2"};
+        _Float16* frag = static_cast<_Float16*>(cached_buffer(frag_names[x_from][x_set], bpad * cols * 4));
         float* inv = static_cast<float*>(cached_buffer("q4_x_inv_scale", 64 * 4));
-        float* blk_scale = !block_scales ? nullptr : static_cast<float*>(cached_buffer(
-            feeds_silu ? "q4_x_block_scales_silu" : feeds_attn ? "q4_x_block_scales_attention" : "q4_x_block_scales_norm",
-            bpad * nblocks * 4));
-        float* ssq = feeds_rms ? static_cast<float*>(cached_buffer("q4_norm_partial_sums", nblocks * 64 * 4)) : nullptr;
+        float* blk_scale = !block_scales ? nullptr : static_cast<float*>(cached_buffer(scale_names[x_from][x_set], bpad * nblocks * 4));
+        float* ssq = feeds_rms ? static_cast<float*>(cached_buffer(ssq_names[x_set], nblocks * 64 * 4)) : nullptr;
         if (feeds_rms && !ssq) return fail("q4 matmul: scratch allocation failed");
         Q4Args norm{};   // (what this matmul needs to finish the norm)
         if (!frag || !inv || (block_scales && !blk_scale)) return fail("q4 matmul: scratch allocation failed");
@@ -213,6 +218,8 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             m.active = true;
             m.silu = false;
             m.block_scales = block_scales;
+            m.x_from = x_from;
+            m.x_set = x_set;
             m.a = a;
             m.out = out;
             m.batch = batch;
