@@ -117,6 +117,7 @@ struct Ctx {
         void* raw = nullptr;
         void* q = nullptr;
         void* d = nullptr;
+        bool is(size_t b, size_t r, size_t c, size_t s) const { return raw && bytes == b && rows == r && cols == c && stride == s; }
     };
     std::unordered_map<std::string, Q4Weight> q4_weights;
     struct Q6KWeight {
@@ -396,6 +397,8 @@ void slot_mark(MetaSlot& s) { s.use = ++g.slot_uses; }
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
+int settle_gemm(const RopeArgs* rope);
+
 // Device copy of a small host blob, uploaded only when (kind, key, bytes) has not been seen
 // with this content.  The copy is ordered on the library stream, so kernels already enqueued
 // that read the previous content are not disturbed.  nullptr on failure (error recorded).
@@ -421,6 +424,8 @@ const void* resident_blob(int kind, const void* key, const void* blob, size_t by
         if (hipMalloc(&r.dev, cap) != hipSuccess) { r.dev = nullptr; fail("resident: hipMalloc failed"); return nullptr; }
         r.cap = cap;
     }
+    // (a held-back matmul that finishes an RMSNorm reads the weights as they were: it goes out in front of the copy)
+    if (r.dev && g.gemm.active && g.gemm.a.rms_gamma == r.dev && !settle_gemm(nullptr)) return nullptr;
     r.content.clear();  // not valid until the copy has been enqueued
     MetaSlot& s = g.ring[g.ring_next];
     g.ring_next = (g.ring_next + 1) % 8;
@@ -471,7 +476,7 @@ int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a, size_t ksplit = 1) 
 
 // Launches the held-back matmul, with the split + RoPE + cast of its output as epilogue when
 // `rope` is given.
-int settle_gemm(const RopeArgs* rope = nullptr) {
+int settle_gemm(const RopeArgs* rope) {
     Ctx::GemmPending& m = g.gemm;
     if (!m.active) return 1;
     m.active = false;
@@ -582,15 +587,19 @@ int settle_kv() {
 
 // Launches what is pending, in the order it was encoded: a pending KV write is always older
 // than a pending chain (whatever starts the KV write launches the chain first, and a scatter
-// only joins while no chain is pending).
-int settle() {
+// only joins while no chain is pending).  settle_before_rows() leaves the chain pending.
+int settle_before_rows() {
     // a held-back attention launch is older than anything else: whatever was pending when it was
     // encoded has been launched, and nothing joins a chain behind it before it is launched
     if (!settle_decode()) return 0;
     // a held-back matmul is older than anything else pending, unless the pending KV write is
     // its own epilogue
-    if (g.gemm.active && !(g.kv.active && g.kv.rope && g.kv.from_gemm) && !settle_gemm()) return 0;
-    if (!settle_kv()) return 0;
+    if (g.gemm.active && !(g.kv.active && g.kv.rope && g.kv.from_gemm) && !settle_gemm(nullptr)) return 0;
+    return settle_kv();
+}
+
+int settle() {
+    if (!settle_before_rows()) return 0;
     Ctx::RowPending& r = g.rows;
     if (!r.active) return 1;
     r.active = false;

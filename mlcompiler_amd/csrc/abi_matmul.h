@@ -24,7 +24,7 @@ bool upload_weights(void* dst, const void* host, size_t bytes) {
 Ctx::Q4Weight* q4_weight(const char* name, const uint8_t* host, size_t bytes, size_t rows, size_t cols,
                          size_t stride) {
     Ctx::Q4Weight& w = g.q4_weights[name];
-    if (w.raw && w.bytes == bytes && w.rows == rows && w.cols == cols && w.stride == stride) return &w;
+    if (w.is(bytes, rows, cols, stride)) return &w;
     if (g_capturing) { fail("q4 matmul: the weights are not on the device yet (run the pass once uncaptured first)"); return nullptr; }
     (void)hipStreamSynchronize(g.stream);
     for (void** p : {&w.raw, &w.q, &w.d})
@@ -66,6 +66,9 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     if (batch * rows > 0x7FFFFFFFull || batch * cols > 0x7FFFFFFFull) return fail("q4 matmul: too many elements");
     const size_t ki = known_bytes(in), ko = known_bytes(out);
     if ((ki && batch * cols * 4 > ki) || (ko && batch * rows * 4 > ko)) return fail("q4 matmul: buffer too small");
+    // (another matrix under a name that is known: a held-back matmul may read the one it replaces)
+    const auto known = g.q4_weights.find(weight_name);
+    if (known != g.q4_weights.end() && !known->second.is(weight_bytes, rows, cols, row_stride) && !settle()) return 0;
     // does the pending chain end in this matmul's input?  (decided before anything below can
     // replace a buffer the chain still refers to)
     const bool feeds = batch <= 64 && !g.opt_q4_force_generic && !(reinterpret_cast<uintptr_t>(out) & 15u) &&
@@ -103,7 +106,8 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     // norm and starts the next one) the two inputs take turns between two sets of buffers: some of its workgroups
     // still read the one when others are done and write the other.
     const int x_set = (feeds_silu || feeds_rms) && g.gemm.x_from == x_from ? 1 - g.gemm.x_set : 0;
-    if (!feeds && !block_scales && !settle()) return 0;
+    // (a held-back matmul that does not take the chain over goes out now: it may read a buffer that is replaced below)
+    if (feeds && !feeds_rms ? !settle_before_rows() : !block_scales && !settle()) return 0;
     Ctx::Q4Weight* w = q4_weight(weight_name, static_cast<const uint8_t*>(weights), weight_bytes, rows, cols, row_stride);
     if (!w) return 0;
 
@@ -323,7 +327,7 @@ int mlc_hip_matmul_q6_k_batched(const char* weight_name, const void* weights, si
     if ((ki && batch * cols * 4 > ki) || (ko && batch * rows * 4 > ko)) return fail("q6_k matmul: buffer too small");
     const bool fast = q6k_fast_shape(rows, cols, row_stride) && !g.opt_q4_force_generic;
     const bool feeds = fast && batch <= 64 && row_len_ok(cols) && rows_continue(in, batch, cols);
-    if (!feeds && !settle()) return 0;
+    if (feeds ? !settle_before_rows() : !settle()) return 0;   // (a held-back matmul may read a buffer that is replaced below)
     Ctx::Q6KWeight* w = q6k_weight(weight_name, static_cast<const uint8_t*>(weights), weight_bytes, rows, cols, row_stride);
     if (!w) return 0;
 

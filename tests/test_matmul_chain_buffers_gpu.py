@@ -94,3 +94,46 @@ def test_gate_up_behind_gate_up(exe, batch, ffn):
     for i in range(2):
         _, _, want = po.gate_up_split_silu_mul(got[f"y{i}"], batch, ffn[i], 2 * ffn[i])
         assert np.max(np.abs(got[f"m{i}"] - want) / (np.abs(want) + 1e-30)) < 5e-6
+
+
+@pytest.mark.parametrize("what", ["fragments", "weights", "norm_weights"])
+def test_a_held_back_matmul_keeps_what_it_reads(exe, what):
+    """Calls behind a held-back matmul that replace what it reads: a matmul with a longer row than any before it
+    ("q4_x_fragments" grows; it has too few rows to take the norm over), another matrix under the same name, other norm
+    weights in the same host array."""
+    batch = 64 if what == "fragments" else 16
+    widths = {"fragments": (64, 8192, 64), "weights": (256, 512, 1024), "norm_weights": (256, 512, 512, 1024)}[what]
+    rng = np.random.default_rng(7)
+    n = len(widths) - 1
+    w = [_weights(rng, widths[i + 1], widths[i]) for i in range(n)]
+    x = rng.standard_normal((batch, widths[0])).astype(np.float32)
+    resid = [rng.standard_normal((batch, v)).astype(np.float32) for v in widths[1:-1]]
+    gammas = [(1.0 + 0.3 * rng.standard_normal(v)).astype(np.float32) for v in widths[1:-1]]
+    gamma = gammas[0].copy()
+    like = {f"{m}{i}": np.empty((batch, widths[i + 1]), np.float32) for i in range(n) for m in "phn"}
+    dev = {m: _pool(exe, np.full_like(a, np.nan)) for m, a in like.items()}
+    src = [_pool(exe, a) for a in [x] + resid]
+    try:
+        a = src[0]
+        assert exe.beginForwardPassCB()
+        for i in range(n):
+            name = "kept" if what == "weights" else f"kept.{what}.{i}"
+            assert exe.encodeMatMulQ4_0Batched(name, w[i], a, batch, widths[i + 1], widths[i], w[i].shape[1], 1,
+                                               dev[f"p{i}"]), exe.lastError()
+            if i < n - 1:
+                gamma[:] = gammas[i]
+                a = dev[f"n{i}"]
+                assert exe.encodeAddBatched(dev[f"p{i}"], src[i + 1], dev[f"h{i}"], batch * widths[i + 1])
+                assert exe.encodeRmsNormBatched(dev[f"h{i}"], gamma, EPS, batch, widths[i + 1], a)
+        assert exe.flushForwardPassCB(), exe.lastError()
+        got = {m: _read(exe, dev[m], like[m]) for m in like}
+    finally:
+        for buf in list(dev.values()) + src:
+            exe.releaseScratchBuffer(buf)
+    a = x
+    for i in range(n):
+        check(got[f"p{i}"], q4.dequant(w[i], widths[i]), a)
+        if i < n - 1:
+            a = got[f"n{i}"]
+            want = po.rms_norm_batched(got[f"h{i}"], gammas[i], EPS, batch, widths[i + 1])
+            assert (np.abs(a - want) <= 2e-6 * np.abs(want).max(axis=1, keepdims=True)).all()
