@@ -22,11 +22,10 @@ bool upload_weights(void* dst, const void* host, size_t bytes) {
 
 // Gives up a matrix whose layout for the matrix cores is not complete, so that the next call starts over (hipFree waits
 // for what still reads it).
-template <class W, class... P>
-void drop_weight(W& w, P*... parts) {
-    for (void* p : {static_cast<void*>(parts)...})
+void drop_weight(Ctx::Q4Weight& w) {
+    for (void* p : {w.raw, w.q, w.d})
         if (p) (void)hipFree(p);
-    w = W{};
+    w = Ctx::Q4Weight{};
 }
 
 // Uploads the weight matrix on first use of its name (or when its size changed).
@@ -47,14 +46,14 @@ Ctx::Q4Weight* q4_weight(const char* name, const uint8_t* host, size_t bytes, si
         const size_t nb = cols / 32, quads = (nb + 3) / 4, tiles = rows / 16, units = tiles * quads * 64;
         if (hipMalloc(&w.q, units * 16) != hipSuccess || hipMalloc(&w.d, tiles * quads * 16 * 8) != hipSuccess) {
             (void)hipGetLastError();
-            drop_weight(w, w.raw, w.q, w.d);
+            drop_weight(w);
             fail("q4 matmul: hipMalloc failed");
             return nullptr;
         }
         hipLaunchKernelGGL(q4_repack_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, g.stream,
                            static_cast<const uint8_t*>(w.raw), static_cast<uint4*>(w.q), static_cast<uint16_t*>(w.d),
                            (uint32_t)tiles, (uint32_t)nb, (uint32_t)quads, stride);
-        if (hipGetLastError() != hipSuccess) { drop_weight(w, w.raw, w.q, w.d); fail("q4 matmul: repacking failed"); return nullptr; }
+        if (hipGetLastError() != hipSuccess) { drop_weight(w); fail("q4 matmul: repacking failed"); return nullptr; }
     }
     return &w;
 }
@@ -312,7 +311,9 @@ Ctx::Q6KWeight* q6k_weight(const char* name, const uint8_t* host, size_t bytes, 
             !upload_weights(w.qa, qa.data(), qa.size()) || !upload_weights(w.sc, sc.data(), sc.size()) ||
             !upload_weights(w.d, d.data(), d.size() * 2)) {
             (void)hipGetLastError();
-            drop_weight(w, w.raw, w.qa, w.sc, w.d);
+            for (void* p : {w.raw, w.qa, w.sc, w.d})
+                if (p) (void)hipFree(p);
+            w = Ctx::Q6KWeight{};
             fail("q6_k matmul: repacked upload failed");
             return nullptr;
         }
