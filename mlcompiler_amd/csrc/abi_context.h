@@ -498,6 +498,21 @@ int settle_gemm(const RopeArgs* rope) {
     return launch_q4(form, m.block_scales, a);
 }
 
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
+}
+
+// Two buffers of one launch whose element i belongs to the same thread: do they meet at other elements than their own?
+bool shifted(const void* a, const void* b, size_t bytes) { return a != b && overlap(a, bytes, b, bytes); }
+
+// A matmul that finishes an RMSNorm reads the norm's input and writes its output in all its workgroups, in no order
+// with what the others do: nothing else that the launch writes may lie there (and nothing that it reads in the output).
+bool meets_norm(const Q4Args& a, const void* p, size_t bytes, bool written = true) {
+    const size_t norm_bytes = (size_t)a.batch * a.rms_len * 4;
+    return a.ssq_in && ((written && overlap(p, bytes, a.rms_src, norm_bytes)) || overlap(p, bytes, a.rms_out, norm_bytes));
+}
+
 // True when the held-back matmul's output is exactly the fused qkv rows a split + RoPE + cast
 // call describes, so that the matmul's epilogue can do that call's work.
 bool gemm_feeds_rope(const void* qkv, size_t batch, size_t qkv_rows, size_t q_rows, size_t k_rows, size_t v_rows) {

@@ -92,11 +92,20 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     if (feeds && scales_fit && g.gemm.active && g.opt_q4_int_operand) {
         const Ctx::GemmPending& m = g.gemm;
         const RowProgram& p = g.rows.p;
+        const size_t row_bytes = batch * cols * 4;
         feeds_rms = !m.silu && !q4_wide(m.rows) && !g.kv.active && p.src == m.out && p.n_slices == 1 &&
                     !p.src_store && !p.silu && p.addend && p.rms && !p.frag && g.rows.batch == batch &&
                     g.rows.len == cols && m.batch == batch && m.rows == cols && cols / 32 <= 128 &&
-                    batch * cols <= rows / (q4_wide(rows) ? 64 : 32) * 1024;   // (every thread of the reader writes at most one
+                    batch * cols <= rows / (q4_wide(rows) ? 64 : 32) * 1024 &&   // (every thread of the reader writes at most one
                                                                               // element of its z group's part of the norm)
+                    // The buffers of either launch lie apart, or exactly on each other where a thread has the same
+                    // element of both: the held-back matmul's (it reads the addend before it writes anything),
+                    !overlap(p.addend, row_bytes, m.out, row_bytes) && !shifted(p.add_out, m.out, row_bytes) &&
+                    !shifted(p.add_out, p.addend, row_bytes) && !meets_norm(m.a, p.add_out, row_bytes) &&
+                    !meets_norm(m.a, p.addend, row_bytes, false) &&
+                    // and this one's, which reads the sum and writes the norm.
+                    !shifted(p.rms_out, p.add_out, row_bytes) && !overlap(out, batch * rows * 4, p.add_out, row_bytes) &&
+                    !overlap(out, batch * rows * 4, p.rms_out, row_bytes);
     }
     // ... or is the input the SiLU * up product that the held-back gate/up projection's epilogue
     // will write?  Then that epilogue also splits it, per (request, block of 32 columns).

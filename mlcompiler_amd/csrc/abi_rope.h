@@ -43,7 +43,9 @@ int mlc_hip_qkv_split_rope_cast(const void* qkv, void* q, void* k, void* v, void
                                 size_t q_rows, size_t k_rows, size_t v_rows, size_t rotary_dim,
                                 int sync) {
     if (!init_once()) return fail("GPU unavailable");
-    const bool from_gemm = gemm_feeds_rope(qkv, batch, qkv_rows, q_rows, k_rows, v_rows);
+    const bool from_gemm = gemm_feeds_rope(qkv, batch, qkv_rows, q_rows, k_rows, v_rows) && !meets_norm(g.gemm.a, q, batch * q_rows * 4) &&
+                           !meets_norm(g.gemm.a, k, batch * k_rows * 4) && !meets_norm(g.gemm.a, v, batch * v_rows * 4) &&
+                           !meets_norm(g.gemm.a, k_f16, batch * k_rows * 2) && !meets_norm(g.gemm.a, v_f16, batch * v_rows * 2);
     if (!from_gemm && !settle()) return 0;
     if (!sync && !g.pass_open) return fail("encode: no open forward pass");  // :7936
     if (const char* why = rope_args_problem(qkv, q, cos_buf, sin_buf, batch, num_heads, kv_heads,
@@ -91,7 +93,8 @@ int mlc_hip_qkv_split_rope_scatter(const void* qkv, void* q, void* k_pages, void
                                    size_t kv_heads, size_t head_dim, size_t qkv_rows, size_t q_rows,
                                    size_t k_rows, size_t v_rows, size_t rotary_dim, int sync) {
     if (!init_once()) return fail("GPU unavailable");
-    const bool from_gemm = gemm_feeds_rope(qkv, batch, qkv_rows, q_rows, k_rows, v_rows);
+    const bool from_gemm = gemm_feeds_rope(qkv, batch, qkv_rows, q_rows, k_rows, v_rows) && !meets_norm(g.gemm.a, q, batch * q_rows * 4) &&
+                           !meets_norm(g.gemm.a, k_f32, batch * k_rows * 4) && !meets_norm(g.gemm.a, v_f32, batch * v_rows * 4);
     if (!from_gemm && !settle()) return 0;
     if (!sync && !g.pass_open) return fail("encode: no open forward pass");
     if (const char* why = rope_args_problem(qkv, q, cos_buf, sin_buf, batch, num_heads, kv_heads,

@@ -137,3 +137,115 @@ def test_a_held_back_matmul_keeps_what_it_reads(exe, what):
             a = got[f"n{i}"]
             want = po.rms_norm_batched(got[f"h{i}"], gammas[i], EPS, batch, widths[i + 1])
             assert (np.abs(a - want) <= 2e-6 * np.abs(want).max(axis=1, keepdims=True)).all()
+
+
+# Buffers that a chain  p0 = W0 x; h0 = r0 + p0; n0 = norm(h0); p1 = W1 n0; h1 = r1 + p1; n1 = norm(h1); y = W2 n1
+# may share, as long as nobody reads what was overwritten: {buffer: the one that it is}, and how many of the two norms
+# the matmuls can still take over then.
+SHARED = {
+    "sums_over_residuals": ({"h0": "r0", "h1": "r1"}, 2),
+    "sum_over_the_sum_before": ({"h1": "h0"}, 1),
+    "sum_over_the_norm_before": ({"h1": "n0"}, 1),
+    "norm_before_as_residual": ({"r1": "n0"}, 1),
+    "sum_before_as_residual": ({"r1": "h0"}, 2),
+    "residual_over_and_over": ({"h0": "r0", "r1": "r0", "h1": "r0"}, 1),
+    "output_over_the_sum_before": ({"p1": "h0"}, 1),
+    "output_over_its_input": ({"p1": "n0"}, 1),
+    "output_added_to_itself": ({"r1": "p1"}, 1),
+    "sum_over_the_output": ({"h0": "p0", "h1": "p1"}, 2),
+    "norms_in_place": ({"n0": "h0", "n1": "h1"}, 2),
+    "last_output_over_the_sum": ({"y": "h1"}, 1),
+    "last_output_over_the_norm": ({"y": "n1"}, 1),
+    "everything_in_two": ({"p0": "x", "h0": "x", "n0": "x", "p1": "r0", "h1": "r0", "n1": "r0", "r1": "x", "y": "x"}, 1),
+}
+
+
+@pytest.mark.parametrize("batch", [3, 32])
+@pytest.mark.parametrize("shared", list(SHARED), ids=list(SHARED))
+def test_shared_buffers(exe, shared, batch):
+    """The chain with its launches fused gives what its calls one by one give, whichever buffers are the same.
+    (Tolerance as in test_row_chain_fuzz_gpu.py: the fused norm's sum runs in another order.)"""
+    same, fused = SHARED[shared]
+    rng = np.random.default_rng(batch)
+    n = 512
+    w = [_weights(rng, n, n) for _ in range(3)]
+    gamma = [(1.0 + 0.3 * rng.standard_normal(n)).astype(np.float32) for _ in range(2)]
+    init = {m: rng.standard_normal((batch, n)).astype(np.float32) for m in ("x", "r0", "r1", "p0", "h0", "n0", "p1", "h1", "n1", "y")}
+    out = {}
+    for fuse in (0, 1):
+        dev = {m: _pool(exe, a) for m, a in init.items()}
+        at = lambda m: dev[same.get(m, m)]
+        assert exe.setOption("fuse_row_ops", fuse)
+        before = exe.fusedMatmulNormLaunches()
+        try:
+            a = "x"
+            assert exe.beginForwardPassCB()
+            for i, dst in enumerate(("p0", "p1", "y")):
+                assert exe.encodeMatMulQ4_0Batched(f"shared{batch}.{i}", w[i], at(a), batch, n, n, w[i].shape[1], 1, at(dst)), exe.lastError()
+                if i < 2:
+                    a = f"n{i}"
+                    assert exe.encodeAddBatched(at(f"r{i}"), at(dst), at(f"h{i}"), batch * n)
+                    assert exe.encodeRmsNormBatched(at(f"h{i}"), gamma[i], EPS, batch, n, at(a))
+            assert exe.flushForwardPassCB(), exe.lastError()
+            out[fuse] = {m: _read(exe, b, init[m]) for m, b in dev.items()}
+        finally:
+            exe.setOption("fuse_row_ops", 1)
+            for buf in dev.values():
+                exe.releaseScratchBuffer(buf)
+        assert exe.fusedMatmulNormLaunches() - before == (fused if fuse else 0)
+    for m, want in out[0].items():
+        assert np.isfinite(want).all() and np.abs(out[1][m] - want).max() <= 1e-4 * np.abs(want).max(), m
+
+
+@pytest.mark.parametrize("over", ["sum", "norm"])
+@pytest.mark.parametrize("reader", ["silu", "rope", "rope_scatter"])
+def test_epilogues_over_the_norm(exe, reader, over):
+    """A matmul that finishes a norm, followed by an operator that it would take over, whose output lies over the
+    norm's input or output."""
+    rng = np.random.default_rng(11)
+    batch, n, heads, kv_heads, d = 6, 4096, 32, 4, 128
+    kv = kv_heads * d
+    rows = 2 * n + 64 * 2 if reader == "silu" else n + 2 * kv
+    w = [_weights(rng, n, 64), _weights(rng, rows, n)]
+    gamma = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    cos, sin = (np.stack(t) for t in zip(*(po.rotary_coefficients(int(p), d) for p in rng.integers(0, 2000, batch))))
+    ids, slots = np.arange(batch, dtype=np.uint32), rng.integers(0, 8, batch).astype(np.uint32)
+    half = rows // 2
+    init = {"x": (batch, 64), "p": (batch, n), "r": (batch, n), "h": (batch, max(n, half)), "n": (batch, max(n, half)), "y": (batch, rows),
+            "a": (batch, max(n, half)), "b": (batch, max(kv, half)), "c": (batch, max(kv, half))}
+    init = {m: rng.standard_normal(s).astype(np.float32) for m, s in init.items()}
+    init |= {"cos": cos.astype(np.float32), "sin": sin.astype(np.float32)}
+    init |= {m: np.zeros((batch, 8, kv), np.uint16) for m in ("k16", "v16", "kp", "vp")}
+    out = {}
+    for fuse in (0, 1):
+        dev = {m: _pool(exe, a) for m, a in init.items()}
+        first = dev["h" if over == "sum" else "n"]
+        assert exe.setOption("fuse_row_ops", fuse)
+        before = exe.fusedMatmulNormLaunches(), exe.fusedMatmulSiluLaunches() + exe.fusedMatmulRopeLaunches()
+        try:
+            assert exe.beginForwardPassCB()
+            assert exe.encodeMatMulQ4_0Batched("over.0", w[0], dev["x"], batch, n, 64, w[0].shape[1], 1, dev["p"]), exe.lastError()
+            assert exe.encodeAddBatched(dev["r"], dev["p"], dev["h"], batch * n)
+            assert exe.encodeRmsNormBatched(dev["h"], gamma, EPS, batch, n, dev["n"])
+            assert exe.encodeMatMulQ4_0Batched(f"over.{reader}", w[1], dev["n"], batch, rows, n, w[1].shape[1], 1, dev["y"]), exe.lastError()
+            if reader == "silu":
+                assert exe.encodeGateUpSplitSiluMul(dev["y"], dev["a"], dev["b"], first, batch, half, rows), exe.lastError()
+            elif reader == "rope":
+                assert exe.encodeQkvSplitRopeCast(dev["y"], first, dev["b"], dev["c"], dev["k16"], dev["v16"], dev["cos"], dev["sin"],
+                                                  batch, heads, kv_heads, d, rows, n, kv, kv, d), exe.lastError()
+            else:
+                assert exe.encodeQkvSplitRopeScatter(dev["y"], first, dev["kp"], dev["vp"], dev["cos"], dev["sin"], ids, slots, 8,
+                                                     batch, heads, kv_heads, d, rows, n, kv, kv, d), exe.lastError()
+            assert exe.flushForwardPassCB(), exe.lastError()
+            out[fuse] = {m: _read(exe, b, init[m]) for m, b in dev.items()}
+        finally:
+            exe.setOption("fuse_row_ops", 1)
+            for buf in dev.values():
+                exe.releaseScratchBuffer(buf)
+        assert exe.fusedMatmulNormLaunches() - before[0] == fuse
+        assert exe.fusedMatmulSiluLaunches() + exe.fusedMatmulRopeLaunches() == before[1]
+    for m, want in out[0].items():
+        got = out[1][m]
+        if want.dtype == np.uint16:      # fp16: one step of its rounding
+            want, got = want.view(np.float16).astype(np.float32), got.view(np.float16).astype(np.float32)
+        assert np.abs(got - want).max() <= (1e-3 if m in ("kp", "vp", "k16", "v16") else 1e-4) * max(np.abs(want).max(), 1e-30), m
