@@ -656,6 +656,20 @@ bool rows_continue(const void* buf, size_t batch, size_t len) {
     return r.batch == batch && r.len == len;  // callers check that the length they go on with fits
 }
 
+// A chain's workgroups each do one row from the first operator to the last, in no order with the other rows: an operator
+// may join only if its rows `p` of `len` floats meet what the chain reads and writes in the same row and column or
+// not at all (written = false: what the chain writes).
+bool rows_apart(const void* p, size_t len, bool written = true) {
+    const Ctx::RowPending& r = g.rows;
+    const RowProgram& c = r.p;
+    const size_t half = c.silu ? c.len_src / 2 : c.len_src;
+    auto apart = [&](const void* q, size_t q_len) {
+        return !q || (p == q && len == q_len) || !overlap(p, r.batch * len * 4, q, r.batch * q_len * 4);
+    };
+    return apart(c.src_store, c.len_src) && (!c.silu || (apart(c.gate_out, half) && apart(c.up_out, half) && apart(c.silu_out, half))) &&
+           apart(c.add_out, half) && (!written || (apart(c.n_slices == 1 ? c.src : nullptr, c.len_src) && apart(c.addend, half)));
+}
+
 // Starts a chain whose source is a plain buffer of rows.
 void rows_begin(const void* src, size_t batch, size_t len) {
     Ctx::RowPending& r = g.rows;

@@ -18,7 +18,7 @@ int mlc_hip_rms_norm_batched(const void* in, const float* weight, size_t n_weigh
     if ((ki && batch * length * 4 > ki) || (ko && batch * length * 4 > ko))
         return fail("rms norm: buffer too small");
     const bool fusable = row_len_ok(length) && aligned16(in) && aligned16(out);
-    const bool joins = fusable && !g.rows.p.rms && rows_continue(in, batch, length);
+    const bool joins = fusable && !g.rows.p.rms && rows_continue(in, batch, length) && rows_apart(out, length);
     if (!joins && !settle()) return 0;  // before the weight's device copy may be replaced
     // the weight vector is borrowed for the call; its device copy is kept between calls
     const float one = 1.0f;
@@ -62,7 +62,8 @@ int mlc_hip_add_batched(const void* a, const void* b, void* out, size_t total_el
     const bool fusable = g.opt_fuse_rows && total_elements % 8 == 0 && aligned16(a) && aligned16(b) && aligned16(out);
     Ctx::RowPending& r = g.rows;
     const bool joins = fusable && r.active && (r.cur == a || r.cur == b) && !r.p.addend && !r.p.rms && !r.p.frag &&
-                       (r.batch ? r.batch * r.len == total_elements && row_len_ok(r.len) : r.n_flat == total_elements);
+                       r.batch && r.batch * r.len == total_elements && row_len_ok(r.len) && rows_apart(out, r.len) &&
+                       rows_apart(r.cur == a ? b : a, r.len, false);
     // A residual add on top of the held-back matmul's output (the out-projection): the matmul stays
     // held back while the chain add -> RMSNorm builds up behind it; if a Q4_0 matmul then reads the
     // norm, the two matmuls do the chain's work (mlc_hip_matmul_q4_0_batched), and if anything
@@ -141,7 +142,8 @@ int mlc_hip_gate_up_split_silu_mul(const void* gate_up, void* gate, void* up, vo
         Ctx::RowPending& r = g.rows;
         const bool joins = ffn_gate_up_rows == 2 * ffn_inner && row_len_ok(ffn_inner) && aligned16(gate) &&
                            aligned16(up) && aligned16(out) && !r.p.silu && !r.p.addend && !r.p.rms &&
-                           rows_continue(gate_up, batch, ffn_gate_up_rows);
+                           rows_continue(gate_up, batch, ffn_gate_up_rows) && rows_apart(gate, ffn_inner) &&
+                           rows_apart(up, ffn_inner) && rows_apart(out, ffn_inner);
         if (joins) {
             r.p.silu = 1;
             r.p.gate_out = static_cast<float*>(gate);
