@@ -367,7 +367,8 @@ long mlc_hip_fused_matmul_norm_launches(void);
 /* Number of decode attention launches so far that carried the step's KV write (a pair of
  * batched K / V scatters of every request's newest position encoded just before it). */
 long mlc_hip_kv_writes_in_decode_launches(void);
-/* Number of fused row-operator launches so far (for tests of "fuse_row_ops"). */
+/* Number of launches of held-back row operators so far: chains of them, and an add behind a held-back matmul
+ * (for tests of "fuse_row_ops"). */
 long mlc_hip_row_program_launches(void);
 /* Number of times so far the decode path copied a page table to the device: the copy is
  * reused while the table's content stays the same (for tests and benchmarks). */
