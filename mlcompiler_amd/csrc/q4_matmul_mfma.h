@@ -264,7 +264,7 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // its K slices -> 8 with the residual add and no slices; a step of 22 layers 1 145 -> 801 (845 with the
 // fragments of 32 requests as they are for larger batches).  32 requests: qkv 7.5 -> 6.9,
 // gate/up 13.3 -> 13.3, a step 1 330 -> 1 199.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
-// a layer 140 -> 112.  2-norm error against float64: 0.95e-7 .. 1.15e-7, before 1.03e-7 .. 1.34e-7.
+// a layer 140 -> 112.  2-norm error against float64 of rows of 2048 to 14336: 0.95e-7 .. 1.17e-7, before 1.03e-7 .. 1.62e-7.
 template <int NI, int RT, int WAVES, bool BS, int FORM>
 __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
@@ -413,11 +413,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     q4_float4 zero;
 #pragma unroll
     for (int i = 0; i < 4; ++i) zero[i] = 0.f;
-    float acc[RT][NI];
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int i = 0; i < NI; ++i) acc[r][i] = 0.f;
+    float acc[RT][NI] = {};
     auto multiply = [&](const QuadW& w, int j, const BlockX& x) __attribute__((always_inline)) {
         // (the scales of this lane's requests in block j, see `turn`)
         [[maybe_unused]] float sc[NI];
@@ -440,6 +436,27 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
             for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(acc[r][i]));
         }
         if constexpr (PACKED && RT == 4 && (WAVES == 16 || !BS)) __builtin_amdgcn_sched_barrier(0);   // (for the same reason)
+    };
+    // Rounding errors grow with the number of blocks added up in a row: a quad's sums go to a second set of registers
+    // where there is room for one, else four quads' to LDS, where the waves' sums meet anyway.  (2-norm error against
+    // float64, with one level -> now: 9216 x 14336 at 17 requests 1.58e-7 -> 1.17e-7, 512 x 11008 1.22e-7 -> 1.07e-7.
+    // No measurable time; adding to LDS after every quad with ds_add costs 1.3 to 5 times the kernel.)
+    constexpr bool TWO_LEVELS = RT * NI <= 8;
+    [[maybe_unused]] float total[RT][NI] = {};
+    [[maybe_unused]] uint32_t in_a_row = 0;
+    [[maybe_unused]] bool flushed = false;
+    auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) f(red[(wave * RT + r) * TILE_PITCH + i * 64 + lane], total[r][i], acc[r][i]);
+    };
+    auto flush = [&]() __attribute__((always_inline)) {
+        if constexpr (TWO_LEVELS) each([](float&, float& sum, float& v) __attribute__((always_inline)) { sum += v; });
+        else if (flushed) each([](float& sum, float&, float& v) __attribute__((always_inline)) { sum += v; });
+        else each([](float& sum, float&, float& v) __attribute__((always_inline)) { sum = v; });
+        each([](float&, float&, float& v) __attribute__((always_inline)) { v = 0.f; });
+        flushed = true;
     };
     // A wave's quads are first, first + WAVES, ...  While one is multiplied the next one's weights are on the way, and
     // activations XD blocks ahead.  The last one is a copy of the code that fetches nothing: a load costs its share
@@ -491,16 +508,21 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
             for (int r = 0; r < RT; ++r) asm volatile("" : "+v"(next.q[r]), "+v"(next.d[r]));
             w = next;
             load_w(quad + 2 * WAVES, next);
+            // (behind the loads: a branch in front of them makes the compiler wait for more of them)
+            if constexpr (TWO_LEVELS) {
+                flush();
+            } else if (++in_a_row == 4) {
+                flush();
+                in_a_row = 0;
+            }
         }
         turn(quad, std::false_type());
     }
 
     // ---- the waves' sums meet in LDS.  A lane holds weight row l16 of the tile and, in register i, request
     // kg * NI + i.
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int i = 0; i < NI; ++i) red[(wave * RT + r) * TILE_PITCH + i * 64 + lane] = acc[r][i];
+    flush();
+    if constexpr (TWO_LEVELS) each([](float& sum, float& v, float&) __attribute__((always_inline)) { sum = v; });
     __syncthreads();
     if constexpr (BS) {
         // the norm's own output: h * factor * gamma, the arithmetic of rms_norm_batched_kernel
