@@ -68,10 +68,12 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
     // ---- which kernel: the tile-balanced one wherever it applies
     int s_hpw = 0, s_nw = 0;
     uint64_t total_tiles = 0;
+    uint32_t with_tiles = 0;
     for (size_t r = 0; r < batch; ++r) {
         uint64_t lim = seq_lens[r];
         if (apply_causal && (uint64_t)q_positions[r] + 1 < lim) lim = (uint64_t)q_positions[r] + 1;  // :2286
         total_tiles += (lim + tile - 1) / tile;
+        with_tiles += lim > 0;
     }
     total_tiles *= kv_heads;
     // (the kernel counts in units: tiles plus at most 64 per (request, KV head) pair)
@@ -187,7 +189,7 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
             c.causal = apply_causal ? 1 : 0;
             c.carried_kv = c.carried_kv || carries_kv;
         }
-        g.last_items = (int)std::min<uint64_t>(n_wg, total_tiles);
+        g.last_items = (int)stream_workgroups((uint32_t)(total_tiles / kv_heads), with_tiles, (uint32_t)kv_heads, n_wg);
         std::snprintf(g.last_kernel, sizeof g.last_kernel, "stream<%zu,%d,%d,%s,%s,%d>", head_dim, s_hpw, s_nw,
                       stream_pv_name(s_hpw, s_nw), batch <= 64 ? "regs" : "lds", nbuf);
         if (carries_kv) {
@@ -269,12 +271,14 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
         (reinterpret_cast<uintptr_t>(page_tables_flat_device) & 3u))
         return fail("decode (no allocation): buffers must be 16-byte aligned");
     uint64_t total_tiles = 0;
+    uint32_t with_tiles = 0;
     for (size_t r = 0; r < batch; ++r) {
         const size_t pages = ((size_t)seq_lens[r] + page_size_tokens - 1) / page_size_tokens;
         if ((size_t)page_table_offsets[r] + pages > n_flat) return fail("decode: page table does not cover seq_len");
         uint64_t lim = seq_lens[r];
         if (apply_causal && (uint64_t)q_positions[r] + 1 < lim) lim = (uint64_t)q_positions[r] + 1;  // :2286
         total_tiles += (lim + tile - 1) / tile;
+        with_tiles += lim > 0;
     }
     total_tiles *= kv_heads;
     if (total_tiles + 64ull * batch * kv_heads >= 0x7FFFFFFFull) return fail("decode (no allocation): too many KV tiles");
@@ -307,7 +311,7 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
     if (!launch_stream_variant(head_dim, hpw, nw, nbuf, a, n_wg, dyn_lds, st))
         return fail("decode: kernel variant not built");
     HIP_OK(hipGetLastError());
-    g.last_items = (int)std::min<uint64_t>(n_wg, total_tiles);
+    g.last_items = (int)stream_workgroups((uint32_t)(total_tiles / kv_heads), with_tiles, (uint32_t)kv_heads, n_wg);
     std::snprintf(g.last_kernel, sizeof g.last_kernel, "stream<%zu,%d,%d,%s,%s,%d>", head_dim, hpw, nw,
                   stream_pv_name(hpw, nw), batch <= 64 ? "regs" : "lds", nbuf);
     g.last_launches = 1;

@@ -10,7 +10,7 @@ struct TokensArgs {
     const uint2* q;          // repacked weights: Q4Args::q / Q6KArgs::qa
     const uint32_t* sc;      // Q6KArgs::sc (Q4_0: not read)
     const _Float16* d;       // Q4Args::d / Q6KArgs::d
-    const _Float16* xfrag;   // split activations of token_blocks * 64 rows (q4_split_activations_kernel)
+    const _Float16* xfrag;   // split activations of token_blocks * 64 rows, 32 requests wide (fragments.h, tokens_split_kernel)
     const float* inv_scale;  // [tokens]
     float* out;              // [tokens][rows], or the slice buffer [ksplit][tokens][rows]
     uint32_t tokens, rows;

@@ -41,6 +41,22 @@ static constexpr size_t kStreamProbeWord = kStreamPartBytes / 8;  // probe build
 // workgroup has room for (heads per wave x waves).
 constexpr size_t stream_partial_bytes(size_t GP, size_t D, size_t NW) { return (GP * D + 64 * NW) * 8; }
 
+// Workgroups with tiles, of a grid of `grid`: tiles_head tiles of 64 (head_dim 128: 32) tokens per KV head, of nz_head
+// requests that have any.  A workgroup gets at least 1 << `least` tiles.  A pair that is spread over more workgroups reads
+// its tiles sooner, but is summed up from more partials, eight per memory round trip: with n tiles per pair the sum of
+// the two is least at about sqrt(n) / 2 tiles (by 3 the pairs' ends rarely fall on a range's end: powers of
+// two), and two tiles go to one workgroup, which then sums up nothing.
+// (Whole calls, one tile per workgroup where there were places -> now, us; 32 query and 4 KV heads of 64, one
+// request of 128, 1024, 2048, 4096, 8192 tokens: 16.7 -> 15.8, 19.7 -> 18.9, 23.7 -> 20.7, 31.8 -> 22.4,
+// 51.8 -> 26.4; 8 KV heads of 128, one request of 2048: 34.3 -> 23.4, four of 512: 23.6 -> 20.1.)
+__host__ __device__ __forceinline__ uint32_t stream_workgroups(uint32_t tiles_head, uint32_t nz_head, uint32_t kv_heads, uint32_t grid) {
+    const uint32_t twice = (uint32_t)(tiles_head * 4u > nz_head * 7u && tiles_head * 4u < nz_head * 9u);
+    const uint32_t least = twice + (uint32_t)(tiles_head > nz_head * 8u) + (uint32_t)(tiles_head >= nz_head * 48u) +
+                           (uint32_t)(tiles_head >= nz_head * 160u);
+    const uint32_t places = (tiles_head * kv_heads + (1u << least) - 1u) >> least;
+    return grid < places ? grid : places;
+}
+
 struct StreamArgs {
     const float* q;             // [B][H][D]
     const uint4* k_pages;       // fp16 pages, viewed as 16-byte chunks
@@ -397,17 +413,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     // workgroup whose range crosses from one pair into the next gets fewer tiles.  Unit numbering:
     // [request][kv head][the pair's tiles, then PC units that stand for its end].
     const uint32_t T = tiles_head * Hkv;                       // the host keeps this below 2^31
-    // A workgroup gets at least 1 << `least` tiles.  A pair that is spread over more workgroups reads its tiles
-    // sooner, but is summed up from more partials, eight per memory round trip: with n tiles per pair the sum of
-    // the two is least at about sqrt(n) / 2 tiles (by 3 the pairs' ends rarely fall on a range's end: powers of
-    // two), and two tiles go to one workgroup, which then sums up nothing.
-    // (Whole calls, one tile per workgroup where there were places -> now, us; 32 query and 4 KV heads of 64, one
-    // request of 128, 1024, 2048, 4096, 8192 tokens: 16.7 -> 15.8, 19.7 -> 18.9, 23.7 -> 20.7, 31.8 -> 22.4,
-    // 51.8 -> 26.4; 8 KV heads of 128, one request of 2048: 34.3 -> 23.4, four of 512: 23.6 -> 20.1.)
-    const uint32_t twice = (uint32_t)(tiles_head * 4u > nz_head * 7u && tiles_head * 4u < nz_head * 9u);
-    const uint32_t least = twice + (uint32_t)(tiles_head > nz_head * 8u) + (uint32_t)(tiles_head >= nz_head * 48u) +
-                           (uint32_t)(tiles_head >= nz_head * 160u);
-    const uint32_t places = min((uint32_t)gridDim.x, (T + (1u << least) - 1u) >> least);
+    const uint32_t places = stream_workgroups(tiles_head, nz_head, Hkv, gridDim.x);
     // (nothing to balance where every tile gets a workgroup of its own)
     const uint32_t PC = T > places ? a.pair_cost : 0u;
     const uint32_t UT = T + PC * nz_head * Hkv;                // ... and this

@@ -8,6 +8,8 @@ from paged_cases import DeviceCase, assert_parity, make_case, oracle_decode
 
 pytestmark = pytest.mark.gpu
 
+CUS = 256   # (two workgroups to a CU)
+
 
 @pytest.mark.parametrize("ratio", [1, 8])
 @pytest.mark.parametrize("batch", [1, 3, 66])
@@ -25,5 +27,7 @@ def test_least_share(exe, tiles, batch, ratio):
     dev = DeviceCase(exe, case)
     try:
         assert_parity(dev.run(sync=True), oracle_decode(case), 64, case.name)
+        total, share = max(batch - 1, 1) * tiles, 1 + (tiles == 2 or tiles > 8) + 2 * (tiles >= 48) + 4 * (tiles >= 160)
+        assert exe.lastDecodeWorkItems() == min(-(-total // share), CUS * 2)
     finally:
         dev.free()
