@@ -451,22 +451,33 @@ constexpr size_t kRowMaxLen = 16384;  // row_program_kernel: 8 groups of 8 eleme
 
 bool row_len_ok(size_t len) { return len > 0 && len % 8 == 0 && len <= kRowMaxLen; }
 
-// Rows of a Q4_0 matmul that come as 64 per workgroup, in tiles of 16.
+// Rows of a Q4_0 matmul that is taken for a gate/up projection (kQ4Silu), and not for one that a residual add follows.
 bool q4_wide(size_t rows) { return rows > 8192; }
 
-// Launches q4_matmul_kernel in one of its forms.  Tiles per workgroup: 4 for matrices of more than 8192 rows
-// and for the SiLU epilogue, 2 for the residual add's, else 1 where that leaves no more workgroups than CUs
-// (a workgroup of 16 waves has a CU to itself) and 2 where it does not.  RoPE: at most 2.
+// Tiles of 16 rows per workgroup of q4_matmul_kernel: as few as leave no more workgroups than CUs (one of 16 waves has
+// a CU to itself), and 4 where there are more in any case: the activations that a CU fetches for a weight halve with
+// every step.  (Whole calls, us, by rows > 8192 -> by this rule, and one workgroup of 32 x 32 products per 32 rows and 64
+// requests: 6144 x 4096 at 17, 32, 33 and 64 requests 25.8, 27.0, 31.3, 34.2 -> 23.3, 23.6, 28.7, 29.9, 23.5, 24.5, 29.5,
+// 31.4; 4096 x 4096 at 64 28.1 -> 24.8, 29.9; 4096 x 14336 at 64 70.4 -> 58.8, 62.5; 8192 x 4096 at 64 40.3 -> 32.8, 34.9.)
+// The SiLU epilogue's workgroups have 4, the residual add's at least 2, and those of up to 8 requests with
+// RoPE or the residual add at most 2 (the kernels of 4 do not fit the registers).
+int q4_tiles(Q4Form form, size_t rows, size_t batch, size_t ksplit) {
+    const size_t wgs = rows / 16 * ((batch + 15) / 16) * ksplit, n_cu = (size_t)g.n_cu;
+    if (form == kQ4Silu) return 4;
+    const int least = form == kQ4Add ? 2 : 1, most = form != kQ4Plain && batch <= 8 ? 2 : 4;
+    return std::min(most, std::max(least, wgs > 2 * n_cu ? 4 : wgs > n_cu ? 2 : 1));
+}
+
+// Launches q4_matmul_kernel in one of its forms.
 int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a, size_t ksplit = 1) {
     const uint32_t tiles = a.rows / 16;
     a.z_groups = (a.batch + 15) / 16;
-    int rt = (size_t)tiles * a.z_groups * ksplit <= (size_t)g.n_cu ? 1 : 2;
-    if (form == kQ4Silu || (form == kQ4Plain && q4_wide(a.rows))) rt = 4;
-    else if (form == kQ4Add) rt = 2;
+    const int rt = q4_tiles(form, a.rows, a.batch, ksplit);
     a.row_groups = tiles / rt;
-    // Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; a wide matrix with more
-    // row groups than CUs runs with 8, two workgroups to a CU, so that one's first loads overlap the other's products.
-    const int waves = q4_wide(a.rows) && (size_t)(tiles / 4) * a.z_groups * ksplit > (size_t)g.n_cu ? 8 : 16;
+    // Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; where there are more
+    // workgroups than CUs, with 4 tiles each, they have 8, two workgroups to a CU, so that one's first loads overlap the
+    // other's products.
+    const int waves = (size_t)(tiles / 4) * a.z_groups * ksplit > (size_t)g.n_cu ? 8 : 16;
     const dim3 grid((a.row_groups + 7) / 8 * 8 * a.z_groups, (unsigned)ksplit);
     const auto launch = a.batch <= 4 ? launch_q4_matmul_1 : a.batch <= 8 ? launch_q4_matmul_2 : launch_q4_matmul_4;
     if (!launch(form, rt, waves, block_scales, grid, a, g.stream)) return fail("q4 matmul: kernel variant not built");

@@ -14,6 +14,20 @@ bool q4_fast_shape(size_t rows, size_t cols, size_t row_stride) {
     return rows % 64 == 0 && cols % 32 == 0 && cols <= (1u << 24) && row_stride >= cols / 32 * 18;
 }
 
+// K slices of a Q4_0 matmul on the matrix cores and the quads of blocks in each.  K is split over workgroups (of 32 rows)
+// only where there are too few of them for the CUs and K is long: from 96 quads (K = 12288) on, so that each of a slice's
+// 16 waves keeps three.
+struct Q4Slices { size_t n, quads; };
+Q4Slices q4_slices(size_t rows, size_t cols) {
+    const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
+    size_t n = (size_t)g.opt_q4_ksplit;
+    if (n == 0) n = std::max<size_t>(1, std::min<size_t>((size_t)g.n_cu / (rows / 32), quads / 48));
+    n = std::min(n, std::max<size_t>(1, nblocks / 16));
+    if (!g.opt_q4_int_operand) n = 1;
+    const size_t per_slice = (quads + n - 1) / n;
+    return {(quads + per_slice - 1) / per_slice, per_slice};
+}
+
 // Copies weights to the device in the order of the library's stream (a plain hipMemcpy may return before the data is
 // there, and the library's stream does not wait for it), and waits.
 bool upload_weights(void* dst, const void* host, size_t bytes) {
@@ -96,8 +110,10 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         feeds_rms = !m.silu && !q4_wide(m.rows) && !g.kv.active && p.src == m.out && p.n_slices == 1 &&
                     !p.src_store && !p.silu && p.addend && p.rms && !p.frag && g.rows.batch == batch &&
                     g.rows.len == cols && m.batch == batch && m.rows == cols && cols / 32 <= 128 &&
-                    batch * cols <= rows / (q4_wide(rows) ? 64 : 32) * 1024 &&   // (every thread of the reader writes at most one
-                                                                              // element of its z group's part of the norm)
+                    // (every thread of the reader writes at most one element of its z group's part of the norm)
+                    batch * cols <= rows / (q4_wide(rows) ? 64 : 32) * 1024 &&
+                    std::min<size_t>(batch, 16) * cols <=
+                        rows / 16 / q4_tiles(q4_wide(rows) ? kQ4Silu : kQ4Add, rows, batch, q4_slices(rows, cols).n) * 1024 &&
                     // The buffers of either launch lie apart, or exactly on each other where a thread has the same
                     // element of both: the held-back matmul's (it reads the addend before it writes anything),
                     !overlap(p.addend, row_bytes, m.out, row_bytes) && !shifted(p.add_out, m.out, row_bytes) &&
@@ -151,16 +167,9 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             return finish(sync);
     }
 
-    // MFMA path, one pass over at most 64 requests at a time.  K is split over workgroups (of 32 rows) only where there
-    // are too few of them for the CUs and K is long: from 96 quads of blocks (K = 12288) on, so that each of a slice's
-    // 16 waves keeps three.
+    // MFMA path, one pass over at most 64 requests at a time.
     const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
-    size_t ksplit = (size_t)g.opt_q4_ksplit;
-    if (ksplit == 0) ksplit = std::max<size_t>(1, std::min<size_t>((size_t)g.n_cu / (rows / 32), quads / 48));
-    ksplit = std::min(ksplit, std::max<size_t>(1, nblocks / 16));
-    if (!g.opt_q4_int_operand) ksplit = 1;
-    const size_t per_slice = (quads + ksplit - 1) / ksplit;
-    ksplit = (quads + per_slice - 1) / per_slice;
+    const size_t ksplit = q4_slices(rows, cols).n, per_slice = q4_slices(rows, cols).quads;
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;

@@ -17,8 +17,15 @@ bool MLC_CAT(launch_q4_matmul_, MLC_Q4_NI)(int form, int rt, int waves, bool blo
     }
     MLC_Q4(kQ4Plain, 1, 16, plain) MLC_Q4(kQ4Plain, 2, 16, plain) MLC_Q4(kQ4Plain, 4, 16, plain) MLC_Q4(kQ4Plain, 4, 8, plain)
     MLC_Q4(kQ4Silu, 4, 16, plain) MLC_Q4(kQ4Silu, 4, 8, plain)
-    MLC_Q4(kQ4Rope, 1, 16, a) MLC_Q4(kQ4Rope, 2, 16, a) MLC_Q4(kQ4Rope, 2, 8, a)
+    MLC_Q4(kQ4Rope, 1, 16, a) MLC_Q4(kQ4Rope, 2, 16, a)
     MLC_Q4(kQ4Add, 2, 16, plain)
+#if MLC_Q4_NI < 4
+    MLC_Q4(kQ4Rope, 2, 8, a)
+    MLC_Q4(kQ4Add, 2, 8, plain)
+#else
+    MLC_Q4(kQ4Rope, 4, 16, a) MLC_Q4(kQ4Rope, 4, 8, a)
+    MLC_Q4(kQ4Add, 4, 16, plain) MLC_Q4(kQ4Add, 4, 8, plain)
+#endif
 #undef MLC_Q4
     return false;
 }

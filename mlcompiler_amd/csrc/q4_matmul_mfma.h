@@ -71,9 +71,9 @@ struct Q4Args {
     float* silu_out;
     _Float16* split_frag;
     float* split_blk_scale;
-    // ADD (32 rows per workgroup, ksplit == 1): the epilogue also does the residual add that follows
+    // ADD (32 or 64 rows per workgroup, ksplit == 1): the epilogue also does the residual add that follows
     // the matmul (add_out = out + add_resid, [batch][rows]), leaves every request's sum of squares over
-    // the workgroup's 32 columns in ssq_out[request][rows / 32] (the RMSNorm that follows is
+    // every 32 columns in ssq_out[request][rows / 32] (the RMSNorm that follows is
     // finished by the matmul that reads it, see ssq_in) and writes add_out * add_gamma as the
     // split-fp16 fragments of that matmul (split_frag / split_blk_scale, K = rows).  add_gamma[c] for
     // c < add_n_gamma, 1 beyond.
@@ -269,7 +269,7 @@ template <int NI, int RT, int WAVES, bool BS, int FORM>
 __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
     static_assert(FORM != kQ4Silu || RT == 4, "SiLU epilogue: 32 rows of gate and 32 of up");
-    static_assert(FORM != kQ4Add || RT == 2, "residual add: 32 rows, one block of the next matmul's K");
+    static_assert(FORM != kQ4Add || RT % 2 == 0, "residual add: whole blocks of the next matmul's K");
     // Up to 8 requests: a quad's activations come 1 KB per load, without the places of requests that do not
     // exist, and each lane's operand from LDS.  (16-byte loads of 64 lanes cost 16 clocks of the return path, however
     // many of them ask for the same bytes or for none.)
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     // ---- thread -> output: row `row` of the workgroup's (SiLU: column of its 32), request req0 + q
     constexpr uint32_t ROWS = FORM == kQ4Silu ? 32 : 16 * RT, PER_PASS = WAVES * 64 / ROWS;
     constexpr int PASSES = (QR + PER_PASS - 1) / PER_PASS;   // outputs per thread
-    static_assert(PASSES == 1 || FORM == kQ4Plain, "the other epilogues: one output per thread");
+    static_assert(PASSES == 1 || FORM != kQ4Silu, "SiLU epilogue: one output per thread");
     const uint32_t row = threadIdx.x % ROWS, qi = threadIdx.x / ROWS;
     // (which request: so that the 64 lanes of a wave read 64 different banks)
     constexpr uint32_t SB = 2 * NI;
@@ -315,19 +315,23 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
 
     // ---- what the epilogue reads besides the sums is fetched before the main loop, so that it adds no memory
     // round trip to the kernel's tail
-    [[maybe_unused]] Q4RopeFetch rope_pre = {1.0f, 0.0f, 0ull};
-    if constexpr (FORM == kQ4Rope)
-        if (has_out) rope_pre = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4RopeOffset), b, col);
-    [[maybe_unused]] float resid_pre = 0.f, gamma_pre = 1.0f, inv_pre[PASSES] = {};
-    if constexpr (FORM == kQ4Add) {
-        if (has_out) resid_pre = a.add_resid[(size_t)b * a.rows + col];
-        if (col < a.add_n_gamma) gamma_pre = a.add_gamma[col];
-    }
-    if constexpr (!BS) {
+    [[maybe_unused]] Q4RopeFetch rope_pre[PASSES];
+    [[maybe_unused]] float resid_pre[PASSES] = {}, gamma_pre = 1.0f, inv_pre[PASSES] = {};
 #pragma unroll
-        for (int p = 0; p < PASSES; ++p)
-            if (q + p * PER_PASS < live) inv_pre[p] = a.inv_scale[b + p * PER_PASS];
+    for (int p = 0; p < PASSES; ++p) {
+        const uint32_t bp = b + p * PER_PASS;
+        const bool has = has_out && q + p * PER_PASS < live;
+        if constexpr (FORM == kQ4Rope) {
+            rope_pre[p] = {1.0f, 0.0f, 0ull};
+            if (has) rope_pre[p] = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4RopeOffset), bp, col);
+        }
+        if constexpr (FORM == kQ4Add)
+            if (has) resid_pre[p] = a.add_resid[(size_t)bp * a.rows + col];
+        if constexpr (!BS)
+            if (has) inv_pre[p] = a.inv_scale[bp];
     }
+    if constexpr (FORM == kQ4Add)
+        if (col < a.add_n_gamma) gamma_pre = a.add_gamma[col];
     // The RMSNorm that the producer of the activations left unfinished (ssq_in): a wave sums up the partials of
     // one or two requests, and the row group writes 1024 elements of the norm's own output at the end.
     constexpr int RMS_N = 16 / WAVES;   // requests per wave, and elements per thread
@@ -438,9 +442,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         if constexpr (PACKED && RT == 4 && (WAVES == 16 || !BS)) __builtin_amdgcn_sched_barrier(0);   // (for the same reason)
     };
     // Rounding errors grow with the number of blocks added up in a row: a quad's sums go to a second set of registers
-    // where there is room for one, else four quads' to LDS, where the waves' sums meet anyway.  (2-norm error against
-    // float64, with one level -> now: 9216 x 14336 at 17 requests 1.58e-7 -> 1.17e-7, 512 x 11008 1.22e-7 -> 1.07e-7.
-    // No measurable time; adding to LDS after every quad with ds_add costs 1.3 to 5 times the kernel.)
+    // where there is room for one, else those of four quads (of two where 8 waves share K: as many blocks of 4096 columns
+    // as 16 waves add up) to LDS, where the waves' sums meet anyway.  (2-norm error against float64, with one level -> now:
+    // 9216 x 14336 at 17 requests 1.58e-7 -> 1.11e-7, 512 x 11008 at 33 1.22e-7 -> 1.07e-7, 28672 x 4096 at 17 1.10e-7 ->
+    // 1.02e-7.  No measurable time; adding to LDS after every quad with ds_add costs 1.3 to 5 times the kernel.)
     constexpr bool TWO_LEVELS = RT * NI <= 8;
     [[maybe_unused]] float total[RT][NI] = {};
     [[maybe_unused]] uint32_t in_a_row = 0;
@@ -511,7 +516,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
             // (behind the loads: a branch in front of them makes the compiler wait for more of them)
             if constexpr (TWO_LEVELS) {
                 flush();
-            } else if (++in_a_row == 4) {
+            } else if (++in_a_row == WAVES / 4) {
                 flush();
                 in_a_row = 0;
             }
@@ -567,14 +572,14 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         if (qp >= live) break;
         const float val = sum_of(row, qp, inv_pre[p]);
         store_through(&out[(size_t)bp * a.rows + col], val);
-        if constexpr (FORM == kQ4Rope) q4_rope_epilogue(a.rope, rope_pre, bp, col, val);   // (the lanes of a pair share b)
+        if constexpr (FORM == kQ4Rope) q4_rope_epilogue(a.rope, rope_pre[p], bp, col, val);   // (the lanes of a pair share b)
         if constexpr (FORM == kQ4Add) {
-            // residual add, this request's sum of squares over the 32 columns, and h * gamma as the next
+            // residual add, this request's sum of squares over a half wave's 32 columns, and h * gamma as the next
             // matmul's fragments
-            const float hv = val + resid_pre;
+            const float hv = val + resid_pre[p];
             store_through(&a.add_out[(size_t)bp * a.rows + col], hv);
             const float ssq = q4_half_wave_sum(hv * hv);
-            if (row == 0) store_through(&a.ssq_out[(size_t)bp * (a.rows / 32) + row_group], ssq);
+            if (row % 32 == 0) store_through(&a.ssq_out[(size_t)bp * (a.rows / 32) + col / 32], ssq);
             q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale, WIDTH);
         }
     }

@@ -17,9 +17,10 @@ def _weights(rng, rows, cols):
 
 
 @pytest.mark.parametrize("batch,widths,fused", [
-    # 512 workgroups of 16 waves, one to a CU, in the middle: its second half starts when the first has written the
-    # next input, which is wider than its own
+    # as many workgroups as CUs in the middle: the first write the next input, which is wider than their own, when
+    # others still read theirs
     (64, (64, 2048, 4096, 8192), 2),
+    (33, (160, 3072, 4096, 8192), 2),               # four tiles each, of 16 waves and at the end of 8
     (16, (128, 512, 512, 1024, 512, 1024), 4),      # the buffers change three times
     (5, (64, 1024, 256, 4096), 2),                  # ... get narrower, and wider
 ])

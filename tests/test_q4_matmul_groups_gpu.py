@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import test_decode_split_fusion_gpu as split
+import test_matmul_rope_fusion_gpu as rope
 import test_matmul_silu_fusion_gpu as silu
 import test_q4_matmul_gpu as q4
 from oracle import paged_oracle as po
@@ -28,6 +29,20 @@ def test_divisions(exe, rows, cols, batch):
     got = q4.run(exe, f"groups_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride)
     check(got, q4.dequant(q, cols), x)
     assert np.array_equal(got, q4.run(exe, f"groups_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride, sync=False))
+
+
+@pytest.mark.parametrize("batch", [17, 32, 33, 64])    # four tiles per workgroup of 16 waves, of 8 from 33 requests on
+def test_rope_of_four_tiles(exe, batch):
+    c = rope.Case(B=batch, H=40, Hkv=4, D=128, hid=1184, seed=batch)
+    plain, _ = rope._run(exe, c, "scatter", fuse=0)
+    fused, n = rope._run(exe, c, "scatter", fuse=1)
+    assert n == 1
+    for m in ("qkv", "q", "k", "v", "kp", "vp"):
+        assert np.array_equal(plain[m].view(np.uint8), fused[m].view(np.uint8)), m
+    check(fused["qkv"], q4.dequant(c.w, c.hid), c.x)
+    wants = po.qkv_split_rope_cast(fused["qkv"], c.cos, c.sin, c.B, c.H, c.Hkv, c.D, c.rows, c.q_rows, c.kv_rows, c.kv_rows, c.rotary)
+    for m, want in zip("qkv", wants):
+        assert np.array_equal(fused[m].view(np.uint8), np.ascontiguousarray(want).view(np.uint8)), m
 
 
 @pytest.mark.parametrize("batch", [1, 6, 16, 21, 40])
