@@ -470,17 +470,30 @@ int q4_tiles(Q4Form form, size_t rows, size_t batch, size_t ksplit) {
 
 // Launches q4_matmul_kernel in one of its forms.
 int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a, size_t ksplit = 1) {
-    const uint32_t tiles = a.rows / 16;
-    a.z_groups = (a.batch + 15) / 16;
+    const size_t tiles = a.rows / 16, z = (a.batch + 15) / 16, n_cu = (size_t)g.n_cu;
     const int rt = q4_tiles(form, a.rows, a.batch, ksplit);
-    a.row_groups = tiles / rt;
+    a.row_groups = (uint32_t)(tiles / rt);
     // Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; where there are more
     // workgroups than CUs, with 4 tiles each, they have 8, two workgroups to a CU, so that one's first loads overlap the
     // other's products.
-    const int waves = (size_t)(tiles / 4) * a.z_groups * ksplit > (size_t)g.n_cu ? 8 : 16;
+    const int waves = tiles / 4 * z * ksplit > n_cu ? 8 : 16;
+    // Such workgroups take four or two groups of 16 requests each, one workgroup to a CU, where those are one round of at
+    // least five eighths of the CUs, or rounds of which the last is at least half full, with no group missing.  (Whole calls,
+    // us, one group per workgroup -> now, and one workgroup of 32 x 32 products per 64 requests: 28672 x 4096 at 32, 49 and
+    // 64 requests 46.5, 70, 74 -> 42.4, 58.4, 62, 44.4, 64.3, 66.5; 16384 x 4096 at 64 47.0 -> 38.9, 41.8; 11264 x 2048 at 32
+    // 24.5 -> 23.3, 23.6.  Two groups elsewhere: 11264 x 2048 at 33, 352 workgroups, 26.3 -> 29.5; 8256 x 1024 at 32, 129
+    // workgroups, 19.3 -> 19.8; 28672 x 4096 at 33, where half of 896 have one group only, 55.6 -> 63.6.)
+    int zt = 1;
+    for (const int n : {4, 2}) {
+        const size_t wgs = tiles / 4 * ((z + n - 1) / n) * ksplit, last = wgs % n_cu;
+        if (zt == 1 && waves == 8 && (form == kQ4Plain || form == kQ4Silu) && z > 1 && (n == 2 || (z == 4 && !block_scales)) &&
+            (wgs <= n_cu ? wgs * 8 >= n_cu * 5 : z % n == 0 && (last == 0 || last * 2 >= n_cu)))
+            zt = n;
+    }
+    a.z_groups = (uint32_t)((z + zt - 1) / zt);
     const dim3 grid((a.row_groups + 7) / 8 * 8 * a.z_groups, (unsigned)ksplit);
     const auto launch = a.batch <= 4 ? launch_q4_matmul_1 : a.batch <= 8 ? launch_q4_matmul_2 : launch_q4_matmul_4;
-    if (!launch(form, rt, waves, block_scales, grid, a, g.stream)) return fail("q4 matmul: kernel variant not built");
+    if (!launch(form, rt, waves, zt, block_scales, grid, a, g.stream)) return fail("q4 matmul: kernel variant not built");
     HIP_OK(hipGetLastError());
     return 1;
 }

@@ -39,9 +39,9 @@ MLC_DECL(64, 1) MLC_DECL(64, 2) MLC_DECL(64, 4) MLC_DECL(64, 8)
 MLC_DECL(128, 1) MLC_DECL(128, 2) MLC_DECL(128, 4) MLC_DECL(128, 8)
 #undef MLC_DECL
 // Defined in q4_matmul_inst.hip, one object per number of accumulator registers.
-bool launch_q4_matmul_1(int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
-bool launch_q4_matmul_2(int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
-bool launch_q4_matmul_4(int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
+bool launch_q4_matmul_1(int, int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
+bool launch_q4_matmul_2(int, int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
+bool launch_q4_matmul_4(int, int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
 }  // namespace mlc_hip
 
 // The sections of this translation unit, in the order they build on one another.

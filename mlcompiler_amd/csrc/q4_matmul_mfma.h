@@ -256,7 +256,9 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // More than 16 requests: z groups of 16, workgroups of their own that read the same weights at the same
 // time on the same XCD (workgroup x: row group x / (8 Z) * 8 + x % 8, z group x / 8 % Z).  Each fetches its
 // own activations only, 4 bytes per request and column through one CU's memory path, which would be the
-// longest stream of a workgroup that had them all.
+// longest stream of a workgroup that had them all.  ZT = 2 or 4: so many groups in one
+// workgroup, which unpacks a weight once for all of them.  That takes 158 or 245 registers, one workgroup of 8 waves to a
+// CU, and so pays where such workgroups fill their rounds (launch_q4).
 //
 // Measured, kernel times in us, before (32 x 32 products, one workgroup per 32 rows, branches or clamps around the loads of
 // a wave's last blocks) -> now.  One request of the 1 B shape: qkv (2560 x 2048) 7.0 -> 4.5, out-projection with the
@@ -265,8 +267,8 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // fragments of 32 requests as they are for larger batches).  32 requests: qkv 7.5 -> 6.9,
 // gate/up 13.3 -> 13.3, a step 1 330 -> 1 199.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
 // a layer 140 -> 112.  2-norm error against float64 of rows of 2048 to 14336: 0.95e-7 .. 1.17e-7, before 1.03e-7 .. 1.62e-7.
-template <int NI, int RT, int WAVES, bool BS, int FORM>
-__global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
+template <int NI, int RT, int WAVES, bool BS, int FORM, int ZT = 1>
+__global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
     static_assert(FORM != kQ4Silu || RT == 4, "SiLU epilogue: 32 rows of gate and 32 of up");
     static_assert(FORM != kQ4Add || RT % 2 == 0, "residual add: whole blocks of the next matmul's K");
@@ -278,13 +280,15 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     constexpr int XQ = PACKED ? 2 * NI : 1;          // loads per quad
     // blocks of activations in registers: as far as 128 registers per wave go
     constexpr int XD = PACKED ? (RT == 4 ? 1 : 2) : RT == 4 ? 2 : 4;
-    constexpr int QR = 4 * NI;                       // requests of the workgroup
+    static_assert(ZT == 1 || (RT == 4 && WAVES == 8 && !PACKED), "more than one group of 16 requests: one workgroup of 8 waves to a CU");
+    constexpr int X_TILES = (ZT + 1) / 2;            // batch tiles of 32 that the workgroup has a part of
+    constexpr int QR = 4 * NI * ZT;                       // requests of the workgroup
     constexpr int TILE_PITCH = NI * 64 + 16;         // floats per tile in LDS (16: bank spread)
-    __shared__ float red[WAVES * RT * TILE_PITCH];
+    __shared__ float red[WAVES * RT * ZT * TILE_PITCH];
     // BS: a quad's scales, [block][request]: fetched by a load of 4 bytes per lane, handed out from here.  (A load of
     // every lane's own scales per block would take as long as one of the block's two fragments: what bounds these
     // kernels next to the vector pipe is the 64 bytes a clock that a CU's loads return.)
-    __shared__ __attribute__((aligned(16))) float scales[BS ? WAVES : 1][64];
+    __shared__ __attribute__((aligned(16))) float scales[BS ? WAVES : 1][ZT][64];
     __shared__ q4_u32x4 packed[PACKED ? WAVES : 1][XQ * 64];
     __shared__ float rms_scale[BS ? QR : 1];         // BS with ssq_in: every request's RMSNorm factor
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -293,7 +297,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     const uint32_t row_group = blockIdx.x / z8 * 8 + blockIdx.x % 8, zg = blockIdx.x / 8 % a.z_groups;
     if (row_group >= a.row_groups) return;           // (the grid is a multiple of 8 row groups)
     const uint32_t slice = blockIdx.y;
-    const uint32_t req0 = zg * 16, live = min((uint32_t)QR, a.batch - req0);   // (the last group may be smaller)
+    const uint32_t req0 = zg * (16 * ZT), live = min((uint32_t)QR, a.batch - req0);   // (the last group may be smaller)
     // tile r of the workgroup
     const uint32_t tile0 = FORM == kQ4Silu ? row_group * 2 : row_group * RT;
     auto tile_of = [&](int r) __attribute__((always_inline)) {
@@ -303,7 +307,6 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     // ---- thread -> output: row `row` of the workgroup's (SiLU: column of its 32), request req0 + q
     constexpr uint32_t ROWS = FORM == kQ4Silu ? 32 : 16 * RT, PER_PASS = WAVES * 64 / ROWS;
     constexpr int PASSES = (QR + PER_PASS - 1) / PER_PASS;   // outputs per thread
-    static_assert(PASSES == 1 || FORM != kQ4Silu, "SiLU epilogue: one output per thread");
     const uint32_t row = threadIdx.x % ROWS, qi = threadIdx.x / ROWS;
     // (which request: so that the 64 lanes of a wave read 64 different banks)
     constexpr uint32_t SB = 2 * NI;
@@ -334,10 +337,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         if (col < a.add_n_gamma) gamma_pre = a.add_gamma[col];
     // The RMSNorm that the producer of the activations left unfinished (ssq_in): a wave sums up the partials of
     // one or two requests, and the row group writes 1024 elements of the norm's own output at the end.
-    constexpr int RMS_N = 16 / WAVES;   // requests per wave, and elements per thread
+    constexpr int RMS_N = 16 * ZT / WAVES;   // requests per wave, and elements per thread
     constexpr int SSQ_NL = 2;           // partials per lane: up to 128 tiles, rows of 4096 (the host checks)
     [[maybe_unused]] float ssq_part[RMS_N][SSQ_NL] = {}, rms_h[RMS_N] = {}, rms_gamma[RMS_N];
-    const uint32_t rms_el = row_group * 1024 + threadIdx.x;
+    const uint32_t rms_el = row_group * (1024 * ZT) + threadIdx.x;
     if constexpr (BS) {
         if (a.ssq_in) {
 #pragma unroll
@@ -363,11 +366,11 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     struct QuadW {
         q4_u32x4 q[RT];
         q4_u32x2 d[RT];
-        float sc;   // BS: the scale of request l16 in block kg of the quad
+        float sc[ZT];   // BS: the scale of request l16 in block kg of the quad
         q4_u32x4 x[XQ];   // PACKED: the quad's activations
     };
     struct BlockX {
-        q4_half8 hi, lo;
+        q4_half8 hi[ZT], lo[ZT];
     };
     // Everything is fetched with buffer loads: a descriptor per stream in scalar registers and 32 bits per lane.  Their
     // descriptors end where the data does; what lies behind (the last blocks of an incomplete quad, the weights
@@ -380,15 +383,26 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         q_desc[r] = q4_buffer(a.q + tile * 64, end * 1024);
         d_desc[r] = q4_buffer(a.d + tile * 16, end * 128);
     }
-    const __amdgpu_buffer_rsrc_t x_desc = q4_buffer(a.xfrag + (size_t)(req0 / 32) * a.nblocks * 2048, a.nblocks * WIDTH * 128);
+    __amdgpu_buffer_rsrc_t x_desc[X_TILES];
+#pragma unroll
+    for (int t = 0; t < X_TILES; ++t) x_desc[t] = q4_buffer(a.xfrag + (size_t)(req0 / 32 + t) * a.nblocks * 2048, a.nblocks * WIDTH * 128);
     const __amdgpu_buffer_rsrc_t s_desc = q4_buffer(BS ? a.blk_scale + (size_t)(req0 / 32) * a.nblocks * 32 : nullptr, a.nblocks * 128);
-    // (request of this lane's row of the A operand; rows without one repeat another's)
-    const uint32_t xreq = min(l16 / 4 * NI + min(l16 % 4, (uint32_t)NI - 1u), live - 1u) + req0 % 32;
-    const uint32_t x_lane = (kg / 2 * 4 * WIDTH + kg % 2 * WIDTH + xreq) * 16;   // (two 16-column steps, hi and lo of each)
+    // (request of this lane's row of the A operand; rows without one repeat another's.  Four groups: more than 48 requests,
+    // so that the third and the fourth group's are in the second batch tile)
+    uint32_t x_lane[ZT];   // (two 16-column steps, hi and lo of each)
+#pragma unroll
+    for (int z = 0; z < ZT; ++z) {
+        const uint32_t xreq = min(l16 / 4 * NI + min(l16 % 4, (uint32_t)NI - 1u) + z * 16, live - 1u) + req0 % 32 - z / 2 * 32;
+        x_lane[z] = (kg / 2 * 4 * WIDTH + kg % 2 * WIDTH + xreq) * 16;
+    }
     const uint32_t s_lane = kg * 128 + (req0 % 32 + l16) * 4;
     auto load_w = [&](uint32_t quad, QuadW& k) __attribute__((always_inline)) {
         constexpr int NT = 2;   // (non-temporal: a weight is read once per launch and need not stay in the L2)
-        if constexpr (BS) k.sc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s_desc, quad * 512 + s_lane, 0, 0));
+        if constexpr (BS) {
+#pragma unroll
+            for (int z = 0; z < ZT; ++z)
+                k.sc[z] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s_desc, quad * 512 + s_lane + z * 64, 0, 0));
+        }
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             k.q[r] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_desc[r], quad * 1024 + lane * 16, 0, NT));
@@ -397,47 +411,55 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
         if constexpr (PACKED) {
 #pragma unroll
             for (int i = 0; i < XQ; ++i)
-                k.x[i] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_desc, quad * (XQ * 1024) + i * 1024 + lane * 16, 0, 0));
+                k.x[i] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_desc[0], quad * (XQ * 1024) + i * 1024 + lane * 16, 0, 0));
         }
         asm volatile("" ::: "memory");
     };
     auto load_x = [&](uint32_t blk, BlockX& k) __attribute__((always_inline)) {
         if constexpr (PACKED) return;
-        k.hi = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc, blk * 4096 + x_lane, 0, 0));
-        k.lo = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc, blk * 4096 + x_lane + 1024, 0, 0));
+#pragma unroll
+        for (int z = 0; z < ZT; ++z) {
+            k.hi[z] = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc[z / 2], blk * 4096 + x_lane[z], 0, 0));
+            k.lo[z] = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc[z / 2], blk * 4096 + x_lane[z] + 1024, 0, 0));
+        }
         asm volatile("" ::: "memory");
     };
     auto read_x = [&](int j, BlockX& k) __attribute__((always_inline)) {
-        const uint32_t piece = j * 8 * WIDTH + x_lane / 16;
-        k.hi = __builtin_bit_cast(q4_half8, packed[wave][piece]);
-        k.lo = __builtin_bit_cast(q4_half8, packed[wave][piece + 2 * WIDTH]);
+        const uint32_t piece = j * 8 * WIDTH + x_lane[0] / 16;
+        k.hi[0] = __builtin_bit_cast(q4_half8, packed[wave][piece]);
+        k.lo[0] = __builtin_bit_cast(q4_half8, packed[wave][piece + 2 * WIDTH]);
         asm volatile("" ::: "memory");
     };
     const uint32_t ones = q4_ones();
     q4_float4 zero;
 #pragma unroll
     for (int i = 0; i < 4; ++i) zero[i] = 0.f;
-    float acc[RT][NI] = {};
+    float acc[RT][ZT][NI] = {};
     auto multiply = [&](const QuadW& w, int j, const BlockX& x) __attribute__((always_inline)) {
         // (the scales of this lane's requests in block j, see `turn`)
-        [[maybe_unused]] float sc[NI];
+        [[maybe_unused]] float sc[ZT][NI];
         if constexpr (BS) {
 #pragma unroll
-            for (int i = 0; i < NI; ++i) sc[i] = scales[wave][j * 16 + kg * NI + i];
+            for (int z = 0; z < ZT; ++z)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) sc[z][i] = scales[wave][z][j * 16 + kg * NI + i];
         }
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             const q4_half2 dd = __builtin_bit_cast(q4_half2, (uint32_t)w.d[r][j / 2]);
             const float d = (float)dd[j % 2];
             const q4_half8 wk = q4_unpack(w.q[r][j], ones);
-            q4_float4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.hi, wk, zero, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.lo, wk, s, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) acc[r][i] = fmaf(BS ? d * sc[i] : d, s[i], acc[r][i]);
-            // (here, and not further down, where the compiler would move it: a quad's products do not fit
-            // the 128 registers a wave has)
+            for (int z = 0; z < ZT; ++z) {
+                q4_float4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.hi[z], wk, zero, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.lo[z], wk, s, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(acc[r][i]));
+                for (int i = 0; i < NI; ++i) acc[r][z][i] = fmaf(BS ? d * sc[z][i] : d, s[i], acc[r][z][i]);
+                // (here, and not further down, where the compiler would move it: a quad's products do not fit
+                // the 128 registers a wave has)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(acc[r][z][i]));
+            }
         }
         if constexpr (PACKED && RT == 4 && (WAVES == 16 || !BS)) __builtin_amdgcn_sched_barrier(0);   // (for the same reason)
     };
@@ -446,15 +468,17 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     // as 16 waves add up) to LDS, where the waves' sums meet anyway.  (2-norm error against float64, with one level -> now:
     // 9216 x 14336 at 17 requests 1.58e-7 -> 1.11e-7, 512 x 11008 at 33 1.22e-7 -> 1.07e-7, 28672 x 4096 at 17 1.10e-7 ->
     // 1.02e-7.  No measurable time; adding to LDS after every quad with ds_add costs 1.3 to 5 times the kernel.)
-    constexpr bool TWO_LEVELS = RT * NI <= 8;
-    [[maybe_unused]] float total[RT][NI] = {};
+    constexpr bool TWO_LEVELS = RT * NI * ZT <= 8;
+    [[maybe_unused]] float total[RT][ZT][NI] = {};
     [[maybe_unused]] uint32_t in_a_row = 0;
     [[maybe_unused]] bool flushed = false;
     auto each = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
-            for (int i = 0; i < NI; ++i) f(red[(wave * RT + r) * TILE_PITCH + i * 64 + lane], total[r][i], acc[r][i]);
+            for (int z = 0; z < ZT; ++z)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) f(red[((wave * RT + r) * ZT + z) * TILE_PITCH + i * 64 + lane], total[r][z][i], acc[r][z][i]);
     };
     auto flush = [&]() __attribute__((always_inline)) {
         if constexpr (TWO_LEVELS) each([](float&, float& sum, float& v) __attribute__((always_inline)) { sum += v; });
@@ -471,7 +495,10 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     QuadW w, next;
     BlockX x[XD];
     auto turn = [&](uint32_t quad, auto more) __attribute__((always_inline)) {
-        if constexpr (BS) scales[wave][lane] = w.sc;   // (a wave's own: LDS operations of a wave are in order)
+        if constexpr (BS) {   // (a wave's own: LDS operations of a wave are in order)
+#pragma unroll
+            for (int z = 0; z < ZT; ++z) scales[wave][z][lane] = w.sc[z];
+        }
         if constexpr (PACKED) {
 #pragma unroll
             for (int i = 0; i < XQ; ++i) packed[wave][i * 64 + lane] = w.x[i];
@@ -542,10 +569,11 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     }
     if (!has_out) return;   // (whole half waves where the epilogue works across lanes: 32 rows share q)
     auto sum_of = [&](uint32_t tile_row, uint32_t sq, float inv) __attribute__((always_inline)) {
-        const float* p = red + tile_row / 16 * TILE_PITCH + (sq % NI) * 64 + sq / NI * 16 + tile_row % 16;
+        const uint32_t s16 = sq % (4 * NI);
+        const float* p = red + (tile_row / 16 * ZT + sq / (4 * NI)) * TILE_PITCH + (s16 % NI) * 64 + s16 / NI * 16 + tile_row % 16;
         float sum[WAVES];   // (added up in pairs: fewer roundings on the way of each)
 #pragma unroll
-        for (int k = 0; k < WAVES; ++k) sum[k] = p[k * RT * TILE_PITCH];
+        for (int k = 0; k < WAVES; ++k) sum[k] = p[k * RT * ZT * TILE_PITCH];
 #pragma unroll
         for (int step = 1; step < WAVES; step *= 2)
 #pragma unroll
@@ -555,14 +583,19 @@ __global__ __launch_bounds__(WAVES * 64, 4) void q4_matmul_kernel(
     };
     if constexpr (FORM == kQ4Silu) {
         // the 32 lanes of a half wave hold one request's 32 columns, one block of the consuming matmul's K
-        const float gv = sum_of(row, q, inv_pre[0]), uv = sum_of(32 + row, q, inv_pre[0]);
-        const float prod = q4_silu_times(gv, uv);
-        store_through(&a.out[(size_t)b * a.rows + col], gv);
-        store_through(&a.out[(size_t)b * a.rows + a.ffn_inner + col], uv);
-        store_through(&a.gate[(size_t)b * a.ffn_inner + col], gv);
-        store_through(&a.up[(size_t)b * a.ffn_inner + col], uv);
-        store_through(&a.silu_out[(size_t)b * a.ffn_inner + col], prod);
-        if (a.split_frag) q4_emit_block(prod, b, col, a.ffn_inner, a.split_frag, a.split_blk_scale, WIDTH);
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) {
+            const uint32_t qp = q + p * PER_PASS, bp = b + p * PER_PASS;
+            if (qp >= live) break;
+            const float gv = sum_of(row, qp, inv_pre[p]), uv = sum_of(32 + row, qp, inv_pre[p]);
+            const float prod = q4_silu_times(gv, uv);
+            store_through(&a.out[(size_t)bp * a.rows + col], gv);
+            store_through(&a.out[(size_t)bp * a.rows + a.ffn_inner + col], uv);
+            store_through(&a.gate[(size_t)bp * a.ffn_inner + col], gv);
+            store_through(&a.up[(size_t)bp * a.ffn_inner + col], uv);
+            store_through(&a.silu_out[(size_t)bp * a.ffn_inner + col], prod);
+            if (a.split_frag) q4_emit_block(prod, bp, col, a.ffn_inner, a.split_frag, a.split_blk_scale, WIDTH);
+        }
         return;
     }
     float* out = a.out + (size_t)slice * a.batch * a.rows;

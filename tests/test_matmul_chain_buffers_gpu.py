@@ -21,6 +21,7 @@ def _weights(rng, rows, cols):
     # others still read theirs
     (64, (64, 2048, 4096, 8192), 2),
     (33, (160, 3072, 4096, 8192), 2),               # four tiles each, of 16 waves and at the end of 8
+    (21, (160, 4096, 10240), 1), (32, (160, 2048, 10240), 1),   # the reader's workgroups have two groups of requests each
     (16, (128, 512, 512, 1024, 512, 1024), 4),      # the buffers change three times
     (5, (64, 1024, 256, 4096), 2),                  # ... get narrower, and wider
 ])

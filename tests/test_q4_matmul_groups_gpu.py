@@ -31,6 +31,33 @@ def test_divisions(exe, rows, cols, batch):
     assert np.array_equal(got, q4.run(exe, f"groups_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride, sync=False))
 
 
+@pytest.mark.parametrize("rows,cols,batch", [
+    (10240, 160, 17), (10240, 1184, 32),      # two groups of 16 requests in a workgroup, the second with one request and full
+    (6144, 2080, 33), (6144, 160, 48), (28672, 96, 31),    # ... the last one missing, two rounds of the CUs
+    (10240, 96, 49), (10240, 1184, 64),       # four groups
+])
+def test_groups_that_share_a_workgroup(exe, rows, cols, batch):
+    q, x, stride = q4.make(rows, cols, batch, rows + cols + batch)
+    name = f"share_{rows}_{cols}_{batch}"
+    got = q4.run(exe, name, q, x, batch, rows, cols, stride)
+    check(got, q4.dequant(q, cols), x)
+    bad = batch - 17 if batch > 32 else batch - 1
+    x[bad] = np.inf                # stays in its row, also where the last quad of blocks is incomplete
+    keep = np.arange(batch) != bad
+    assert np.array_equal(got[keep], q4.run(exe, name, q, x, batch, rows, cols, stride)[keep])
+
+
+@pytest.mark.parametrize("batch", [17, 32, 49, 64])
+def test_silu_of_groups_that_share_a_workgroup(exe, batch):
+    c = silu.Case(batch, 160, 5120, 192, seed=batch)
+    got, n = silu._run(exe, c, "down", fuse=1)
+    assert n == (1, 1)
+    check(got["gate_up"], q4.dequant(c.w_gu, 160), c.x)
+    _, _, want = po.gate_up_split_silu_mul(got["gate_up"], batch, 5120, 10240)
+    assert np.max(np.abs(got["prod"] - want) / (np.abs(want) + 1e-30)) < 5e-6      # (as in test_matmul_silu_fusion_gpu.py)
+    check(got["down"], q4.dequant(c.w_down, 5120), got["prod"])
+
+
 @pytest.mark.parametrize("batch", [17, 32, 33, 64])    # four tiles per workgroup of 16 waves, of 8 from 33 requests on
 def test_rope_of_four_tiles(exe, batch):
     c = rope.Case(B=batch, H=40, Hkv=4, D=128, hid=1184, seed=batch)
