@@ -392,7 +392,9 @@ long mlc_hip_decode_table_uploads(void);
  *   "q4_ksplit"             K slices of the Q4_0 MFMA matmul (0 = automatic)
  *   "q4_int_operand"        1 (default) = the Q4_0 MFMA matmul multiplies the integers q - 8 and
  *                           applies the block scale to each block's sum in fp32; 0 = it
- *                           multiplies d * (q - 8) as an exact pair of fp16 numbers
+ *                           multiplies d * (q - 8) as an exact pair of fp16 numbers, always as a
+ *                           launch of its own ("fuse_row_ops" then fuses nothing into the matmuls
+ *                           but the split of their input)
  *   "fuse_row_ops"          1 (default) = row-local operators encoded back to back in a pass
  *                           (sum of matmul K slices, add, RMSNorm, gate/up SiLU, the fp16 split
  *                           of the next matmul's input) are collected and launched as one

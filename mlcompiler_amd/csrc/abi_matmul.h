@@ -23,7 +23,6 @@ Q4Slices q4_slices(size_t rows, size_t cols) {
     size_t n = (size_t)g.opt_q4_ksplit;
     if (n == 0) n = std::max<size_t>(1, std::min<size_t>((size_t)g.n_cu / (rows / 32), quads / 48));
     n = std::min(n, std::max<size_t>(1, nblocks / 16));
-    if (!g.opt_q4_int_operand) n = 1;
     const size_t per_slice = (quads + n - 1) / n;
     return {(quads + per_slice - 1) / per_slice, per_slice};
 }
@@ -239,11 +238,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         a.out = ksplit > 1 ? slices : o;
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)nblocks;
         a.nquads = (uint32_t)quads; a.quads_per_slice = (uint32_t)per_slice;
-        if (!g.opt_q4_int_operand) {
-            hipLaunchKernelGGL(q4_pairs_kernel, dim3((unsigned)(rows / 16), (unsigned)((bn + 15) / 16)), dim3(512), 0, g.stream, a);
-            continue;
-        }
-        if (g.opt_fuse_rows && !sync && ksplit == 1 && batch <= 64) {
+        if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && ksplit == 1 && batch <= 64) {
             // held back for one call: a split + RoPE + cast of this output becomes the epilogue
             Ctx::GemmPending& m = g.gemm;
             m.active = true;
@@ -257,7 +252,15 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             m.rows = rows;
             return finish(sync);
         }
-        if (!launch_q4(kQ4Plain, block_scales, ra, ksplit)) return 0;
+        if (!g.opt_q4_int_operand) {
+            const size_t z = (bn + 15) / 16, n_cu = (size_t)g.n_cu, pairs = rows / 64 * (z / 2) * ksplit;
+            const int rt = rows / 16 * z * ksplit > 2 * n_cu ? 4 : 1, zt = rt == 4 && z % 2 == 0 && pairs * 8 >= n_cu * 5 ? 2 : 1;
+            const auto kernel = zt == 2 ? q4_pairs_kernel<4, 2, 8> : rt == 4 ? q4_pairs_kernel<4, 1, 16> : q4_pairs_kernel<1, 1, 16>;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(rows / 16 / rt), (unsigned)(z / zt), (unsigned)ksplit), dim3(zt == 2 ? 512 : 1024), 0,
+                               g.stream, a);
+        } else if (!launch_q4(kQ4Plain, block_scales, ra, ksplit)) {
+            return 0;
+        }
         if (ksplit > 1) {
             const uint32_t n = (uint32_t)(bn * rows);
             if (g.opt_fuse_rows && batch <= 64 && rows <= 2 * kRowMaxLen) {

@@ -130,38 +130,79 @@ __global__ __launch_bounds__(256) void q4_repack_kernel(const uint8_t* __restric
 }
 
 // Option q4_int_operand = 0: the weights as exact fp16 pairs d * (q - 8) = w_hi + w_lo, three products per block.
-// One workgroup of 8 waves: 16 rows x 16 requests (grid y), all of K.
-__global__ __launch_bounds__(512) void q4_pairs_kernel(const Q4Args a) {
-    constexpr int WAVES = 8;
-    __shared__ float red[WAVES * 4 * 64];
+// One workgroup of 16 waves: RT tiles of 16 rows x ZT groups of 16 requests (grid y) x one K slice (grid z); a wave takes
+// every sixteenth quad of blocks.  A workgroup fetches 2 KB of activations per block and group beside a tile's 256 bytes of
+// weights, and 17 instructions make a weight word an operand: four tiles where there are workgroups for it, and then two
+// groups (8 waves: 132 registers) where those fill five eighths of the CUs.  (Whole calls, us, one tile and group, no quads ->
+// now: 28672 x 4096 at 1, 32 and 64 requests 50, 89, 160 -> 35, 46, 76; 4096 x 14336 at 64 96 -> 56; 2048 x 2048 at 32
+// 18.8 -> 17.2.)
+template <int RT, int ZT, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void q4_pairs_kernel(const Q4Args a) {
+    __shared__ float red[WAVES * RT * ZT * 4 * 64];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t lane = threadIdx.x % 64, l16 = lane % 16, kg = lane / 16;
-    const uint32_t tile = blockIdx.x, req0 = blockIdx.y * 16, live = min(16u, a.batch - req0);
-    const uint32_t width = frag_width(a.batch), req = req0 + min(l16, live - 1u);
-    q4_float4 acc;
+    const uint32_t tile0 = blockIdx.x * RT, req0 = blockIdx.y * (16 * ZT), live = min(16u * ZT, a.batch - req0);
+    const uint32_t width = frag_width(a.batch), cols = a.nblocks * 32;
+    const uint32_t end = min((blockIdx.z + 1) * a.quads_per_slice, a.nquads);
+    q4_float4 acc[RT][ZT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = 0.f;
-    for (uint32_t blk = wave; blk < a.nblocks; blk += WAVES) {
-        const size_t tq = (size_t)tile * a.nquads + blk / 4;
-        const uint32_t word = reinterpret_cast<const uint32_t*>(a.q)[(tq * 64 + lane) * 4 + blk % 4];
-        const _Float16 d = reinterpret_cast<const _Float16*>(a.d)[(tq * 16 + l16) * 4 + blk % 4];
-        const q4_half8 n = q4_unpack(word, 0x64006400u), d8 = {d, d, d, d, d, d, d, d};
-        const q4_half8 whi = d8 * n, wlo = __builtin_elementwise_fma(d8, n, -whi);
-        const q4_half8 hi = *reinterpret_cast<const q4_half8*>(a.xfrag + frag_piece(req, blk * 4 + kg, 0, a.nblocks * 32, width));
-        const q4_half8 lo = *reinterpret_cast<const q4_half8*>(a.xfrag + frag_piece(req, blk * 4 + kg, 1, a.nblocks * 32, width));
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, whi, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, whi, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, wlo, acc, 0, 0, 0);
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int z = 0; z < ZT; ++z)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[r][z][i] = 0.f;
+    for (uint32_t quad = blockIdx.z * a.quads_per_slice + wave; quad < end; quad += WAVES) {
+        uint4 word[RT];
+        uint2 scale[RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const size_t tq = (size_t)(tile0 + r) * a.nquads + quad;
+            word[r] = a.q[tq * 64 + lane];
+            scale[r] = a.d[tq * 16 + l16];
+        }
+        q4_half8 hi[4][ZT], lo[4][ZT];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {   // (a block that an incomplete quad lacks has scale 0: the last one again)
+            const uint32_t blk = min(quad * 4 + j, a.nblocks - 1u);
+#pragma unroll
+            for (uint32_t z = 0; z < ZT; ++z) {
+                const uint32_t req = req0 + min(z * 16 + l16, live - 1u);
+                hi[j][z] = *reinterpret_cast<const q4_half8*>(a.xfrag + frag_piece(req, blk * 4 + kg, 0, cols, width));
+                lo[j][z] = *reinterpret_cast<const q4_half8*>(a.xfrag + frag_piece(req, blk * 4 + kg, 1, cols, width));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                const uint32_t w = j == 0 ? word[r].x : j == 1 ? word[r].y : j == 2 ? word[r].z : word[r].w;
+                const _Float16 d = __builtin_bit_cast(q4_half2, j < 2 ? scale[r].x : scale[r].y)[j % 2];
+                const q4_half8 n = q4_unpack(w, 0x64006400u), d8 = {d, d, d, d, d, d, d, d};
+                const q4_half8 whi = d8 * n, wlo = __builtin_elementwise_fma(d8, n, -whi);
+#pragma unroll
+                for (int z = 0; z < ZT; ++z) {
+                    acc[r][z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[j][z], whi, acc[r][z], 0, 0, 0);
+                    acc[r][z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[j][z], whi, acc[r][z], 0, 0, 0);
+                    acc[r][z] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[j][z], wlo, acc[r][z], 0, 0, 0);
+                }
+            }
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[(wave * 4 + i) * 64 + lane] = acc[i];
-    __syncthreads();
-    const uint32_t i = threadIdx.x / 64, q = kg * 4 + i;
-    if (i >= 4 || q >= live) return;
-    float sum = 0.f;
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) sum += red[(w * 4 + i) * 64 + lane];
-    a.out[(size_t)(req0 + q) * a.rows + tile * 16 + l16] = sum * a.inv_scale[req0 + q];
+        for (int z = 0; z < ZT; ++z)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) red[(((wave * RT + r) * ZT + z) * 4 + i) * 64 + lane] = acc[r][z][i];
+    __syncthreads();
+    for (uint32_t o = threadIdx.x; o < RT * ZT * 256; o += WAVES * 64) {
+        const uint32_t r = o / (ZT * 256), z = o / 256 % ZT, i = o / 64 % 4, q = z * 16 + kg * 4 + i;
+        if (q >= live) continue;
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += red[(((w * RT + r) * ZT + z) * 4 + i) * 64 + lane];
+        a.out[((size_t)blockIdx.z * a.batch + req0 + q) * a.rows + (tile0 + r) * 16 + l16] = sum * a.inv_scale[req0 + q];
+    }
 }
 
 // out[i] = slice 0 + slice 1 + ... in that order, eight loads at a time: what this takes is the way to memory and back

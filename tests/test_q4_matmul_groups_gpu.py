@@ -47,6 +47,25 @@ def test_groups_that_share_a_workgroup(exe, rows, cols, batch):
     assert np.array_equal(got[keep], q4.run(exe, name, q, x, batch, rows, cols, stride)[keep])
 
 
+@pytest.mark.parametrize("rows,cols,batch,ksplit", [
+    (64, 96, 3, 0), (192, 2080, 17, 0),                       # one tile and group per workgroup; incomplete quads
+    (8256, 160, 5, 0), (10240, 1184, 33, 0),                  # four tiles
+    (10240, 160, 17, 0), (10240, 1184, 64, 0), (4160, 96, 100, 0),    # ... and two groups of requests
+    (512, 14336, 9, 0), (512, 4096, 21, 3), (192, 2080, 70, 2),       # K slices
+])
+def test_weights_as_pairs(exe, rows, cols, batch, ksplit):
+    q, x, stride = q4.make(rows, cols, batch, rows + cols + batch)
+    assert exe.setOption("q4_int_operand", 0) and exe.setOption("q4_ksplit", ksplit)
+    try:
+        got = q4.run(exe, f"pairs_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride)
+        again = q4.run(exe, f"pairs_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride, sync=False)
+    finally:
+        exe.setOption("q4_int_operand", 1)
+        exe.setOption("q4_ksplit", 0)
+    check(got, q4.dequant(q, cols), x)
+    assert np.array_equal(got, again)
+
+
 @pytest.mark.parametrize("batch", [17, 32, 49, 64])
 def test_silu_of_groups_that_share_a_workgroup(exe, batch):
     c = silu.Case(batch, 160, 5120, 192, seed=batch)
