@@ -70,13 +70,13 @@ def _run(exe, c: Case, form: str, fuse: int):
     return got, (exe.fusedMatmulSiluLaunches() - before[0], exe.fusedMatmulSiluSplitLaunches() - before[1])
 
 
-# fused where the gate/up rows make more than 256 tiles of 32 (two row tiles per workgroup)
+# fused where there are more than 8192 gate/up rows
 SHAPES = {
     "tinyllama": dict(B=32, hid=2048, ffn=5632, rows_out=2048, fused=True),
     "two_batch_tiles": dict(B=40, hid=256, ffn=4128, rows_out=192, fused=True),
     "ragged_batch": dict(B=5, hid=128, ffn=4160, rows_out=64, fused=True, spread=True),
     "down_not_split_over_k": dict(B=20, hid=64, ffn=4128, rows_out=8192 + 64, fused=True, spread=True),
-    # (two batch tiles and two row tiles per workgroup: no kernel for block-wise scales, the split stays a launch)
+    # (a wide reader of more than 32 requests takes no block-wise scales: the split stays a launch)
     "down_two_tiles_each_way": dict(B=33, hid=64, ffn=4128, rows_out=8192 + 64, fused=True, split=False, spread=True),
     "few_rows": dict(B=9, hid=256, ffn=512, rows_out=256, fused=False),
 }

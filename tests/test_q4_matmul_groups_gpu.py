@@ -1,5 +1,5 @@
 """Q4_0 matmuls of up to 64 requests at the edges of the kernel's division: 1, 2 or 4 accumulator registers per
-product (batches 4 | 5, 8 | 9), groups of 16 requests, incomplete quads of blocks, waves without a quad and with one or
+product (batches 4 | 5, 8 | 9), groups of 16 requests (one, two or four to a workgroup), incomplete quads of blocks, waves without a quad and with one or
 two, 1, 2 or 4 tiles of 16 rows per workgroup, 8 or 16 waves; and a matmul that both finishes one RMSNorm and
 carries the residual add of the next (its two norms have weights of their own)."""
 import numpy as np
@@ -20,7 +20,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("batch", [1, 4, 5, 8, 9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("rows,cols", [
     (64, 64),        # half a quad of blocks, most waves without one
-    (4160, 160),     # a quad and one block; two tiles per workgroup (one of 65 row groups)
+    (4160, 160),     # a quad and one block; two tiles per workgroup, four from 17 requests on (65 row groups)
     (192, 2080),     # 17 quads, the last incomplete: one wave has two
     (8256, 1184),    # wide: four tiles per workgroup, 16 waves (8 from 17 requests on), 10 quads
 ])
