@@ -111,8 +111,10 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
                     g.rows.len == cols && m.batch == batch && m.rows == cols && cols / 32 <= 128 &&
                     // (every thread of the reader writes at most one element of its z group's part of the norm)
                     batch * cols <= rows / (q4_wide(rows) ? 64 : 32) * 1024 &&
+                    // (in whichever form it will be launched), and its workgroups share no element: one slice of K
                     std::min<size_t>(batch, 16) * cols <=
-                        rows / 16 / q4_tiles(q4_wide(rows) ? kQ4Silu : kQ4Add, rows, batch, q4_slices(rows, cols).n) * 1024 &&
+                        rows / 16 / std::max(q4_tiles(q4_wide(rows) ? kQ4Silu : kQ4Add, rows, batch, 1), q4_tiles(kQ4Plain, rows, batch, 1)) * 1024 &&
+                    q4_slices(rows, cols).n == 1 &&
                     // The buffers of either launch lie apart, or exactly on each other where a thread has the same
                     // element of both: the held-back matmul's (it reads the addend before it writes anything),
                     !overlap(p.addend, row_bytes, m.out, row_bytes) && !shifted(p.add_out, m.out, row_bytes) &&

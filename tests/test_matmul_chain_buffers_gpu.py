@@ -199,6 +199,43 @@ def test_shared_buffers(exe, shared, batch):
         assert np.isfinite(want).all() and np.abs(out[1][m] - want).max() <= 1e-4 * np.abs(want).max(), m
 
 
+@pytest.mark.parametrize("batch,rows,ksplit", [(8, 1536, 6), (5, 1088, 8), (8, 1536, 1), (8, 1536, 0)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_norm_in_front_of_k_slices(exe, batch, rows, ksplit, in_place):
+    """A norm whose reader splits its K: every element is written, and once.  (Slices would each finish the norm, and have
+    fewer row groups than the other forms.)"""
+    rng = np.random.default_rng(ksplit)
+    n = 4096
+    w = [_weights(rng, n, 512), _weights(rng, rows, n)]
+    gamma = (1.0 + 0.3 * rng.standard_normal(n)).astype(np.float32)
+    init = {"x": rng.standard_normal((batch, 512)), "r": rng.standard_normal((batch, n)), "p": np.zeros((batch, n)),
+            "h": np.full((batch, n), np.nan), "n": np.full((batch, n), np.nan), "y": np.full((batch, rows), np.nan)}
+    dev = {m: _pool(exe, a.astype(np.float32)) for m, a in init.items()}
+    norm = dev["h" if in_place else "n"]
+    before = exe.fusedMatmulNormLaunches()
+    assert exe.setOption("q4_ksplit", ksplit)
+    try:
+        assert exe.beginForwardPassCB()
+        assert exe.encodeMatMulQ4_0Batched(f"sliced.{ksplit}.0", w[0], dev["x"], batch, n, 512, w[0].shape[1], 1, dev["p"]), exe.lastError()
+        assert exe.encodeAddBatched(dev["p"], dev["r"], dev["h"], batch * n)
+        assert exe.encodeRmsNormBatched(dev["h"], gamma, EPS, batch, n, norm)
+        assert exe.encodeMatMulQ4_0Batched(f"sliced.{ksplit}.{rows}", w[1], norm, batch, rows, n, w[1].shape[1], 1, dev["y"]), exe.lastError()
+        assert exe.flushForwardPassCB(), exe.lastError()
+        got = {m: _read(exe, b, np.empty(init[m].shape, np.float32)) for m, b in dev.items()}
+    finally:
+        exe.setOption("q4_ksplit", 0)
+        for buf in dev.values():
+            exe.releaseScratchBuffer(buf)
+    total = got["r"] + got["p"]
+    want = po.rms_norm_batched(total, gamma, EPS, batch, n)
+    if not in_place:
+        assert np.array_equal(got["h"], total)
+    a = got["h" if in_place else "n"]
+    assert (np.abs(a - want) <= 2e-6 * np.abs(want).max(axis=1, keepdims=True)).all()
+    check(got["y"], q4.dequant(w[1], n), a)
+    assert exe.fusedMatmulNormLaunches() - before == (1 if ksplit < 2 else 0)
+
+
 @pytest.mark.parametrize("over", ["sum", "norm"])
 @pytest.mark.parametrize("reader", ["silu", "rope", "rope_scatter"])
 def test_epilogues_over_the_norm(exe, reader, over):
