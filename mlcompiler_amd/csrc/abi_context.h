@@ -55,11 +55,11 @@ constexpr size_t kScratchReplayWordOffset = kStreamPartBytes + kScratchProbeByte
 constexpr size_t kScratchBytes = kScratchReplayWordOffset + 256;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-// First launch of every captured pass: moves the replay word on, so that the decode launches of
+// First launch of every captured pass: moves the replay word on, so that the launches of
 // this replay (whose arguments, tag included, are the same at every replay) use tags that the
 // replay before did not.
 __global__ void replay_word_kernel(uint32_t* word, uint32_t step) { *word += step; }
-constexpr uint32_t kReplayTagStep = 4096;   // decode launches of one captured pass, at most
+constexpr uint32_t kReplayTagStep = 4096;   // launches of one captured pass that need a tag, at most
 
 // Device copy of the flat page table (and, where the per-request arrays do not travel inside the
 // kernel arguments, of those arrays) as the tile-balanced decode kernel reads it; uploaded only
@@ -244,7 +244,7 @@ struct Ctx {
     char last_kernel[96] = "";   // kernel variant of the last decode launch (for benchmarks)
     int n_cu = 256;
     unsigned char* scratch_ptr = nullptr;   // device address of `scratch` on g.device
-    uint32_t next_tag = 0;                  // tag of the last tile-balanced decode launch (never zero)
+    uint32_t next_tag = 0;                  // tag of the last launch that needed one (never zero)
     // Every decode launch on this GPU uses the one scratch array, so launches on different
     // streams must follow each other: the stream of the last launch is remembered, and a launch
     // on another stream first waits for that one (one event, created at set-up; launches that
@@ -252,7 +252,7 @@ struct Ctx {
     hipStream_t scratch_stream = nullptr;
     bool scratch_in_use = false;
     hipEvent_t scratch_ev = nullptr;
-    // One word of pinned host memory that the decode kernel sets (through its device address) when a
+    // One word of pinned host memory that a kernel sets (through its device address) when a
     // merge gives up waiting for another workgroup's partial; looked at wherever the host has
     // waited for the stream.
     volatile uint32_t* fault_host = nullptr;
@@ -284,6 +284,7 @@ struct Ctx {
         int causal = 0;
         bool carried_kv = false;             // ... and does the step's KV write
         size_t n_decode = 0;                 // tile-balanced decode launches of the pass
+        size_t n_tags = 0;                   // launches of the pass that needed a tag
         uint64_t buffer_generation = 0;      // Ctx::buffer_generation when the pass was captured
         const void* rows_dev = nullptr;      // device copy of the KV write's page rows
         size_t rows_batch = 0, rows_page_size = 0;
@@ -399,6 +400,30 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 int settle_gemm(const RopeArgs* rope);
 
+// Numbers a launch whose workgroups leave each other tagged words.
+TagArgs next_tags() {
+    TagArgs t;
+    t.fault = g.fault_dev;
+    t.spin_limit = (uint32_t)g.opt_spin_limit;
+    t.test_flags = (uint32_t)g.opt_test_flags;
+    if (g_capturing) {
+        // the arguments of a captured launch are the same at every replay: its tag is its number in
+        // the pass plus the replay word, which the pass's first launch moves on by kReplayTagStep
+        t.tag = 0x80000000u | (uint32_t)g.cap.n_tags++;
+        t.tag_dev = reinterpret_cast<const uint32_t*>(g.scratch_ptr + kScratchReplayWordOffset);
+    } else {
+        if (++g.next_tag == 0) ++g.next_tag;   // (zero is what untouched memory holds)
+        t.tag = g.next_tag;
+        t.tag_dev = nullptr;
+    }
+    return t;
+}
+bool too_many_tags() {
+    if (!g_capturing || g.cap.n_tags <= kReplayTagStep) return false;
+    fail("capture: more launches in one pass than its tags can tell apart");
+    return true;
+}
+
 // Device copy of a small host blob, uploaded only when (kind, key, bytes) has not been seen
 // with this content.  The copy is ordered on the library stream, so kernels already enqueued
 // that read the previous content are not disturbed.  nullptr on failure (error recorded).
@@ -469,8 +494,12 @@ int q4_tiles(Q4Form form, size_t rows, size_t batch, size_t ksplit) {
 }
 
 // Launches q4_matmul_kernel in one of its forms.
-int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a, size_t ksplit = 1) {
-    const size_t tiles = a.rows / 16, z = (a.batch + 15) / 16, n_cu = (size_t)g.n_cu;
+int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a) {
+    const size_t tiles = a.rows / 16, z = (a.batch + 15) / 16, n_cu = (size_t)g.n_cu, ksplit = a.slices;
+    if (ksplit > 1) {
+        a.tags = next_tags();
+        if (too_many_tags()) return 0;
+    }
     const int rt = q4_tiles(form, a.rows, a.batch, ksplit);
     a.row_groups = (uint32_t)(tiles / rt);
     // Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; where there are more
@@ -637,9 +666,30 @@ int settle_before_rows() {
     return settle_kv();
 }
 
+// The held-back matmul's epilogue can do the pending chain's residual add of its output: the buffers lie apart, or exactly
+// on each other where a thread has the same element of both (it reads the addend before it writes anything).
+bool gemm_adds() {
+    const Ctx::GemmPending& m = g.gemm;
+    const RowProgram& p = g.rows.p;
+    const size_t bytes = m.batch * m.rows * 4;
+    return g.rows.active && m.active && !m.silu && !q4_wide(m.rows) && !g.kv.active && g.rows.batch == m.batch && g.rows.len == m.rows &&
+           p.src == m.out && p.n_slices == 1 && !p.src_store && !p.silu && p.addend && !p.frag &&
+           !overlap(p.addend, bytes, m.out, bytes) && !shifted(p.add_out, m.out, bytes) && !shifted(p.add_out, p.addend, bytes) &&
+           !meets_norm(m.a, p.add_out, bytes) && !meets_norm(m.a, p.addend, bytes, false);
+}
+
 int settle() {
-    if (!settle_before_rows()) return 0;
     Ctx::RowPending& r = g.rows;
+    if (r.active && !r.p.rms && gemm_adds()) {
+        // nothing but the add: 1.6 to 4 us for a launch of its own
+        g.gemm.a.add_resid = r.p.addend;
+        g.gemm.a.add_out = r.p.add_out;
+        g.gemm.a.ssq_out = nullptr;
+        g.gemm.a.split_frag = nullptr;
+        r.active = false;
+        ++g.row_launches;
+    }
+    if (!settle_before_rows()) return 0;
     if (!r.active) return 1;
     r.active = false;
     const RowProgram& p = r.p;
@@ -712,11 +762,11 @@ void rows_begin(const void* src, size_t batch, size_t len) {
     r.cur = src;
 }
 
-// After a wait for the stream: did a decode launch give up on a partial?
+// After a wait for the stream: did a launch give up on a partial?
 int check_fault() {
     if (g.fault_host && *g.fault_host) {
         *g.fault_host = 0;
-        return fail("decode: a workgroup gave up waiting for another workgroup's partial result; the outputs of this "
+        return fail("a workgroup gave up waiting for another workgroup's partial result; the outputs of this "
                     "pass are not valid (launches that share the library's scratch memory must not overlap)");
     }
     return 1;

@@ -342,19 +342,13 @@ void stream_fill_common(StreamArgs& a, const void* q, const void* k_pages, const
     a.v_pages = static_cast<const uint4*>(v_pages);
     a.o = static_cast<float*>(o);
     a.part = reinterpret_cast<uint64_t*>(g.scratch_ptr);
-    a.fault = g.fault_dev;
-    a.spin_limit = (uint32_t)g.opt_spin_limit;
-    a.test_flags = (uint32_t)g.opt_test_flags;
-    if (g_capturing) {
-        // the arguments of a captured launch are the same at every replay: its tag is its number in
-        // the pass plus the replay word, which the pass's first launch moves on by kReplayTagStep
-        a.tag = 0x80000000u | (uint32_t)g.cap.n_decode++;
-        a.tag_dev = reinterpret_cast<const uint32_t*>(g.scratch_ptr + kScratchReplayWordOffset);
-    } else {
-        if (++g.next_tag == 0) ++g.next_tag;   // (zero is what untouched memory holds)
-        a.tag = g.next_tag;
-        a.tag_dev = nullptr;
-    }
+    const TagArgs tags = next_tags();
+    a.fault = tags.fault;
+    a.spin_limit = tags.spin_limit;
+    a.test_flags = tags.test_flags;
+    a.tag = tags.tag;
+    a.tag_dev = tags.tag_dev;
+    if (g_capturing) ++g.cap.n_decode;
     a.batch = (uint32_t)B;
     a.num_heads = (uint32_t)H;
     a.kv_heads = (uint32_t)Hkv;

@@ -15,16 +15,29 @@ bool q4_fast_shape(size_t rows, size_t cols, size_t row_stride) {
 }
 
 // K slices of a Q4_0 matmul on the matrix cores and the quads of blocks in each.  K is split over workgroups (of 32 rows)
-// only where there are too few of them for the CUs and K is long: from 96 quads (K = 12288) on, so that each of a slice's
-// 16 waves keeps three.
+// where there are too few of them for the CUs, as far as that leaves a wave fewer quads in a row: a round of quads takes
+// a wave about 1.5 us, the slices' meeting inside the launch 0.8.  (Kernel times, us, one slice, or two summed by a
+// launch behind -> now: 2048 x 5632 with the residual add at one request 8.2 -> 5.8 (three slices), at 32 requests 10.5 -> 8.6;
+// 4096 x 4096 with it at 16 8.8 -> 7.6; 4096 x 14336 at 16 14.1 and 4.2 for sum and add -> 15.2.)
 struct Q4Slices { size_t n, quads; };
-Q4Slices q4_slices(size_t rows, size_t cols) {
-    const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
+Q4Slices q4_slices(size_t rows, size_t cols, size_t batch) {
+    const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4, n_cu = (size_t)g.n_cu, z = (batch + 15) / 16;
     size_t n = (size_t)g.opt_q4_ksplit;
-    if (n == 0) n = std::max<size_t>(1, std::min<size_t>((size_t)g.n_cu / (rows / 32), quads / 48));
-    n = std::min(n, std::max<size_t>(1, nblocks / 16));
+    if (n == 0 && !g.opt_q4_int_operand) n = std::min(n_cu / (rows / 32), quads / 48);
+    else if (n == 0) n = std::max(std::min(n_cu / (rows / 32 * z), (quads + 15) / 16), std::min(n_cu / (rows / 32), quads / 48));
+    n = std::max<size_t>(1, std::min(n, nblocks / 16));
     const size_t per_slice = (quads + n - 1) / n;
     return {(quads + per_slice - 1) / per_slice, per_slice};
+}
+
+// Where the slices of a matmul leave their sums (zeros to begin with: no launch's tag).
+uint64_t* q4_meet(size_t words) {
+    const size_t bytes = std::max<size_t>(words * 8, 2u << 20);
+    const auto it = g.cached.find("q4_k_meet");
+    const bool there = it != g.cached.end() && it->second.second >= bytes;
+    void* p = cached_buffer("q4_k_meet", bytes);
+    if (p && !there && hipMemsetAsync(p, 0, bytes, g.stream) != hipSuccess) return nullptr;
+    return static_cast<uint64_t*>(p);
 }
 
 // Copies weights to the device in the order of the library's stream (a plain hipMemcpy may return before the data is
@@ -103,24 +116,17 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
     const bool scales_fit = batch <= 32 || !q4_wide(rows);
     bool feeds_rms = false;
     if (feeds && scales_fit && g.gemm.active && g.opt_q4_int_operand) {
-        const Ctx::GemmPending& m = g.gemm;
         const RowProgram& p = g.rows.p;
         const size_t row_bytes = batch * cols * 4;
-        feeds_rms = !m.silu && !q4_wide(m.rows) && !g.kv.active && p.src == m.out && p.n_slices == 1 &&
-                    !p.src_store && !p.silu && p.addend && p.rms && !p.frag && g.rows.batch == batch &&
-                    g.rows.len == cols && m.batch == batch && m.rows == cols && cols / 32 <= 128 &&
-                    // (every thread of the reader writes at most one element of its z group's part of the norm)
+        feeds_rms = gemm_adds() && p.rms && g.rows.batch == batch && g.rows.len == cols && cols / 32 <= 128 &&
+                    // (as many elements as the reader's threads, over all requests: tests of the launch counts pin it)
                     batch * cols <= rows / (q4_wide(rows) ? 64 : 32) * 1024 &&
-                    // (in whichever form it will be launched), and its workgroups share no element: one slice of K
+                    // Every row group of the reader writes 1024 elements of its z group's part of the norm (in whichever
+                    // form it will be launched), and no element belongs to two: one slice of K,
                     std::min<size_t>(batch, 16) * cols <=
                         rows / 16 / std::max(q4_tiles(q4_wide(rows) ? kQ4Silu : kQ4Add, rows, batch, 1), q4_tiles(kQ4Plain, rows, batch, 1)) * 1024 &&
-                    q4_slices(rows, cols).n == 1 &&
-                    // The buffers of either launch lie apart, or exactly on each other where a thread has the same
-                    // element of both: the held-back matmul's (it reads the addend before it writes anything),
-                    !overlap(p.addend, row_bytes, m.out, row_bytes) && !shifted(p.add_out, m.out, row_bytes) &&
-                    !shifted(p.add_out, p.addend, row_bytes) && !meets_norm(m.a, p.add_out, row_bytes) &&
-                    !meets_norm(m.a, p.addend, row_bytes, false) &&
-                    // and this one's, which reads the sum and writes the norm.
+                    g.opt_q4_ksplit <= 1 &&
+                    // and its buffers lie apart, too: it reads the sum and writes the norm
                     !shifted(p.rms_out, p.add_out, row_bytes) && !overlap(out, batch * rows * 4, p.add_out, row_bytes) &&
                     !overlap(out, batch * rows * 4, p.rms_out, row_bytes);
     }
@@ -170,7 +176,9 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
 
     // MFMA path, one pass over at most 64 requests at a time.
     const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
-    const size_t ksplit = q4_slices(rows, cols).n, per_slice = q4_slices(rows, cols).quads;
+    const Q4Slices split = feeds_rms ? Q4Slices{1, quads} : q4_slices(rows, cols, std::min<size_t>(batch, 64));
+    const size_t ksplit = split.n, per_slice = split.quads;
+    const bool meet = ksplit > 1 && g.opt_q4_int_operand;   // (the slices' sums meet in the launch)
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;
@@ -227,8 +235,9 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
                                inv, (uint32_t)bn, (uint32_t)cols);
         }
         // (the chain has been launched: its K-slice source may be replaced now)
-        float* slices = ksplit > 1 ? static_cast<float*>(cached_buffer("q4_k_slices", ksplit * bn * rows * 4)) : nullptr;
-        if (ksplit > 1 && !slices) return fail("q4 matmul: scratch allocation failed");
+        float* slices = ksplit > 1 && !meet ? static_cast<float*>(cached_buffer("q4_k_slices", ksplit * bn * rows * 4)) : nullptr;
+        uint64_t* words = meet ? q4_meet((ksplit - 1) * bn * rows) : nullptr;
+        if (ksplit > 1 && !slices && !words) return fail("q4 matmul: scratch allocation failed");
         Q4RopeArgs ra;
         Q4Args& a = ra;
         a = norm;
@@ -237,10 +246,12 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         a.xfrag = frag;
         a.blk_scale = blk_scale;
         a.inv_scale = inv;
-        a.out = ksplit > 1 ? slices : o;
+        a.out = slices ? slices : o;
+        a.slices = (uint32_t)ksplit;
+        a.meet = words;
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)nblocks;
         a.nquads = (uint32_t)quads; a.quads_per_slice = (uint32_t)per_slice;
-        if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && ksplit == 1 && batch <= 64) {
+        if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && batch <= 64) {
             // held back for one call: a split + RoPE + cast of this output becomes the epilogue
             Ctx::GemmPending& m = g.gemm;
             m.active = true;
@@ -260,10 +271,10 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             const auto kernel = zt == 2 ? q4_pairs_kernel<4, 2, 8> : rt == 4 ? q4_pairs_kernel<4, 1, 16> : q4_pairs_kernel<1, 1, 16>;
             hipLaunchKernelGGL(kernel, dim3((unsigned)(rows / 16 / rt), (unsigned)(z / zt), (unsigned)ksplit), dim3(zt == 2 ? 512 : 1024), 0,
                                g.stream, a);
-        } else if (!launch_q4(kQ4Plain, block_scales, ra, ksplit)) {
+        } else if (!launch_q4(kQ4Plain, block_scales, ra)) {
             return 0;
         }
-        if (ksplit > 1) {
+        if (slices) {
             const uint32_t n = (uint32_t)(bn * rows);
             if (g.opt_fuse_rows && batch <= 64 && rows <= 2 * kRowMaxLen) {
                 // the sum over the slices starts the next chain: whatever row-local operator

@@ -125,7 +125,7 @@ int mlc_hip_gate_up_split_silu_mul(const void* gate_up, void* gate, void* up, vo
         Ctx::GemmPending& m = g.gemm;
         const size_t half_bytes = batch * ffn_inner * 4;
         if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && m.active && !m.silu && !g.rows.active && !g.kv.active &&
-            q4_wide(m.rows) && m.out == gate_up && m.batch == batch && m.rows == ffn_gate_up_rows &&
+            q4_wide(m.rows) && m.a.slices == 1 && m.out == gate_up && m.batch == batch && m.rows == ffn_gate_up_rows &&
             ffn_gate_up_rows == 2 * ffn_inner && ffn_inner % 32 == 0 && aligned16(gate) && aligned16(up) && aligned16(out) &&
             !meets_norm(m.a, gate, half_bytes) && !meets_norm(m.a, up, half_bytes) && !meets_norm(m.a, out, half_bytes)) {
             m.silu = true;

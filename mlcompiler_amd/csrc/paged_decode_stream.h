@@ -27,6 +27,7 @@
 
 #include "fragments.h"
 #include "paged_decode_kernels.h"
+#include "tagged_words.h"
 
 namespace mlc_hip {
 
@@ -177,15 +178,6 @@ __device__ __forceinline__ void sd_wait_vmcnt() {
 // Workgroup barrier that orders LDS traffic only (global -> LDS loads stay in flight across it).
 __device__ __forceinline__ void sd_barrier() {
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// A word of a partial: {value, tag}, written and read whole (64-bit relaxed atomics at device
-// scope: the store is written through to memory, the load bypasses the per-XCD L2 caches).
-__device__ __forceinline__ void st_tagged(uint64_t* p, uint64_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint64_t ld_tagged(const uint64_t* p) {
-    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // exclusive-to-inclusive prefix sum over the 64 lanes in six DPP steps (no LDS traffic)
@@ -1188,8 +1180,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     // are the lane's un-normalised outputs, word OPL carries m of head i in lane i < HPW and l of
     // head i - HPW in lanes HPW .. 2*HPW-1 (m in log2 units).
     constexpr int PW = OPL + 1;
-    const uint32_t tag_sum = a.tag + tag_add;
-    const uint32_t tag = tag_sum ? tag_sum : 0x9E3779B9u;   // (zero is what untouched memory holds)
+    const uint32_t tag = launch_tag(a.tag, tag_add);
     auto partial_of = [&](uint32_t wg) { return a.part + ((size_t)(wg * NW + (uint32_t)hg) * PW) * 64 + lane; };
     auto publish = [&](const float (&o_un)[OPL], const float (&m_all)[HPW], const float (&l_all)[HPW]) {
         uint64_t* dst = partial_of(w);
@@ -1250,7 +1241,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
                 }
                 if (__all(ok)) break;
                 if (++spins >= a.spin_limit) {   // a sharer never wrote: give up, tell the host
-                    if (lane == 0) __hip_atomic_store(a.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    if (lane == 0) report_fault(a.fault);
                     break;
                 }
             }

@@ -29,6 +29,7 @@
 
 #include "fragments.h"
 #include "store_through.h"
+#include "tagged_words.h"
 #include "paged_decode_kernels.h"
 #include "paged_rope_kernels.h"
 
@@ -51,15 +52,18 @@ struct Q4Args {
     const uint2* d;
     const _Float16* xfrag;      // split activations (fragments.h)
     const float* inv_scale;     // [batch]
-    float* out;                 // [batch][rows], or the slice buffer [ksplit][batch][rows]
-    uint32_t batch, rows, nblocks, nquads, quads_per_slice;
+    float* out;                 // [batch][rows]; q4_pairs_kernel with K slices: the slice buffer [slices][batch][rows]
+    uint32_t batch, rows, nblocks, nquads, quads_per_slice, slices;
+    // slices > 1: where the workgroups of all slices but the last leave their sums for those of the last
+    uint64_t* meet;             // [slices - 1][batch][rows] tagged words
+    TagArgs tags;
     // The grid's x dimension: row groups (of RT tiles) times z groups of 16 requests, see q4_matmul_kernel.
     uint32_t row_groups, z_groups;
     // Kernels built with BS: the activations were split with one power-of-two scale per (request,
     // block of 32 columns) instead of one per request: x = (hi + lo) * scale.  The scales are
     // [batch tile of 32][nblocks][32 requests]; inv_scale is not read.
     const float* blk_scale;
-    // SILU (ksplit == 1, rows = 2 * ffn_inner): the output is a fused gate/up row; row group j takes columns
+    // SILU (slices == 1, rows = 2 * ffn_inner): the output is a fused gate/up row; row group j takes columns
     // 32 j .. 32 j + 31 of the gate half and of the up half and its epilogue also does the gate/up split and
     // SiLU(gate) * up -> gate, up, silu_out ([batch][ffn_inner] each).  With split_frag set it goes on
     // to split the 32 products of every request into the fragments of the matmul that consumes
@@ -71,8 +75,8 @@ struct Q4Args {
     float* silu_out;
     _Float16* split_frag;
     float* split_blk_scale;
-    // ADD (32 or 64 rows per workgroup, ksplit == 1): the epilogue also does the residual add that follows
-    // the matmul (add_out = out + add_resid, [batch][rows]), leaves every request's sum of squares over
+    // ADD (32 or 64 rows per workgroup): the epilogue also does the residual add that follows
+    // the matmul (add_out = out + add_resid, [batch][rows]) and, with split_frag set, leaves every request's sum of squares over
     // every 32 columns in ssq_out[request][rows / 32] (the RMSNorm that follows is
     // finished by the matmul that reads it, see ssq_in) and writes add_out * add_gamma as the
     // split-fp16 fragments of that matmul (split_frag / split_blk_scale, K = rows).  add_gamma[c] for
@@ -95,7 +99,7 @@ struct Q4Args {
     const float* rms_gamma;     // as add_gamma
     uint32_t rms_n_gamma;
 };
-// ... and for the kernels built for ROPE (ksplit == 1, out is a fused qkv row of rope.qkv_rows = rows
+// ... and for the kernels built for ROPE (out is a fused qkv row of rope.qkv_rows = rows
 // floats per request), whose epilogue also does what qkv_split_rope_cast_kernel would do with that row.
 // (A type of its own: the launches without it need not carry its page rows.)
 struct Q4RopeArgs : Q4Args {
@@ -360,6 +364,8 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
             }
         }
     }
+    uint32_t tag_add = 0;
+    if (a.slices > 1 && a.tags.tag_dev) tag_add = *a.tags.tag_dev;
     asm volatile("" ::: "memory");
 
     // ---- main loop
@@ -599,22 +605,64 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         }
         return;
     }
-    float* out = a.out + (size_t)slice * a.batch * a.rows;
+    // K slices: all but the last leave their sums as tagged words and are done; the last one's workgroups, which the
+    // hardware starts behind them, add them to their own in slice order.  (The wait is bounded all the same.)
+    const uint32_t tag = launch_tag(a.tags.tag, tag_add);
+    if (slice + 1 < a.slices) {
+        if (a.tags.test_flags & 1u) return;
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) {
+            const uint32_t qp = q + p * PER_PASS, bp = b + p * PER_PASS;
+            if (qp >= live) break;
+            st_tagged(a.meet + ((size_t)slice * a.batch + bp) * a.rows + col,
+                      (uint64_t)tag << 32 | __float_as_uint(sum_of(row, qp, inv_pre[p])));
+        }
+        return;
+    }
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
         const uint32_t qp = q + p * PER_PASS, bp = b + p * PER_PASS;
         if (qp >= live) break;
-        const float val = sum_of(row, qp, inv_pre[p]);
-        store_through(&out[(size_t)bp * a.rows + col], val);
+        float val = sum_of(row, qp, inv_pre[p]);
+        if (a.slices > 1) {
+            constexpr uint32_t AT_ONCE = 4;
+            float others = 0.f;
+            uint32_t spins = 0;
+            for (uint32_t s0 = 0; s0 + 1 < a.slices; s0 += AT_ONCE) {
+                const uint64_t* src = a.meet + ((size_t)s0 * a.batch + bp) * a.rows + col;
+                uint64_t word[AT_ONCE];
+                for (;;) {
+                    bool ok = true;
+#pragma unroll
+                    for (uint32_t s = 0; s < AT_ONCE; ++s)
+                        if (s0 + s + 1 < a.slices) word[s] = ld_tagged(src + (size_t)s * a.batch * a.rows);
+#pragma unroll
+                    for (uint32_t s = 0; s < AT_ONCE; ++s)
+                        if (s0 + s + 1 < a.slices) ok = ok && (uint32_t)(word[s] >> 32) == tag;
+                    if (__all(ok)) break;
+                    if (++spins >= a.tags.spin_limit) {
+                        if (!ok) report_fault(a.tags.fault);
+                        break;
+                    }
+                }
+#pragma unroll
+                for (uint32_t s = 0; s < AT_ONCE; ++s)
+                    if (s0 + s + 1 < a.slices) others += __uint_as_float((uint32_t)word[s]);
+            }
+            val = others + val;
+        }
+        store_through(&a.out[(size_t)bp * a.rows + col], val);
         if constexpr (FORM == kQ4Rope) q4_rope_epilogue(a.rope, rope_pre[p], bp, col, val);   // (the lanes of a pair share b)
         if constexpr (FORM == kQ4Add) {
             // residual add, this request's sum of squares over a half wave's 32 columns, and h * gamma as the next
             // matmul's fragments
             const float hv = val + resid_pre[p];
             store_through(&a.add_out[(size_t)bp * a.rows + col], hv);
-            const float ssq = q4_half_wave_sum(hv * hv);
-            if (row % 32 == 0) store_through(&a.ssq_out[(size_t)bp * (a.rows / 32) + col / 32], ssq);
-            q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale, WIDTH);
+            if (a.split_frag) {   // (else the add is all)
+                const float ssq = q4_half_wave_sum(hv * hv);
+                if (row % 32 == 0) store_through(&a.ssq_out[(size_t)bp * (a.rows / 32) + col / 32], ssq);
+                q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale, WIDTH);
+            }
         }
     }
 }

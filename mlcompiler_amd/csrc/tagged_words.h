@@ -1,0 +1,41 @@
+// Words that workgroups of one launch leave each other in memory: {value, tag}, written and read whole (64-bit relaxed
+// atomics at device scope: the store is written through to memory, the load bypasses the per-XCD L2 caches).  The tag is
+// the launch's, never seen in the buffer before, so every word says by itself whether it has been written in this
+// launch: no order among the stores, no acknowledgement, no arrival counter, nothing to clear.  A word gets from one
+// workgroup to another in 0.5 us, on the same XCD or not.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace mlc_hip {
+
+__device__ __forceinline__ void st_tagged(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t ld_tagged(const uint64_t* p) {
+    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The tag of a launch: its own number, and in a captured pass, whose arguments are the same at every replay, the replay
+// word on top.  Never zero, which is what untouched memory holds.
+__device__ __forceinline__ uint32_t launch_tag(uint32_t tag, uint32_t replay_word) {
+    const uint32_t sum = tag + replay_word;
+    return sum ? sum : 0x9E3779B9u;
+}
+
+// Tells the host that a wait for such words was given up.
+__device__ __forceinline__ void report_fault(uint32_t* fault) {
+    __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// What a launch needs to know for it.
+struct TagArgs {
+    const uint32_t* tag_dev;    // null, or a device word that is added to `tag` (captured passes)
+    uint32_t* fault;            // host-visible word, set when a wait was given up
+    uint32_t tag;               // this launch's tag: differs from that of every earlier launch whose words may still lie there
+    uint32_t spin_limit;        // rounds a wait polls before it gives up
+    uint32_t test_flags;        // bit 0: words are not published (tests of the give-up path)
+};
+
+}  // namespace mlc_hip
