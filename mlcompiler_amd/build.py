@@ -31,6 +31,8 @@ STAMP_PATH = os.path.join(CSRC, "libmlc_hip.stamp")   # hash of the sources the 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-fno-honor-nans",
+    # the first 14 words of scalar kernel arguments arrive in registers with a wave (the Q4_0 matmul's first loads need no others)
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wno-inline-asm",  # the global->LDS load in paged_prefill_kernels.h names m0 as clobbered
 ]
 

@@ -11,8 +11,9 @@ bool MLC_CAT(launch_q4_matmul_, MLC_Q4_NI)(int form, int rt, int waves, int zt, 
     const Q4Args& plain = a;
 #define MLC_Q4Z(ZT, FORM, RT, WAVES, ARGS)                                                                                     \
     if (form == FORM && rt == RT && waves == WAVES && zt == ZT) {                                                              \
-        if (block_scales) hipLaunchKernelGGL((q4_matmul_kernel<MLC_Q4_NI, RT, WAVES, ZT < 4, FORM, ZT>), grid, dim3(WAVES * 64), 0, stream, ARGS); \
-        else hipLaunchKernelGGL((q4_matmul_kernel<MLC_Q4_NI, RT, WAVES, false, FORM, ZT>), grid, dim3(WAVES * 64), 0, stream, ARGS);             \
+        const auto kernel = block_scales ? q4_matmul_kernel<MLC_Q4_NI, RT, WAVES, ZT < 4, FORM, ZT> : q4_matmul_kernel<MLC_Q4_NI, RT, WAVES, false, FORM, ZT>; \
+        hipLaunchKernelGGL(kernel, grid, dim3(WAVES * 64), 0, stream, a.q, a.d, a.xfrag, a.blk_scale, a.ssq_in, a.nblocks, a.quads_per_slice, \
+                           a.row_groups, a.batch | a.z_groups << 16, ARGS);                                                     \
         return true;                                                                                                           \
     }
 #define MLC_Q4(...) MLC_Q4Z(1, __VA_ARGS__)

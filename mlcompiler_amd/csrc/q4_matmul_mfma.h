@@ -107,6 +107,8 @@ struct Q4RopeArgs : Q4Args {
 };
 static constexpr uint32_t kQ4RopeOffset = (sizeof(Q4Args) + alignof(RopeArgs) - 1) / alignof(RopeArgs) * alignof(RopeArgs);
 static_assert(sizeof(Q4RopeArgs) == kQ4RopeOffset + sizeof(RopeArgs), "where the kernel finds rope in its arguments");
+static constexpr uint32_t kQ4LeadBytes = 5 * 8 + 4 * 4;   // arguments in front of them
+static_assert(kQ4LeadBytes % alignof(Q4RopeArgs) == 0, "no padding behind them");
 
 // Maximum / sum over the 32 lanes of a half wave, every lane gets the result.
 __device__ __forceinline__ float q4_half_wave_max(float v) {
@@ -271,8 +273,15 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // fragments of 32 requests as they are for larger batches).  32 requests: qkv 7.5 -> 6.9,
 // gate/up 13.3 -> 13.3, a step 1 330 -> 1 199.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
 // a layer 140 -> 112.  2-norm error against float64 of rows of 2048 to 14336: 0.95e-7 .. 1.17e-7, before 1.03e-7 .. 1.62e-7.
+//
+// The arguments that the first loads need come in front and as scalars: they are in registers when a wave starts (kernel
+// argument preload, build.py), so that weights and activations are requested at once and what the epilogue reads, whose
+// addresses take a fetch of the other arguments, behind them.  (From the argument segment, epilogue first -> now: steps of
+// 22 layers of the 1 B shape 757 -> 740 us at one request, 1 160 -> 1 121 at 32, a layer of the 8 B shape at 16 109.2 -> 107.)
 template <int NI, int RT, int WAVES, bool BS, int FORM, int ZT = 1>
 __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
+    const uint4* const w_q, const uint2* const w_d, const _Float16* const xfrag, const float* const blk_scale, const float* const ssq_in,
+    const uint32_t nblocks, const uint32_t quads_per_slice, const uint32_t row_groups, const uint32_t batch_z,
     const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
     static_assert(FORM != kQ4Silu || RT == 4, "SiLU epilogue: 32 rows of gate and 32 of up");
     static_assert(FORM != kQ4Add || RT % 2 == 0, "residual add: whole blocks of the next matmul's K");
@@ -297,15 +306,16 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     __shared__ float rms_scale[BS ? QR : 1];         // BS with ssq_in: every request's RMSNorm factor
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t lane = threadIdx.x % 64, l16 = lane % 16, kg = lane / 16;
-    const uint32_t z8 = 8 * a.z_groups;
-    const uint32_t row_group = blockIdx.x / z8 * 8 + blockIdx.x % 8, zg = blockIdx.x / 8 % a.z_groups;
-    if (row_group >= a.row_groups) return;           // (the grid is a multiple of 8 row groups)
+    const uint32_t batch = batch_z & 0xFFFFu, z_groups = batch_z >> 16, nquads = (nblocks + 3) / 4;
+    const uint32_t z8 = 8 * z_groups;
+    const uint32_t row_group = blockIdx.x / z8 * 8 + blockIdx.x % 8, zg = blockIdx.x / 8 % z_groups;
+    if (row_group >= row_groups) return;           // (the grid is a multiple of 8 row groups)
     const uint32_t slice = blockIdx.y;
-    const uint32_t req0 = zg * (16 * ZT), live = min((uint32_t)QR, a.batch - req0);   // (the last group may be smaller)
+    const uint32_t req0 = zg * (16 * ZT), live = min((uint32_t)QR, batch - req0);   // (the last group may be smaller)
     // tile r of the workgroup
     const uint32_t tile0 = FORM == kQ4Silu ? row_group * 2 : row_group * RT;
     auto tile_of = [&](int r) __attribute__((always_inline)) {
-        return FORM == kQ4Silu && r >= 2 ? a.ffn_inner / 16 + tile0 + (uint32_t)r - 2u : tile0 + (uint32_t)r;
+        return FORM == kQ4Silu && r >= 2 ? row_groups * 2 + tile0 + (uint32_t)r - 2u : tile0 + (uint32_t)r;
     };
 
     // ---- thread -> output: row `row` of the workgroup's (SiLU: column of its 32), request req0 + q
@@ -320,54 +330,6 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     const bool has_out = qi < QR && q < live;
     const uint32_t b = req0 + q, col = tile0 * 16 + row;
 
-    // ---- what the epilogue reads besides the sums is fetched before the main loop, so that it adds no memory
-    // round trip to the kernel's tail
-    [[maybe_unused]] Q4RopeFetch rope_pre[PASSES];
-    [[maybe_unused]] float resid_pre[PASSES] = {}, gamma_pre = 1.0f, inv_pre[PASSES] = {};
-#pragma unroll
-    for (int p = 0; p < PASSES; ++p) {
-        const uint32_t bp = b + p * PER_PASS;
-        const bool has = has_out && q + p * PER_PASS < live;
-        if constexpr (FORM == kQ4Rope) {
-            rope_pre[p] = {1.0f, 0.0f, 0ull};
-            if (has) rope_pre[p] = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4RopeOffset), bp, col);
-        }
-        if constexpr (FORM == kQ4Add)
-            if (has) resid_pre[p] = a.add_resid[(size_t)bp * a.rows + col];
-        if constexpr (!BS)
-            if (has) inv_pre[p] = a.inv_scale[bp];
-    }
-    if constexpr (FORM == kQ4Add)
-        if (col < a.add_n_gamma) gamma_pre = a.add_gamma[col];
-    // The RMSNorm that the producer of the activations left unfinished (ssq_in): a wave sums up the partials of
-    // one or two requests, and the row group writes 1024 elements of the norm's own output at the end.
-    constexpr int RMS_N = 16 * ZT / WAVES;   // requests per wave, and elements per thread
-    constexpr int SSQ_NL = 2;           // partials per lane: up to 128 tiles, rows of 4096 (the host checks)
-    [[maybe_unused]] float ssq_part[RMS_N][SSQ_NL] = {}, rms_h[RMS_N] = {}, rms_gamma[RMS_N];
-    const uint32_t rms_el = row_group * (1024 * ZT) + threadIdx.x;
-    if constexpr (BS) {
-        if (a.ssq_in) {
-#pragma unroll
-            for (int n = 0; n < RMS_N; ++n) {
-                const uint32_t sq = wave + n * WAVES, el = rms_el + n * WAVES * 64;
-#pragma unroll
-                for (int j = 0; j < SSQ_NL; ++j) {
-                    const uint32_t tl = lane + j * 64;
-                    if (sq < live && tl < a.ssq_tiles) ssq_part[n][j] = a.ssq_in[(size_t)(req0 + sq) * a.ssq_tiles + tl];
-                }
-                rms_gamma[n] = 1.0f;
-                if (el < live * a.rms_len) {
-                    const uint32_t rc = el % a.rms_len;
-                    rms_h[n] = a.rms_src[(size_t)req0 * a.rms_len + el];
-                    if (rc < a.rms_n_gamma) rms_gamma[n] = a.rms_gamma[rc];
-                }
-            }
-        }
-    }
-    uint32_t tag_add = 0;
-    if (a.slices > 1 && a.tags.tag_dev) tag_add = *a.tags.tag_dev;
-    asm volatile("" ::: "memory");
-
     // ---- main loop
     struct QuadW {
         q4_u32x4 q[RT];
@@ -381,18 +343,18 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     // Everything is fetched with buffer loads: a descriptor per stream in scalar registers and 32 bits per lane.  Their
     // descriptors end where the data does; what lies behind (the last blocks of an incomplete quad, the weights
     // behind a wave's last quad) reads as zero.
-    const uint32_t first = slice * a.quads_per_slice + wave, end = min((slice + 1) * a.quads_per_slice, a.nquads);
+    const uint32_t first = slice * quads_per_slice + wave, end = min((slice + 1) * quads_per_slice, nquads);
     __amdgpu_buffer_rsrc_t q_desc[RT], d_desc[RT];
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
-        const size_t tile = (size_t)tile_of(r) * a.nquads;
-        q_desc[r] = q4_buffer(a.q + tile * 64, end * 1024);
-        d_desc[r] = q4_buffer(a.d + tile * 16, end * 128);
+        const size_t tile = (size_t)tile_of(r) * nquads;
+        q_desc[r] = q4_buffer(w_q + tile * 64, end * 1024);
+        d_desc[r] = q4_buffer(w_d + tile * 16, end * 128);
     }
     __amdgpu_buffer_rsrc_t x_desc[X_TILES];
 #pragma unroll
-    for (int t = 0; t < X_TILES; ++t) x_desc[t] = q4_buffer(a.xfrag + (size_t)(req0 / 32 + t) * a.nblocks * 2048, a.nblocks * WIDTH * 128);
-    const __amdgpu_buffer_rsrc_t s_desc = q4_buffer(BS ? a.blk_scale + (size_t)(req0 / 32) * a.nblocks * 32 : nullptr, a.nblocks * 128);
+    for (int t = 0; t < X_TILES; ++t) x_desc[t] = q4_buffer(xfrag + (size_t)(req0 / 32 + t) * nblocks * 2048, nblocks * WIDTH * 128);
+    const __amdgpu_buffer_rsrc_t s_desc = q4_buffer(BS ? blk_scale + (size_t)(req0 / 32) * nblocks * 32 : nullptr, nblocks * 128);
     // (request of this lane's row of the A operand; rows without one repeat another's.  Four groups: more than 48 requests,
     // so that the third and the fourth group's are in the second batch tile)
     uint32_t x_lane[ZT];   // (two 16-column steps, hi and lo of each)
@@ -526,8 +488,56 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         for (int i = 0; i < XD; ++i) load_x(first * 4 + i, x[i]);
         if (first + WAVES < end) load_w(first + WAVES, next);
     }
+    // ---- what the epilogue reads besides the sums is fetched before the main loop, so that it adds no memory
+    // round trip to the kernel's tail
+    [[maybe_unused]] Q4RopeFetch rope_pre[PASSES];
+    [[maybe_unused]] float resid_pre[PASSES] = {}, gamma_pre = 1.0f, inv_pre[PASSES] = {};
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+        const uint32_t bp = b + p * PER_PASS;
+        const bool has = has_out && q + p * PER_PASS < live;
+        if constexpr (FORM == kQ4Rope) {
+            rope_pre[p] = {1.0f, 0.0f, 0ull};
+            if (has) rope_pre[p] = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4LeadBytes + kQ4RopeOffset), bp, col);
+        }
+        if constexpr (FORM == kQ4Add)
+            if (has) resid_pre[p] = a.add_resid[(size_t)bp * a.rows + col];
+        if constexpr (!BS)
+            if (has) inv_pre[p] = a.inv_scale[bp];
+    }
+    if constexpr (FORM == kQ4Add)
+        if (col < a.add_n_gamma) gamma_pre = a.add_gamma[col];
+    // The RMSNorm that the producer of the activations left unfinished (ssq_in): a wave sums up the partials of
+    // one or two requests, and the row group writes 1024 elements of the norm's own output at the end.
+    constexpr int RMS_N = 16 * ZT / WAVES;   // requests per wave, and elements per thread
+    constexpr int SSQ_NL = 2;           // partials per lane: up to 128 tiles, rows of 4096 (the host checks)
+    [[maybe_unused]] float ssq_part[RMS_N][SSQ_NL] = {}, rms_h[RMS_N] = {}, rms_gamma[RMS_N];
+    const uint32_t rms_el = row_group * (1024 * ZT) + threadIdx.x;
     if constexpr (BS) {
-        if (a.ssq_in) {
+        if (ssq_in) {
+#pragma unroll
+            for (int n = 0; n < RMS_N; ++n) {
+                const uint32_t sq = wave + n * WAVES, el = rms_el + n * WAVES * 64;
+#pragma unroll
+                for (int j = 0; j < SSQ_NL; ++j) {
+                    const uint32_t tl = lane + j * 64;
+                    if (sq < live && tl < a.ssq_tiles) ssq_part[n][j] = ssq_in[(size_t)(req0 + sq) * a.ssq_tiles + tl];
+                }
+                rms_gamma[n] = 1.0f;
+                if (el < live * a.rms_len) {
+                    const uint32_t rc = el % a.rms_len;
+                    rms_h[n] = a.rms_src[(size_t)req0 * a.rms_len + el];
+                    if (rc < a.rms_n_gamma) rms_gamma[n] = a.rms_gamma[rc];
+                }
+            }
+        }
+    }
+    uint32_t tag_add = 0;   // (K slices of a captured pass)
+    if (a.slices > 1 && a.tags.tag_dev) tag_add = *a.tags.tag_dev;
+    asm volatile("" ::: "memory");
+
+    if constexpr (BS) {
+        if (ssq_in) {
 #pragma unroll
             for (int m = 0; m < RMS_N; ++m) {
                 float part = q4_half_wave_sum(ssq_part[m][0] + ssq_part[m][1]);
@@ -565,7 +575,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     __syncthreads();
     if constexpr (BS) {
         // the norm's own output: h * factor * gamma, the arithmetic of rms_norm_batched_kernel
-        if (a.ssq_in) {
+        if (ssq_in) {
 #pragma unroll
             for (int m = 0; m < RMS_N; ++m) {
                 const uint32_t el = rms_el + m * WAVES * 64;
@@ -585,7 +595,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         for (int step = 1; step < WAVES; step *= 2)
 #pragma unroll
             for (int k = 0; k < WAVES; k += 2 * step) sum[k] += sum[k + step];
-        if constexpr (BS) return a.ssq_in ? sum[0] * rms_scale[sq] : sum[0];
+        if constexpr (BS) return ssq_in ? sum[0] * rms_scale[sq] : sum[0];
         else return sum[0] * inv;
     };
     if constexpr (FORM == kQ4Silu) {
@@ -614,7 +624,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         for (int p = 0; p < PASSES; ++p) {
             const uint32_t qp = q + p * PER_PASS, bp = b + p * PER_PASS;
             if (qp >= live) break;
-            st_tagged(a.meet + ((size_t)slice * a.batch + bp) * a.rows + col,
+            st_tagged(a.meet + ((size_t)slice * batch + bp) * a.rows + col,
                       (uint64_t)tag << 32 | __float_as_uint(sum_of(row, qp, inv_pre[p])));
         }
         return;
@@ -629,13 +639,13 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
             float others = 0.f;
             uint32_t spins = 0;
             for (uint32_t s0 = 0; s0 + 1 < a.slices; s0 += AT_ONCE) {
-                const uint64_t* src = a.meet + ((size_t)s0 * a.batch + bp) * a.rows + col;
+                const uint64_t* src = a.meet + ((size_t)s0 * batch + bp) * a.rows + col;
                 uint64_t word[AT_ONCE];
                 for (;;) {
                     bool ok = true;
 #pragma unroll
                     for (uint32_t s = 0; s < AT_ONCE; ++s)
-                        if (s0 + s + 1 < a.slices) word[s] = ld_tagged(src + (size_t)s * a.batch * a.rows);
+                        if (s0 + s + 1 < a.slices) word[s] = ld_tagged(src + (size_t)s * batch * a.rows);
 #pragma unroll
                     for (uint32_t s = 0; s < AT_ONCE; ++s)
                         if (s0 + s + 1 < a.slices) ok = ok && (uint32_t)(word[s] >> 32) == tag;
