@@ -50,10 +50,12 @@ constexpr size_t stream_partial_bytes(size_t GP, size_t D, size_t NW) { return (
 // (Whole calls, one tile per workgroup where there were places -> now, us; 32 query and 4 KV heads of 64, one
 // request of 128, 1024, 2048, 4096, 8192 tokens: 16.7 -> 15.8, 19.7 -> 18.9, 23.7 -> 20.7, 31.8 -> 22.4,
 // 51.8 -> 26.4; 8 KV heads of 128, one request of 2048: 34.3 -> 23.4, four of 512: 23.6 -> 20.1.)
-__host__ __device__ __forceinline__ uint32_t stream_workgroups(uint32_t tiles_head, uint32_t nz_head, uint32_t kv_heads, uint32_t grid) {
+__host__ __device__ __forceinline__ uint32_t stream_least(uint32_t tiles_head, uint32_t nz_head) {
     const uint32_t twice = (uint32_t)(tiles_head * 4u > nz_head * 7u && tiles_head * 4u < nz_head * 9u);
-    const uint32_t least = twice + (uint32_t)(tiles_head > nz_head * 8u) + (uint32_t)(tiles_head >= nz_head * 48u) +
-                           (uint32_t)(tiles_head >= nz_head * 160u);
+    return twice + (uint32_t)(tiles_head > nz_head * 8u) + (uint32_t)(tiles_head >= nz_head * 48u) + (uint32_t)(tiles_head >= nz_head * 160u);
+}
+__host__ __device__ __forceinline__ uint32_t stream_workgroups(uint32_t tiles_head, uint32_t nz_head, uint32_t kv_heads, uint32_t grid) {
+    const uint32_t least = stream_least(tiles_head, nz_head);
     const uint32_t places = (tiles_head * kv_heads + (1u << least) - 1u) >> least;
     return grid < places ? grid : places;
 }
@@ -406,8 +408,14 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
     // [request][kv head][the pair's tiles, then PC units that stand for its end].
     const uint32_t T = tiles_head * Hkv;                       // the host keeps this below 2^31
     const uint32_t places = stream_workgroups(tiles_head, nz_head, Hkv, gridDim.x);
-    // (nothing to balance where every tile gets a workgroup of its own)
-    const uint32_t PC = T > places ? a.pair_cost : 0u;
+    // (nothing to balance where every tile gets a workgroup of its own, or where every pair is a whole number of least
+    // shares, whose ranges then end where pairs end: 10 tiles in each of four pairs, two to a workgroup, 8.7 -> 7.9 us a launch
+    // of a captured step; without the condition, where ranges cross pairs, calls of 2 to 8 requests took up to 1 us more)
+    uint32_t PC = T > places ? a.pair_cost : 0u;
+    if constexpr (SMALL) {
+        const uint32_t least = stream_least(tiles_head, nz_head);
+        if (T == places << least && __ballot((v_tiles & ((1u << least) - 1u)) != 0) == 0) PC = 0;
+    }
     const uint32_t UT = T + PC * nz_head * Hkv;                // ... and this
     const uint32_t W = places < UT ? places : UT;
     const uint32_t w = blockIdx.x;
@@ -1265,8 +1273,6 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         store_direct(po.orow, acc_o, l_run);
     };
 
-    // ---- the stream: the first NBUF tiles of the range go out together, then one tile per step
-    // into the stage the step before has left
     // ---- the step's KV write: this workgroup owns the last tile of every pair that ends in
     // its range, so it writes those pairs' slices of the new rows before it loads the tiles
     // that hold them.  A new row is its request's newest position, so it lies in the pair's
