@@ -298,7 +298,8 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
 namespace {
 
 bool q6k_fast_shape(size_t rows, size_t cols, size_t row_stride) {
-    return rows % 32 == 0 && cols % 256 == 0 && row_stride >= cols / 256 * 210;
+    // (the kernel addresses a tile's weights and a batch tile's fragments with 32 bits)
+    return rows % 32 == 0 && cols % 256 == 0 && cols <= (1u << 24) && row_stride >= cols / 256 * 210;
 }
 
 // Uploads the weight matrix on first use of its name (or when its size changed); shapes the
@@ -398,9 +399,7 @@ int mlc_hip_matmul_q6_k_batched(const char* weight_name, const void* weights, si
             return finish(sync);
     }
 
-    // matrix cores, at most 64 requests per pass; two row tiles per workgroup when one would give
-    // more workgroups than CUs (and the batch fits one batch tile)
-    const size_t tiles = rows / 32;
+    // matrix cores, at most 64 requests per pass
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;
@@ -425,12 +424,7 @@ int mlc_hip_matmul_q6_k_batched(const char* weight_name, const void* weights, si
         a.inv_scale = inv;
         a.out = static_cast<float*>(out) + bo * rows;
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)(cols / 256);
-        if (bpad == 32 && tiles > 256 && tiles % 2 == 0)
-            hipLaunchKernelGGL((q6_k_matmul_mfma_kernel<1, 2>), dim3((unsigned)(tiles / 2)), dim3(512), 0, g.stream, a);
-        else if (bpad == 32)
-            hipLaunchKernelGGL((q6_k_matmul_mfma_kernel<1, 1>), dim3((unsigned)tiles), dim3(512), 0, g.stream, a);
-        else
-            hipLaunchKernelGGL((q6_k_matmul_mfma_kernel<2, 1>), dim3((unsigned)tiles), dim3(512), 0, g.stream, a);
+        launch_q6k_matmul(a, (size_t)g.n_cu, g.stream);
     }
     return finish(sync);
 }
