@@ -43,7 +43,7 @@ int kv_copy(const void* src, void* dst, const uint32_t* page_table, size_t pages
     const size_t head_bytes = head_dim * dtype_bytes;
     if ((head_bytes % 16) == 0 && aligned16(src) && aligned16(dst)) {
         a.head_units = (uint32_t)(head_bytes / 16);
-        launch_kv_copy<uint4, TO_PAGES>(a);
+        launch_kv_copy<copy_u32x4, TO_PAGES>(a);
     } else {
         a.head_units = (uint32_t)head_dim;
         if (dtype_bytes == 4) launch_kv_copy<uint32_t, TO_PAGES>(a);

@@ -49,6 +49,10 @@ __global__ void scatter_kv_pair_kernel(const ScatterPairArgs a) {
 // row.  The page table travels inside the kernel arguments where it fits: a call of 1 500 tokens is
 // then one launch of 3 us instead of a copy of 3 us and the launch behind it.
 static constexpr size_t kKvCopyEmbPages = 960;
+// (16 bytes as a vector of the compiler's own: an array of HIP's uint4 was given a home in LDS, at an address made from the
+// dispatch packet, which lies in host memory.  Two scatters and two gathers of 8 heads of 128 halves, 4096 and 8192 tokens:
+// 115 and 123 us -> 61 and 72, of which 48 are four calls' launch and wait.)
+typedef uint32_t copy_u32x4 __attribute__((ext_vector_type(4)));
 struct KvCopyArgs {
     const void* src;
     void* dst;
