@@ -24,6 +24,7 @@
 #pragma once
 
 #include <cstddef>
+#include <type_traits>
 
 #include "fragments.h"
 #include "paged_decode_kernels.h"
@@ -1200,9 +1201,12 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
         for (int h = 0; h < HPW; ++h) x = lane == h ? m_all[h] : lane == HPW + h ? l_all[h] : x;
         st_tagged(dst + OPL * 64, hi | __float_as_uint(x));
     };
-    // Sums up the pair this workgroup ends: the partials of workgroups po.w_lo .. w-1, eight at a
-    // time, then this workgroup's own part.
-    constexpr int MUNR = 8;
+    // Sums up the pair this workgroup ends: the partials of workgroups po.w_lo .. w-1, four or eight at a
+    // time (the first round's loads are one trip through memory), then this workgroup's own part.  What this takes is the
+    // latency of its instructions, with one or two waves on a SIMD: hence one address for a round's partials and all weights of a
+    // round from one maximum.  (Whole calls, every partial fetched again in every round and folded one after the other ->
+    // now, us: 32 requests of 32/4 heads of 64 24.3 -> 23.6, 64 with the KV write 43.9 -> 43.0, 12 of 24/8 heads of 128 and pages
+    // of 16 32.8 -> 31.6.  Fetching places without a partial, too, instead of a branch: 25.0 at 32 requests.)
     auto merge_pair = [&](const PairOut& po, const float (&own_o)[OPL], const float (&own_m)[HPW],
                           const float (&own_l)[HPW]) {
         float acc_o[OPL], m_run[HPW], l_run[HPW];
@@ -1213,63 +1217,83 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             m_run[h] = kNegBig;
             l_run[h] = 0.f;
         }
-        auto fold = [&](const float (&o)[OPL], const float (&m)[HPW], const float (&l)[HPW]) {
-#pragma unroll
-            for (int h = 0; h < HPW; ++h) {
-                const float m_new = max_nn(m_run[h], m[h]);
-                const float keep = fast_exp2(m_run[h] - m_new);
-                const float wgt = fast_exp2(m[h] - m_new);
-                l_run[h] = l_run[h] * keep + l[h] * wgt;
-                m_run[h] = m_new;
-#pragma unroll
-                for (int kk = 0; kk < HPK; ++kk) acc_o[h * HPK + kk] = acc_o[h * HPK + kk] * keep + o[h * HPK + kk] * wgt;
-            }
-        };
         const uint32_t n_others = w - po.w_lo;
         uint32_t spins = 0;
-        for (uint32_t s0 = 0; s0 < n_others; s0 += MUNR) {
-            const uint32_t cnt = min((uint32_t)MUNR, n_others - s0);
-            uint64_t wd[MUNR][PW];
+        auto round = [&](uint32_t s0, auto places) {
+            constexpr int N = decltype(places)::value;
+            uint64_t wd[N][PW] = {};
+            uint32_t missing = (1u << min((uint32_t)N, n_others - s0)) - 1u;
+            const uint64_t* const src = a.part + ((size_t)((po.w_lo + s0) * NW + (uint32_t)hg) * PW) * 64 + lane;
             for (;;) {
-                bool ok = true;
+                // (only what has not come yet: every round goes to memory, beside the other workgroups' tiles)
 #pragma unroll
-                for (int u = 0; u < MUNR; ++u) {
-                    if ((uint32_t)u < cnt) {
-                        const uint64_t* src = partial_of(po.w_lo + s0 + (uint32_t)u);
+                for (int u = 0; u < N; ++u) {
+                    if (missing >> u & 1u) {
 #pragma unroll
-                        for (int k = 0; k < PW; ++k) wd[u][k] = ld_tagged(src + k * 64);
+                        for (int k = 0; k < PW; ++k) wd[u][k] = ld_tagged(src + (u * NW * PW + k) * 64);
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < MUNR; ++u) {
-                    if ((uint32_t)u < cnt) {
+                for (int u = 0; u < N; ++u) {
+                    bool ok = true;
 #pragma unroll
-                        for (int k = 0; k < PW; ++k) ok = ok && (uint32_t)(wd[u][k] >> 32) == tag;
-                    }
+                    for (int k = 0; k < PW; ++k) ok = ok && (uint32_t)(wd[u][k] >> 32) == tag;
+                    if (__all(ok)) missing &= ~(1u << u);
                 }
-                if (__all(ok)) break;
+                if (missing == 0) break;
                 if (++spins >= a.spin_limit) {   // a sharer never wrote: give up, tell the host
                     if (lane == 0) report_fault(a.fault);
                     break;
                 }
             }
+            float m[N][HPW], l[N][HPW];
 #pragma unroll
-            for (int u = 0; u < MUNR; ++u) {
-                if ((uint32_t)u < cnt) {
-                    float o[OPL], m[HPW], l[HPW];
+            for (int u = 0; u < N; ++u) {
+                const int x = (int)(uint32_t)wd[u][OPL];
+                const bool real = s0 + (uint32_t)u < n_others;
 #pragma unroll
-                    for (int k = 0; k < OPL; ++k) o[k] = __uint_as_float((uint32_t)wd[u][k]);
-                    const int x = (int)(uint32_t)wd[u][OPL];
-#pragma unroll
-                    for (int h = 0; h < HPW; ++h) {
-                        m[h] = __int_as_float(__builtin_amdgcn_readlane(x, h));
-                        l[h] = __int_as_float(__builtin_amdgcn_readlane(x, HPW + h));
-                    }
-                    fold(o, m, l);
+                for (int h = 0; h < HPW; ++h) {
+                    m[u][h] = real ? __int_as_float(__builtin_amdgcn_readlane(x, h)) : kNegBig;
+                    l[u][h] = real ? __int_as_float(__builtin_amdgcn_readlane(x, HPW + h)) : 0.f;
                 }
             }
+#pragma unroll
+            for (int h = 0; h < HPW; ++h) {
+                float top[N];
+#pragma unroll
+                for (int u = 0; u < N; ++u) top[u] = m[u][h];
+#pragma unroll
+                for (int step = 1; step < N; step *= 2)
+#pragma unroll
+                    for (int u = 0; u + step < N; u += 2 * step) top[u] = max_nn(top[u], top[u + step]);
+                const float m_new = max_nn(m_run[h], top[0]);
+                const float keep = fast_exp2(m_run[h] - m_new);
+                m_run[h] = m_new;
+                l_run[h] *= keep;
+#pragma unroll
+                for (int kk = 0; kk < HPK; ++kk) acc_o[h * HPK + kk] *= keep;
+#pragma unroll
+                for (int u = 0; u < N; ++u) {
+                    const float wgt = s0 + (uint32_t)u < n_others ? fast_exp2(m[u][h] - m_new) : 0.f;
+                    l_run[h] += l[u][h] * wgt;
+#pragma unroll
+                    for (int kk = 0; kk < HPK; ++kk) acc_o[h * HPK + kk] += __uint_as_float((uint32_t)wd[u][h * HPK + kk]) * wgt;
+                }
+            }
+        };
+        if (n_others - 1u < 4u) {
+            round(0u, std::integral_constant<int, 4>());
+        } else {
+            for (uint32_t s0 = 0; s0 < n_others; s0 += 8u) round(s0, std::integral_constant<int, 8>());
         }
-        fold(own_o, own_m, own_l);
+#pragma unroll
+        for (int h = 0; h < HPW; ++h) {
+            const float m_new = max_nn(m_run[h], own_m[h]);
+            const float keep = fast_exp2(m_run[h] - m_new), wgt = fast_exp2(own_m[h] - m_new);
+            l_run[h] = l_run[h] * keep + own_l[h] * wgt;
+#pragma unroll
+            for (int kk = 0; kk < HPK; ++kk) acc_o[h * HPK + kk] = acc_o[h * HPK + kk] * keep + own_o[h * HPK + kk] * wgt;
+        }
         store_direct(po.orow, acc_o, l_run);
     };
 
@@ -1424,8 +1448,17 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
 #ifndef MLC_NO_TAIL
             if (range_done && (kept || cur) && has_heads) {
                 MLC_PROBE(28);
-                if (kept) merge_pair(kept_po, kept_o, kept_m, kept_l);
-                else merge_pair(cur_po, o_un, m_all, l_all);
+                if (cur) {   // (one call: the code is long)
+                    kept_po = cur_po;
+#pragma unroll
+                    for (int i = 0; i < OPL; ++i) kept_o[i] = o_un[i];
+#pragma unroll
+                    for (int h = 0; h < HPW; ++h) {
+                        kept_m[h] = m_all[h];
+                        kept_l[h] = l_all[h];
+                    }
+                }
+                merge_pair(kept_po, kept_o, kept_m, kept_l);
             }
 #endif
             reset_state();
