@@ -26,6 +26,11 @@
 // this load): vector and matrix work together fill 80 % of the cycles.  Two row tiles per wave (half the
 // LDS reads, 79 us at 512 tokens, 238 against 243 at 2047) and three smaller workgroups per CU without the
 // overlap of blocks (64 us at 512, but 10 % behind on K = 14336 and on Q6_K) were measured as well.
+// Vector instructions per Q4_0 block and wave 75 -> 59 (addresses through buffer descriptors, nine instead of 13 for an
+// unpacked operand): 11264 x 2048 at 512 tokens 78.4 -> 75.8 us, at 2047 236.9 -> 228.6; 4096 x 14336 at 200 99.2 -> 95.2;
+// Q6_K 32000 x 2048 at 65 and 700 61.1 -> 59.7 and 255.7 -> 252.  Not kept then: a fresh product in place of clearing the
+// first-level sums, with a first level of 256 columns throughout (78 -> 81.6: another schedule); a higher priority for a wave
+// in its products (Q6_K at 65 tokens 58.8 -> 57.1, at 700 256 -> 270); the split's stores through the L2 (57 instead of 56).
 // Error against 64-bit products, 2-norm: 1.00e-7 to 1.4e-7 relative, before 1.03e-7 to 1.34e-7.
 #pragma once
 
@@ -107,51 +112,76 @@ __global__ __launch_bounds__(THREADS) void tokens_split_kernel(const float* __re
     }
 }
 
-// One stage's weights of one row tile: 4 k steps of 16 columns.
+// One stage's weights of one row tile: 4 k steps of 16 columns.  What a tile holds is read through buffer
+// descriptors: a lane's place in a stage is one register for good and the stage a scalar, where a 64-bit address costs
+// vector instructions per load.
 struct TokensQ4 {
     static constexpr int KSTEPS_PER_SCALE = 2, UNPACK = 0, VALU_PER_PRODUCT = 0;   // (the compiler's order)
     // (the layout is that of 16-row tiles and quads of blocks: a stage is half a quad, and k step s of its blocks
     // takes the column groups 2 s and 2 s + 1)
+    struct Place {
+        __amdgpu_buffer_rsrc_t q, d;
+        uint32_t q_lane, d_lane;
+        uint32_t ones;   // 0x64006400, in a vector register: with a literal, and + or are two instructions
+        __device__ __forceinline__ Place(const TokensArgs& a, uint32_t tile, uint32_t lane) {
+            const uint32_t nquads = (a.nblocks + 3) / 4, half = lane % 32 / 16;
+            q = q4_buffer(a.q + (size_t)tile * 2 * nquads * 128, 2 * nquads * 1024);
+            d = q4_buffer(a.d + (size_t)tile * 2 * nquads * 64, 2 * nquads * 128);
+            q_lane = half * nquads * 1024 + (lane / 32 * 16 + lane % 16) * 16;
+            d_lane = half * nquads * 128 + lane % 16 * 8;
+            ones = 0x64006400u;
+            asm volatile("" : "+v"(ones));
+        }
+    };
     uint2 q[2];     // [k step of a block]: a word per block
     q4_half2 d;     // a scale per block
     bool real;
-    __device__ __forceinline__ void load(const TokensArgs& a, uint32_t tile, uint32_t stage, uint32_t end, uint32_t lane) {
+    __device__ __forceinline__ void load(const TokensArgs& a, const Place& at, uint32_t stage, uint32_t end) {
         const uint32_t st = min(stage, a.stages - 1u);   // past the end: the last stage again, with scale 0
         real = stage < end;
-        const size_t tq = (size_t)(tile * 2 + lane % 32 / 16) * ((a.nblocks + 3) / 4) + st / 2;
 #pragma unroll
-        for (uint32_t s = 0; s < 2; ++s) q[s] = a.q[(tq * 64 + (s * 2 + lane / 32) * 16 + lane % 16) * 2 + st % 2];
-        d = reinterpret_cast<const q4_half2*>(a.d)[(tq * 16 + lane % 16) * 2 + st % 2];
+        for (uint32_t s = 0; s < 2; ++s)
+            q[s] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(at.q, at.q_lane + s * 512, st / 2 * 1024 + st % 2 * 8, 0));
+        d = __builtin_bit_cast(q4_half2, __builtin_amdgcn_raw_buffer_load_b32(at.d, at.d_lane, st / 2 * 128 + st % 2 * 4, 0));
     }
     static __device__ __forceinline__ uint32_t kstep(const TokensArgs& a, uint32_t stage, uint32_t k) {
         return min(stage * 2 + k / 2, a.nblocks - 1u) * 2 + (k & 1u);
     }
-    __device__ __forceinline__ q4_half8 operand(int k) const {
-        return q4_unpack(k < 2 ? q[k & 1].x : q[k & 1].y, 0x64006400u);
+    __device__ __forceinline__ q4_half8 operand(int k, const Place& at) const {
+        return q4_unpack(k < 2 ? q[k & 1].x : q[k & 1].y, at.ones);
     }
     __device__ __forceinline__ float scale(int k) const { return real ? (float)d[k / 2] : 0.0f; }
 };
 
 struct TokensQ6 {   // a stage is one group (see Q6KArgs): k step = quarter
     static constexpr int KSTEPS_PER_SCALE = 1, UNPACK = 12, VALU_PER_PRODUCT = 10;
+    struct Place {
+        __amdgpu_buffer_rsrc_t q, sc, d;
+        uint32_t lane;
+        __device__ __forceinline__ Place(const TokensArgs& a, uint32_t tile, uint32_t l) : lane(l) {
+            q = q4_buffer(a.q + (size_t)tile * a.stages * 192, a.stages * 1536);
+            sc = q4_buffer(a.sc + (size_t)tile * a.stages * 32, a.stages * 128);
+            d = q4_buffer(a.d + (size_t)tile * a.nblocks * 32, a.nblocks * 64);
+        }
+    };
     uint2 p[3];
     uint32_t s;
     _Float16 d;
     bool real;
-    __device__ __forceinline__ void load(const TokensArgs& a, uint32_t tile, uint32_t stage, uint32_t end, uint32_t lane) {
+    __device__ __forceinline__ void load(const TokensArgs& a, const Place& at, uint32_t stage, uint32_t end) {
         const uint32_t gi = min(stage, a.stages - 1u);
         real = stage < end;
-        const size_t tg = (size_t)tile * a.stages + gi;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) p[i] = a.q[(tg * 3 + i) * 64 + lane];
-        s = a.sc[tg * 32 + lane % 32];
-        d = a.d[((size_t)tile * a.nblocks + gi / 4) * 32 + lane % 32];
+        for (uint32_t i = 0; i < 3; ++i)
+            p[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(at.q, at.lane * 8 + i * 512, gi * 1536, 0));
+        s = __builtin_amdgcn_raw_buffer_load_b32(at.sc, at.lane % 32 * 4, gi * 128, 0);
+        d = __builtin_bit_cast(_Float16, __builtin_amdgcn_raw_buffer_load_b16(at.d, at.lane % 32 * 2, gi / 4 * 64, 0));
     }
     static __device__ __forceinline__ uint32_t kstep(const TokensArgs& a, uint32_t stage, uint32_t k) {
         const uint32_t gi = min(stage, a.stages - 1u);
         return gi / 4 * 16 + (gi / 2) % 2 * 8 + k * 2 + gi % 2;
     }
-    __device__ __forceinline__ q4_half8 operand(int k) const {
+    __device__ __forceinline__ q4_half8 operand(int k, const Place&) const {
         const uint2 ql = p[k & 1], qh = p[2];
         const uint32_t v0 = ((k >= 2 ? ql.x >> 4 : ql.x) & 0x0F0F0F0Fu) | (((qh.x >> (2 * k)) & 0x03030303u) << 4);
         const uint32_t v1 = ((k >= 2 ? ql.y >> 4 : ql.y) & 0x0F0F0F0Fu) | (((qh.y >> (2 * k)) & 0x03030303u) << 4);
@@ -193,6 +223,9 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[x][e] = total[x][e] = 0.f;
 
+    const typename W::Place at(a, tile_in, lane);
+    const __amdgpu_buffer_rsrc_t x_desc = q4_buffer(a.xfrag + (size_t)token_block * 2 * a.ksteps * 1024, 2 * a.ksteps * 2048);
+    // (the stage in the lane's offset: as a scalar offset Q6_K 32000 x 2048 at 700 tokens took 271 us instead of 256)
     q4_half8 st[2][2];   // this thread's part of the next stage: k step `wave`
     auto fetch_x = [&](uint32_t stage) __attribute__((always_inline)) {
         const uint32_t ks = W::kstep(a, stage, wave);
@@ -200,8 +233,8 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
         for (int x = 0; x < 2; ++x)
 #pragma unroll
             for (int p = 0; p < 2; ++p)
-                st[x][p] = *reinterpret_cast<const q4_half8*>(
-                    a.xfrag + ((((size_t)(token_block * 2 + x) * a.ksteps + ks) * 2 + p) * 64 + lane) * 8);
+                st[x][p] = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(
+                    x_desc, lane * 16 + p * 1024 + (x * a.ksteps + ks) * 2048, 0, 0));
     };
     auto store_x = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -218,8 +251,8 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
 
     W w[2];
     fetch_x(s0);
-    w[0].load(a, tile_in, s0, s1, lane);
-    w[1].load(a, tile_in, s0 + 1, s1, lane);
+    w[0].load(a, at, s0, s1);
+    w[1].load(a, at, s0 + 1, s1);
     asm volatile("" ::: "memory");   // (this and the ones below keep the loads where they are written)
     store_x(0);
     barrier();
@@ -253,7 +286,7 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
                         for (int x = 0; x < 2; ++x) xa[k][p][x] = xs[i % 2][x][step * KS + k][p][lane];
                 sc[n] = w[i % 2].scale(step * KS);
 #pragma unroll
-                for (int k = 0; k < KS; ++k) wk[k] = w[i % 2].operand(step * KS + k);
+                for (int k = 0; k < KS; ++k) wk[k] = w[i % 2].operand(step * KS + k, at);
 #pragma unroll
                 for (int x = 0; x < 2; ++x)
 #pragma unroll
@@ -277,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
                     }
                 }
             }
-            w[i % 2].load(a, tile_in, base + i + 2, s1, lane);
+            w[i % 2].load(a, at, base + i + 2, s1);
             asm volatile("" ::: "memory");
             store_x((i + 1) % 2);   // (last read before the barrier in front of this stage)
             barrier();
