@@ -9,6 +9,10 @@ namespace {
 // size for good (a buffer that grows would put an end to the captured passes).
 constexpr size_t kTokensFragBytes = 64u << 20, kTokensSliceBytes = 32u << 20;
 
+// The last round's K slices: at least so many stages each, at most so many of them, and what they leave each other (64 x 128
+// words of 8 bytes for each of fewer than `slots` workgroups).
+constexpr size_t kTokensTailStages = 8, kTokensTailSlices = 4, kTokensMeetBytes = 32u << 20;
+
 // How one piece is divided: K is split where the workgroups would leave CUs idle (two fit one), in whole groups of
 // 4 stages, and never into more slices than the buffer holds.
 struct TokensPlan {
@@ -21,17 +25,47 @@ TokensPlan tokens_plan(size_t wgs, size_t slots, size_t stages, size_t out_bytes
     return {(uint32_t)per, (stages + per - 1) / per};   // (rounding up leaves no more slices than before)
 }
 
+// The tiles left over by whole rounds of the slots: a quarter of a round or less leaves every CU one workgroup or none, and
+// two to a CU do more than one.  They go to several workgroups each, a slice of K for every one, whose sums meet inside the
+// launch.  That costs about 5 us, hence the longer K the more such tiles (whole calls, us, whole K / slices; Q4_0):
+//   tiles left | 16 stages   | 32 stages    | 64 stages     | 88, 224
+//   32         | 52.5 / 51.2 | 80.1 / 68.6  | 254.8 / 235.2 | 404 / 317 (8 slices at most: 312)
+//   64         | 51.4 / 51.3 | 77.9 / 69.7  |               | 177 / 152 (157)
+//   96         | 51.3 / 52.4 | 78.1 / 73.2  | 125.5 / 116.2 |
+//   128        | 50.7 / 53.0 | 76.5 / 77.8  | 124.8 / 119.0 | 388 / 357
+// 192 tiles in two slices (11264 x 2048, 512 tokens): 75.8 / 78.5.  Q6_K, 32 tiles, 32 stages: 82.4 / 72.2.
+struct TokensTail {
+    uint32_t whole, rest, slices, stages;
+};
+TokensTail tokens_tail(size_t wgs, size_t slots, size_t stages) {
+    const size_t rest = wgs % slots;
+    if (wgs < slots || rest == 0 || rest > std::min(slots / 4, 3 * stages)) return {(uint32_t)wgs, 0, 1, 0};
+    const size_t n = std::min({slots / rest, stages / kTokensTailStages, kTokensTailSlices});
+    if (n < 2) return {(uint32_t)wgs, 0, 1, 0};
+    const size_t per = ((stages + n - 1) / n + 3) / 4 * 4;
+    return {(uint32_t)(wgs - rest), (uint32_t)rest, (uint32_t)((stages + per - 1) / per), (uint32_t)per};
+}
+
+// Where they meet (zeros to begin with: no launch's tag).
+uint64_t* tokens_meet() {
+    const bool there = g.cached.count("tokens_k_meet");
+    void* p = cached_buffer("tokens_k_meet", kTokensMeetBytes);
+    if (p && !there && hipMemsetAsync(p, 0, kTokensMeetBytes, g.stream) != hipSuccess) return nullptr;
+    return static_cast<uint64_t*>(p);
+}
+
 // All tokens of a call with more than 64 in one launch per piece (matmul_tokens_kernels.h).
 // Returns 0 where the call has to go 64 requests at a time instead: workspaces not at hand.
 int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t batch, size_t rows, size_t cols) {
     const size_t piece = kTokensFragBytes / (4 * cols) / 64 * 64;
     if (piece == 0) return 0;
-    for (const char* name : {"tokens_x_fragments", "tokens_x_inv_scale", "tokens_k_slices"})
+    for (const char* name : {"tokens_x_fragments", "tokens_x_inv_scale", "tokens_k_slices", "tokens_k_meet"})
         if (g_capturing && !g.cached.count(name)) return 0;
     _Float16* frag = static_cast<_Float16*>(cached_buffer("tokens_x_fragments", kTokensFragBytes));
     float* inv = static_cast<float*>(cached_buffer("tokens_x_inv_scale", kTokensFragBytes / 64));   // (cols >= 64)
     float* slices = static_cast<float*>(cached_buffer("tokens_k_slices", kTokensSliceBytes));
-    if (!frag || !inv || !slices) return 0;
+    a.meet = tokens_meet();
+    if (!frag || !inv || !slices || !a.meet) return 0;
     a.xfrag = frag;
     a.inv_scale = inv;
     a.rows = (uint32_t)rows;
@@ -45,12 +79,21 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
         a.token_blocks = (uint32_t)((bn + 63) / 64);
         launch_tokens_split(in + bo * cols, frag, inv, (uint32_t)bn, (uint32_t)cols, a.token_blocks * 16, g.stream);
         const size_t wgs = (size_t)a.token_blocks * a.row_blocks;
-        const TokensPlan plan = tokens_plan(wgs, 2 * (size_t)g.n_cu, a.stages, bn * rows * 4);
+        const size_t slots = 2 * (size_t)g.n_cu;
+        const TokensPlan plan = tokens_plan(wgs, slots, a.stages, bn * rows * 4);
         a.stages_per_slice = plan.stages_per_slice;
         // (first-level sums of 4, 8 or 16 stages: about as many as there are of them)
         a.flush_mask = a.stages_per_slice <= 48 ? 0 : a.stages_per_slice <= 512 ? 1 : 3;
         a.out = plan.ksplit > 1 ? slices : o;
-        launch_matmul_tokens(q6, a, (unsigned)(wgs * plan.ksplit), g.stream);
+        const bool tags_left = !g_capturing || g.cap.n_tags < kReplayTagStep;
+        const TokensTail tail = plan.ksplit == 1 && tags_left && (slots - 1) * 65536 <= kTokensMeetBytes
+                                    ? tokens_tail(wgs, slots, a.stages) : TokensTail{(uint32_t)(wgs * plan.ksplit), 0, 1, 0};
+        a.whole = tail.whole;
+        a.rest = tail.rest;
+        a.tail_slices = tail.slices;
+        a.tail_stages = tail.stages;
+        a.tags = tail.rest ? next_tags() : TagArgs{};
+        launch_matmul_tokens(q6, a, tail.whole + tail.rest * tail.slices, g.stream);
         if (plan.ksplit > 1) {
             const uint32_t n = (uint32_t)(bn * rows);
             hipLaunchKernelGGL(q4_sum_slices_kernel, dim3((n + 255) / 256), dim3(256), 0, g.stream, slices, o, n,

@@ -17,7 +17,9 @@
 //     11264 x 2048 and 512 tokens);
 //   * fp32 sums are kept in two levels (4 stages = 256 columns or more, then those sums), so that an
 //     element is rounded no more often than in the waves' partial sums of the other kernels;
-//   * workgroups of one XCD share row blocks and groups of 8 token blocks.
+//   * workgroups of one XCD share row blocks and groups of 8 token blocks;
+//   * what is left over by whole rounds of workgroups is split over K where it is a small part of a round
+//     (tokens_tail): 4096 x 14336 at 1030 tokens 404 -> 317 us, 28672 x 4096 at 420 255 -> 235.
 // Measured (whole synchronous calls, before -> after, us): Q4_0 11264 x 2048 at 128 tokens 51 -> 48, 512
 // tokens 161 -> 81, 2047 tokens 609 -> 260; 2048 x 5632 at 512 tokens 171 -> 65; 2048 x 2048 at 2048 tokens
 // 443 -> 66; Q6_K 32000 x 2048 at 700 tokens 584 -> 281, at 65 tokens 94 -> 72.  Of the 512-token call the
@@ -203,11 +205,15 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
 
     // workgroup -> (slice, group of 8 token blocks, row block, token block); XCD x (workgroups x,
     // x + 8, ...) takes a contiguous run of that order
-    const uint32_t n = gridDim.x, xcd = blockIdx.x % 8, per = n / 8, rem = n % 8;
-    uint32_t t = xcd * per + min(xcd, rem) + blockIdx.x / 8;
+    const bool tail = blockIdx.x >= a.whole;
+    const uint32_t n = tail ? a.rest : a.whole, tail_slice = tail ? (blockIdx.x - a.whole) / a.rest : 0u;
+    const uint32_t id = tail ? (blockIdx.x - a.whole) - tail_slice * a.rest : blockIdx.x;
+    const uint32_t xcd = id % 8, per = n / 8, rem = n % 8;
+    uint32_t t = xcd * per + min(xcd, rem) + id / 8;
+    const uint32_t in_tail = t;
     const uint32_t per_k = a.token_blocks * a.row_blocks;
-    const uint32_t slice = t / per_k;
-    t -= slice * per_k;
+    const uint32_t slice = tail ? 0u : t / per_k;
+    t = tail ? a.whole + t : t - slice * per_k;
     const uint32_t group = t / (8 * a.row_blocks);
     t -= group * 8 * a.row_blocks;
     const uint32_t in_group = min(8u, a.token_blocks - group * 8);
@@ -215,7 +221,8 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
 
     const uint32_t tile = row_block * 4 + wave, tiles = a.rows / 32;
     const uint32_t tile_in = min(tile, tiles - 1u);   // (a tile past the end: the last one again, not stored)
-    const uint32_t s0 = slice * a.stages_per_slice, s1 = min(s0 + a.stages_per_slice, a.stages);
+    const uint32_t s0 = tail ? tail_slice * a.tail_stages : slice * a.stages_per_slice;
+    const uint32_t s1 = min(s0 + (tail ? a.tail_stages : a.stages_per_slice), a.stages);
 
     q4_float16 acc[2], total[2];
 #pragma unroll
@@ -328,6 +335,46 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
     }
 
     if (tile >= tiles) return;
+    if (tail) {
+        // (the hardware starts the slices of an XCD in order, so that nobody waits for a workgroup that is not running
+        // or done; the wait is bounded all the same)
+        const uint32_t tag = launch_tag(a.tags.tag, a.tags.tag_dev ? *a.tags.tag_dev : 0u);
+        uint64_t* const mine = a.meet + (size_t)in_tail * 8192 + wave * 2048 + lane;
+        if (tail_slice + 1 < a.tail_slices) {
+            if (a.tags.test_flags & 1u) return;
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    st_tagged(mine + (size_t)tail_slice * a.rest * 8192 + (x * 16 + e) * 64, (uint64_t)tag << 32 | __float_as_uint(total[x][e]));
+            return;
+        }
+        uint32_t spins = 0;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            float others[16] = {};
+            for (uint32_t sl = 0; sl + 1 < a.tail_slices; ++sl) {
+                const uint64_t* src = mine + (size_t)sl * a.rest * 8192 + x * 1024;
+                uint64_t word[16];
+                for (;;) {
+                    bool ok = true;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) word[e] = ld_tagged(src + e * 64);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) ok = ok && (uint32_t)(word[e] >> 32) == tag;
+                    if (__all(ok)) break;
+                    if (++spins >= a.tags.spin_limit) {
+                        if (!ok) report_fault(a.tags.fault);
+                        break;
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 16; ++e) others[e] += __uint_as_float((uint32_t)word[e]);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) total[x][e] = others[e] + total[x][e];
+        }
+    }
     // lane: weight row lane % 32 of the tile; register e: token (e/4)*8 + (lane/32)*4 + e%4
     float* out = a.out + (size_t)slice * a.tokens * a.rows + tile * 32 + lane % 32;
 #pragma unroll
