@@ -23,7 +23,7 @@
 // Measured (whole synchronous calls, before -> after, us): Q4_0 11264 x 2048 at 128 tokens 51 -> 48, 512
 // tokens 161 -> 81, 2047 tokens 609 -> 260; 2048 x 5632 at 512 tokens 171 -> 65; 2048 x 2048 at 2048 tokens
 // 443 -> 66; Q6_K 32000 x 2048 at 700 tokens 584 -> 281, at 65 tokens 94 -> 72.  Of the 512-token call the
-// kernel takes 70 us and the split 7 (before: 8 x (15.6 + 4.4)).  At 2047 tokens it does 777 TFLOP/s of fp16
+// kernel took 70 us (64 since) and the split 7 (before: 8 x (15.6 + 4.4)).  At 2047 tokens it did 777 TFLOP/s of fp16
 // products, where a large library product reaches 1 180 on the same card at the same clock (2.1 GHz under
 // this load): vector and matrix work together fill 80 % of the cycles.  Two row tiles per wave (half the
 // LDS reads, 79 us at 512 tokens, 238 against 243 at 2047) and three smaller workgroups per CU without the
