@@ -84,17 +84,23 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
         a.stages_per_slice = plan.stages_per_slice;
         // (first-level sums of 4, 8 or 16 stages: about as many as there are of them)
         a.flush_mask = a.stages_per_slice <= 48 ? 0 : a.stages_per_slice <= 512 ? 1 : 3;
-        a.out = plan.ksplit > 1 ? slices : o;
-        const bool tags_left = !g_capturing || g.cap.n_tags < kReplayTagStep;
-        const TokensTail tail = plan.ksplit == 1 && tags_left && (slots - 1) * 65536 <= kTokensMeetBytes
-                                    ? tokens_tail(wgs, slots, a.stages) : TokensTail{(uint32_t)(wgs * plan.ksplit), 0, 1, 0};
+        // All tiles in slices: they meet inside the launch too where they are few or short (rows x columns at tokens, summed by
+        // a kernel behind / in the launch, us: two slices 6144 x 4096 at 300 64.2 / 60.9, 11264 x 2048 at 128 45.1 / 41.7; four
+        // of 8 stages 2048 x 2048 at 512 42.3 / 39.2, of 16 4096 x 4096 at 256 47.8 / 47.4, of 24 2048 x 5632 at 512 56.6 /
+        // 58.4, of 56 4096 x 14336 at 200 98.5 / 100.3).
+        TokensTail tail{(uint32_t)(wgs * plan.ksplit), 0, 1, 0};
+        const bool meet = (!g_capturing || g.cap.n_tags < kReplayTagStep) && (slots - 1) * 65536 <= kTokensMeetBytes;
+        if (meet && plan.ksplit == 1) tail = tokens_tail(wgs, slots, a.stages);
+        else if (meet && plan.ksplit <= (plan.stages_per_slice <= 16 ? kTokensTailSlices : 3)) tail = {0, (uint32_t)wgs, (uint32_t)plan.ksplit, plan.stages_per_slice};
+        const bool sum = plan.ksplit > 1 && !tail.rest;
+        a.out = sum ? slices : o;
         a.whole = tail.whole;
         a.rest = tail.rest;
         a.tail_slices = tail.slices;
         a.tail_stages = tail.stages;
         a.tags = tail.rest ? next_tags() : TagArgs{};
         launch_matmul_tokens(q6, a, tail.whole + tail.rest * tail.slices, g.stream);
-        if (plan.ksplit > 1) {
+        if (sum) {
             const uint32_t n = (uint32_t)(bn * rows);
             hipLaunchKernelGGL(q4_sum_slices_kernel, dim3((n + 255) / 256), dim3(256), 0, g.stream, slices, o, n,
                                (uint32_t)plan.ksplit);

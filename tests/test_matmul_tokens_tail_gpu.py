@@ -18,6 +18,9 @@ pytestmark = pytest.mark.gpu
     ("q4", 8192, 2688, 640),     # ... K too short for so many
     ("q4", 6144, 1024, 1024),    # 256 left: none split
     ("q4", 4096, 960, 1030),     # too short to be split
+    ("q4", 2048, 2048, 500),     # all 128 tiles in four slices
+    ("q4", 6144, 2080, 300),     # 240 tiles in two, the second one shorter
+    ("q6", 4128, 768, 200),      # 132 tiles in three
     ("q6", 4128, 2048, 1000), ("q6", 6144, 1024, 700),
 ])
 def test_tail(exe, fmt, rows, cols, tokens):
