@@ -59,7 +59,7 @@ static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 // this replay (whose arguments, tag included, are the same at every replay) use tags that the
 // replay before did not.
 __global__ void replay_word_kernel(uint32_t* word, uint32_t step) { *word += step; }
-constexpr uint32_t kReplayTagStep = 4096;   // launches of one captured pass that need a tag, at most
+constexpr uint32_t kReplayTagStep = 4096;   // decode launches of one captured pass, at most, and sliced matmuls with a tag
 
 // Device copy of the flat page table (and, where the per-request arrays do not travel inside the
 // kernel arguments, of those arrays) as the tile-balanced decode kernel reads it; uploaded only
@@ -284,7 +284,7 @@ struct Ctx {
         int causal = 0;
         bool carried_kv = false;             // ... and does the step's KV write
         size_t n_decode = 0;                 // tile-balanced decode launches of the pass
-        size_t n_tags = 0;                   // launches of the pass that needed a tag
+        size_t n_sliced = 0;                 // matmuls of the pass whose K slices meet inside the launch
         uint64_t buffer_generation = 0;      // Ctx::buffer_generation when the pass was captured
         const void* rows_dev = nullptr;      // device copy of the KV write's page rows
         size_t rows_batch = 0, rows_page_size = 0;
@@ -400,8 +400,9 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 int settle_gemm(const RopeArgs* rope);
 
-// Numbers a launch whose workgroups leave each other tagged words.
-TagArgs next_tags() {
+// Numbers a launch whose workgroups leave each other tagged words.  `in_pass` counts those of its kind in a captured pass:
+// launches whose words lie in different buffers may have the same tag.
+TagArgs next_tags(size_t& in_pass) {
     TagArgs t;
     t.fault = g.fault_dev;
     t.spin_limit = (uint32_t)g.opt_spin_limit;
@@ -409,7 +410,7 @@ TagArgs next_tags() {
     if (g_capturing) {
         // the arguments of a captured launch are the same at every replay: its tag is its number in
         // the pass plus the replay word, which the pass's first launch moves on by kReplayTagStep
-        t.tag = 0x80000000u | (uint32_t)g.cap.n_tags++;
+        t.tag = 0x80000000u | (uint32_t)in_pass++;
         t.tag_dev = reinterpret_cast<const uint32_t*>(g.scratch_ptr + kScratchReplayWordOffset);
     } else {
         if (++g.next_tag == 0) ++g.next_tag;   // (zero is what untouched memory holds)
@@ -418,11 +419,7 @@ TagArgs next_tags() {
     }
     return t;
 }
-bool too_many_tags() {
-    if (!g_capturing || g.cap.n_tags <= kReplayTagStep) return false;
-    fail("capture: more launches in one pass than its tags can tell apart");
-    return true;
-}
+bool sliced_tags_left() { return !g_capturing || g.cap.n_sliced < kReplayTagStep; }
 
 // Device copy of a small host blob, uploaded only when (kind, key, bytes) has not been seen
 // with this content.  The copy is ordered on the library stream, so kernels already enqueued
@@ -496,10 +493,6 @@ int q4_tiles(Q4Form form, size_t rows, size_t batch, size_t ksplit) {
 // Launches q4_matmul_kernel in one of its forms.
 int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a) {
     const size_t tiles = a.rows / 16, z = (a.batch + 15) / 16, n_cu = (size_t)g.n_cu, ksplit = a.slices;
-    if (ksplit > 1) {
-        a.tags = next_tags();
-        if (too_many_tags()) return 0;
-    }
     const int rt = q4_tiles(form, a.rows, a.batch, ksplit);
     a.row_groups = (uint32_t)(tiles / rt);
     // Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; where there are more

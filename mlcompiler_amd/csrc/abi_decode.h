@@ -158,7 +158,8 @@ int mlc_hip_paged_attn_decode(const void* q, const void* k_pages, const void* v_
             a.new_k = static_cast<const uint4*>(g.kv.src[0]);
             a.new_v = static_cast<const uint4*>(g.kv.src[1]);
         }
-        if (too_many_tags()) return 0;
+        if (g_capturing && g.cap.n_decode > kReplayTagStep)
+            return fail("capture: more decode launches in one pass than its tags can tell apart");
         // Held back for one call where a Q4_0 matmul reading o could take its activations from
         // this launch (see Ctx::DecodePending); launched now otherwise.
         const size_t o_cols = num_heads * head_dim;

@@ -342,13 +342,12 @@ void stream_fill_common(StreamArgs& a, const void* q, const void* k_pages, const
     a.v_pages = static_cast<const uint4*>(v_pages);
     a.o = static_cast<float*>(o);
     a.part = reinterpret_cast<uint64_t*>(g.scratch_ptr);
-    const TagArgs tags = next_tags();
+    const TagArgs tags = next_tags(g.cap.n_decode);
     a.fault = tags.fault;
     a.spin_limit = tags.spin_limit;
     a.test_flags = tags.test_flags;
     a.tag = tags.tag;
     a.tag_dev = tags.tag_dev;
-    if (g_capturing) ++g.cap.n_decode;
     a.batch = (uint32_t)B;
     a.num_heads = (uint32_t)H;
     a.kv_heads = (uint32_t)Hkv;

@@ -176,9 +176,6 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
 
     // MFMA path, one pass over at most 64 requests at a time.
     const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
-    const Q4Slices split = feeds_rms ? Q4Slices{1, quads} : q4_slices(rows, cols, std::min<size_t>(batch, 64));
-    const size_t ksplit = split.n, per_slice = split.quads;
-    const bool meet = ksplit > 1 && g.opt_q4_int_operand;   // (the slices' sums meet in the launch)
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;
@@ -234,6 +231,11 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bn), dim3(256), 0, g.stream, xin, frag,
                                inv, (uint32_t)bn, (uint32_t)cols);
         }
+        // The slices' sums meet in the launch; a matmul that has no tag for that takes all of K.
+        const bool whole = feeds_rms || (g.opt_q4_int_operand && !sliced_tags_left());
+        const Q4Slices split = whole ? Q4Slices{1, quads} : q4_slices(rows, cols, std::min<size_t>(batch, 64));
+        const size_t ksplit = split.n, per_slice = split.quads;
+        const bool meet = ksplit > 1 && g.opt_q4_int_operand;
         // (the chain has been launched: its K-slice source may be replaced now)
         float* slices = ksplit > 1 && !meet ? static_cast<float*>(cached_buffer("q4_k_slices", ksplit * bn * rows * 4)) : nullptr;
         uint64_t* words = meet ? q4_meet((ksplit - 1) * bn * rows) : nullptr;
@@ -249,6 +251,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         a.out = slices ? slices : o;
         a.slices = (uint32_t)ksplit;
         a.meet = words;
+        if (meet) a.tags = next_tags(g.cap.n_sliced);
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)nblocks;
         a.nquads = (uint32_t)quads; a.quads_per_slice = (uint32_t)per_slice;
         if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && batch <= 64) {

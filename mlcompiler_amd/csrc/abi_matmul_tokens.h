@@ -89,7 +89,7 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
         // of 8 stages 2048 x 2048 at 512 42.3 / 39.2, of 16 4096 x 4096 at 256 47.8 / 47.4, of 24 2048 x 5632 at 512 56.6 /
         // 58.4, of 56 4096 x 14336 at 200 98.5 / 100.3).
         TokensTail tail{(uint32_t)(wgs * plan.ksplit), 0, 1, 0};
-        const bool meet = (!g_capturing || g.cap.n_tags < kReplayTagStep) && (slots - 1) * 65536 <= kTokensMeetBytes;
+        const bool meet = sliced_tags_left() && (slots - 1) * 65536 <= kTokensMeetBytes;
         if (meet && plan.ksplit == 1) tail = tokens_tail(wgs, slots, a.stages);
         else if (meet && plan.ksplit <= (plan.stages_per_slice <= 16 ? kTokensTailSlices : 3)) tail = {0, (uint32_t)wgs, (uint32_t)plan.ksplit, plan.stages_per_slice};
         const bool sum = plan.ksplit > 1 && !tail.rest;
@@ -98,7 +98,7 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
         a.rest = tail.rest;
         a.tail_slices = tail.slices;
         a.tail_stages = tail.stages;
-        a.tags = tail.rest ? next_tags() : TagArgs{};
+        a.tags = tail.rest ? next_tags(g.cap.n_sliced) : TagArgs{};
         launch_matmul_tokens(q6, a, tail.whole + tail.rest * tail.slices, g.stream);
         if (sum) {
             const uint32_t n = (uint32_t)(bn * rows);
