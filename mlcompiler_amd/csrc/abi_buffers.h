@@ -56,6 +56,21 @@ void* cached_buffer(const char* name, size_t bytes) {
     g.allocs[p] = bytes;
     return p;
 }
+
+// Words for the workgroups of a launch to meet in (tagged_words.h), zeros to begin with: no launch's tag.  Null where they
+// are not at hand and cannot be had, which includes any time while a pass is being captured.
+uint64_t* meeting_words(const char* name, size_t bytes) {
+    const auto it = g.cached.find(name);
+    if (it != g.cached.end() && it->second.second >= bytes) return static_cast<uint64_t*>(it->second.first);
+    if (g_capturing) return nullptr;
+    void* p = cached_buffer(name, bytes);
+    if (p && hipMemsetAsync(p, 0, bytes, g.stream) != hipSuccess) {
+        (void)hipGetLastError();
+        g.cached[name].second = 0;   // (as good as not there)
+        return nullptr;
+    }
+    return static_cast<uint64_t*>(p);
+}
 }  // namespace
 
 void* mlc_hip_cached(const char* name, size_t bytes) {

@@ -30,16 +30,6 @@ Q4Slices q4_slices(size_t rows, size_t cols, size_t batch) {
     return {(quads + per_slice - 1) / per_slice, per_slice};
 }
 
-// Where the slices of a matmul leave their sums (zeros to begin with: no launch's tag).
-uint64_t* q4_meet(size_t words) {
-    const size_t bytes = std::max<size_t>(words * 8, 2u << 20);
-    const auto it = g.cached.find("q4_k_meet");
-    const bool there = it != g.cached.end() && it->second.second >= bytes;
-    void* p = cached_buffer("q4_k_meet", bytes);
-    if (p && !there && hipMemsetAsync(p, 0, bytes, g.stream) != hipSuccess) return nullptr;
-    return static_cast<uint64_t*>(p);
-}
-
 // Copies weights to the device in the order of the library's stream (a plain hipMemcpy may return before the data is
 // there, and the library's stream does not wait for it), and waits.
 bool upload_weights(void* dst, const void* host, size_t bytes) {
@@ -231,14 +221,16 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bn), dim3(256), 0, g.stream, xin, frag,
                                inv, (uint32_t)bn, (uint32_t)cols);
         }
-        // The slices' sums meet in the launch; a matmul that has no tag for that takes all of K.
-        const bool whole = feeds_rms || (g.opt_q4_int_operand && !sliced_tags_left());
-        const Q4Slices split = whole ? Q4Slices{1, quads} : q4_slices(rows, cols, std::min<size_t>(batch, 64));
+        // The slices' sums meet in the launch; a matmul that has no tag or no memory for that takes all of K.  (Everything
+        // held back has been launched: buffers that it reads may be replaced now.)
+        Q4Slices split = feeds_rms ? Q4Slices{1, quads} : q4_slices(rows, cols, std::min<size_t>(batch, 64));
+        uint64_t* words = nullptr;
+        if (split.n > 1 && g.opt_q4_int_operand) {
+            if (sliced_tags_left()) words = meeting_words("q4_k_meet", std::max<size_t>((split.n - 1) * bn * rows * 8, 2u << 20));
+            if (!words) split = {1, quads};
+        }
         const size_t ksplit = split.n, per_slice = split.quads;
-        const bool meet = ksplit > 1 && g.opt_q4_int_operand;
-        // (the chain has been launched: its K-slice source may be replaced now)
-        float* slices = ksplit > 1 && !meet ? static_cast<float*>(cached_buffer("q4_k_slices", ksplit * bn * rows * 4)) : nullptr;
-        uint64_t* words = meet ? q4_meet((ksplit - 1) * bn * rows) : nullptr;
+        float* slices = ksplit > 1 && !words ? static_cast<float*>(cached_buffer("q4_k_slices", ksplit * bn * rows * 4)) : nullptr;
         if (ksplit > 1 && !slices && !words) return fail("q4 matmul: scratch allocation failed");
         Q4RopeArgs ra;
         Q4Args& a = ra;
@@ -251,7 +243,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         a.out = slices ? slices : o;
         a.slices = (uint32_t)ksplit;
         a.meet = words;
-        if (meet) a.tags = next_tags(g.cap.n_sliced);
+        if (words) a.tags = next_tags(g.cap.n_sliced);
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)nblocks;
         a.nquads = (uint32_t)quads; a.quads_per_slice = (uint32_t)per_slice;
         if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && batch <= 64) {

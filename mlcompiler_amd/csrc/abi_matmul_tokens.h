@@ -46,14 +46,6 @@ TokensTail tokens_tail(size_t wgs, size_t slots, size_t stages) {
     return {(uint32_t)(wgs - rest), (uint32_t)rest, (uint32_t)((stages + per - 1) / per), (uint32_t)per};
 }
 
-// Where they meet (zeros to begin with: no launch's tag).
-uint64_t* tokens_meet() {
-    const bool there = g.cached.count("tokens_k_meet");
-    void* p = cached_buffer("tokens_k_meet", kTokensMeetBytes);
-    if (p && !there && hipMemsetAsync(p, 0, kTokensMeetBytes, g.stream) != hipSuccess) return nullptr;
-    return static_cast<uint64_t*>(p);
-}
-
 // All tokens of a call with more than 64 in one launch per piece (matmul_tokens_kernels.h).
 // Returns 0 where the call has to go 64 requests at a time instead: workspaces not at hand.
 int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t batch, size_t rows, size_t cols) {
@@ -64,7 +56,7 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
     _Float16* frag = static_cast<_Float16*>(cached_buffer("tokens_x_fragments", kTokensFragBytes));
     float* inv = static_cast<float*>(cached_buffer("tokens_x_inv_scale", kTokensFragBytes / 64));   // (cols >= 64)
     float* slices = static_cast<float*>(cached_buffer("tokens_k_slices", kTokensSliceBytes));
-    a.meet = tokens_meet();
+    a.meet = meeting_words("tokens_k_meet", kTokensMeetBytes);
     if (!frag || !inv || !slices || !a.meet) return 0;
     a.xfrag = frag;
     a.inv_scale = inv;

@@ -42,3 +42,31 @@ def test_more_sliced_matmuls_in_a_captured_pass_than_tags(exe):
             exe.captureRelease(handle)
         exe.releaseScratchBuffer(d_x)
         exe.releaseScratchBuffer(d_y)
+
+
+def test_slices_without_room_for_their_words_in_a_captured_pass(exe):
+    """Captured with more requests than have been seen: the words' buffer cannot grow, and the matmul takes all of K."""
+    rng = np.random.default_rng(2)
+    rows, cols = 512, 32768
+    w, x = _weights(rng, rows, cols), rng.standard_normal((64, cols)).astype(np.float32)
+    d_x, d_y = _pool(exe, x), exe.allocateScratchBuffer(64 * rows * 4)
+    call = lambda batch: exe.encodeMatMulQ4_0Batched("meet.room", w, d_x, batch, rows, cols, w.shape[1], 1, d_y)
+    handle = 0
+    try:
+        assert exe.setOption("q4_ksplit", 64)     # (more words than any other call needs)
+        assert exe.beginForwardPassCB() and call(33) and exe.flushForwardPassCB(), exe.lastError()
+        assert exe.beginForwardPassCB() and exe.captureBegin()
+        ok = call(64)
+        handle = exe.captureEnd()
+        assert ok and handle > 0, exe.lastError()
+        assert exe.flushForwardPassCB()
+        for _ in range(2):
+            assert exe.uploadToBuffer(d_y, np.full((64, rows), np.nan, np.float32))
+            assert exe.beginForwardPassCB() and exe.replay(handle) and exe.flushForwardPassCB(), exe.lastError()
+            check(_read(exe, d_y, np.empty((64, rows), np.float32)), q4.dequant(w, cols), x)
+    finally:
+        exe.setOption("q4_ksplit", 0)
+        if handle > 0:
+            exe.captureRelease(handle)
+        exe.releaseScratchBuffer(d_x)
+        exe.releaseScratchBuffer(d_y)
