@@ -24,11 +24,12 @@ int mlc_hip_capture_begin(void) {
         !resident_page_rows(g.last_ids.data(), g.last_slots.data(), g.last_ids.size(), g.last_page_size))
         return 0;
     g.cap = Ctx::Captured{};
+    g.cap.tag_step = tag_step(kReplayTagStep);
     g_capture_failed = false;
     HIP_OK(hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal));
     g_capturing = true;
     hipLaunchKernelGGL(replay_word_kernel, dim3(1), dim3(1), 0, g.stream,
-                       reinterpret_cast<uint32_t*>(g.scratch_ptr + kScratchReplayWordOffset), kReplayTagStep);
+                       reinterpret_cast<uint32_t*>(g.scratch_ptr + kScratchReplayWordOffset), g.cap.tag_step);
     return 1;
 }
 
@@ -159,6 +160,9 @@ int mlc_hip_replay(int handle) {
     if (it->second.buffer_generation != g.buffer_generation)
         return fail("replay: a device buffer of the library was freed or moved since the capture (capture again)");
     if (!settle()) return 0;
+    const uint32_t step = it->second.tag_step;
+    if (g.replay_word > kLastReplayWord - step && !renew_tags()) return 0;
+    g.replay_word += step;
     if (it->second.n_decode && !scratch_follow(g.stream)) return 0;
     HIP_OK(hipGraphLaunch(it->second.exec, g.stream));
     if (it->second.n_decode && !scratch_launched(g.stream)) return 0;

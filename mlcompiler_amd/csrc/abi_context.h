@@ -55,11 +55,23 @@ constexpr size_t kScratchReplayWordOffset = kStreamPartBytes + kScratchProbeByte
 constexpr size_t kScratchBytes = kScratchReplayWordOffset + 256;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
+// The buffers in which the K slices of matmuls meet (meeting_words) hold tagged words as well.
+constexpr const char* kMeetingWords[] = {"q4_k_meet", "tokens_k_meet"};
+
 // First launch of every captured pass: moves the replay word on, so that the launches of
 // this replay (whose arguments, tag included, are the same at every replay) use tags that the
 // replay before did not.
 __global__ void replay_word_kernel(uint32_t* word, uint32_t step) { *word += step; }
 constexpr uint32_t kReplayTagStep = 4096;   // decode launches of one captured pass, at most, and sliced matmuls with a tag
+
+// The tags of launches are numbers up to the first of these, those of captured passes lie above, at replay words up to the second.
+constexpr uint32_t kLastLaunchTag = 0x7FFFFFFFu, kLastReplayWord = 0x80000000u - kReplayTagStep;
+
+// Words that have been written once stay in memory until the same place is written again: before the tags start over, every
+// buffer of such words is cleared (renew_tags).
+__global__ void clear_words_kernel(uint4* p, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = make_uint4(0u, 0u, 0u, 0u);
+}
 
 // Device copy of the flat page table (and, where the per-request arrays do not travel inside the
 // kernel arguments, of those arrays) as the tile-balanced decode kernel reads it; uploaded only
@@ -245,6 +257,7 @@ struct Ctx {
     int n_cu = 256;
     unsigned char* scratch_ptr = nullptr;   // device address of `scratch` on g.device
     uint32_t next_tag = 0;                  // tag of the last launch that needed one (never zero)
+    uint32_t replay_word = 0;               // the replay word behind the last replay
     // Every decode launch on this GPU uses the one scratch array, so launches on different
     // streams must follow each other: the stream of the last launch is remembered, and a launch
     // on another stream first waits for that one (one event, created at set-up; launches that
@@ -258,7 +271,9 @@ struct Ctx {
     volatile uint32_t* fault_host = nullptr;
     uint32_t* fault_dev = nullptr;
     long opt_spin_limit = 200000;           // rounds a merge polls before it gives up (about 0.1 s)
-    long opt_test_flags = 0;                // bit 0: workgroups do not publish their partials (tests of the give-up path)
+    // Bit 0: workgroups do not publish their partials (tests of the give-up path); bit 1: a launch and a replay take 2^30 tags
+    // (tests of what happens when they run out).
+    long opt_test_flags = 0;
     StreamTables tables;
     long opt_wgs_per_cu = 0;        // tile-balanced kernel: workgroups per CU (0 = automatic)
     long opt_stream_stages = 0;     // tile-balanced kernel: LDS stages per workgroup (0 = automatic)
@@ -285,6 +300,7 @@ struct Ctx {
         bool carried_kv = false;             // ... and does the step's KV write
         size_t n_decode = 0;                 // tile-balanced decode launches of the pass
         size_t n_sliced = 0;                 // matmuls of the pass whose K slices meet inside the launch
+        uint32_t tag_step = 0;               // what a replay moves the replay word on by
         uint64_t buffer_generation = 0;      // Ctx::buffer_generation when the pass was captured
         const void* rows_dev = nullptr;      // device copy of the KV write's page rows
         size_t rows_batch = 0, rows_page_size = 0;
@@ -400,20 +416,45 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 int settle_gemm(const RopeArgs* rope);
 
+int scratch_follow(hipStream_t stream);
+int scratch_launched(hipStream_t stream);
+
+uint32_t tag_step(uint32_t step) { return g.opt_test_flags & 2 ? 1u << 30 : step; }
+
+// No tag is left that none of the words in memory can have: clears them, behind every launch that uses them, and starts over.
+int renew_tags() {
+    if (!scratch_follow(g.stream)) return 0;
+    auto clear = [&](void* p, size_t bytes) {
+        const unsigned grid = (unsigned)std::min<size_t>((bytes / 16 + 255) / 256, 1024);
+        hipLaunchKernelGGL(clear_words_kernel, dim3(grid), dim3(256), 0, g.stream, static_cast<uint4*>(p), bytes / 16);
+    };
+    clear(g.scratch_ptr, kStreamPartBytes);
+    clear(g.scratch_ptr + kScratchReplayWordOffset, 256);
+    for (const char* name : kMeetingWords) {
+        const auto it = g.cached.find(name);
+        if (it != g.cached.end()) clear(it->second.first, it->second.second);
+    }
+    HIP_OK(hipGetLastError());
+    g.next_tag = g.replay_word = 0;
+    return scratch_launched(g.stream);
+}
+
 // Numbers a launch whose workgroups leave each other tagged words.  `in_pass` counts those of its kind in a captured pass:
 // launches whose words lie in different buffers may have the same tag.
 TagArgs next_tags(size_t& in_pass) {
     TagArgs t;
     t.fault = g.fault_dev;
     t.spin_limit = (uint32_t)g.opt_spin_limit;
-    t.test_flags = (uint32_t)g.opt_test_flags;
+    t.test_flags = (uint32_t)g.opt_test_flags & 1u;
     if (g_capturing) {
         // the arguments of a captured launch are the same at every replay: its tag is its number in
         // the pass plus the replay word, which the pass's first launch moves on by kReplayTagStep
         t.tag = 0x80000000u | (uint32_t)in_pass++;
         t.tag_dev = reinterpret_cast<const uint32_t*>(g.scratch_ptr + kScratchReplayWordOffset);
     } else {
-        if (++g.next_tag == 0) ++g.next_tag;   // (zero is what untouched memory holds)
+        const uint32_t step = tag_step(1);
+        if (g.next_tag > kLastLaunchTag - step) (void)renew_tags();   // (a failure shows at the launch behind it)
+        g.next_tag += step;
         t.tag = g.next_tag;
         t.tag_dev = nullptr;
     }

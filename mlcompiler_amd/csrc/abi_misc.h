@@ -96,7 +96,7 @@ int mlc_hip_set_option(const char* name, long value) {
         return 1;
     }
     if (!std::strcmp(name, "decode_test_flags")) {
-        if (value < 0 || value > 1) return 0;
+        if (value < 0 || value > 3) return 0;
         g.opt_test_flags = value;
         return 1;
     }

@@ -70,3 +70,66 @@ def test_slices_without_room_for_their_words_in_a_captured_pass(exe):
             exe.captureRelease(handle)
         exe.releaseScratchBuffer(d_x)
         exe.releaseScratchBuffer(d_y)
+
+
+def _decode(exe):
+    """A decode attention whose pairs are split over workgroups."""
+    from paged_cases import DeviceCase, baseline_config
+    case = baseline_config(2, batch=6)
+    dev = DeviceCase(exe, case)
+    out = np.empty((case.batch, case.num_heads, case.head_dim), np.float32)
+    call = lambda: exe.encodePagedFlashAttention(dev.q_buf, dev.k_buf, dev.v_buf, dev.o_buf, case.page_tables_flat, case.page_table_offsets,
+                                                 case.seq_lens, case.q_positions, case.batch, case.num_heads, case.kv_heads,
+                                                 case.head_dim, case.page_size, case.apply_causal)
+    return call, lambda: _read(exe, dev.o_buf, out), dev.free
+
+
+def _matmul(rows, cols, batch):
+    def make(exe):
+        rng = np.random.default_rng(rows)
+        w, x = _weights(rng, rows, cols), rng.standard_normal((batch, cols)).astype(np.float32)
+        d_x, d_y = _pool(exe, x), exe.allocateScratchBuffer(batch * rows * 4)
+        call = lambda: exe.encodeMatMulQ4_0Batched(f"meet.{rows}.{cols}", w, d_x, batch, rows, cols, w.shape[1], 1, d_y)
+        return call, lambda: _read(exe, d_y, np.empty((batch, rows), np.float32)), lambda: [exe.releaseScratchBuffer(b) for b in (d_x, d_y)]
+    return make
+
+
+KINDS = {"decode": _decode, "slices": _matmul(64, 4096, 5), "tail": _matmul(4160, 1024, 1000)}
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("captured", [False, True])
+def test_tags_that_come_again(exe, kind, captured):
+    """Every launch (replay) takes 2^30 tags, so that they start over at once, and the second one does not write
+    its words: those of the first, which had the same tag, are gone, and the wait for the second's is given up."""
+    call, read, free = KINDS[kind](exe)
+    handles = []
+
+    def run(flags):
+        assert exe.setOption("decode_test_flags", flags) and exe.setOption("decode_spin_limit", 3 if flags & 1 else 200000)
+        if captured:
+            assert exe.beginForwardPassCB() and exe.captureBegin()
+            assert call(), exe.lastError()
+            handles.append(exe.captureEnd())
+            assert handles[-1] > 0 and exe.flushForwardPassCB(), exe.lastError()
+            assert exe.beginForwardPassCB() and exe.replay(handles[-1]), exe.lastError()
+        else:
+            assert exe.beginForwardPassCB() and call(), exe.lastError()
+        return exe.flushForwardPassCB()
+
+    try:
+        assert run(0) if not captured else (exe.beginForwardPassCB() and call() and exe.flushForwardPassCB()), exe.lastError()
+        want = read()
+        for _ in range(3):
+            assert run(2), exe.lastError()
+            assert np.array_equal(read(), want)
+        assert not run(3) and "gave up" in exe.lastError()
+        for _ in range(3):
+            assert run(0), exe.lastError()
+            assert np.array_equal(read(), want)
+    finally:
+        exe.setOption("decode_test_flags", 0)
+        exe.setOption("decode_spin_limit", 200000)
+        for h in handles:
+            exe.captureRelease(h)
+        free()
