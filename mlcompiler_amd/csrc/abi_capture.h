@@ -163,9 +163,10 @@ int mlc_hip_replay(int handle) {
     const uint32_t step = it->second.tag_step;
     if (g.replay_word > kLastReplayWord - step && !renew_tags()) return 0;
     g.replay_word += step;
-    if (it->second.n_decode && !scratch_follow(g.stream)) return 0;
+    const bool waits = it->second.n_decode || it->second.n_sliced;
+    if (waits && !scratch_follow(g.stream)) return 0;
     HIP_OK(hipGraphLaunch(it->second.exec, g.stream));
-    if (it->second.n_decode && !scratch_launched(g.stream)) return 0;
+    if (waits && !scratch_launched(g.stream)) return 0;
     return 1;
 }
 

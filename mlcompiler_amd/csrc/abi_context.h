@@ -258,10 +258,11 @@ struct Ctx {
     unsigned char* scratch_ptr = nullptr;   // device address of `scratch` on g.device
     uint32_t next_tag = 0;                  // tag of the last launch that needed one (never zero)
     uint32_t replay_word = 0;               // the replay word behind the last replay
-    // Every decode launch on this GPU uses the one scratch array, so launches on different
-    // streams must follow each other: the stream of the last launch is remembered, and a launch
-    // on another stream first waits for that one (one event, created at set-up; launches that
-    // stay on the library's stream cost nothing).
+    // Launches whose workgroups wait for each other (the decode attention, matmuls whose K slices meet inside the launch)
+    // must follow each other also on different streams: decode launches share the one scratch array, and any two side
+    // by side could each hold the CUs that workgroups need for which the other one's wait.  The stream of the last
+    // such launch is remembered, and a launch on another stream first waits for that one (one event, created at
+    // set-up; launches that stay on the library's stream cost nothing).
     hipStream_t scratch_stream = nullptr;
     bool scratch_in_use = false;
     hipEvent_t scratch_ev = nullptr;
@@ -555,10 +556,11 @@ int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a) {
     }
     a.z_groups = (uint32_t)((z + zt - 1) / zt);
     const dim3 grid((a.row_groups + 7) / 8 * 8 * a.z_groups, (unsigned)ksplit);
+    if (ksplit > 1 && !scratch_follow(g.stream)) return 0;
     const auto launch = a.batch <= 4 ? launch_q4_matmul_1 : a.batch <= 8 ? launch_q4_matmul_2 : launch_q4_matmul_4;
     if (!launch(form, rt, waves, zt, block_scales, grid, a, g.stream)) return fail("q4 matmul: kernel variant not built");
     HIP_OK(hipGetLastError());
-    return 1;
+    return ksplit > 1 ? scratch_launched(g.stream) : 1;
 }
 
 // Launches the held-back matmul, with the split + RoPE + cast of its output as epilogue when

@@ -300,13 +300,18 @@ const char* stream_pv_name(int hpw, int nw) {
     return m == 3 ? "mfma-p32" : m == 2 ? "mfma" : m == 1 ? "pv16" : "pv32";
 }
 
-// Orders a launch that uses the scratch array on `stream` behind the last one that did (see
+// Orders a launch whose workgroups wait for each other on `stream` behind the last one (see
 // Ctx::scratch_stream).  The library's own stream lives as long as the library, so the event that
 // marks its last launch is recorded only when another stream shows up; a caller's stream may be
 // gone by then, so the event is recorded right behind a launch on one.  A captured pass runs on
-// the library's stream, where its replays are ordered like any other launch there.
+// the library's stream, where its replays are ordered like any other launch there.  (A launch that a caller records into
+// a graph of its own does not run now: when that graph runs is the caller's to order.)
+bool caller_records(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return stream != g.stream && hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
 int scratch_follow(hipStream_t stream) {
-    if (g_capturing) return 1;
+    if (g_capturing || caller_records(stream)) return 1;
     if (g.scratch_in_use && g.scratch_stream != stream) {
         if (g.scratch_stream == g.stream) HIP_OK(hipEventRecord(g.scratch_ev, g.stream));
         HIP_OK(hipStreamWaitEvent(stream, g.scratch_ev, 0));
@@ -314,7 +319,7 @@ int scratch_follow(hipStream_t stream) {
     return 1;
 }
 int scratch_launched(hipStream_t stream) {
-    if (g_capturing) return 1;
+    if (g_capturing || caller_records(stream)) return 1;
     g.scratch_stream = stream;
     g.scratch_in_use = true;
     if (stream != g.stream) HIP_OK(hipEventRecord(g.scratch_ev, stream));

@@ -91,7 +91,9 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
         a.tail_slices = tail.slices;
         a.tail_stages = tail.stages;
         a.tags = tail.rest ? next_tags(g.cap.n_sliced) : TagArgs{};
+        if (tail.rest && !scratch_follow(g.stream)) return 0;
         launch_matmul_tokens(q6, a, tail.whole + tail.rest * tail.slices, g.stream);
+        if (tail.rest && !scratch_launched(g.stream)) return 0;
         if (sum) {
             const uint32_t n = (uint32_t)(bn * rows);
             hipLaunchKernelGGL(q4_sum_slices_kernel, dim3((n + 255) / 256), dim3(256), 0, g.stream, slices, o, n,

@@ -133,3 +133,114 @@ def test_tags_that_come_again(exe, kind, captured):
         for h in handles:
             exe.captureRelease(h)
         free()
+
+
+def _hip():
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+    for name in ("hipStreamCreate", "hipStreamSynchronize", "hipStreamDestroy", "hipStreamQuery", "hipMemcpyAsync"):
+        getattr(hip, name).argtypes = {"hipStreamCreate": [C.POINTER(C.c_void_p)],
+                                       "hipMemcpyAsync": [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p]}.get(name, [C.c_void_p])
+    return hip
+
+
+@pytest.mark.parametrize("kind", ["slices", "tail", "replayed"])
+def test_waiting_launches_on_two_streams_follow_each_other(exe, kind):
+    """A matmul whose slices meet and a decode attention on a caller's stream: side by side, each could hold the CUs
+    that workgroups need for which the other one's wait."""
+    import ctypes as C
+    from mlcompiler_amd._lib import load
+    from paged_cases import DeviceCase, baseline_config
+    lib, hip, stream = load(), _hip(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+    library = C.c_void_p(lib.mlc_hip_stream())
+    call, read, free = KINDS["tail" if kind == "tail" else "slices"](exe)
+    case = baseline_config(2, batch=6)
+    dev = DeviceCase(exe, case)
+    arrays = [np.ascontiguousarray(a, np.uint32) for a in (case.page_tables_flat, case.page_table_offsets, case.seq_lens, case.q_positions)]
+    d_flat = _pool(exe, arrays[0])
+    u32p = lambda a: a.ctypes.data_as(C.POINTER(C.c_uint32))
+    big = 1 << 28
+    d_a, d_b = exe.allocateScratchBuffer(big), exe.allocateScratchBuffer(big)
+    handle = 0
+
+    def decode():
+        return lib.mlc_hip_paged_attn_decode_noalloc(dev.q_buf, dev.k_buf, dev.v_buf, dev.o_buf, d_flat, arrays[0].size, u32p(arrays[1]),
+                                                     u32p(arrays[2]), u32p(arrays[3]), case.batch, case.num_heads, case.kv_heads,
+                                                     case.head_dim, case.page_size, int(case.apply_causal), stream)
+
+    def busy(s):     # some milliseconds of copies
+        for _ in range(40):
+            assert hip.hipMemcpyAsync(d_a, d_b, big, 3, s) == 0
+        assert hip.hipStreamQuery(s) == 600      # (not ready)
+
+    try:
+        want_o = dev.run()
+        assert exe.setOption("fuse_row_ops", 0)      # (nothing held back: that orders the streams by itself)
+        assert exe.beginForwardPassCB() and call() and exe.flushForwardPassCB(), exe.lastError()
+        want = read()
+        if kind == "replayed":
+            assert exe.beginForwardPassCB() and exe.captureBegin() and call()
+            handle = exe.captureEnd()
+            assert handle > 0 and exe.flushForwardPassCB(), exe.lastError()
+        launch = (lambda: exe.replay(handle)) if handle else call
+        # a matmul behind the other stream's decode
+        busy(stream)
+        assert decode(), exe.lastError()
+        assert exe.beginForwardPassCB() and launch() and exe.flushForwardPassCB(), exe.lastError()
+        assert hip.hipStreamQuery(stream) == 0
+        assert np.array_equal(read(), want)
+        # and the decode behind the matmul
+        busy(library)
+        assert exe.beginForwardPassCB() and launch(), exe.lastError()
+        assert decode(), exe.lastError()
+        assert hip.hipStreamSynchronize(stream) == 0 and hip.hipStreamQuery(library) == 0
+        assert exe.flushForwardPassCB(), exe.lastError()
+        assert np.array_equal(read(), want)
+        assert np.array_equal(_read(exe, dev.o_buf, want_o), want_o)
+    finally:
+        exe.setOption("fuse_row_ops", 1)
+        if handle > 0:
+            exe.captureRelease(handle)
+        hip.hipStreamSynchronize(stream)
+        hip.hipStreamDestroy(stream)
+        for b in (d_flat, d_a, d_b):
+            exe.releaseScratchBuffer(b)
+        dev.free()
+        free()
+
+
+def test_a_decode_recorded_into_a_callers_graph_orders_nothing(exe):
+    """It does not run when it is recorded: the library's launches behind it neither wait for it nor fail."""
+    import ctypes as C
+    from mlcompiler_amd._lib import load
+    from paged_cases import DeviceCase, baseline_config
+    lib, hip, stream, graph = load(), _hip(), C.c_void_p(), C.c_void_p()
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+    call, read, free = KINDS["slices"](exe)
+    case = baseline_config(2, batch=6)
+    dev = DeviceCase(exe, case)
+    arrays = [np.ascontiguousarray(a, np.uint32) for a in (case.page_tables_flat, case.page_table_offsets, case.seq_lens, case.q_positions)]
+    d_flat = _pool(exe, arrays[0])
+    u32p = lambda a: a.ctypes.data_as(C.POINTER(C.c_uint32))
+    try:
+        want_o = dev.run()
+        assert exe.beginForwardPassCB() and call() and exe.flushForwardPassCB(), exe.lastError()
+        want = read()
+        assert hip.hipStreamBeginCapture(stream, 1) == 0       # (this thread's calls)
+        ok = lib.mlc_hip_paged_attn_decode_noalloc(dev.q_buf, dev.k_buf, dev.v_buf, dev.o_buf, d_flat, arrays[0].size, u32p(arrays[1]),
+                                                   u32p(arrays[2]), u32p(arrays[3]), case.batch, case.num_heads, case.kv_heads,
+                                                   case.head_dim, case.page_size, int(case.apply_causal), stream)
+        ended = hip.hipStreamEndCapture(stream, C.byref(graph))
+        assert ok and ended == 0 and graph, exe.lastError()
+        assert hip.hipGraphDestroy(graph) == 0
+        assert exe.beginForwardPassCB() and call() and exe.flushForwardPassCB(), exe.lastError()
+        assert np.array_equal(read(), want) and np.array_equal(dev.run(), want_o)
+    finally:
+        hip.hipStreamDestroy(stream)
+        exe.releaseScratchBuffer(d_flat)
+        dev.free()
+        free()
