@@ -64,6 +64,9 @@ constexpr const char* kMeetingWords[] = {"q4_k_meet", "tokens_k_meet"};
 __global__ void replay_word_kernel(uint32_t* word, uint32_t step) { *word += step; }
 constexpr uint32_t kReplayTagStep = 4096;   // decode launches of one captured pass, at most, and sliced matmuls with a tag
 
+// Rounds that a wait for tagged words polls before it is given up (about 0.1 s).
+constexpr long kSpinLimit = 200000;
+
 // The tags of launches are numbers up to the first of these, those of captured passes lie above, at replay words up to the second.
 constexpr uint32_t kLastLaunchTag = 0x7FFFFFFFu, kLastReplayWord = 0x80000000u - kReplayTagStep;
 
@@ -271,7 +274,7 @@ struct Ctx {
     // waited for the stream.
     volatile uint32_t* fault_host = nullptr;
     uint32_t* fault_dev = nullptr;
-    long opt_spin_limit = 200000;           // rounds a merge polls before it gives up (about 0.1 s)
+    long opt_spin_limit = kSpinLimit;       // rounds a merge of the decode attention polls before it gives up
     // Bit 0: workgroups do not publish their partials (tests of the give-up path); bit 1: a launch and a replay take 2^30 tags
     // (tests of what happens when they run out).
     long opt_test_flags = 0;
@@ -459,6 +462,12 @@ TagArgs next_tags(size_t& in_pass) {
         t.tag = g.next_tag;
         t.tag_dev = nullptr;
     }
+    return t;
+}
+// The same for a matmul whose K slices meet.  The option cuts the wait of the decode attention, and this one only in tests of it.
+TagArgs next_sliced_tags() {
+    TagArgs t = next_tags(g.cap.n_sliced);
+    if (!t.test_flags) t.spin_limit = (uint32_t)std::max(g.opt_spin_limit, kSpinLimit);
     return t;
 }
 bool sliced_tags_left() { return !g_capturing || g.cap.n_sliced < kReplayTagStep; }

@@ -243,7 +243,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         a.out = slices ? slices : o;
         a.slices = (uint32_t)ksplit;
         a.meet = words;
-        if (words) a.tags = next_tags(g.cap.n_sliced);
+        if (words) a.tags = next_sliced_tags();
         a.batch = (uint32_t)bn; a.rows = (uint32_t)rows; a.nblocks = (uint32_t)nblocks;
         a.nquads = (uint32_t)quads; a.quads_per_slice = (uint32_t)per_slice;
         if (g.opt_fuse_rows && g.opt_q4_int_operand && !sync && batch <= 64) {

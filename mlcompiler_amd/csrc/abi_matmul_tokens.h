@@ -90,7 +90,7 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
         a.rest = tail.rest;
         a.tail_slices = tail.slices;
         a.tail_stages = tail.stages;
-        a.tags = tail.rest ? next_tags(g.cap.n_sliced) : TagArgs{};
+        a.tags = tail.rest ? next_sliced_tags() : TagArgs{};
         if (tail.rest && !scratch_follow(g.stream)) return 0;
         launch_matmul_tokens(q6, a, tail.whole + tail.rest * tail.slices, g.stream);
         if (tail.rest && !scratch_launched(g.stream)) return 0;

@@ -72,6 +72,23 @@ def test_slices_without_room_for_their_words_in_a_captured_pass(exe):
         exe.releaseScratchBuffer(d_y)
 
 
+@pytest.mark.parametrize("rows,cols,batch", [(64, 4096, 5), (4160, 2080, 1000)])
+def test_the_decode_spin_limit_is_not_the_matmuls(exe, rows, cols, batch):
+    """A matmul waits for its slices as long as ever where the decode attention's wait is cut short."""
+    rng = np.random.default_rng(3)
+    w, x = _weights(rng, rows, cols), rng.standard_normal((batch, cols)).astype(np.float32)
+    d_x, d_y = _pool(exe, x), exe.allocateScratchBuffer(batch * rows * 4)
+    try:
+        assert exe.setOption("decode_spin_limit", 1)
+        for _ in range(20):
+            assert exe.encodeMatMulQ4_0Batched("meet.spin", w, d_x, batch, rows, cols, w.shape[1], 1, d_y, True), exe.lastError()
+        check(_read(exe, d_y, np.empty((batch, rows), np.float32)), q4.dequant(w, cols), x)
+    finally:
+        exe.setOption("decode_spin_limit", 200000)
+        exe.releaseScratchBuffer(d_x)
+        exe.releaseScratchBuffer(d_y)
+
+
 def _decode(exe):
     """A decode attention whose pairs are split over workgroups."""
     from paged_cases import DeviceCase, baseline_config
