@@ -51,13 +51,12 @@ TokensTail tokens_tail(size_t wgs, size_t slots, size_t stages) {
 int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t batch, size_t rows, size_t cols) {
     const size_t piece = kTokensFragBytes / (4 * cols) / 64 * 64;
     if (piece == 0) return 0;
-    for (const char* name : {"tokens_x_fragments", "tokens_x_inv_scale", "tokens_k_slices", "tokens_k_meet"})
+    for (const char* name : {"tokens_x_fragments", "tokens_x_inv_scale", "tokens_k_slices"})
         if (g_capturing && !g.cached.count(name)) return 0;
     _Float16* frag = static_cast<_Float16*>(cached_buffer("tokens_x_fragments", kTokensFragBytes));
     float* inv = static_cast<float*>(cached_buffer("tokens_x_inv_scale", kTokensFragBytes / 64));   // (cols >= 64)
     float* slices = static_cast<float*>(cached_buffer("tokens_k_slices", kTokensSliceBytes));
-    a.meet = meeting_words("tokens_k_meet", kTokensMeetBytes);
-    if (!frag || !inv || !slices || !a.meet) return 0;
+    if (!frag || !inv || !slices) return 0;
     a.xfrag = frag;
     a.inv_scale = inv;
     a.rows = (uint32_t)rows;
@@ -80,10 +79,14 @@ int matmul_tokens(bool q6, TokensArgs a, const float* in, float* out, size_t bat
         // a kernel behind / in the launch, us: two slices 6144 x 4096 at 300 64.2 / 60.9, 11264 x 2048 at 128 45.1 / 41.7; four
         // of 8 stages 2048 x 2048 at 512 42.3 / 39.2, of 16 4096 x 4096 at 256 47.8 / 47.4, of 24 2048 x 5632 at 512 56.6 /
         // 58.4, of 56 4096 x 14336 at 200 98.5 / 100.3).
-        TokensTail tail{(uint32_t)(wgs * plan.ksplit), 0, 1, 0};
+        const TokensTail none{(uint32_t)(wgs * plan.ksplit), 0, 1, 0};
+        TokensTail tail = none;
         const bool meet = sliced_tags_left() && (slots - 1) * 65536 <= kTokensMeetBytes;
         if (meet && plan.ksplit == 1) tail = tokens_tail(wgs, slots, a.stages);
         else if (meet && plan.ksplit <= (plan.stages_per_slice <= 16 ? kTokensTailSlices : 3)) tail = {0, (uint32_t)wgs, (uint32_t)plan.ksplit, plan.stages_per_slice};
+        // (room to meet in is taken by the first call that has use for it, and a call that finds none does without)
+        a.meet = tail.rest ? meeting_words("tokens_k_meet", kTokensMeetBytes) : nullptr;
+        if (!a.meet) tail = none;
         const bool sum = plan.ksplit > 1 && !tail.rest;
         a.out = sum ? slices : o;
         a.whole = tail.whole;

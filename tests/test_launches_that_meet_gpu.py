@@ -89,6 +89,38 @@ def test_the_decode_spin_limit_is_not_the_matmuls(exe, rows, cols, batch):
         exe.releaseScratchBuffer(d_y)
 
 
+MEMORY = """
+import ctypes as C, numpy as np, sys
+sys.path[:0] = ["tests", "."]
+from mlcompiler_amd import HipExecutor
+import test_q4_matmul_gpu as q4
+exe, hip = HipExecutor.Instance(), C.CDLL("libamdhip64.so")
+exe.requireAvailable()
+used = []
+# 80 tiles, too short to be split; 128 and 32 tiles left over by whole rounds, too short and long enough
+for rows, cols, tokens in ((64, 256, 5120), (4096, 960, 1030), (4096, 1024, 1030)):
+    q, x, stride = q4.make(rows, cols, tokens, rows)
+    q4.run(exe, f"memory_{rows}_{cols}", q, x, tokens, rows, cols, stride)
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    used.append(total.value - free.value)
+print("used", *used)
+"""
+
+
+def test_only_split_tiles_take_memory_to_meet_in():
+    """(A process of its own: the library's buffers are for good.)"""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", MEMORY], cwd=root, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr
+    first, whole, split = (int(v) >> 20 for v in out.stdout.split("used")[1].split())
+    print(f"in use: {first}, {whole}, {split} MiB")
+    assert whole - first < 32 <= split - whole
+
+
 def _decode(exe):
     """A decode attention whose pairs are split over workgroups."""
     from paged_cases import DeviceCase, baseline_config
