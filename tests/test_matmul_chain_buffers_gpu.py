@@ -290,25 +290,27 @@ def test_epilogues_over_the_norm(exe, reader, over):
         assert np.abs(got - want).max() <= (1e-3 if m in ("kp", "vp", "k16", "v16") else 1e-4) * max(np.abs(want).max(), 1e-30), m
 
 
-@pytest.mark.parametrize("what", ["sum_over_gate_up", "norm_over_residual_one_row_down", "slices_sum_over_gate_up", "gate_as_residual"])
+@pytest.mark.parametrize("what", ["sum_over_gate_up", "norm_over_residual_one_row_down", "slices_sum_over_gate_up", "gate_as_residual",
+                                  "slices_of_pairs_sum_over_gate_up"])
 def test_row_chains_over_shared_buffers(exe, what):
     """Row operators of one chain whose buffers meet in other rows than their own: the chain's workgroups run in no order."""
     rng = np.random.default_rng(3)
-    batch, n = 300, 1024       # (more rows than run at once)
+    batch, n, k = 300, 1024, 512       # (more rows than run at once)
+    pairs = what.startswith("slices_of_pairs")      # (the chain starts with the sum over the matmul's slices)
     if what.startswith("slices"):
-        batch = 40
-    w = _weights(rng, 2 * n, 512)
+        batch, k = 40, 1024 if pairs else 512
+    w = _weights(rng, 2 * n, k)
     gamma = rng.uniform(0.5, 1.5, n).astype(np.float32)
-    init = {"gu": (batch, 2 * n), "g": (batch, n), "u": (batch, n), "m": (batch, n), "r": (batch + 1, n), "s": (batch, n), "x": (batch, 512)}
+    init = {"gu": (batch, 2 * n), "g": (batch, n), "u": (batch, n), "m": (batch, n), "r": (batch + 1, n), "s": (batch, n), "x": (batch, k)}
     init = {m: rng.standard_normal(s).astype(np.float32) for m, s in init.items()}
     out = {}
     for fuse in (0, 1):
         dev = {m: _pool(exe, a) for m, a in init.items()}
-        assert exe.setOption("fuse_row_ops", fuse) and exe.setOption("q4_ksplit", 2)
+        assert exe.setOption("fuse_row_ops", fuse) and exe.setOption("q4_ksplit", 2) and exe.setOption("q4_int_operand", 0 if pairs else 1)
         try:
             assert exe.beginForwardPassCB()
             if what.startswith("slices"):
-                assert exe.encodeMatMulQ4_0Batched("rows.shared", w, dev["x"], batch, 2 * n, 512, w.shape[1], 1, dev["gu"]), exe.lastError()
+                assert exe.encodeMatMulQ4_0Batched(f"rows.shared.{k}", w, dev["x"], batch, 2 * n, k, w.shape[1], 1, dev["gu"]), exe.lastError()
             assert exe.encodeGateUpSplitSiluMul(dev["gu"], dev["g"], dev["u"], dev["m"], batch, n, 2 * n)
             resid, total = dev["g" if what == "gate_as_residual" else "r"], dev["gu" if "gate_up" in what else "s"]
             assert exe.encodeAddBatched(dev["m"], resid, total, batch * n)
@@ -319,6 +321,7 @@ def test_row_chains_over_shared_buffers(exe, what):
         finally:
             exe.setOption("fuse_row_ops", 1)
             exe.setOption("q4_ksplit", 0)
+            exe.setOption("q4_int_operand", 1)
             for buf in dev.values():
                 exe.releaseScratchBuffer(buf)
     for m, want in out[0].items():

@@ -92,6 +92,14 @@ SHAPES = {
     "partial_rotary": dict(B=5, H=8, Hkv=4, D=64, hid=256, rotary=32),
     "no_rotary": dict(B=3, H=4, Hkv=2, D=64, hid=128, rotary=0),
     "two_row_tiles": dict(B=7, H=64, Hkv=8, D=128, hid=256),
+    "k_slices": dict(B=8, H=8, Hkv=2, D=64, hid=4096),             # two of 16 quads, meeting in front of the epilogue
+    "k_slices_two_groups": dict(B=21, H=12, Hkv=2, D=64, hid=5600),
+}
+
+
+# the matmuls of the captured-pass test: one slice, two, and two with a second group of requests
+REPLAYED = {
+    "one": dict(B=9, H=8, Hkv=2, D=64, hid=256), "two": SHAPES["k_slices"], "two_groups": SHAPES["k_slices_two_groups"],
 }
 
 
@@ -163,3 +171,55 @@ def test_matmul_followed_by_something_else_is_launched_as_it_is(exe):
                                 c.rotary)[0]
     assert np.array_equal(q, wq)
     assert np.array_equal(a, got) and np.array_equal(b, got)
+
+
+@pytest.mark.parametrize("shape", list(REPLAYED))
+@pytest.mark.parametrize("form", ["scatter", "cast"])
+def test_replayed(exe, shape, form):
+    """Captured once, replayed with other inputs: what the same calls give one by one."""
+    c = Case(seed=7, **REPLAYED[shape])
+    rng = np.random.default_rng(8)
+    B, out = c.B, {"qkv": c.rows, "q": c.q_rows, "k": c.kv_rows, "v": c.kv_rows, "k16": c.kv_rows, "v16": c.kv_rows}
+    like = {n: np.zeros((B, cols), np.uint16 if n.endswith("16") else np.float32) for n, cols in out.items()}
+    like |= {"kp": c.k_pool, "vp": c.v_pool}
+    d = {n: _pool(exe, a) for n, a in like.items()}
+    d_x, d_cos, d_sin = (_pool(exe, a) for a in (c.x, c.cos, c.sin))
+
+    def encode():
+        assert exe.encodeMatMulQ4_0Batched(c.name, c.w, d_x, B, c.rows, c.hid, po.q4_0_row_bytes(c.hid), 1, d["qkv"]), exe.lastError()
+        if form == "scatter":
+            assert exe.encodeQkvSplitRopeScatter(d["qkv"], d["q"], d["kp"], d["vp"], d_cos, d_sin, c.ids, c.slots, c.P, B, c.H, c.Hkv,
+                                                 c.D, c.rows, c.q_rows, c.kv_rows, c.kv_rows, c.rotary, k_f32_buf=d["k"],
+                                                 v_f32_buf=d["v"]), exe.lastError()
+        else:
+            assert exe.encodeQkvSplitRopeCast(d["qkv"], d["q"], d["k"], d["v"], d["k16"], d["v16"], d_cos, d_sin, B, c.H, c.Hkv, c.D,
+                                              c.rows, c.q_rows, c.kv_rows, c.kv_rows, c.rotary), exe.lastError()
+
+    def read():
+        return {n: _read(exe, d[n], a) for n, a in like.items()}
+
+    handle = 0
+    try:
+        assert exe.beginForwardPassCB()
+        encode()
+        assert exe.flushForwardPassCB()
+        before = exe.fusedMatmulRopeLaunches()
+        assert exe.beginForwardPassCB() and exe.captureBegin()
+        encode()
+        handle = exe.captureEnd()
+        assert handle > 0 and exe.flushForwardPassCB(), exe.lastError()
+        assert exe.fusedMatmulRopeLaunches() == before + 1
+        for _ in range(4):
+            assert exe.uploadToBuffer(d_x, rng.standard_normal(c.x.shape).astype(np.float32))
+            assert exe.beginForwardPassCB() and exe.replay(handle) and exe.flushForwardPassCB(), exe.lastError()
+            got = read()
+            assert exe.beginForwardPassCB()
+            encode()
+            assert exe.flushForwardPassCB(), exe.lastError()
+            for n, a in read().items():
+                assert np.array_equal(a.view(np.uint8), got[n].view(np.uint8)), n
+    finally:
+        if handle > 0:
+            exe.captureRelease(handle)
+        for b in list(d.values()) + [d_x, d_cos, d_sin]:
+            exe.releaseScratchBuffer(b)

@@ -22,6 +22,9 @@ pytestmark = pytest.mark.gpu
     ("q4", 6144, 2080, 300),     # 240 tiles in two, the second one shorter
     ("q6", 4128, 768, 200),      # 132 tiles in three
     ("q6", 4128, 2048, 1000), ("q6", 6144, 1024, 700),
+    ("q4", 4160, 4160, 1000),    # 65 stages, 20 in a slice: first-level sums of 8, by the whole K, the slice's last one shorter
+    ("q4", 4096, 7232, 1030),    # 113 stages
+    ("q6", 4128, 4352, 1000),    # 68
 ])
 def test_tail(exe, fmt, rows, cols, tokens):
     print(f"[tokens tail] {fmt} rows={rows} cols={cols} tokens={tokens}", flush=True)
@@ -54,5 +57,27 @@ def test_tail_replayed(exe):
             q4.run(exe, "tail_replay", q, -x, tokens, rows, cols, stride)
     finally:
         exe.captureRelease(handle)
+        exe.releaseScratchBuffer(d_in)
+        exe.releaseScratchBuffer(d_out)
+
+
+@pytest.mark.parametrize("rows,cols,tokens", [(4160, 1024, 1000), (2048, 2048, 500)])    # a tail; all tiles
+def test_a_slice_that_never_comes(exe, rows, cols, tokens):
+    """The bounded wait ends, the pass fails, and the next one works."""
+    q, x, stride = q4.make(rows, cols, tokens, 9)
+    d_in, d_out = exe.allocateScratchBuffer(x.nbytes), exe.allocateScratchBuffer(tokens * rows * 4)
+    call = lambda: exe.encodeMatMulQ4_0Batched(f"tail_never_{rows}", q, d_in, tokens, rows, cols, stride, 1, d_out, True)
+    try:
+        assert exe.uploadToBuffer(d_in, x) and call()
+        assert exe.setOption("decode_test_flags", 1) and exe.setOption("decode_spin_limit", 3)
+        assert not call() and "gave up" in exe.lastError()
+        assert exe.setOption("decode_test_flags", 0) and exe.setOption("decode_spin_limit", 200000)
+        assert call()
+        got = np.empty((tokens, rows), np.float32)
+        assert exe.downloadFromBuffer(d_out, got)
+        check(got, q4.dequant(q, cols), x)
+    finally:
+        exe.setOption("decode_test_flags", 0)
+        exe.setOption("decode_spin_limit", 200000)
         exe.releaseScratchBuffer(d_in)
         exe.releaseScratchBuffer(d_out)

@@ -139,7 +139,7 @@ def test_fused_and_unfused_sequences_agree(exe, seed):
     weights = {"n": po.quantize_q4_0((rng.standard_normal((L, L)) * 0.06).astype(np.float32)),
                "w": po.quantize_q4_0((rng.standard_normal((2 * L, L)) * 0.06).astype(np.float32))}
     gammas = [rng.uniform(0.5, 1.5, L).astype(np.float32) for _ in range(2)]
-    ksplit = int(rng.choice([0, 2]))     # 2: the matmuls leave K slices for the next chain to sum
+    ksplit = int(rng.choice([0, 2]))     # (rows of 256 columns are too short for two slices: the option must change nothing)
     cos, sin = np.zeros((B, D // 2), np.float32), np.zeros((B, D // 2), np.float32)
     for r in range(B):
         cos[r], sin[r] = po.rotary_coefficients(int(rng.integers(0, 2000)), D)

@@ -200,7 +200,7 @@ def test_gate_up_then_matmul_then_add_in_one_pass(exe, batch, hid, ffn, rows, fu
     bufs = [d_gu, d_res, d_gate, d_upb, d_mix, d_down, d_out]
     assert exe.setOption("fuse_row_ops", fuse)
     try:
-        for ks in (0, 2):   # automatic, and a forced K split (the sum of the slices joins the add)
+        for ks in (0, 2):   # automatic, and a forced K split (whose slices meet inside the matmul's launch)
             assert exe.setOption("q4_ksplit", ks)
             assert exe.beginForwardPassCB()
             assert exe.encodeGateUpSplitSiluMul(d_gu, d_gate, d_upb, d_mix, batch, ffn, 2 * ffn)
@@ -224,9 +224,8 @@ def test_gate_up_then_matmul_then_add_in_one_pass(exe, batch, hid, ffn, rows, fu
 
 
 def test_long_rows_between_two_matmuls(exe):
-    """A matmul whose output rows are longer than the fused row kernel handles (20480 > 16384),
-    split over K so that the sum of its slices is pending, feeding another matmul directly: the
-    sum and the split of the second matmul's input then run as separate kernels."""
+    """A matmul whose output rows are longer than the fused row kernel handles (20480 > 16384), with its K
+    split, feeding another matmul directly: the split of the second matmul's input runs as a kernel of its own."""
     rng = np.random.default_rng(21)
     batch, k1, mid, rows2 = 3, 1024, 20480, 64
     w1 = po.quantize_q4_0((rng.standard_normal((mid, k1)) * 0.05).astype(np.float32))
@@ -248,3 +247,67 @@ def test_long_rows_between_two_matmuls(exe):
             exe.releaseScratchBuffer(b)
     assert np.max(np.abs(got_mid - want_mid)) < 2e-5 * float(np.max(np.abs(want_mid)))
     assert np.max(np.abs(got - want)) < 1e-4 * float(np.max(np.abs(want)))
+
+
+@pytest.mark.parametrize("behind", ["add", "norm", "silu", "silu_add", "matmul", "long_rows"])
+@pytest.mark.parametrize("fuse", [1, 0])
+def test_chains_that_start_with_a_sum_of_k_slices(exe, behind, fuse):
+    """With the weights as fp16 pairs (q4_int_operand = 0) the K slices of a matmul are summed by whatever row operators come
+    behind it, in one launch with them; rows too long for that are summed by a kernel of their own."""
+    rng = np.random.default_rng(31)
+    batch, k, n = 5, 2048, 20480 if behind == "long_rows" else 1024      # (two slices of 16 quads)
+    rows = 2 * n if behind.startswith("silu") else n
+    w = po.quantize_q4_0((rng.standard_normal((rows, k)) * 0.05).astype(np.float32))
+    w2 = po.quantize_q4_0((rng.standard_normal((64, n)) * 0.05).astype(np.float32))
+    x, r = (rng.standard_normal((batch, c)).astype(np.float32) for c in (k, n))
+    gamma = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    d_x, d_r = _up(exe, x), _up(exe, r)
+    d = {m: _up(exe, np.full((batch, c), np.nan, np.float32))
+         for m, c in (("p", rows), ("h", n), ("n", n), ("g", n), ("u", n), ("m", n), ("y", 64))}
+    before = exe.rowProgramLaunches()
+    assert exe.setOption("fuse_row_ops", fuse) and exe.setOption("q4_int_operand", 0) and exe.setOption("q4_ksplit", 2)
+    try:
+        assert exe.beginForwardPassCB()
+        assert exe.encodeMatMulQ4_0Batched(f"slices.a.{behind}", w, d_x, batch, rows, k, w.shape[1], 1, d["p"]), exe.lastError()
+        last = d["p"]
+        if behind.startswith("silu"):
+            assert exe.encodeGateUpSplitSiluMul(d["p"], d["g"], d["u"], d["m"], batch, n, 2 * n)
+            last = d["m"]
+        if behind in ("add", "norm", "silu_add"):
+            assert exe.encodeAddBatched(last, d_r, d["h"], batch * n)
+            last = d["h"]
+        if behind == "norm":
+            assert exe.encodeRmsNormBatched(d["h"], gamma, 1e-5, batch, n, d["n"])
+            last = d["n"]
+        if behind != "add":
+            assert exe.encodeMatMulQ4_0Batched(f"slices.b.{behind}", w2, last, batch, 64, n, w2.shape[1], 1, d["y"]), exe.lastError()
+        assert exe.flushForwardPassCB(), exe.lastError()
+        p = _down(exe, d["p"], (batch, rows))
+        h, norm, g, u, m = (_down(exe, d[b], (batch, n)) for b in "hngum")
+        y = _down(exe, d["y"], (batch, 64))
+    finally:
+        exe.setOption("fuse_row_ops", 1)
+        exe.setOption("q4_int_operand", 1)
+        exe.setOption("q4_ksplit", 0)
+        for b in [d_x, d_r, *d.values()]:
+            exe.releaseScratchBuffer(b)
+    want = po.matmul_q4_0_batched(w, x, batch, rows, k)
+    assert np.max(np.abs(p - want)) < 2e-5 * np.max(np.abs(want))
+    last = p
+    if behind.startswith("silu"):
+        assert np.array_equal(g, p[:, :n]) and np.array_equal(u, p[:, n:])
+        want_m = po.gate_up_split_silu_mul(p, batch, n, 2 * n)[2]
+        assert np.max(np.abs(m - want_m) / (np.abs(want_m) + 1e-6)) < 5e-6
+        last = m
+    if behind in ("add", "norm", "silu_add"):
+        assert np.array_equal(h, r + last)
+        last = h
+    if behind == "norm":
+        want_n = po.rms_norm_batched(h, gamma, 1e-5, batch, n)
+        assert np.max(np.abs(norm - want_n) / (np.abs(want_n) + 1e-6)) < 5e-6
+        last = norm
+    if behind != "add":
+        want_y = po.matmul_q4_0_batched(w2, last, batch, 64, n)
+        assert np.max(np.abs(y - want_y)) < 1e-4 * np.max(np.abs(want_y))
+    # a chain behind the first matmul, and the sum of the second one's two slices; none joins rows that are too long
+    assert exe.rowProgramLaunches() - before == (0 if not fuse else 1 if behind in ("add", "long_rows") else 2)
