@@ -268,8 +268,9 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
  * 128); q, o and the pools 16-byte aligned.  mlc_hip_available() must have returned 1 before (set-up creates the
  * library's stream and looks up the scratch array's device address).  The call returns when the
  * kernel is enqueued (no synchronisation).  Every decode launch of this library on one GPU
- * uses the same scratch array, so they must follow each other: the library remembers the stream
- * of the last one and puts a launch on another stream behind what that stream held at the time
+ * uses the same scratch array, so they must follow each other, and so must they and matmuls whose
+ * K slices meet inside the launch (both wait for workgroups of their own): the library remembers the
+ * stream of the last one and puts a launch on another stream behind what that stream held at the time
  * (events created at set-up); what the caller enqueues on its own streams by other means is the
  * caller's to order.  Operators that earlier encode calls held back are launched first, on the
  * library's stream, and a caller's stream is put behind them.  Not possible while a pass is
@@ -304,8 +305,10 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
  * 128, page sizes and GQA ratios as in the call above, 16-byte aligned buffers).  mlc_hip_capture_end returns a
  * handle > 0, or 0 (then nothing was kept; encode the pass uncaptured).  mlc_hip_captured_launches
  * counts the launches of the encode calls; the pass holds one more, the library's own first launch,
- * which moves a device word on by which the decode launches of one replay tell their split-K
- * partials from those of the replay before.
+ * which moves a device word on by which the decode launches of one replay, and its matmuls whose K
+ * slices meet inside the launch, tell their partials from those of the replay before.  A pass holds at
+ * most 4096 decode launches; matmuls beyond 4096 such ones, and ones that find no buffer to meet in from
+ * an uncaptured call, take K whole.
  *
  * mlc_hip_replay_update copies the step's tables (seq_lens [batch], q_positions [batch],
  * page_table_offsets [batch + 1], the flat table; page_ids / slots_in_page [batch]) over the
@@ -367,8 +370,8 @@ long mlc_hip_fused_matmul_norm_launches(void);
 /* Number of decode attention launches so far that carried the step's KV write (a pair of
  * batched K / V scatters of every request's newest position encoded just before it). */
 long mlc_hip_kv_writes_in_decode_launches(void);
-/* Number of launches of held-back row operators so far: chains of them, and an add behind a held-back matmul
- * (for tests of "fuse_row_ops"). */
+/* Number of held-back row operators' chains that went out so far, and of adds behind a held-back matmul, as a
+ * launch of their own or in the matmul's epilogue (for tests of "fuse_row_ops"). */
 long mlc_hip_row_program_launches(void);
 /* Number of times so far the decode path copied a page table to the device: the copy is
  * reused while the table's content stays the same (for tests and benchmarks). */
@@ -382,8 +385,12 @@ long mlc_hip_decode_table_uploads(void);
  *   "decode_heads_per_wave" 1, 2, 4 or 8: the most query heads one wavefront handles;
  *                           the GQA group is spread over group/that many waves (0 = automatic)
  *   "decode_spin_limit"     rounds a workgroup that sums up a split pair polls for the other workgroups'
- *                           partials before it gives up and the pass fails (default 200000, about 0.1 s)
- *   "decode_test_flags"     bit 0: partials are not published (tests of the give-up path)
+ *                           partials before it gives up and the pass fails (default 200000, about 0.1 s);
+ *                           a matmul whose K slices meet inside its launch never waits for less than the
+ *                           default
+ *   "decode_test_flags"     for tests.  Bit 0: partials of the decode attention and sums of K slices are not
+ *                           published, and decode_spin_limit goes for both (the give-up path); bit 1: a
+ *                           launch, or a replay of a pass captured then, takes 2^30 tags (they start over)
  *   "decode_pv_fp16"        0 (default) = fp32-grade softmax weights: fp32 on the vector pipe, the sum
  *                           of two fp16 numbers on the matrix pipe; 1 = weights rounded to fp16
  *                           for the P.V product (fp32 accumulate)

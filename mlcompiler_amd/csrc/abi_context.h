@@ -244,7 +244,7 @@ struct Ctx {
     long kv_fused = 0;               // KV writes that went out fused with a neighbour (for tests)
     long kv_in_decode = 0;           // ... of which inside the attention launch
     long opt_fuse_rows = 1;          // 0 = every operator is launched when it is encoded
-    long row_launches = 0;           // launches of row chains and of adds behind a held-back matmul (for tests)
+    long row_launches = 0;           // row chains, and adds behind a held-back matmul, also in its epilogue (for tests)
     MetaSlot plan_slots[4];
     int plan_next = 0;
     DecodePlan plan;
@@ -726,7 +726,7 @@ bool gemm_adds() {
 int settle() {
     Ctx::RowPending& r = g.rows;
     if (r.active && !r.p.rms && gemm_adds()) {
-        // nothing but the add: 1.6 to 4 us for a launch of its own
+        // nothing but the add: 1.6 to 4 us for a launch of its own (counted like one)
         g.gemm.a.add_resid = r.p.addend;
         g.gemm.a.add_out = r.p.add_out;
         g.gemm.a.ssq_out = nullptr;

@@ -336,8 +336,7 @@ __global__ __launch_bounds__(256, 2) void matmul_tokens_kernel(const TokensArgs 
 
     if (tile >= tiles) return;
     if (tail) {
-        // (the hardware starts the slices of an XCD in order, so that nobody waits for a workgroup that is not running
-        // or done; the wait is bounded all the same)
+        // (who waits for whom: tagged_words.h)
         const uint32_t tag = launch_tag(a.tags.tag, a.tags.tag_dev ? *a.tags.tag_dev : 0u);
         uint64_t* const mine = a.meet + (size_t)in_tail * 8192 + wave * 2048 + lane;
         if (tail_slice + 1 < a.tail_slices) {

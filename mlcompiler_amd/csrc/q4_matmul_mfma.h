@@ -201,13 +201,8 @@ __device__ __forceinline__ void q4_rope_epilogue(const RopeArgs& p, const Q4Rope
     if (pool) store_through(&pool[(size_t)f.page_row * rows + local], h);
 }
 
-// 8- and 16-byte non-temporal loads (data that is read once and need not displace anything in the L2).
 typedef uint32_t q4_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t q4_u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint2 q4_stream_u2(const uint2* p) {
-    const q4_u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const q4_u32x2*>(p));
-    return make_uint2(v[0], v[1]);
-}
 
 // A buffer descriptor of `bytes` bytes: loads behind its end return zero and move no data.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t q4_buffer(const void* p, uint32_t bytes) {
@@ -615,8 +610,8 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         }
         return;
     }
-    // K slices: all but the last leave their sums as tagged words and are done; the last one's workgroups, which the
-    // hardware starts behind them, add them to their own in slice order.  (The wait is bounded all the same.)
+    // K slices: all but the last leave their sums as tagged words and are done; the last one's workgroups, which are the
+    // last of the launch, add them to their own in slice order (tagged_words.h: why the wait ends).
     const uint32_t tag = launch_tag(a.tags.tag, tag_add);
     if (slice + 1 < a.slices) {
         if (a.tags.test_flags & 1u) return;

@@ -261,7 +261,7 @@ class HipExecutor:
         return int(self._lib.mlc_hip_fused_matmul_norm_launches())
 
     def rowProgramLaunches(self) -> int:
-        """Fused row-operator launches so far (option "fuse_row_ops")."""
+        """Held-back row operators so far that went out as one: chains, and adds behind a matmul (option "fuse_row_ops")."""
         return int(self._lib.mlc_hip_row_program_launches())
 
     def setOption(self, name: str, value: int) -> bool:
