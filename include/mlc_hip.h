@@ -272,7 +272,9 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
  * K slices meet inside the launch (both wait for workgroups of their own): the library remembers the
  * stream of the last one and puts a launch on another stream behind what that stream held at the time
  * (events created at set-up); what the caller enqueues on its own streams by other means is the
- * caller's to order.  Operators that earlier encode calls held back are launched first, on the
+ * caller's to order.  A caller that records the call into a graph of its own may replay it: the launch
+ * keeps this call's lengths and reads everything else anew, and one small launch in front of it tells
+ * the replay's partials from those of the replay before.  Operators that earlier encode calls held back are launched first, on the
  * library's stream, and a caller's stream is put behind them.  Not possible while a pass is
  * being captured.  The page ids cannot be checked on the host; for pools obtained from
  * mlc_hip_alloc the kernel clamps them below the pool's size. */
@@ -390,7 +392,8 @@ long mlc_hip_decode_table_uploads(void);
  *                           default
  *   "decode_test_flags"     for tests.  Bit 0: partials of the decode attention and sums of K slices are not
  *                           published, and decode_spin_limit goes for both (the give-up path); bit 1: a
- *                           launch, or a replay of a pass captured then, takes 2^30 tags (they start over)
+ *                           launch, or a replay of a pass captured then, takes more than half of the tags
+ *                           there are (they start over)
  *   "decode_pv_fp16"        0 (default) = fp32-grade softmax weights: fp32 on the vector pipe, the sum
  *                           of two fp16 numbers on the matrix pipe; 1 = weights rounded to fp16
  *                           for the P.V product (fp32 accumulate)

@@ -24,7 +24,7 @@ int mlc_hip_capture_begin(void) {
         !resident_page_rows(g.last_ids.data(), g.last_slots.data(), g.last_ids.size(), g.last_page_size))
         return 0;
     g.cap = Ctx::Captured{};
-    g.cap.tag_step = tag_step(kReplayTagStep);
+    g.cap.tag_step = tag_step(kReplayTagStep, kLastReplayWord);
     g_capture_failed = false;
     HIP_OK(hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal));
     g_capturing = true;

@@ -67,14 +67,29 @@ constexpr uint32_t kReplayTagStep = 4096;   // decode launches of one captured p
 // Rounds that a wait for tagged words polls before it is given up (about 0.1 s).
 constexpr long kSpinLimit = 200000;
 
-// The tags of launches are numbers up to the first of these, those of captured passes lie above, at replay words up to the second.
-constexpr uint32_t kLastLaunchTag = 0x7FFFFFFFu, kLastReplayWord = 0x80000000u - kReplayTagStep;
+// Tags: those of launches are their numbers, up to the first of these; those of launches that a caller records into a graph of
+// its own lie behind, and behind them those of captured passes, at replay words up to the last.
+constexpr uint32_t kLastLaunchTag = 0x3FFFFFFFu, kRecordedTag = 0x40000000u, kLastRecordedWord = 0x3FFFFFFFu,
+                   kLastReplayWord = 0x80000000u - kReplayTagStep;
 
 // Words that have been written once stay in memory until the same place is written again: before the tags start over, every
 // buffer of such words is cleared (renew_tags).
 __global__ void clear_words_kernel(uint4* p, size_t n) {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = make_uint4(0u, 0u, 0u, 0u);
 }
+
+// In front of every decode launch that a caller records into a graph of its own: numbers this replay's launch, whose arguments
+// are the same at every replay.  When the numbers start over, which the host does not learn, the partials are cleared here
+// (one workgroup, about a millisecond every 2^30 such launches).
+__global__ __launch_bounds__(1024) void recorded_word_kernel(uint32_t* word, uint32_t step, uint4* part, uint32_t n) {
+    const uint32_t last = *word;
+    const bool over = last > kLastRecordedWord - step;
+    if (over)
+        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) part[i] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    if (threadIdx.x == 0) *word = (over ? 0u : last) + step;
+}
+constexpr size_t kScratchRecordedWordOffset = kScratchReplayWordOffset + 128;
 
 // Device copy of the flat page table (and, where the per-request arrays do not travel inside the
 // kernel arguments, of those arrays) as the tile-balanced decode kernel reads it; uploaded only
@@ -275,8 +290,8 @@ struct Ctx {
     volatile uint32_t* fault_host = nullptr;
     uint32_t* fault_dev = nullptr;
     long opt_spin_limit = kSpinLimit;       // rounds a merge of the decode attention polls before it gives up
-    // Bit 0: workgroups do not publish their partials (tests of the give-up path); bit 1: a launch and a replay take 2^30 tags
-    // (tests of what happens when they run out).
+    // Bit 0: workgroups do not publish their partials (tests of the give-up path); bit 1: a launch and a replay take more than
+    // half of the tags there are (tests of what happens when they run out).
     long opt_test_flags = 0;
     StreamTables tables;
     long opt_wgs_per_cu = 0;        // tile-balanced kernel: workgroups per CU (0 = automatic)
@@ -423,7 +438,8 @@ int settle_gemm(const RopeArgs* rope);
 int scratch_follow(hipStream_t stream);
 int scratch_launched(hipStream_t stream);
 
-uint32_t tag_step(uint32_t step) { return g.opt_test_flags & 2 ? 1u << 30 : step; }
+// Tags that a launch or a replay takes, of a kind that goes up to `last`.
+uint32_t tag_step(uint32_t step, uint32_t last) { return g.opt_test_flags & 2 ? last / 2 + 1 : step; }
 
 // No tag is left that none of the words in memory can have: clears them, behind every launch that uses them, and starts over.
 int renew_tags() {
@@ -456,7 +472,7 @@ TagArgs next_tags(size_t& in_pass) {
         t.tag = 0x80000000u | (uint32_t)in_pass++;
         t.tag_dev = reinterpret_cast<const uint32_t*>(g.scratch_ptr + kScratchReplayWordOffset);
     } else {
-        const uint32_t step = tag_step(1);
+        const uint32_t step = tag_step(1, kLastLaunchTag);
         if (g.next_tag > kLastLaunchTag - step) (void)renew_tags();   // (a failure shows at the launch behind it)
         g.next_tag += step;
         t.tag = g.next_tag;

@@ -308,13 +308,21 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
     std::memcpy(a.emb, seq_lens, batch * 4);
     std::memcpy(a.emb + emb_stride, q_positions, batch * 4);
     std::memcpy(a.emb + 2 * emb_stride, page_table_offsets, batch * 4);
+    const bool recorded = caller_records(st);
+    if (recorded) {
+        uint32_t* word = reinterpret_cast<uint32_t*>(g.scratch_ptr + kScratchRecordedWordOffset);
+        hipLaunchKernelGGL(recorded_word_kernel, dim3(1), dim3(1024), 0, st, word, tag_step(1, kLastRecordedWord),
+                           reinterpret_cast<uint4*>(g.scratch_ptr), (uint32_t)(kStreamPartBytes / 16));
+        a.tag = kRecordedTag;
+        a.tag_dev = word;
+    }
     if (!launch_stream_variant(head_dim, hpw, nw, nbuf, a, n_wg, dyn_lds, st))
         return fail("decode: kernel variant not built");
     HIP_OK(hipGetLastError());
     g.last_items = (int)stream_workgroups((uint32_t)(total_tiles / kv_heads), with_tiles, (uint32_t)kv_heads, n_wg);
     std::snprintf(g.last_kernel, sizeof g.last_kernel, "stream<%zu,%d,%d,%s,%s,%d>", head_dim, hpw, nw,
                   stream_pv_name(hpw, nw), batch <= 64 ? "regs" : "lds", nbuf);
-    g.last_launches = 1;
+    g.last_launches = recorded ? 2 : 1;
     return 1;
 }
 

@@ -308,10 +308,10 @@ const char* stream_pv_name(int hpw, int nw) {
 // a graph of its own does not run now: when that graph runs is the caller's to order.)
 bool caller_records(hipStream_t stream) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    return stream != g.stream && hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
 }
 int scratch_follow(hipStream_t stream) {
-    if (g_capturing || caller_records(stream)) return 1;
+    if (g_capturing || (stream != g.stream && caller_records(stream))) return 1;
     if (g.scratch_in_use && g.scratch_stream != stream) {
         if (g.scratch_stream == g.stream) HIP_OK(hipEventRecord(g.scratch_ev, g.stream));
         HIP_OK(hipStreamWaitEvent(stream, g.scratch_ev, 0));
@@ -319,7 +319,7 @@ int scratch_follow(hipStream_t stream) {
     return 1;
 }
 int scratch_launched(hipStream_t stream) {
-    if (g_capturing || caller_records(stream)) return 1;
+    if (g_capturing || (stream != g.stream && caller_records(stream))) return 1;
     g.scratch_stream = stream;
     g.scratch_in_use = true;
     if (stream != g.stream) HIP_OK(hipEventRecord(g.scratch_ev, stream));

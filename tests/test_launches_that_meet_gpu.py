@@ -149,7 +149,7 @@ KINDS = {"decode": _decode, "slices": _matmul(64, 4096, 5), "tail": _matmul(4160
 @pytest.mark.parametrize("kind", list(KINDS))
 @pytest.mark.parametrize("captured", [False, True])
 def test_tags_that_come_again(exe, kind, captured):
-    """Every launch (replay) takes 2^30 tags, so that they start over at once, and the second one does not write
+    """Every launch (replay) takes more than half of the tags, so that they start over at once, and the second one does not write
     its words: those of the first, which had the same tag, are gone, and the wait for the second's is given up."""
     call, read, free = KINDS[kind](exe)
     handles = []
@@ -293,3 +293,57 @@ def test_a_decode_recorded_into_a_callers_graph_orders_nothing(exe):
         exe.releaseScratchBuffer(d_flat)
         dev.free()
         free()
+
+
+@pytest.mark.parametrize("own", [True, False])      # a stream of the caller's, or the library's
+@pytest.mark.parametrize("flags", [0, 2])
+def test_a_decode_replayed_from_a_callers_graph(exe, flags, own):
+    """Every replay sums the partials of its own, and none of the one before (at once also where the tags start over)."""
+    import ctypes as C
+    from mlcompiler_amd._lib import load
+    from paged_cases import DeviceCase, baseline_config
+    lib, hip, stream, graph, run = load(), _hip(), C.c_void_p(), C.c_void_p(), C.c_void_p()
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    case = baseline_config(2, batch=6)
+    dev = DeviceCase(exe, case)
+    arrays = [np.ascontiguousarray(a, np.uint32) for a in (case.page_tables_flat, case.page_table_offsets, case.seq_lens, case.q_positions)]
+    d_flat, d_o = _pool(exe, arrays[0]), exe.allocateScratchBuffer(case.q.nbytes)
+    u32p = lambda a: a.ctypes.data_as(C.POINTER(C.c_uint32))
+    rng = np.random.default_rng(4)
+    qs = [rng.standard_normal(case.q.shape).astype(np.float32) for _ in range(20)]
+    want = []
+    if own:
+        assert hip.hipStreamCreate(C.byref(stream)) == 0
+    else:
+        stream.value = lib.mlc_hip_stream()
+    try:
+        for q in qs:
+            assert exe.uploadToBuffer(dev.q_buf, q)
+            want.append(dev.run().copy())
+        assert exe.setOption("decode_test_flags", flags)
+        assert hip.hipStreamBeginCapture(stream, 1) == 0       # (this thread's calls)
+        ok = lib.mlc_hip_paged_attn_decode_noalloc(dev.q_buf, dev.k_buf, dev.v_buf, d_o, d_flat, arrays[0].size, u32p(arrays[1]),
+                                                   u32p(arrays[2]), u32p(arrays[3]), case.batch, case.num_heads, case.kv_heads,
+                                                   case.head_dim, case.page_size, int(case.apply_causal), stream)
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and ok, exe.lastError()
+        assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+        assert exe.setOption("decode_test_flags", 0)
+        for q, o in zip(qs, want):
+            assert exe.uploadToBuffer(dev.q_buf, q)
+            assert hip.hipGraphLaunch(run, stream) == 0 and hip.hipStreamSynchronize(stream) == 0
+            assert np.array_equal(_read(exe, d_o, np.empty_like(o)), o)
+    finally:
+        exe.setOption("decode_test_flags", 0)
+        if run:
+            hip.hipGraphExecDestroy(run)
+        if graph:
+            hip.hipGraphDestroy(graph)
+        if own:
+            hip.hipStreamDestroy(stream)
+        for b in (d_flat, d_o):
+            exe.releaseScratchBuffer(b)
+        dev.free()
