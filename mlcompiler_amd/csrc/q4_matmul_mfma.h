@@ -265,9 +265,9 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // a wave's last blocks) -> now.  One request of the 1 B shape: qkv (2560 x 2048) 7.0 -> 4.5, out-projection with the
 // residual add 8.4 -> 4.6, gate/up with SiLU (11264 x 2048) 11.2 -> 7.0, down (2048 x 5632) 8.1 and 5.0 for the sum of
 // its K slices -> 5.5 with the residual add, three slices that meet in here; a step of 22 layers 1 145 -> 801 (845 with the
-// fragments of 32 requests as they are for larger batches).  32 requests: qkv 7.5 -> 6.9,
-// gate/up 13.3 -> 13.3, a step 1 330 -> 1 199.  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
-// a layer 140 -> 112.  2-norm error against float64 of rows of 2048 to 14336: 0.95e-7 .. 1.17e-7, before 1.03e-7 .. 1.62e-7.
+// fragments of 32 requests as they are for larger batches; 703 with everything since).  32 requests: qkv 7.5 -> 6.9,
+// gate/up 13.3 -> 13.3, a step 1 330 -> 1 199 (1 108).  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
+// a layer 140 -> 112 (106).  2-norm error against float64 of rows of 2048 to 14336: 0.95e-7 .. 1.17e-7, before 1.03e-7 .. 1.62e-7.
 //
 // The arguments that the first loads need come in front and as scalars: they are in registers when a wave starts (kernel
 // argument preload, build.py), so that weights and activations are requested at once and what the epilogue reads, whose
