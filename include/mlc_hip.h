@@ -419,6 +419,8 @@ long mlc_hip_decode_table_uploads(void);
  *                           add + RMSNorm; the fp16 split of the matmul that reads their output):
  *                           see the mlc_hip_fused_* counters above.
  *                           0 = each operator is launched when it is encoded
+ *   "q4_chain"              1 (default) = for up to four requests, a Q4_0 matmul with its residual add and the
+ *                           matmul that reads the RMSNorm behind it go out in one launch; 0 = always two
  *   "decode_pair_cost"      0..64: the tile-balanced decode kernel gives every workgroup the same
  *                           number of units, a KV tile counting one and the end of a (request,
  *                           KV head) pair this many; 0 = the same number of tiles; -1 (default) =

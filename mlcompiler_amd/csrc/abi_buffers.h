@@ -40,6 +40,7 @@ void* cached_buffer(const char* name, size_t bytes) {
     if (it != g.cached.end() && it->second.second >= bytes) return it->second.first;
     if (g_capturing) { fail("cached buffer: allocation is not possible while a pass is being captured"); return nullptr; }
     if (it != g.cached.end()) {  // grow-only reallocation, metal_runtime.mm:8222-8241
+        if (!settle_front()) return nullptr;   // (it may read the one that is given up; whatever else is pending is the caller's to launch)
         (void)hipStreamSynchronize(g.stream);
         g.allocs.erase(it->second.first);
         (void)hipFree(it->second.first);

@@ -56,13 +56,16 @@ constexpr size_t kScratchBytes = kScratchReplayWordOffset + 256;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 // The buffers in which the K slices of matmuls meet (meeting_words) hold tagged words as well.
-constexpr const char* kMeetingWords[] = {"q4_k_meet", "tokens_k_meet"};
+constexpr const char* kMeetingWords[] = {"q4_k_meet", "tokens_k_meet", "q4_link_words"};
 
 // First launch of every captured pass: moves the replay word on, so that the launches of
 // this replay (whose arguments, tag included, are the same at every replay) use tags that the
 // replay before did not.
 __global__ void replay_word_kernel(uint32_t* word, uint32_t step) { *word += step; }
 constexpr uint32_t kReplayTagStep = 4096;   // decode launches of one captured pass, at most, and sliced matmuls with a tag
+
+// Room for the words between two matmuls of a launch (q4_link_words): four requests of 4096 columns, eight copies, take 2.2 MB.
+constexpr size_t kLinkBytes = 4u << 20;
 
 // Rounds that a wait for tagged words polls before it is given up (about 0.1 s).
 constexpr long kSpinLimit = 200000;
@@ -234,6 +237,15 @@ struct Ctx {
         const void* silu_out = nullptr;
         size_t ffn_inner = 0;
     } gemm;
+    // The matmul in front of the held-back one, where its epilogue does the residual add and starts the norm that the
+    // held-back one reads: both go out in one launch where they can (launch_chain), and this one alone before anything
+    // that it reads is replaced.
+    struct GemmFront {
+        bool active = false;
+        bool block_scales = false;
+        Q4RopeArgs a{};
+    } front;
+    long opt_q4_chain = 1;           // 0 = always two launches
     // The tile-balanced decode attention launch of the open pass, held back for one call: when that
     // call is a Q4_0 matmul that reads the attention's output (the out-projection), the kernel
     // that writes a row of the output also writes it as that matmul's split-fp16 activations, one
@@ -256,6 +268,7 @@ struct Ctx {
     long gemm_silu_split_fused = 0;  // ... of which also wrote the next matmul's activation fragments
     std::vector<uint32_t> last_ids, last_slots;   // see place_page_rows
     size_t last_page_size = 0;
+    size_t last_page_row = 0;        // the highest row of the last KV write
     long kv_fused = 0;               // KV writes that went out fused with a neighbour (for tests)
     long kv_in_decode = 0;           // ... of which inside the attention launch
     long opt_fuse_rows = 1;          // 0 = every operator is launched when it is encoded
@@ -434,6 +447,8 @@ void slot_mark(MetaSlot& s) { s.use = ++g.slot_uses; }
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 int settle_gemm(const RopeArgs* rope);
+int settle_front();
+uint64_t* meeting_words(const char* name, size_t bytes);
 
 int scratch_follow(hipStream_t stream);
 int scratch_launched(hipStream_t stream);
@@ -494,8 +509,8 @@ bool sliced_tags_left() { return !g_capturing || g.cap.n_sliced < kReplayTagStep
 const void* resident_blob(int kind, const void* key, const void* blob, size_t bytes) {
     // A caller that never repeats itself: start over -- but only while no held-back operator
     // refers to one of the copies (their launches come later).
-    if (g.resident.size() > 1024 && !g.rows.active && !g.kv.active && !g.gemm.active && !g.dec.active && !g_capturing &&
-        g.captures.empty()) {   // (a captured pass keeps the addresses of the copies it read)
+    if (g.resident.size() > 1024 && !g.rows.active && !g.kv.active && !g.gemm.active && !g.front.active && !g.dec.active &&
+        !g_capturing && g.captures.empty()) {   // (a captured pass keeps the addresses of the copies it read)
         if (!wait_stream()) return nullptr;
         for (auto& kv : g.resident)
             if (kv.second.dev) (void)hipFree(kv.second.dev);
@@ -514,6 +529,7 @@ const void* resident_blob(int kind, const void* key, const void* blob, size_t by
         r.cap = cap;
     }
     // (a held-back matmul that finishes an RMSNorm reads the weights as they were: it goes out in front of the copy)
+    if (r.dev && g.front.active && (g.front.a.rms_gamma == r.dev || g.front.a.add_gamma == r.dev) && !settle_front()) return nullptr;
     if (r.dev && g.gemm.active && g.gemm.a.rms_gamma == r.dev && !settle_gemm(nullptr)) return nullptr;
     r.content.clear();  // not valid until the copy has been enqueued
     MetaSlot& s = g.ring[g.ring_next];
@@ -557,15 +573,24 @@ int q4_tiles(Q4Form form, size_t rows, size_t batch, size_t ksplit) {
     return std::min(most, std::max(least, wgs > 2 * n_cu ? 4 : wgs > n_cu ? 2 : 1));
 }
 
+// Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; where there are more
+// workgroups than CUs, with 4 tiles each, they have 8, two workgroups to a CU, so that one's first loads overlap the
+// other's products.
+int q4_waves(const Q4Args& a) { return a.rows / 64 * ((a.batch + 15) / 16) * a.slices > (size_t)g.n_cu ? 8 : 16; }
+
+int launch_chain(Q4Form form, bool block_scales, Q4RopeArgs& a);
+
 // Launches q4_matmul_kernel in one of its forms.
 int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a) {
+    if (g.front.active) {
+        const int chained = launch_chain(form, block_scales, a);
+        if (chained >= 0) return chained;
+        if (!settle_front()) return 0;
+    }
     const size_t tiles = a.rows / 16, z = (a.batch + 15) / 16, n_cu = (size_t)g.n_cu, ksplit = a.slices;
     const int rt = q4_tiles(form, a.rows, a.batch, ksplit);
     a.row_groups = (uint32_t)(tiles / rt);
-    // Waves per workgroup, the same for every form of a call (they divide K).  16 fill a CU; where there are more
-    // workgroups than CUs, with 4 tiles each, they have 8, two workgroups to a CU, so that one's first loads overlap the
-    // other's products.
-    const int waves = tiles / 4 * z * ksplit > n_cu ? 8 : 16;
+    const int waves = q4_waves(a);
     // Such workgroups take four or two groups of 16 requests each, one workgroup to a CU, where those are one round of at
     // least five eighths of the CUs, or rounds of which the last is at least half full, with no group missing.  (Whole calls,
     // us, one group per workgroup -> now, and one workgroup of 32 x 32 products per 64 requests: 28672 x 4096 at 32, 49 and
@@ -588,11 +613,80 @@ int launch_q4(Q4Form form, bool block_scales, Q4RopeArgs& a) {
     return ksplit > 1 ? scratch_launched(g.stream) : 1;
 }
 
+// Launches the matmul in front of the held-back one by itself.
+int settle_front() {
+    if (!g.front.active) return 1;
+    g.front.active = false;
+    return launch_q4(kQ4Add, g.front.block_scales, g.front.a);
+}
+
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
+}
+
+// The matmul in front and the held-back one in one launch (q4_chain_kernel): 1, 0 on failure, -1 where they cannot be.
+int launch_chain(Q4Form form, bool block_scales, Q4RopeArgs& b) {
+    Q4RopeArgs& a = g.front.a;
+    const size_t batch = b.batch;
+    if (!g.opt_q4_chain || (form != kQ4Silu && form != kQ4Rope) || !block_scales || !g.front.block_scales || !b.ssq_in || b.ssq_in != a.ssq_out ||
+        batch > 4 || b.slices != 1 || q4_waves(a) != 16 || q4_waves(b) != 16 || q4_tiles(kQ4Add, a.rows, batch, a.slices) != 2)
+        return -1;
+    const int rt = q4_tiles(form, b.rows, batch, 1);
+    if (rt * ((b.nquads + 15) / 16) > 4) return -1;
+    a.row_groups = a.rows / 32;
+    a.z_groups = b.z_groups = 1;
+    b.row_groups = (uint32_t)(b.rows / 16 / rt);
+    const uint32_t blocks = (a.row_groups + 7) / 8 * 8 * a.slices, grid = blocks + (b.row_groups + 7) / 8 * 8;
+    if (blocks > 0xFFFFu || grid > 2 * (uint32_t)g.n_cu) return -1;
+    // The second matmul's workgroups run beside the first one's: what they write must be nothing that those read or write,
+    // and what they read besides the words nothing that those write.
+    const size_t row = batch * a.rows * 4;
+    bool apart = true;
+    const auto writes = [&](const void* p, size_t bytes) {
+        if (!p) return;
+        for (const void* q : {(const void*)a.out, (const void*)a.add_out, (const void*)a.add_resid}) apart = apart && !overlap(p, bytes, q, row);
+        if (a.ssq_in)
+            for (const void* q : {(const void*)a.rms_src, (const void*)a.rms_out}) apart = apart && !overlap(p, bytes, q, batch * a.rms_len * 4);
+    };
+    const auto reads = [&](const void* p, size_t bytes) {
+        for (const void* q : {(const void*)a.out, (const void*)a.add_out}) apart = apart && !overlap(p, bytes, q, row);
+        if (a.ssq_in) apart = apart && !overlap(p, bytes, a.rms_out, batch * a.rms_len * 4);
+    };
+    writes(b.out, batch * b.rows * 4);
+    writes(b.rms_out, batch * b.rms_len * 4);
+    if (form == kQ4Silu) {
+        for (const void* p : {(const void*)b.gate, (const void*)b.up, (const void*)b.silu_out}) writes(p, batch * b.ffn_inner * 4);
+    } else {
+        const RopeArgs& r = b.rope;
+        writes(r.q, batch * r.q_rows * 4);
+        writes(r.k, batch * r.k_rows * 4);
+        writes(r.v, batch * r.v_rows * 4);
+        writes(r.k_f16, batch * r.k_rows * 2);
+        writes(r.v_f16, batch * r.v_rows * 2);
+        writes(r.k_pages, (g.last_page_row + 1) * r.k_rows * 2);
+        writes(r.v_pages, (g.last_page_row + 1) * r.v_rows * 2);
+        reads(r.cos_table, batch * (r.rotary_dim / 2) * 4);
+        reads(r.sin_table, batch * (r.rotary_dim / 2) * 4);
+    }
+    const size_t bytes = q4_link_words(a.rows, b.batch) * 8 * kQ4LinkCopies;
+    if (!apart || bytes > kLinkBytes || !sliced_tags_left()) return -1;
+    Q4Link link;
+    link.words = meeting_words("q4_link_words", kLinkBytes);
+    if (!link.words) return -1;
+    link.tags = next_sliced_tags();
+    g.front.active = false;
+    if (!scratch_follow(g.stream)) return 0;
+    if (!launch_q4_chain(form, rt, blocks, grid, a, b, link, g.stream)) return fail("q4 matmul: kernel variant not built");
+    HIP_OK(hipGetLastError());
+    return scratch_launched(g.stream);
+}
+
 // Launches the held-back matmul, with the split + RoPE + cast of its output as epilogue when
 // `rope` is given.
 int settle_gemm(const RopeArgs* rope) {
     Ctx::GemmPending& m = g.gemm;
-    if (!m.active) return 1;
+    if (!m.active) return settle_front();
     m.active = false;
     Q4RopeArgs a;
     static_cast<Q4Args&>(a) = m.a;
@@ -610,11 +704,6 @@ int settle_gemm(const RopeArgs* rope) {
         form = kQ4Add;
     }
     return launch_q4(form, m.block_scales, a);
-}
-
-bool overlap(const void* a, size_t na, const void* b, size_t nb) {
-    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-    return x < y + nb && y < x + na;
 }
 
 // Two buffers of one launch whose element i belongs to the same thread: do they meet at other elements than their own?
@@ -677,6 +766,8 @@ bool place_page_rows(const uint32_t* page_ids, const uint32_t* slots, size_t bat
         g.last_slots.assign(slots, slots + batch);
         g.last_page_size = page_size;
     }
+    g.last_page_row = 0;
+    for (size_t r = 0; r < batch; ++r) g.last_page_row = std::max(g.last_page_row, (size_t)page_ids[r] * page_size + slots[r]);
     if (batch > most || g_capturing) return (*dev = resident_page_rows(page_ids, slots, batch, page_size)) != nullptr;
     for (size_t r = 0; r < batch; ++r) emb[r] = (uint64_t)page_ids[r] * page_size + slots[r];
     return true;
@@ -723,7 +814,7 @@ int settle_before_rows() {
     if (!settle_decode()) return 0;
     // a held-back matmul is older than anything else pending, unless the pending KV write is
     // its own epilogue
-    if (g.gemm.active && !(g.kv.active && g.kv.rope && g.kv.from_gemm) && !settle_gemm(nullptr)) return 0;
+    if ((g.gemm.active || g.front.active) && !(g.kv.active && g.kv.rope && g.kv.from_gemm) && !settle_gemm(nullptr)) return 0;
     return settle_kv();
 }
 

@@ -246,7 +246,7 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
     {
         // operators held back by earlier encode calls are launched now, on the library's stream
         // (kernel launches only); a caller's stream of its own is put behind them
-        const bool pending = g.rows.active || g.kv.active || g.gemm.active || g.dec.active;
+        const bool pending = g.rows.active || g.kv.active || g.gemm.active || g.front.active || g.dec.active;
         if (!settle()) return 0;
         if (pending && st != g.stream) {
             HIP_OK(hipEventRecord(g.scratch_ev, g.stream));

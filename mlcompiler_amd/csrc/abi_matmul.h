@@ -211,7 +211,12 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             norm.rms_n_gamma = p.n_weight;
             g.rows.active = false;   // the two matmuls do the chain's work
             ++g.gemm_rms_fused;
-            if (!settle()) return 0;
+            // (nothing else is pending: settle() would launch it, and does where this matmul turns out to go out alone)
+            if (!settle_front()) return 0;
+            m.active = false;
+            g.front.active = true;
+            g.front.block_scales = m.block_scales;
+            static_cast<Q4Args&>(g.front.a) = m.a;
         } else if (feeds) {  // the chain that produces the input also splits it (batch <= 64: one round)
             g.rows.p.frag = frag;
             g.rows.p.inv_scale = inv;

@@ -75,6 +75,7 @@ int mlc_hip_set_option(const char* name, long value) {
     if (!std::strcmp(name, "decode_pv_fp16")) { g.opt_pv_fp16 = value ? 1 : 0; return 1; }
     if (!std::strcmp(name, "q4_force_generic")) { g.opt_q4_force_generic = value ? 1 : 0; return 1; }
     if (!std::strcmp(name, "q4_int_operand")) { g.opt_q4_int_operand = value ? 1 : 0; return 1; }
+    if (!std::strcmp(name, "q4_chain")) { g.opt_q4_chain = value ? 1 : 0; return 1; }
     if (!std::strcmp(name, "q4_ksplit")) {
         if (value < 0 || value > 64) return 0;
         g.opt_q4_ksplit = value;

@@ -42,6 +42,7 @@ MLC_DECL(128, 1) MLC_DECL(128, 2) MLC_DECL(128, 4) MLC_DECL(128, 8)
 bool launch_q4_matmul_1(int, int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
 bool launch_q4_matmul_2(int, int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
 bool launch_q4_matmul_4(int, int, int, int, bool, dim3, const Q4RopeArgs&, hipStream_t);
+bool launch_q4_chain(int, int, uint32_t, uint32_t, const Q4Args&, const Q4RopeArgs&, const Q4Link&, hipStream_t);
 }  // namespace mlc_hip
 
 // The sections of this translation unit, in the order they build on one another.

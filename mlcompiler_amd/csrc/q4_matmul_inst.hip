@@ -35,4 +35,21 @@ bool MLC_CAT(launch_q4_matmul_, MLC_Q4_NI)(int form, int rt, int waves, int zt, 
     return false;
 }
 
+#if MLC_Q4_NI == 1
+// Two matmuls in one launch, `blocks` workgroups of them the first one's; false: there is no such variant
+bool launch_q4_chain(int form, int rt, uint32_t blocks, uint32_t grid, const Q4Args& a, const Q4RopeArgs& b, const Q4Link& link,
+                     hipStream_t stream) {
+    const auto launch = [&](auto kernel, const auto& args) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(1024), 0, stream, a.q, a.d, a.xfrag, a.blk_scale, a.ssq_in, a.nblocks, a.quads_per_slice,
+                           a.row_groups, a.batch | blocks << 16, args);
+        return true;
+    };
+    const uint32_t quads = (b.nquads + 15) / 16;   // per wave of the second matmul
+    if (form == kQ4Silu && rt == 4 && quads == 1) return launch(q4_chain_kernel<4, 1, kQ4Silu>, Q4ChainArgs<kQ4Silu>{a, b, link});
+    if (form == kQ4Rope && rt == 1 && quads <= 2) return launch(q4_chain_kernel<1, 2, kQ4Rope>, Q4ChainArgs<kQ4Rope>{a, b, link});
+    if (form == kQ4Rope && rt == 2 && quads <= 2) return launch(q4_chain_kernel<2, 2, kQ4Rope>, Q4ChainArgs<kQ4Rope>{a, b, link});
+    return false;
+}
+#endif
+
 }  // namespace mlc_hip

@@ -146,6 +146,46 @@ __device__ __forceinline__ void q4_emit_block(float v, uint32_t b, uint32_t col,
     if (col % 32 == 0) store_through(&blk_scale[((size_t)(b / 32) * (k_cols / 32) + col / 32) * 32 + b % 32], __builtin_ldexpf(1.0f, -se));
 }
 
+// Two matmuls in one launch (q4_chain_kernel): what the first one's workgroups leave for the second one's, K columns of R
+// requests, as tagged words (tagged_words.h).  First, for every quad of K (128 columns), in lines of its own (every workgroup's
+// waves poll them: with all quads' scales side by side, in the memory of one or two channels, a word took 2 us to arrive):
+//   [4][R]    a block's scale
+//   [4][R]    ... and its sum of squares (of the RMSNorm in between)
+//   [R][128]  {hi, lo} of an activation, the fragments of the second matmul
+// and behind the quads [R][K], the values that the RMSNorm reads.
+// All of it kQ4LinkCopies times, for the workgroups x % copies of the second matmul: a word that all of them poll in one place
+// is late by as much as their loads take turns there.
+struct Q4Link {
+    uint64_t* words;
+    TagArgs tags;
+};
+static constexpr uint32_t kQ4LinkCopies = 8;
+__host__ __device__ __forceinline__ uint32_t q4_link_quad(uint32_t R) { return (R * 136 + 31) / 32 * 32; }
+__host__ __device__ __forceinline__ size_t q4_link_sum(uint32_t K, uint32_t R) { return (size_t)((K + 127) / 128) * q4_link_quad(R); }
+__host__ __device__ __forceinline__ size_t q4_link_words(uint32_t K, uint32_t R) { return q4_link_sum(K, R) + (size_t)K * R; }
+
+// What q4_emit_block does, as those words.
+__device__ __forceinline__ void q4_emit_words(float v, float sum, float ssq, uint32_t b, uint32_t col, uint32_t K, uint32_t R,
+                                              uint64_t* words, uint32_t tag) {
+    const float amax = q4_half_wave_max(fabsf(v));
+    int e = 0;
+    if (amax > 0.f && amax < INFINITY) (void)frexpf(amax, &e);
+    int se = 14 - e;
+    se = se > 100 ? 100 : (se < -100 ? -100 : se);
+    const float tv = __builtin_ldexpf(v, se);
+    const _Float16 hi = (_Float16)tv;
+    const _Float16 lo = (_Float16)(tv - (float)hi);
+    const uint64_t t = (uint64_t)tag << 32;
+    uint64_t* const quad = words + (size_t)(col / 128) * q4_link_quad(R);
+    st_tagged(quad + 8 * R + b * 128 + col % 128, t | __builtin_bit_cast(uint16_t, hi) | (uint32_t)__builtin_bit_cast(uint16_t, lo) << 16);
+    if (col % 32 == 0) {
+        const uint32_t blk = col / 32 % 4 * R + b;
+        st_tagged(quad + blk, t | __float_as_uint(__builtin_ldexpf(1.0f, -se)));
+        st_tagged(quad + 4 * R + blk, t | __float_as_uint(ssq));
+    }
+    st_tagged(words + q4_link_sum(K, R) + (size_t)b * K + col, t | __float_as_uint(sum));
+}
+
 // The split + RoPE + cast (+ paged write) of one element of a request's fused qkv row, by the
 // thread that just produced it; the partner of its (even, odd) pair sits in the neighbouring
 // lane.  Same arithmetic, element for element, as qkv_split_rope_cast_kernel.  What the thread
@@ -257,7 +297,8 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // More than 16 requests: z groups of 16, workgroups of their own that read the same weights at the same
 // time on the same XCD (workgroup x: row group x / (8 Z) * 8 + x % 8, z group x / 8 % Z).  Each fetches its
 // own activations only, 4 bytes per request and column through one CU's memory path, which would be the
-// longest stream of a workgroup that had them all.  ZT = 2 or 4: so many groups in one
+// longest stream of a workgroup that had them all.  (NI < 4: the A operand has room for hi and lo of a request in different rows, and
+// one product does for both.  2-norm error against float64, two products -> one: 0.95e-7 .. 1.07e-7 -> 0.85e-7 .. 0.98e-7.)  ZT = 2 or 4: so many groups in one
 // workgroup, which unpacks a weight once for all of them.  That takes 158 or 245 registers, one workgroup of 8 waves to a
 // CU, and so pays where such workgroups fill their rounds (launch_q4).
 //
@@ -273,11 +314,35 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
 // argument preload, build.py), so that weights and activations are requested at once and what the epilogue reads, whose
 // addresses take a fetch of the other arguments, behind them.  (From the argument segment, epilogue first -> now: steps of
 // 22 layers of the 1 B shape 757 -> 740 us at one request, 1 160 -> 1 121 at 32, a layer of the 8 B shape at 16 109.2 -> 107.)
-template <int NI, int RT, int WAVES, bool BS, int FORM, int ZT = 1>
-__global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
+//
+// LINK: the kernel is one of two matmuls in a launch (q4_chain_kernel): kQ4LinkOut, the first (residual add), leaves the
+// second one's activations as tagged words, kQ4LinkIn, the second, takes them from there: at most QUADS quads per wave, whose
+// weights are unpacked while the wave has to wait.
+enum Q4LinkKind { kQ4LinkNone = 0, kQ4LinkOut = 1, kQ4LinkIn = 2 };
+
+template <int NI, int RT, int WAVES, bool BS, int ZT>
+struct Q4Lds {
+    static constexpr bool PACKED = NI < 4;
+    static constexpr int XQ = PACKED ? 2 * NI : 1, QR = 4 * NI * ZT;
+    static constexpr int TILE_PITCH = NI * 64 + 16;         // floats per tile (16: bank spread)
+    float red[WAVES * RT * ZT * TILE_PITCH];
+    // BS: a quad's scales, [block][request]: fetched by a load of 4 bytes per lane, handed out from here.  (A load of
+    // every lane's own scales per block would take as long as one of the block's two fragments: what bounds these
+    // kernels next to the vector pipe is the 64 bytes a clock that a CU's loads return.)
+    __attribute__((aligned(16))) float scales[BS ? WAVES : 1][ZT][64];
+    q4_u32x4 packed[PACKED ? WAVES : 1][PACKED ? XQ * 64 : 1];
+    float rms_scale[BS ? QR : 1];         // BS with ssq_in: every request's RMSNorm factor
+};
+
+template <int NI, int RT, int WAVES, bool BS, int FORM, int ZT, int LINK, int QUADS, class Args>
+__device__ __forceinline__ void q4_matmul_workgroup(
+    Q4Lds<NI, RT, WAVES, BS, ZT>& lds, const uint32_t block_x, const uint32_t slice, const uint32_t rope_args_offset,
     const uint4* const w_q, const uint2* const w_d, const _Float16* const xfrag, const float* const blk_scale, const float* const ssq_in,
-    const uint32_t nblocks, const uint32_t quads_per_slice, const uint32_t row_groups, const uint32_t batch_z,
-    const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
+    const uint32_t nblocks, const uint32_t quads_per_slice, const uint32_t row_groups, const uint32_t batch_z, const Args& a,
+    const Q4Link& link) {
+    constexpr bool LINKED = LINK == kQ4LinkIn;
+    static_assert(LINK == kQ4LinkNone || (NI == 1 && WAVES == 16 && BS && ZT == 1), "two matmuls in a launch: up to 4 requests");
+    static_assert(LINK != kQ4LinkOut || FORM == kQ4Add, "the first of two: with the residual add");
     static_assert(FORM != kQ4Silu || RT == 4, "SiLU epilogue: 32 rows of gate and 32 of up");
     static_assert(FORM != kQ4Add || RT % 2 == 0, "residual add: whole blocks of the next matmul's K");
     // Up to 8 requests: a quad's activations come 1 KB per load, without the places of requests that do not
@@ -291,21 +356,17 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     static_assert(ZT == 1 || (RT == 4 && WAVES == 8 && !PACKED), "more than one group of 16 requests: one workgroup of 8 waves to a CU");
     constexpr int X_TILES = (ZT + 1) / 2;            // batch tiles of 32 that the workgroup has a part of
     constexpr int QR = 4 * NI * ZT;                       // requests of the workgroup
-    constexpr int TILE_PITCH = NI * 64 + 16;         // floats per tile in LDS (16: bank spread)
-    __shared__ float red[WAVES * RT * ZT * TILE_PITCH];
-    // BS: a quad's scales, [block][request]: fetched by a load of 4 bytes per lane, handed out from here.  (A load of
-    // every lane's own scales per block would take as long as one of the block's two fragments: what bounds these
-    // kernels next to the vector pipe is the 64 bytes a clock that a CU's loads return.)
-    __shared__ __attribute__((aligned(16))) float scales[BS ? WAVES : 1][ZT][64];
-    __shared__ q4_u32x4 packed[PACKED ? WAVES : 1][XQ * 64];
-    __shared__ float rms_scale[BS ? QR : 1];         // BS with ssq_in: every request's RMSNorm factor
+    constexpr int TILE_PITCH = Q4Lds<NI, RT, WAVES, BS, ZT>::TILE_PITCH;
+    auto& red = lds.red;
+    auto& scales = lds.scales;
+    auto& packed = lds.packed;
+    auto& rms_scale = lds.rms_scale;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t lane = threadIdx.x % 64, l16 = lane % 16, kg = lane / 16;
     const uint32_t batch = batch_z & 0xFFFFu, z_groups = batch_z >> 16, nquads = (nblocks + 3) / 4;
     const uint32_t z8 = 8 * z_groups;
-    const uint32_t row_group = blockIdx.x / z8 * 8 + blockIdx.x % 8, zg = blockIdx.x / 8 % z_groups;
+    const uint32_t row_group = block_x / z8 * 8 + block_x % 8, zg = block_x / 8 % z_groups;
     if (row_group >= row_groups) return;           // (the grid is a multiple of 8 row groups)
-    const uint32_t slice = blockIdx.y;
     const uint32_t req0 = zg * (16 * ZT), live = min((uint32_t)QR, batch - req0);   // (the last group may be smaller)
     // tile r of the workgroup
     const uint32_t tile0 = FORM == kQ4Silu ? row_group * 2 : row_group * RT;
@@ -319,10 +380,13 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     const uint32_t row = threadIdx.x % ROWS, qi = threadIdx.x / ROWS;
     // (which request: so that the 64 lanes of a wave read 64 different banks)
     constexpr uint32_t SB = 2 * NI;
-    const uint32_t q = ROWS == 16   ? (qi % 4) * NI + qi / 4
-                       : ROWS == 32 ? (qi & ~(1u | SB)) | ((qi & 1u) ? SB : 0u) | ((qi & SB) ? 1u : 0u)
-                                    : qi;
-    const bool has_out = qi < QR && q < live;
+    const uint32_t q_any = ROWS == 16   ? (qi % 4) * NI + qi / 4
+                           : ROWS == 32 ? (qi & ~(1u | SB)) | ((qi & 1u) ? SB : 0u) | ((qi & SB) ? 1u : 0u)
+                                        : qi;
+    // (kQ4LinkOut: the threads that would have nothing to do leave the other matmul copies of its words)
+    static_assert(LINK != kQ4LinkOut || (ROWS == 32 && PASSES == 1 && PER_PASS / QR == kQ4LinkCopies), "a thread per word and copy");
+    const uint32_t q = LINK == kQ4LinkOut ? q_any % QR : q_any, copy = LINK == kQ4LinkOut ? q_any / QR : 0u;
+    const bool has_out = (LINK == kQ4LinkOut || qi < QR) && q < live;
     const uint32_t b = req0 + q, col = tile0 * 16 + row;
 
     // ---- main loop
@@ -333,7 +397,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         q4_u32x4 x[XQ];   // PACKED: the quad's activations
     };
     struct BlockX {
-        q4_half8 hi[ZT], lo[ZT];
+        q4_half8 hi[ZT], lo[ZT];   // (PACKED: hi[0] has both)
     };
     // Everything is fetched with buffer loads: a descriptor per stream in scalar registers and 32 bits per lane.  Their
     // descriptors end where the data does; what lies behind (the last blocks of an incomplete quad, the weights
@@ -353,15 +417,20 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     // (request of this lane's row of the A operand; rows without one repeat another's.  Four groups: more than 48 requests,
     // so that the third and the fourth group's are in the second batch tile)
     uint32_t x_lane[ZT];   // (two 16-column steps, hi and lo of each)
+    if constexpr (PACKED) {
+        // up to 8 requests: hi of request r in row (r / NI) * 4 + r % NI and lo NI rows further, so that one product has both
+        const uint32_t m = l16 % 4, xreq = min(l16 / 4 * NI + m % NI, live - 1u);
+        x_lane[0] = (kg / 2 * 4 * WIDTH + kg % 2 * WIDTH + min(m / NI, 1u) * 2 * WIDTH + xreq) * 16;
+    }
 #pragma unroll
-    for (int z = 0; z < ZT; ++z) {
+    for (int z = 0; z < (PACKED ? 0 : ZT); ++z) {
         const uint32_t xreq = min(l16 / 4 * NI + min(l16 % 4, (uint32_t)NI - 1u) + z * 16, live - 1u) + req0 % 32 - z / 2 * 32;
         x_lane[z] = (kg / 2 * 4 * WIDTH + kg % 2 * WIDTH + xreq) * 16;
     }
     const uint32_t s_lane = kg * 128 + (req0 % 32 + l16) * 4;
     auto load_w = [&](uint32_t quad, QuadW& k) __attribute__((always_inline)) {
         constexpr int NT = 2;   // (non-temporal: a weight is read once per launch and need not stay in the L2)
-        if constexpr (BS) {
+        if constexpr (BS && !LINKED) {
 #pragma unroll
             for (int z = 0; z < ZT; ++z)
                 k.sc[z] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s_desc, quad * 512 + s_lane + z * 64, 0, 0));
@@ -371,7 +440,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
             k.q[r] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_desc[r], quad * 1024 + lane * 16, 0, NT));
             k.d[r] = __builtin_bit_cast(q4_u32x2, __builtin_amdgcn_raw_buffer_load_b64(d_desc[r], quad * 128 + l16 * 8, 0, NT));
         }
-        if constexpr (PACKED) {
+        if constexpr (PACKED && !LINKED) {
 #pragma unroll
             for (int i = 0; i < XQ; ++i)
                 k.x[i] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_desc[0], quad * (XQ * 1024) + i * 1024 + lane * 16, 0, 0));
@@ -387,10 +456,59 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         }
         asm volatile("" ::: "memory");
     };
+    // The other matmul's words of a quad (LINKED), into the places of LDS that loaded ones would go to.  A word of
+    // every block first: few loads while there is nothing to be had.
+    [[maybe_unused]] uint32_t link_tag = 0, link_spins = 0;
+    [[maybe_unused]] const uint64_t* const link_words =
+        LINKED ? link.words + block_x % kQ4LinkCopies * q4_link_words(nblocks * 32, batch) : nullptr;
+    [[maybe_unused]] auto link_wait = [&](auto get) __attribute__((always_inline)) {
+        while (!__all(get())) {
+            if (++link_spins >= link.tags.spin_limit) {
+                if (lane == 0) report_fault(link.tags.fault);
+                break;
+            }
+        }
+    };
+    [[maybe_unused]] auto receive = [&](uint32_t quad) __attribute__((always_inline)) {
+        const bool has_cols = quad * 128 + lane * 2 < nblocks * 32, has_scale = l16 < live && quad * 4 + kg < nblocks;
+        const uint64_t* const words = link_words + (size_t)quad * q4_link_quad(batch);
+        const uint64_t none = (uint64_t)link_tag << 32;
+        uint64_t sc = none;
+        link_wait([&]() __attribute__((always_inline)) {
+            if (has_scale) sc = ld_tagged(words + kg * batch + l16);
+            return (uint32_t)(sc >> 32) == link_tag;
+        });
+        scales[wave][0][lane] = __uint_as_float((uint32_t)sc);
+        uint32_t* const to = reinterpret_cast<uint32_t*>(packed[wave]);
+        const uint32_t piece = lane / 8 * 4 * WIDTH + lane / 4 % 2 * WIDTH;   // (columns 2 * lane and the next one: k step lane / 8)
+        const uint64_t* const frag = words + 8 * batch + lane * 2;
+        uint64_t wd[4][2];
+#pragma unroll
+        for (uint32_t n = 0; n < 4; ++n) wd[n][0] = wd[n][1] = none;
+        link_wait([&]() __attribute__((always_inline)) {
+            bool ok = true;
+#pragma unroll
+            for (uint32_t n = 0; n < 4; ++n)
+                if (n < live && has_cols) {
+                    wd[n][0] = ld_tagged(frag + n * 128);
+                    wd[n][1] = ld_tagged(frag + n * 128 + 1);
+                }
+#pragma unroll
+            for (uint32_t n = 0; n < 4; ++n) ok = ok && (uint32_t)(wd[n][0] >> 32) == link_tag && (uint32_t)(wd[n][1] >> 32) == link_tag;
+            return ok;
+        });
+#pragma unroll
+        for (uint32_t n = 0; n < 4; ++n) {
+            if (n >= live) break;
+            const uint32_t w0 = (uint32_t)wd[n][0], w1 = (uint32_t)wd[n][1];
+            to[(piece + n) * 4 + lane % 4] = (w0 & 0xFFFFu) | w1 << 16;
+            to[(piece + 2 * WIDTH + n) * 4 + lane % 4] = w0 >> 16 | (w1 & 0xFFFF0000u);
+        }
+        asm volatile("" ::: "memory");
+    };
     auto read_x = [&](int j, BlockX& k) __attribute__((always_inline)) {
         const uint32_t piece = j * 8 * WIDTH + x_lane[0] / 16;
         k.hi[0] = __builtin_bit_cast(q4_half8, packed[wave][piece]);
-        k.lo[0] = __builtin_bit_cast(q4_half8, packed[wave][piece + 2 * WIDTH]);
         asm volatile("" ::: "memory");
     };
     const uint32_t ones = q4_ones();
@@ -398,7 +516,8 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) zero[i] = 0.f;
     float acc[RT][ZT][NI] = {};
-    auto multiply = [&](const QuadW& w, int j, const BlockX& x) __attribute__((always_inline)) {
+    // (wk_of: weights that have been unpacked already)
+    auto multiply = [&](const QuadW& w, int j, const BlockX& x, auto wk_of) __attribute__((always_inline)) {
         // (the scales of this lane's requests in block j, see `turn`)
         [[maybe_unused]] float sc[ZT][NI];
         if constexpr (BS) {
@@ -411,13 +530,14 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         for (int r = 0; r < RT; ++r) {
             const q4_half2 dd = __builtin_bit_cast(q4_half2, (uint32_t)w.d[r][j / 2]);
             const float d = (float)dd[j % 2];
-            const q4_half8 wk = q4_unpack(w.q[r][j], ones);
+            const q4_half8 wk = wk_of(r);
 #pragma unroll
             for (int z = 0; z < ZT; ++z) {
                 q4_float4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.hi[z], wk, zero, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.lo[z], wk, s, 0, 0, 0);
+                if constexpr (!PACKED) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.lo[z], wk, s, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < NI; ++i) acc[r][z][i] = fmaf(BS ? d * sc[z][i] : d, s[i], acc[r][z][i]);
+                for (int i = 0; i < NI; ++i)
+                    acc[r][z][i] = fmaf(BS ? d * sc[z][i] : d, PACKED ? s[i] + s[(i + NI) % 4] : s[i], acc[r][z][i]);
                 // (here, and not further down, where the compiler would move it: a quad's products do not fit
                 // the 128 registers a wave has)
 #pragma unroll
@@ -472,12 +592,16 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         for (int j = 0; j < 4; ++j) {
             if constexpr (PACKED)
                 if (j + XD - 1 < 4) read_x(j + XD - 1, x[(j + XD - 1) % XD]);
-            multiply(w, j, x[j % XD]);
+            multiply(w, j, x[j % XD], [&](int r) __attribute__((always_inline)) { return q4_unpack(w.q[r][j], ones); });
             if (j + XD < 4) load_x(quad * 4 + j + XD, x[j % XD]);
             else if constexpr (decltype(more)::value) load_x((quad + WAVES) * 4 + j + XD - 4, x[j % XD]);
         }
     };
-    if (first < end) {
+    QuadW link_w[LINKED ? QUADS : 1];
+    if constexpr (LINKED) {
+#pragma unroll
+        for (int n = 0; n < QUADS; ++n) load_w(first + n * WAVES, link_w[n]);
+    } else if (first < end) {
         load_w(first, w);
 #pragma unroll
         for (int i = 0; i < XD; ++i) load_x(first * 4 + i, x[i]);
@@ -493,7 +617,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         const bool has = has_out && q + p * PER_PASS < live;
         if constexpr (FORM == kQ4Rope) {
             rope_pre[p] = {1.0f, 0.0f, 0ull};
-            if (has) rope_pre[p] = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, kQ4LeadBytes + kQ4RopeOffset), bp, col);
+            if (has) rope_pre[p] = q4_rope_prefetch(a.rope, rope_page_rows(a.rope, rope_args_offset), bp, col);
         }
         if constexpr (FORM == kQ4Add)
             if (has) resid_pre[p] = a.add_resid[(size_t)bp * a.rows + col];
@@ -509,30 +633,35 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     [[maybe_unused]] float ssq_part[RMS_N][SSQ_NL] = {}, rms_h[RMS_N] = {}, rms_gamma[RMS_N];
     const uint32_t rms_el = row_group * (1024 * ZT) + threadIdx.x;
     if constexpr (BS) {
-        if (ssq_in) {
+        if (LINKED || ssq_in) {
 #pragma unroll
             for (int n = 0; n < RMS_N; ++n) {
                 const uint32_t sq = wave + n * WAVES, el = rms_el + n * WAVES * 64;
 #pragma unroll
                 for (int j = 0; j < SSQ_NL; ++j) {
                     const uint32_t tl = lane + j * 64;
-                    if (sq < live && tl < a.ssq_tiles) ssq_part[n][j] = ssq_in[(size_t)(req0 + sq) * a.ssq_tiles + tl];
+                    if (!LINKED && sq < live && tl < a.ssq_tiles) ssq_part[n][j] = ssq_in[(size_t)(req0 + sq) * a.ssq_tiles + tl];
                 }
                 rms_gamma[n] = 1.0f;
                 if (el < live * a.rms_len) {
                     const uint32_t rc = el % a.rms_len;
-                    rms_h[n] = a.rms_src[(size_t)req0 * a.rms_len + el];
+                    if constexpr (!LINKED) rms_h[n] = a.rms_src[(size_t)req0 * a.rms_len + el];
                     if (rc < a.rms_n_gamma) rms_gamma[n] = a.rms_gamma[rc];
                 }
             }
         }
     }
     uint32_t tag_add = 0;   // (K slices of a captured pass)
-    if (a.slices > 1 && a.tags.tag_dev) tag_add = *a.tags.tag_dev;
+    if constexpr (LINK == kQ4LinkNone) {
+        if (a.slices > 1 && a.tags.tag_dev) tag_add = *a.tags.tag_dev;
+    } else {
+        if (link.tags.tag_dev) tag_add = *link.tags.tag_dev;   // (of the same pass: a.tags has none or the same)
+        link_tag = launch_tag(link.tags.tag, tag_add);
+    }
     asm volatile("" ::: "memory");
 
-    if constexpr (BS) {
-        if (ssq_in) {
+    auto finish_rms = [&]() __attribute__((always_inline)) {
+        if (LINKED || ssq_in) {
 #pragma unroll
             for (int m = 0; m < RMS_N; ++m) {
                 float part = q4_half_wave_sum(ssq_part[m][0] + ssq_part[m][1]);
@@ -542,8 +671,43 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
                 if (lane == 0 && sq < live) rms_scale[sq] = 1.0f / sqrtf(part / (float)a.rms_len + a.rms_eps);
             }
         }
-    }
-    if (first < end) {
+    };
+    [[maybe_unused]] uint64_t ssq_word[SSQ_NL];
+    [[maybe_unused]] auto get_ssq = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < SSQ_NL; ++j) {
+            const uint32_t tl = lane + j * 64;
+            ssq_word[j] = (uint64_t)link_tag << 32;
+            if (tl < nblocks) ssq_word[j] = ld_tagged(link_words + (size_t)(tl / 4) * q4_link_quad(batch) + (4 + tl % 4) * batch + wave);
+        }
+    };
+    if constexpr (BS && !LINKED) finish_rms();
+    if constexpr (LINKED) {
+        static_assert(TWO_LEVELS && RT * QUADS <= 4, "a wave's weights unpacked: at most 64 registers");
+        q4_half8 wk[QUADS][RT][4];
+#pragma unroll
+        for (int n = 0; n < QUADS; ++n)
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    wk[n][r][j] = q4_unpack(link_w[n].q[r][j], ones);
+                    asm volatile("" : "+v"(wk[n][r][j]));   // (now, and not where they are used)
+                }
+#pragma unroll
+        for (int n = 0; n < QUADS; ++n) {
+            const uint32_t quad = first + n * WAVES;
+            if (quad >= end) break;
+            receive(quad);
+            if (n == 0 && wave < live) get_ssq();   // (on their way during the products)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                read_x(j, x[0]);
+                multiply(link_w[n], j, x[0], [&](int r) __attribute__((always_inline)) { return wk[n][r][j]; });
+            }
+            if (n + 1 < QUADS) flush();
+        }
+    } else if (first < end) {
         uint32_t quad = first;
         for (; quad + WAVES < end; quad += WAVES) {
             turn(quad, std::true_type());
@@ -563,6 +727,32 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         turn(quad, std::false_type());
     }
 
+    [[maybe_unused]] uint64_t rms_word = 0;
+    [[maybe_unused]] const uint64_t* rms_at = nullptr;   // this thread's element of the norm, if it has one
+    if constexpr (LINKED) {
+        // the other matmul's sums of squares: wave n adds up request n's
+        static_assert(RMS_N == 1, "one element of the norm per thread");
+        if (wave < live) {
+            if (first >= end) get_ssq();
+            bool again = false;
+            link_wait([&]() __attribute__((always_inline)) {
+                if (again) get_ssq();
+                again = true;
+                bool ok = true;
+#pragma unroll
+                for (int j = 0; j < SSQ_NL; ++j) ok = ok && (uint32_t)(ssq_word[j] >> 32) == link_tag;
+                return ok;
+            });
+#pragma unroll
+            for (int j = 0; j < SSQ_NL; ++j) ssq_part[0][j] = __uint_as_float((uint32_t)ssq_word[j]);
+        }
+        if (rms_el < live * a.rms_len) {
+            rms_at = link_words + q4_link_sum(a.rms_len, batch) + rms_el;
+            rms_word = ld_tagged(rms_at);
+        }
+        finish_rms();
+    }
+
     // ---- the waves' sums meet in LDS.  A lane holds weight row l16 of the tile and, in register i, request
     // kg * NI + i.
     flush();
@@ -570,7 +760,14 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     __syncthreads();
     if constexpr (BS) {
         // the norm's own output: h * factor * gamma, the arithmetic of rms_norm_batched_kernel
-        if (ssq_in) {
+        if constexpr (LINKED) {
+            link_wait([&]() __attribute__((always_inline)) {
+                if (rms_at && (uint32_t)(rms_word >> 32) != link_tag) rms_word = ld_tagged(rms_at);
+                return !rms_at || (uint32_t)(rms_word >> 32) == link_tag;
+            });
+            rms_h[0] = __uint_as_float((uint32_t)rms_word);
+        }
+        if (LINKED || ssq_in) {
 #pragma unroll
             for (int m = 0; m < RMS_N; ++m) {
                 const uint32_t el = rms_el + m * WAVES * 64;
@@ -590,7 +787,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
         for (int step = 1; step < WAVES; step *= 2)
 #pragma unroll
             for (int k = 0; k < WAVES; k += 2 * step) sum[k] += sum[k + step];
-        if constexpr (BS) return ssq_in ? sum[0] * rms_scale[sq] : sum[0];
+        if constexpr (BS) return LINKED || ssq_in ? sum[0] * rms_scale[sq] : sum[0];
         else return sum[0] * inv;
     };
     if constexpr (FORM == kQ4Silu) {
@@ -614,7 +811,7 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     // last of the launch, add them to their own in slice order (tagged_words.h: why the wait ends).
     const uint32_t tag = launch_tag(a.tags.tag, tag_add);
     if (slice + 1 < a.slices) {
-        if (a.tags.test_flags & 1u) return;
+        if ((a.tags.test_flags & 1u) || copy != 0) return;
 #pragma unroll
         for (int p = 0; p < PASSES; ++p) {
             const uint32_t qp = q + p * PER_PASS, bp = b + p * PER_PASS;
@@ -656,6 +853,13 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
             }
             val = others + val;
         }
+        if constexpr (LINK == kQ4LinkOut) {
+            // (what the other matmul waits for first)
+            const float hv = val + resid_pre[p], ssq = q4_half_wave_sum(hv * hv);
+            if (!(link.tags.test_flags & 1u))
+                q4_emit_words(hv * gamma_pre, hv, ssq, bp, col, a.rows, batch, link.words + copy * q4_link_words(a.rows, batch), link_tag);
+            if (copy != 0) return;   // (whole half waves)
+        }
         store_through(&a.out[(size_t)bp * a.rows + col], val);
         if constexpr (FORM == kQ4Rope) q4_rope_epilogue(a.rope, rope_pre[p], bp, col, val);   // (the lanes of a pair share b)
         if constexpr (FORM == kQ4Add) {
@@ -663,12 +867,62 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
             // matmul's fragments
             const float hv = val + resid_pre[p];
             store_through(&a.add_out[(size_t)bp * a.rows + col], hv);
-            if (a.split_frag) {   // (else the add is all)
+            if (LINK == kQ4LinkNone && a.split_frag) {   // (else the add is all)
                 const float ssq = q4_half_wave_sum(hv * hv);
                 if (row % 32 == 0) store_through(&a.ssq_out[(size_t)bp * (a.rows / 32) + col / 32], ssq);
                 q4_emit_block(hv * gamma_pre, bp, col, a.rows, a.split_frag, a.split_blk_scale, WIDTH);
             }
         }
+    }
+}
+
+template <int NI, int RT, int WAVES, bool BS, int FORM, int ZT = 1>
+__global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
+    const uint4* const w_q, const uint2* const w_d, const _Float16* const xfrag, const float* const blk_scale, const float* const ssq_in,
+    const uint32_t nblocks, const uint32_t quads_per_slice, const uint32_t row_groups, const uint32_t batch_z,
+    const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
+    __shared__ Q4Lds<NI, RT, WAVES, BS, ZT> lds;
+    q4_matmul_workgroup<NI, RT, WAVES, BS, FORM, ZT, kQ4LinkNone, 0>(lds, blockIdx.x, blockIdx.y, kQ4LeadBytes + kQ4RopeOffset, w_q, w_d, xfrag,
+                                                                  blk_scale, ssq_in, nblocks, quads_per_slice, row_groups, batch_z, a, Q4Link{});
+}
+
+// Two matmuls of up to 4 requests in one launch: one with the residual add that starts an RMSNorm, and the one that reads
+// the norm.  The first matmul's workgroups come first, in all their K slices; the second one's request their weights, and then wait
+// for the first one's sums as tagged words (tagged_words.h: why the waits end).  That takes a launch's start and end and the second
+// one's way to its first weights off the chain of launches that a step is, and its unpacking, 0.7 us of the vector pipe per four
+// row tiles: while it waits a wave holds its weights as halves in up to 64 registers.
+//
+// Measured: out-projection and gate/up of the 1 B shape at one request 12.0 us in two launches, 8.0 in one, of which, from the
+// start: the first one's weights back 1.5, its sums published 3.5 (vector pipe, 16 waves), seen 4.3, all words in LDS 4.9, products
+// 5.9, waves' sums met 6.3, stored 7.4.  With one copy of the words, a quad's scales in the lines of all the others' they were seen at
+// 5.5.  Steps of 22 layers, us, two launches -> one: 1, 2, 3, 4 requests 683, 696, 702, 705 -> 618, 643, 654, 673; a
+// build for 5 and 8 requests 771, 778 -> 763, 784 (every workgroup fetches 8 bytes per request and column): two launches there.
+template <int FORM>
+struct Q4ChainArgs {
+    Q4Args first;
+    std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> second;
+    Q4Link link;
+};
+static_assert(sizeof(Q4Args) % alignof(Q4RopeArgs) == 0, "where q4_chain_kernel finds the second one's rope in its arguments");
+template <int RT, int QUADS, int FORM>
+__global__ __launch_bounds__(1024, 4) void q4_chain_kernel(
+    const uint4* const w_q, const uint2* const w_d, const _Float16* const xfrag, const float* const blk_scale, const float* const ssq_in,
+    const uint32_t nblocks, const uint32_t quads_per_slice, const uint32_t row_groups, const uint32_t batch_blocks, const Q4ChainArgs<FORM> c) {
+    __shared__ union {
+        Q4Lds<1, 2, 16, true, 1> first;
+        Q4Lds<1, RT, 16, true, 1> second;
+    } lds;
+    const uint32_t batch_z = (batch_blocks & 0xFFFFu) | 1u << 16, blocks = batch_blocks >> 16;   // (of the first matmul)
+    if (blockIdx.x < blocks) {
+        const uint32_t per_slice = (row_groups + 7) / 8 * 8;
+        uint32_t slice = 0, x = blockIdx.x;
+        for (; x >= per_slice; x -= per_slice) ++slice;
+        q4_matmul_workgroup<1, 2, 16, true, kQ4Add, 1, kQ4LinkOut, 0>(lds.first, x, slice, 0, w_q, w_d, xfrag, blk_scale, ssq_in, nblocks,
+                                                                    quads_per_slice, row_groups, batch_z, c.first, c.link);
+    } else {
+        q4_matmul_workgroup<1, RT, 16, true, FORM, 1, kQ4LinkIn, QUADS>(
+            lds.second, blockIdx.x - blocks, 0, kQ4LeadBytes + (uint32_t)sizeof(Q4Args) + kQ4RopeOffset, c.second.q, c.second.d,
+            nullptr, nullptr, nullptr, c.second.nblocks, c.second.quads_per_slice, c.second.row_groups, batch_z, c.second, c.link);
     }
 }
 

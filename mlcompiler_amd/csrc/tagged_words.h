@@ -2,7 +2,8 @@
 // atomics at device scope: the store is written through to memory, the load bypasses the per-XCD L2 caches).  The tag is
 // the launch's, never seen in the buffer before, so every word says by itself whether it has been written in this
 // launch: no order among the stores, no acknowledgement, no arrival counter, nothing to clear until the tags start over
-// (renew_tags).  A word gets from one workgroup to another in 0.5 us, on the same XCD or not.
+// (renew_tags).  A word gets from one workgroup to another in 0.5 us, on the same XCD or not; in 2 us
+// where thousands of waves poll words of the same few lines.
 //
 // Why every wait ends.  Each XCD starts its workgroups of a launch in the launch's order, but the XCDs run ahead of each
 // other, and who shares words with whom need not be on one XCD nor running at the same time.
@@ -11,6 +12,8 @@
 //   * Partials of the decode attention: a workgroup waits for workgroups with lower numbers only, after it has published
 //     its own part.  Take the lowest number that has not published: whatever has started before it on its XCD waits for
 //     lower numbers at most, which all have, and ends.
+//   * Two matmuls in one launch: the second one's workgroups, the last of the launch, wait for the first one's, which wait for
+//     each other's slices at most.  None of the second's has started on an XCD where one of the first's has yet to start.
 // That holds for one such launch at a time (scratch_follow orders them across streams), beside launches that end by
 // themselves.  The waits are bounded all the same: a pass then fails instead of hanging.
 #pragma once
