@@ -25,7 +25,7 @@
 // banks).  One tile ahead of its use every thread reads back the 16 bytes of V its own
 // load delivered and writes them transposed into one of two V^T buffers, so the only
 // wait is on the thread's own oldest loads and there is one barrier per tile.
-// (GQA ratios up to 4 run the second kernel of this file, 64 chunk rows per wave; see there.)
+// (GQA ratios up to 4, and 8 over more than a few key tiles, run the second kernel of this file, 64 chunk rows per wave; see there.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillArgs 
     *reinterpret_cast<float4*>(orow + block * 8 + lane / 32 * 4) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
 }
 
-// ---- the same computation with 64 chunk rows per wave (GQA ratios 1, 2 and 4).  One workgroup
+// ---- the same computation with 64 chunk rows per wave (GQA ratios 1, 2 and 4; 8 as two workgroups of 4 heads).  One workgroup
 // = 4 waves = the G query heads of one KV head x 4/G blocks of 64 consecutive chunk rows (the
 // same 256 (row, head) pairs per K/V tile as above), one wave per SIMD with the whole register
 // file to itself.  Every A operand read from LDS (a K row block, a V^T row block) feeds two
@@ -536,10 +536,11 @@ __device__ __forceinline__ void pf_tie(uint32_t& x, float& y) { asm volatile("" 
 __device__ __forceinline__ void pf_tie(float& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void pf_tie(pf_float16& x) { asm volatile("" : "+v"(x)); }
 
-template <int D, int G, int NST>
+// SUB: workgroups that share a KV head, with G of its query heads each.
+template <int D, int G, int NST, int SUB>
 __global__ __launch_bounds__(256) void paged_prefill_mfma64_kernel(const PrefillArgs a) {
     static_assert(D == 64 || D == 128, "head_dim 64 or 128");
-    static_assert(G == 1 || G == 2 || G == 4, "waves cover whole GQA groups");
+    static_assert(G == 1 || G == 2 || G == 4, "waves cover whole GQA groups, or whole parts of them");
     static_assert(NST >= 4 && NST <= 8 && NST % 2 == 0, "4, 6 or 8 stages");
     constexpr int WAVES = 4;
     constexpr int NT = 64 * WAVES;
@@ -578,11 +579,11 @@ __global__ __launch_bounds__(256) void paged_prefill_mfma64_kernel(const Prefill
     uint32_t wg = blockIdx.x;
     if (gridDim.x % 8u == 0) wg = (wg % 8u) * (gridDim.x / 8u) + wg / 8u;
     const uint32_t rbk = wg % a.row_blocks;
-    const uint32_t kvh = (wg / a.row_blocks) % a.kv_heads;
-    const uint32_t req = wg / (a.row_blocks * a.kv_heads);
+    const uint32_t part = (wg / a.row_blocks) % (a.kv_heads * SUB), kvh = part / SUB;
+    const uint32_t req = wg / (a.row_blocks * a.kv_heads * SUB);
     constexpr uint32_t ROWS_WG = kPfRows * HALVES * RB;
     const uint32_t row0_wg = rbk * ROWS_WG;
-    const uint32_t head = kvh * G + (wave % G);
+    const uint32_t head = part * G + (wave % G);
     const uint32_t row0 = row0_wg + (wave / G) * (kPfRows * HALVES);  // first chunk row of this wave
 
     const uint32_t* tables = pf_tables(a);
@@ -1003,6 +1004,14 @@ __global__ __launch_bounds__(256) void paged_prefill_mfma64_kernel(const Prefill
     }
 }
 
+// GQA ratio 8: 64 rows of four heads per workgroup where there are enough key tiles, else 32 rows of all eight.  Both have 256
+// (row, head) pairs; the kernel with 64 rows reads an operand from LDS for two products, and takes longer until its first tile and in
+// the last row block, half of which a chunk may not fill.  (Whole calls, us, 32 -> 64 rows, by tiles of the longest
+// row block.  head_dim 64: 2 tiles 20.3 -> 21.3, 4 23.3 -> 23.9, 8 25.9 -> 26.2, 34.1 -> 32.8 and 24.5 -> 24.5, 9 30.8 -> 31.5, 10 34.0 -> 31.5
+// and 41.9 -> 41.4, 12 37.5 -> 34.1, 25 47.1 -> 40.4, 128 124 -> 110.  128: 4 28.6 -> 30.1, 8 48.5 -> 51.4 and 30.3 -> 30.6, 10 60.8 -> 63.2,
+// 12 50.8 -> 51.7 and 52.5 -> 51.8, 16 62.5 -> 60.7 and 40.2 -> 38.5, 25 58.1 -> 53.8, 128 162 -> 146.)
+inline bool prefill_rows64_ratio8(size_t head_dim, size_t max_tiles) { return max_tiles >= (head_dim == 64 ? 10u : 16u); }
+
 inline bool prefill_shape_supported(size_t head_dim, size_t page_size, size_t num_heads,
                                     size_t kv_heads) {
     const size_t g = kv_heads ? num_heads / kv_heads : 0;
@@ -1012,19 +1021,18 @@ inline bool prefill_shape_supported(size_t head_dim, size_t page_size, size_t nu
 
 template <int D, int G>
 inline void launch_prefill_dg(PrefillArgs a, int stages, bool rows64, uint32_t splits, hipStream_t stream) {
-    if constexpr (G <= 4) {
-        if (rows64 && splits == 1) {
-            const uint32_t rows_per_wg = kPfRows * 2 * (4 / G);
-            a.row_blocks = (a.chunk + rows_per_wg - 1) / rows_per_wg;
-            const dim3 grid(a.row_blocks * a.kv_heads * a.batch), block(256);
-            switch (stages) {
-                case 2:
-                case 4: hipLaunchKernelGGL((paged_prefill_mfma64_kernel<D, G, 4>), grid, block, 0, stream, a); break;
-                case 8: hipLaunchKernelGGL((paged_prefill_mfma64_kernel<D, G, 8>), grid, block, 0, stream, a); break;
-                default: hipLaunchKernelGGL((paged_prefill_mfma64_kernel<D, G, 6>), grid, block, 0, stream, a); break;
-            }
-            return;
+    if (rows64 && splits == 1) {
+        constexpr int PER = G < 4 ? G : 4, SUB = G / PER;
+        const uint32_t rows_per_wg = kPfRows * 2 * (4 / PER);
+        a.row_blocks = (a.chunk + rows_per_wg - 1) / rows_per_wg;
+        const dim3 grid(a.row_blocks * a.kv_heads * SUB * a.batch), block(256);
+        switch (stages) {
+            case 2:
+            case 4: hipLaunchKernelGGL((paged_prefill_mfma64_kernel<D, PER, 4, SUB>), grid, block, 0, stream, a); break;
+            case 8: hipLaunchKernelGGL((paged_prefill_mfma64_kernel<D, PER, 8, SUB>), grid, block, 0, stream, a); break;
+            default: hipLaunchKernelGGL((paged_prefill_mfma64_kernel<D, PER, 6, SUB>), grid, block, 0, stream, a); break;
         }
+        return;
     }
     const uint32_t rows_per_wg = kPfRows * (kPfWaves / G);
     a.row_blocks = (a.chunk + rows_per_wg - 1) / rows_per_wg;
@@ -1079,7 +1087,7 @@ inline uint32_t prefill_splits(size_t wgs, size_t head_dim, size_t max_tiles, si
 }
 
 // stages: LDS pipeline depth (2, 4, 6 or 8; anything else selects 6).  rows64: 64 chunk rows per
-// wave (GQA ratios up to 4), else 32.  splits: parts into which every workgroup's keys are cut (more than
+// wave, else 32.  splits: parts into which every workgroup's keys are cut (more than
 // one: 32 rows per wave, partial sums in a.part_o / part_ml, prefill_splits() says how many).
 inline void launch_prefill(const PrefillArgs& a, size_t head_dim, int stages, bool rows64, uint32_t splits, hipStream_t stream) {
     if (head_dim == 64) launch_prefill_d<64>(a, stages, rows64, splits, stream);
