@@ -119,6 +119,9 @@ def build_all(verbose: bool = False) -> None:
             obj = os.path.join(obj_dir, f"decode_d{d}_h{h}.o")
             jobs.append(([cc, *HIPCC_FLAGS, f"-DMLC_D={d}", f"-DMLC_HPW={h}", "-c",
                           os.path.join(CSRC, "paged_decode_inst.hip"), "-o", obj], obj))
+    for d in (64, 128):
+        obj = os.path.join(obj_dir, f"prefill_d{d}.o")
+        jobs.append(([cc, *HIPCC_FLAGS, f"-DMLC_D={d}", "-c", os.path.join(CSRC, "paged_prefill_inst.hip"), "-o", obj], obj))
     tok_obj = os.path.join(obj_dir, "matmul_tokens.o")
     jobs.append(([cc, *HIPCC_FLAGS, "-c", os.path.join(CSRC, "matmul_tokens_inst.hip"), "-o", tok_obj], tok_obj))
     for ni in (1, 2, 4):

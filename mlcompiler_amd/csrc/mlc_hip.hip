@@ -25,7 +25,7 @@
 #include "paged_decode_generic.h"
 #include "paged_decode_kernels.h"
 #include "paged_decode_stream.h"
-#include "paged_prefill_kernels.h"
+#include "paged_prefill_args.h"
 #include "paged_rope_kernels.h"
 #include "walker_kernels.h"
 #include "q4_matmul_kernels.h"
