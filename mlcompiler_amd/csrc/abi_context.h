@@ -569,7 +569,7 @@ bool q4_wide(size_t rows) { return rows > 8192; }
 int q4_tiles(Q4Form form, size_t rows, size_t batch, size_t ksplit) {
     const size_t wgs = rows / 16 * ((batch + 15) / 16) * ksplit, n_cu = (size_t)g.n_cu;
     if (form == kQ4Silu) return 4;
-    const int least = form == kQ4Add ? 2 : 1, most = form != kQ4Plain && batch <= 8 ? 2 : 4;
+    const int least = form == kQ4Add ? 2 : 1, most = form != kQ4Plain && form != kQ4Rows && batch <= 8 ? 2 : 4;
     return std::min(most, std::max(least, wgs > 2 * n_cu ? 4 : wgs > n_cu ? 2 : 1));
 }
 

@@ -30,6 +30,30 @@ Q4Slices q4_slices(size_t rows, size_t cols, size_t batch) {
     return {(quads + per_slice - 1) / per_slice, per_slice};
 }
 
+// A matmul that is a call of its own takes its rows of floats as they are and splits them itself, every workgroup all of them: that
+// takes the launch in front away, 2 us and, for long rows, its time.  (The split is of every block by itself, as the fused
+// launches have it.)  Up to four requests that pays everywhere, up to eight where a workgroup has one row tile, or two and K is long:
+// a build for four tiles spills.  Whole calls, us, split in front -> now, and with 5 and 8 tokens in brackets where the split stays in front:
+//   rows x columns | 1           | 4           | 5             | 8
+//   2560 x 2048    | 17.4 / 14.9 | 17.4 / 15.4 | 17.6 / 15.8   | 18.0 / 16.6
+//   11264 x 2048   | 19.2 / 16.9 | 19.3 / 17.6 | (19.9 / 22.0) | (20.0 / 22.6)
+//   2048 x 5632    | 18.7 / 16.0 | 18.7 / 16.8 | 19.2 / 17.6   | 19.3 / 18.2
+//   6144 x 4096    | 20.0 / 17.8 | 20.0 / 18.9 | (20.9 / 20.2) | (20.8 / 21.7)
+//   4096 x 4096    | 18.7 / 16.1 | 18.7 / 16.8 | 19.0 / 17.4   | 19.3 / 18.3
+//   28672 x 4096   | 30.2 / 27.8 | 30.4 / 29.9 | (32.0 / 44.7) | (32.1 / 48.5)
+//   4096 x 14336   | 32.7 / 22.3 | 32.1 / 23.3 | 33.9 / 26.0   | 33.7 / 27.7
+bool q4_splits_rows(size_t rows, size_t cols, size_t batch) {
+    const int tiles = batch <= 8 ? q4_tiles(kQ4Rows, rows, batch, q4_slices(rows, cols, batch).n) : 4;
+    return batch <= 4 || (batch <= 8 && (tiles == 1 || (tiles == 2 && cols > 4096)));
+}
+
+// The split of a batch's rows into fragments: 1024 threads per row from 4096 columns on, where 256 keep no row in registers.
+void launch_q4_split(const float* x, _Float16* frag, float* inv_scale, size_t batch, size_t cols) {
+    const unsigned threads = cols > 4096 ? 1024 : 256;
+    hipLaunchKernelGGL(threads == 1024 ? q4_split_activations_kernel<1024> : q4_split_activations_kernel<256>, dim3((unsigned)batch), dim3(threads),
+                       0, g.stream, x, frag, inv_scale, (uint32_t)batch, (uint32_t)cols);
+}
+
 // Copies weights to the device in the order of the library's stream (a plain hipMemcpy may return before the data is
 // there, and the library's stream does not wait for it), and waits.
 bool upload_weights(void* dst, const void* host, size_t bytes) {
@@ -166,6 +190,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
 
     // MFMA path, one pass over at most 64 requests at a time.
     const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
+    const bool rows_in = sync && g.opt_q4_int_operand && !feeds && !block_scales && aligned16(in) && q4_splits_rows(rows, cols, batch);
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;
@@ -222,9 +247,8 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             g.rows.p.inv_scale = inv;
             g.rows.grid_rows = bn;
             if (!settle()) return 0;
-        } else {
-            hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bn), dim3(256), 0, g.stream, xin, frag,
-                               inv, (uint32_t)bn, (uint32_t)cols);
+        } else if (!rows_in) {
+            launch_q4_split(xin, frag, inv, bn, cols);
         }
         // The slices' sums meet in the launch; a matmul that has no tag or no memory for that takes all of K.  (Everything
         // held back has been launched: buffers that it reads may be replaced now.)
@@ -245,6 +269,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         a.xfrag = frag;
         a.blk_scale = blk_scale;
         a.inv_scale = inv;
+        a.xrows = xin;
         a.out = slices ? slices : o;
         a.slices = (uint32_t)ksplit;
         a.meet = words;
@@ -271,7 +296,7 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             const auto kernel = zt == 2 ? q4_pairs_kernel<4, 2, 8> : rt == 4 ? q4_pairs_kernel<4, 1, 16> : q4_pairs_kernel<1, 1, 16>;
             hipLaunchKernelGGL(kernel, dim3((unsigned)(rows / 16 / rt), (unsigned)(z / zt), (unsigned)ksplit), dim3(zt == 2 ? 512 : 1024), 0,
                                g.stream, a);
-        } else if (!launch_q4(kQ4Plain, block_scales, ra)) {
+        } else if (!launch_q4(rows_in ? kQ4Rows : kQ4Plain, block_scales || rows_in, ra)) {
             return 0;
         }
         if (slices) {
@@ -413,8 +438,7 @@ int mlc_hip_matmul_q6_k_batched(const char* weight_name, const void* weights, si
             g.rows.grid_rows = bn;
             if (!settle()) return 0;
         } else {
-            hipLaunchKernelGGL(q4_split_activations_kernel, dim3((unsigned)bn), dim3(256), 0, g.stream, xin, frag,
-                               inv, (uint32_t)bn, (uint32_t)cols);
+            launch_q4_split(xin, frag, inv, bn, cols);
         }
         Q6KArgs a;
         a.qa = static_cast<const uint2*>(w->qa);

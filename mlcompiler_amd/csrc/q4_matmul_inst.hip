@@ -22,6 +22,18 @@ bool MLC_CAT(launch_q4_matmul_, MLC_Q4_NI)(int form, int rt, int waves, int zt, 
     MLC_Q4(kQ4Rope, 1, 16, a) MLC_Q4(kQ4Rope, 2, 16, a)
     MLC_Q4(kQ4Add, 2, 16, plain)
 #if MLC_Q4_NI < 4
+#define MLC_Q4R(RT, WAVES)                                                                                                     \
+    if (form == kQ4Rows && rt == RT && waves == WAVES && zt == 1) {                                                            \
+        hipLaunchKernelGGL((q4_matmul_kernel<MLC_Q4_NI, RT, WAVES, true, kQ4Rows>), grid, dim3(WAVES * 64), 0, stream, a.q, a.d, \
+                           reinterpret_cast<const _Float16*>(a.xrows), nullptr, nullptr, a.nblocks, a.quads_per_slice, a.row_groups, \
+                           a.batch | a.z_groups << 16, plain);                                                                 \
+        return true;                                                                                                           \
+    }
+    MLC_Q4R(1, 16) MLC_Q4R(2, 16)
+#if MLC_Q4_NI == 1
+    MLC_Q4R(4, 16) MLC_Q4R(4, 8)
+#endif
+#undef MLC_Q4R
     MLC_Q4(kQ4Rope, 2, 8, a)
     MLC_Q4(kQ4Add, 2, 8, plain)
 #else

@@ -37,31 +37,33 @@ __global__ __launch_bounds__(256) void q4_0_matmul_generic_kernel(
 
 // ---- activations -> operand fragments (fragments.h).  One workgroup per request row:
 // s = 2^(14 - exponent(max|x|)).  Rows past `batch` of the last tile are not written here, and nobody reads them.
-__global__ __launch_bounds__(256) void q4_split_activations_kernel(
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void q4_split_activations_kernel(
     const float* __restrict__ x, _Float16* __restrict__ frag, float* __restrict__ inv_scale,
     uint32_t batch, uint32_t cols) {
-    __shared__ float red[4];
-    constexpr int MAXV = 4;  // register-resident groups of 8 columns per thread: cols <= 8192
+    constexpr int WAVES = THREADS / 64;
+    __shared__ float red[WAVES];
+    constexpr int MAXV = 2;  // groups of 8 columns that a thread keeps in registers: cols <= 4096 / 16384
     const uint32_t n = blockIdx.x;
     const uint32_t width = frag_width(batch);
     const uint32_t groups = cols / 8;
     const bool live = n < batch;
     const float4* xr = reinterpret_cast<const float4*>(x + (size_t)(live ? n : 0) * cols);
-    const bool in_regs = groups <= 256 * MAXV;
+    const bool in_regs = groups <= THREADS * MAXV;
     float4 v[MAXV][2];
     float amax = 0.f;
     if (live) {
         if (in_regs) {
 #pragma unroll
             for (int j = 0; j < MAXV; ++j) {
-                const uint32_t k8 = j * 256 + threadIdx.x;
+                const uint32_t k8 = j * THREADS + threadIdx.x;
                 v[j][0] = v[j][1] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (k8 < groups) { v[j][0] = xr[k8 * 2]; v[j][1] = xr[k8 * 2 + 1]; }
                 amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[j][0].x), fabsf(v[j][0].y)), fmaxf(fabsf(v[j][0].z), fabsf(v[j][0].w))));
                 amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[j][1].x), fabsf(v[j][1].y)), fmaxf(fabsf(v[j][1].z), fabsf(v[j][1].w))));
             }
         } else {
-            for (uint32_t k4 = threadIdx.x; k4 < cols / 4; k4 += 256) {
+            for (uint32_t k4 = threadIdx.x; k4 < cols / 4; k4 += THREADS) {
                 const float4 t = xr[k4];
                 amax = fmaxf(amax, fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w))));
             }
@@ -71,7 +73,9 @@ __global__ __launch_bounds__(256) void q4_split_activations_kernel(
     for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
     if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = amax;
     __syncthreads();
-    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    amax = red[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) amax = fmaxf(amax, red[w]);
     int e = 0;
     if (amax > 0.f && amax < INFINITY) (void)frexpf(amax, &e);  // amax = m * 2^e, m in [0.5, 1)
     int se = 14 - e;
@@ -94,11 +98,11 @@ __global__ __launch_bounds__(256) void q4_split_activations_kernel(
     if (in_regs) {
 #pragma unroll
         for (int j = 0; j < MAXV; ++j) {
-            const uint32_t k8 = j * 256 + threadIdx.x;
+            const uint32_t k8 = j * THREADS + threadIdx.x;
             if (k8 < groups) emit(k8, v[j][0], v[j][1]);
         }
     } else {
-        for (uint32_t k8 = threadIdx.x; k8 < groups; k8 += 256) {
+        for (uint32_t k8 = threadIdx.x; k8 < groups; k8 += THREADS) {
             const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
             emit(k8, live ? xr[k8 * 2] : z, live ? xr[k8 * 2 + 1] : z);
         }

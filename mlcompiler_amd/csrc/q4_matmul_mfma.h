@@ -52,6 +52,7 @@ struct Q4Args {
     const uint2* d;
     const _Float16* xfrag;      // split activations (fragments.h)
     const float* inv_scale;     // [batch]
+    const float* xrows;         // kQ4Rows: [batch][nblocks * 32], in place of the fragments
     float* out;                 // [batch][rows]; q4_pairs_kernel with K slices: the slice buffer [slices][batch][rows]
     uint32_t batch, rows, nblocks, nquads, quads_per_slice, slices;
     // slices > 1: where the workgroups of all slices but the last leave their sums for those of the last
@@ -275,7 +276,8 @@ __device__ __forceinline__ float q4_silu_times(float g, float u) {  // walker_ke
 }
 
 // What the epilogue of q4_matmul_kernel does besides storing the result.
-enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3 };
+// kQ4Rows: nothing; its activations come as rows of floats (xrows), which it splits itself.
+enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3, kQ4Rows = 4 };
 
 // One workgroup of 16 (or 8) waves: RT tiles of 16 weight rows x up to 16 requests x one K slice.  The slice's
 // quads of blocks are dealt out to the waves; a wave streams its quads' nibbles and scales (one quad ahead) and
@@ -343,6 +345,8 @@ __device__ __forceinline__ void q4_matmul_workgroup(
     constexpr bool LINKED = LINK == kQ4LinkIn;
     static_assert(LINK == kQ4LinkNone || (NI == 1 && WAVES == 16 && BS && ZT == 1), "two matmuls in a launch: up to 4 requests");
     static_assert(LINK != kQ4LinkOut || FORM == kQ4Add, "the first of two: with the residual add");
+    constexpr bool ROWS_IN = FORM == kQ4Rows;
+    static_assert(!ROWS_IN || (NI < 4 && BS), "rows of floats: up to 8 requests, split by block");
     static_assert(FORM != kQ4Silu || RT == 4, "SiLU epilogue: 32 rows of gate and 32 of up");
     static_assert(FORM != kQ4Add || RT % 2 == 0, "residual add: whole blocks of the next matmul's K");
     // Up to 8 requests: a quad's activations come 1 KB per load, without the places of requests that do not
@@ -412,7 +416,8 @@ __device__ __forceinline__ void q4_matmul_workgroup(
     }
     __amdgpu_buffer_rsrc_t x_desc[X_TILES];
 #pragma unroll
-    for (int t = 0; t < X_TILES; ++t) x_desc[t] = q4_buffer(xfrag + (size_t)(req0 / 32 + t) * nblocks * 2048, nblocks * WIDTH * 128);
+    for (int t = 0; t < X_TILES; ++t)
+        x_desc[t] = ROWS_IN ? q4_buffer(xfrag, batch * nblocks * 128) : q4_buffer(xfrag + (size_t)(req0 / 32 + t) * nblocks * 2048, nblocks * WIDTH * 128);
     const __amdgpu_buffer_rsrc_t s_desc = q4_buffer(BS ? blk_scale + (size_t)(req0 / 32) * nblocks * 32 : nullptr, nblocks * 128);
     // (request of this lane's row of the A operand; rows without one repeat another's.  Four groups: more than 48 requests,
     // so that the third and the fourth group's are in the second batch tile)
@@ -430,7 +435,7 @@ __device__ __forceinline__ void q4_matmul_workgroup(
     const uint32_t s_lane = kg * 128 + (req0 % 32 + l16) * 4;
     auto load_w = [&](uint32_t quad, QuadW& k) __attribute__((always_inline)) {
         constexpr int NT = 2;   // (non-temporal: a weight is read once per launch and need not stay in the L2)
-        if constexpr (BS && !LINKED) {
+        if constexpr (BS && !LINKED && !ROWS_IN) {
 #pragma unroll
             for (int z = 0; z < ZT; ++z)
                 k.sc[z] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(s_desc, quad * 512 + s_lane + z * 64, 0, 0));
@@ -440,7 +445,17 @@ __device__ __forceinline__ void q4_matmul_workgroup(
             k.q[r] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_desc[r], quad * 1024 + lane * 16, 0, NT));
             k.d[r] = __builtin_bit_cast(q4_u32x2, __builtin_amdgcn_raw_buffer_load_b64(d_desc[r], quad * 128 + l16 * 8, 0, NT));
         }
-        if constexpr (PACKED && !LINKED) {
+        if constexpr (ROWS_IN) {
+            // (two requests per register quad, two columns of each; a lane behind the last column fetches the first ones, and drops them)
+            const uint32_t at = quad * 512 + lane * 8;
+#pragma unroll
+            for (int n = 0; n < QR; ++n) {
+                const q4_u32x2 v = __builtin_bit_cast(q4_u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+                    x_desc[0], min((uint32_t)n, live - 1u) * (nblocks * 128) + (at < nblocks * 128 ? at : 0u), 0, 0));
+                k.x[n / 2][n % 2 * 2] = v[0];
+                k.x[n / 2][n % 2 * 2 + 1] = v[1];
+            }
+        } else if constexpr (PACKED && !LINKED) {
 #pragma unroll
             for (int i = 0; i < XQ; ++i)
                 k.x[i] = __builtin_bit_cast(q4_u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_desc[0], quad * (XQ * 1024) + i * 1024 + lane * 16, 0, 0));
@@ -503,6 +518,32 @@ __device__ __forceinline__ void q4_matmul_workgroup(
             const uint32_t w0 = (uint32_t)wd[n][0], w1 = (uint32_t)wd[n][1];
             to[(piece + n) * 4 + lane % 4] = (w0 & 0xFFFFu) | w1 << 16;
             to[(piece + 2 * WIDTH + n) * 4 + lane % 4] = w0 >> 16 | (w1 & 0xFFFF0000u);
+        }
+        asm volatile("" ::: "memory");
+    };
+    // A quad's rows of floats (ROWS_IN) into the places of LDS that its fragments would go to: a block is 16 lanes, one power of two
+    // for it as in q4_emit_block.
+    [[maybe_unused]] auto split_rows = [&](uint32_t quad, const QuadW& k) __attribute__((always_inline)) {
+        const bool has_cols = quad * 128 + lane * 2 < nblocks * 32;
+        uint32_t* const to = reinterpret_cast<uint32_t*>(packed[wave]);
+        const uint32_t piece = lane / 8 * 4 * WIDTH + lane / 4 % 2 * WIDTH;   // (columns 2 * lane and the next one: k step lane / 8)
+#pragma unroll
+        for (int n = 0; n < QR; ++n) {
+            if ((uint32_t)n >= live) break;
+            const float x0 = has_cols ? __uint_as_float(k.x[n / 2][n % 2 * 2]) : 0.f, x1 = has_cols ? __uint_as_float(k.x[n / 2][n % 2 * 2 + 1]) : 0.f;
+            float amax = fmaxf(fabsf(x0), fabsf(x1));
+            amax = fmaxf(amax, dpp_f<kDppQuadXor1>(amax));
+            amax = fmaxf(amax, dpp_f<kDppQuadXor2>(amax));
+            amax = fmaxf(amax, dpp_f<kDppHalfMirror>(amax));
+            amax = fmaxf(amax, dpp_f<kDppRowRor8>(amax));
+            const int e = amax < INFINITY ? __builtin_amdgcn_frexp_expf(amax) : 0;   // (0 where amax is)
+            int se = 14 - e;
+            se = se > 100 ? 100 : (se < -100 ? -100 : se);
+            const float t0 = __builtin_ldexpf(x0, se), t1 = __builtin_ldexpf(x1, se);
+            const q4_half2 hi = {(_Float16)t0, (_Float16)t1}, lo = {(_Float16)(t0 - (float)hi[0]), (_Float16)(t1 - (float)hi[1])};
+            to[(piece + n) * 4 + lane % 4] = __builtin_bit_cast(uint32_t, hi);
+            to[(piece + 2 * WIDTH + n) * 4 + lane % 4] = __builtin_bit_cast(uint32_t, lo);
+            if (l16 == 0) scales[wave][0][kg * 16 + n] = __builtin_ldexpf(1.0f, -se);
         }
         asm volatile("" ::: "memory");
     };
@@ -579,13 +620,17 @@ __device__ __forceinline__ void q4_matmul_workgroup(
     QuadW w, next;
     BlockX x[XD];
     auto turn = [&](uint32_t quad, auto more) __attribute__((always_inline)) {
-        if constexpr (BS) {   // (a wave's own: LDS operations of a wave are in order)
+        if constexpr (ROWS_IN) {
+            split_rows(quad, w);
+        } else if constexpr (BS) {   // (a wave's own: LDS operations of a wave are in order)
 #pragma unroll
             for (int z = 0; z < ZT; ++z) scales[wave][z][lane] = w.sc[z];
         }
         if constexpr (PACKED) {
+            if constexpr (!ROWS_IN) {
 #pragma unroll
-            for (int i = 0; i < XQ; ++i) packed[wave][i * 64 + lane] = w.x[i];
+                for (int i = 0; i < XQ; ++i) packed[wave][i * 64 + lane] = w.x[i];
+            }
             if constexpr (XD > 1) read_x(0, x[0]);
         }
 #pragma unroll

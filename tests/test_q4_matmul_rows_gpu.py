@@ -1,0 +1,62 @@
+"""Q4_0 matmuls that are a call of their own over up to eight requests split their rows of floats themselves: row tiles per
+workgroup, quads that end early, K slices, the requests where another launch splits them instead, and rows whose blocks are far apart."""
+import numpy as np
+import pytest
+
+import test_q4_matmul_gpu as q4
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch", [1, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("rows,cols", [
+    (64, 64), (192, 96),            # half a quad; three blocks
+    (2048, 2080),                   # slices, the last of them with a quad of one block
+    (4160, 160), (8192, 2048),      # two row tiles
+    (8256, 288), (16448, 128),      # four, of 16 and 8 waves
+    (256, 8224),                    # two tiles or one, many quads to a wave
+])
+def test_rows_of_floats(exe, rows, cols, batch):
+    q, x, stride = q4.make(rows, cols, batch, rows + cols + batch)
+    x[batch // 2, ::3] = 0.0
+    got = q4.run(exe, f"rowsin_{rows}_{cols}_{batch}", q, x, batch, rows, cols, stride)
+    q4.check(got, q, x, batch, rows, cols, stride)
+
+
+def test_one_call_reads_its_rows_only(exe):
+    """What lies behind the last row and the last column is not read into the products: infinities there change nothing."""
+    rows, cols, batch = 128, 160, 3
+    q, x, stride = q4.make(rows, cols, batch, 1)
+    want = q4.run(exe, "rowsin_edge", q, x, batch, rows, cols, stride)
+    big = np.full((batch + 2, cols), np.inf, np.float32)
+    big[1:-1] = x
+    d_in, d_out = exe.allocateScratchBuffer(big.nbytes), exe.allocateScratchBuffer(batch * rows * 4)
+    try:
+        assert exe.uploadToBuffer(d_in, big)
+        assert exe.encodeMatMulQ4_0Batched("rowsin_edge", q, d_in + cols * 4, batch, rows, cols, stride, 1, d_out, sync=True), exe.lastError()
+        got = np.empty((batch, rows), np.float32)
+        assert exe.downloadFromBuffer(d_out, got)
+    finally:
+        exe.releaseScratchBuffer(d_in)
+        exe.releaseScratchBuffer(d_out)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("batch", [2, 7])
+def test_blocks_far_apart(exe, batch):
+    """Every block has a power of two of its own: one whose elements are 2^-60 of another's keeps its 22 bits."""
+    rows, cols = 256, 512
+    q, x, stride = q4.make(rows, cols, batch, 5)
+    x[:, :256] *= 2.0 ** 60
+    x[0, 32:64] = 0.0
+    x[1, 64:96] *= 2.0 ** -130          # (denormal numbers)
+    only_small = x.copy()
+    only_small[:, :256] = 0.0
+    for v in (x, only_small):
+        got = q4.run(exe, f"rowsin_far_{batch}", q, v, batch, rows, cols, stride)
+        w = q4.dequant(q, cols)
+        scale = np.abs(v.astype(np.float64)) @ np.abs(w).T
+        assert (np.abs(got - v.astype(np.float64) @ w.T) <= 4e-6 * scale + 1e-300).all()
+    x[0, 100] = np.inf
+    got = q4.run(exe, f"rowsin_far_{batch}", q, x, batch, rows, cols, stride)
+    assert not np.isfinite(got[0]).any() and np.isfinite(got[1:]).all()
