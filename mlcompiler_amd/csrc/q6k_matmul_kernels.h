@@ -86,6 +86,8 @@ struct Q6KArgs {
 // ahead.  Whole calls, us, before -> now: 32000 x 2048 at 1, 16, 32 and 64 requests 34.6, 35.7, 38.1, 65.5 -> 28.7, 30.9, 34.2,
 // 48.3 (the kernel at one and 32: 21.2 and 24.5 -> 15.7 and 20.9), 128256 x 2048 at one and 64 91, 207 -> 72, 141; 4096 x 4096 at
 // 17 to 32 24 -> 23.
+// Up to 16 requests one product does for hi and lo: 32000 x 2048 at 1 and 3 requests 29.1 -> 28.7, 2048 x 2048 at 1 to 16 19.9 -> 19.3, 4096 x
+// 4096 22.8 -> 22.1.  2-norm error against float64 at 2048 and 4096 columns 1.10e-7, 1.31e-7 -> 1.07e-7, 1.29e-7.
 template <int NBT, int RT, int NA>
 __global__ __launch_bounds__(512, 2) void q6_k_matmul_mfma_kernel(const Q6KArgs a) {
     constexpr int WAVES = 8;
@@ -98,9 +100,15 @@ __global__ __launch_bounds__(512, 2) void q6_k_matmul_mfma_kernel(const Q6KArgs 
     const uint32_t ksteps = a.nblocks * 16;
     // (lanes past the last request fetch that one's fragments again; their results are dropped)
     const uint32_t width = frag_width(a.batch);
+    // (up to 16 requests: lo of a request sits 2 NA rows behind its hi, in the registers NA further, and one product does for both)
+    constexpr bool BOTH = NA < 16;
+    static_assert(!BOTH || NBT == 1, "one batch tile");
+    constexpr int XP = BOTH ? 1 : 2;
     uint32_t lane_x[NBT];
 #pragma unroll
-    for (int t = 0; t < NBT; ++t) lane_x[t] = (half * width + min(l32, a.batch - 1u - t * 32)) * 16;
+    for (int t = 0; t < NBT; ++t)
+        lane_x[t] = BOTH ? (half * width + min(l32 % (2 * NA), a.batch - 1u)) * 16 + min(l32 / (2 * NA), 1u) * 32 * width
+                         : (half * width + min(l32, a.batch - 1u - t * 32)) * 16;
 
     float acc[RT][NBT][NA];
 #pragma unroll
@@ -140,13 +148,13 @@ __global__ __launch_bounds__(512, 2) void q6_k_matmul_mfma_kernel(const Q6KArgs 
         }
         asm volatile("" ::: "memory");
     };
-    q4_half8 x[NBT][4][2];  // [batch tile][quarter][hi, lo]
+    q4_half8 x[NBT][4][XP];  // [batch tile][quarter][hi, lo]
     auto load_x = [&](uint32_t g, int q) __attribute__((always_inline)) {
         const uint32_t kstep = g / 4 * 16 + (g / 2) % 2 * 8 + q * 2 + g % 2;
 #pragma unroll
         for (int t = 0; t < NBT; ++t)
 #pragma unroll
-            for (int pt = 0; pt < 2; ++pt)
+            for (int pt = 0; pt < XP; ++pt)
                 x[t][q][pt] = __builtin_bit_cast(q4_half8, __builtin_amdgcn_raw_buffer_load_b128(x_desc[t], (kstep * 2 + pt) * 32 * width + lane_x[t], 0, 0));
         asm volatile("" ::: "memory");
     };
@@ -168,9 +176,9 @@ __global__ __launch_bounds__(512, 2) void q6_k_matmul_mfma_kernel(const Q6KArgs 
 #pragma unroll
                 for (int i = 0; i < 16; ++i) s[i] = 0.f;
                 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[t][q][0], w, s, 0, 0, 0);
-                s = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[t][q][1], w, s, 0, 0, 0);
+                if constexpr (!BOTH) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[t][q][XP - 1], w, s, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < NA; ++i) acc[r][t][i] = fmaf(gscale, s[i], acc[r][t][i]);
+                for (int i = 0; i < NA; ++i) acc[r][t][i] = fmaf(gscale, BOTH ? s[i] + s[(i + NA) % 16] : s[i], acc[r][t][i]);
                 // (here, and not further down, where the compiler would move it with all the products' registers)
 #pragma unroll
                 for (int i = 0; i < NA; ++i) asm volatile("" : "+v"(acc[r][t][i]));
