@@ -299,8 +299,9 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3, kQ4Rows = 4 };
 // More than 16 requests: z groups of 16, workgroups of their own that read the same weights at the same
 // time on the same XCD (workgroup x: row group x / (8 Z) * 8 + x % 8, z group x / 8 % Z).  Each fetches its
 // own activations only, 4 bytes per request and column through one CU's memory path, which would be the
-// longest stream of a workgroup that had them all.  (NI < 4: the A operand has room for hi and lo of a request in different rows, and
-// one product does for both.  2-norm error against float64, two products -> one: 0.95e-7 .. 1.07e-7 -> 0.85e-7 .. 0.98e-7.)  ZT = 2 or 4: so many groups in one
+// longest stream of a workgroup that had them all.  (NI = 1: the A operand has room for hi and lo of a request
+// in different rows, and one product does for both; with NI = 2 that is no faster and spills.  2-norm error against float64, two
+// products -> one: 0.95e-7 .. 1.07e-7 -> 0.85e-7 .. 0.98e-7.)  ZT = 2 or 4: so many groups in one
 // workgroup, which unpacks a weight once for all of them.  That takes 158 or 245 registers, one workgroup of 8 waves to a
 // CU, and so pays where such workgroups fill their rounds (launch_q4).
 //
@@ -352,7 +353,7 @@ __device__ __forceinline__ void q4_matmul_workgroup(
     // Up to 8 requests: a quad's activations come 1 KB per load, without the places of requests that do not
     // exist, and each lane's operand from LDS.  (16-byte loads of 64 lanes cost 16 clocks of the return path, however
     // many of them ask for the same bytes or for none.)
-    constexpr bool PACKED = NI < 4;
+    constexpr bool PACKED = NI < 4, BOTH = NI == 1;
     constexpr uint32_t WIDTH = PACKED ? 4 * NI : 32;
     constexpr int XQ = PACKED ? 2 * NI : 1;          // loads per quad
     // blocks of activations in registers: as far as 128 registers per wave go
@@ -401,7 +402,7 @@ __device__ __forceinline__ void q4_matmul_workgroup(
         q4_u32x4 x[XQ];   // PACKED: the quad's activations
     };
     struct BlockX {
-        q4_half8 hi[ZT], lo[ZT];   // (PACKED: hi[0] has both)
+        q4_half8 hi[ZT], lo[ZT];   // (BOTH: hi[0] has both)
     };
     // Everything is fetched with buffer loads: a descriptor per stream in scalar registers and 32 bits per lane.  Their
     // descriptors end where the data does; what lies behind (the last blocks of an incomplete quad, the weights
@@ -423,9 +424,9 @@ __device__ __forceinline__ void q4_matmul_workgroup(
     // so that the third and the fourth group's are in the second batch tile)
     uint32_t x_lane[ZT];   // (two 16-column steps, hi and lo of each)
     if constexpr (PACKED) {
-        // up to 8 requests: hi of request r in row (r / NI) * 4 + r % NI and lo NI rows further, so that one product has both
-        const uint32_t m = l16 % 4, xreq = min(l16 / 4 * NI + m % NI, live - 1u);
-        x_lane[0] = (kg / 2 * 4 * WIDTH + kg % 2 * WIDTH + min(m / NI, 1u) * 2 * WIDTH + xreq) * 16;
+        // BOTH: hi of request r in row r * 4 and lo in the next one, so that one product has both
+        const uint32_t m = l16 % 4, xreq = min(l16 / 4 * NI + (BOTH ? 0u : min(m, (uint32_t)NI - 1u)), live - 1u);
+        x_lane[0] = (kg / 2 * 4 * WIDTH + kg % 2 * WIDTH + (BOTH ? min(m, 1u) * 2 * WIDTH : 0u) + xreq) * 16;
     }
 #pragma unroll
     for (int z = 0; z < (PACKED ? 0 : ZT); ++z) {
@@ -550,6 +551,7 @@ __device__ __forceinline__ void q4_matmul_workgroup(
     auto read_x = [&](int j, BlockX& k) __attribute__((always_inline)) {
         const uint32_t piece = j * 8 * WIDTH + x_lane[0] / 16;
         k.hi[0] = __builtin_bit_cast(q4_half8, packed[wave][piece]);
+        if constexpr (!BOTH) k.lo[0] = __builtin_bit_cast(q4_half8, packed[wave][piece + 2 * WIDTH]);
         asm volatile("" ::: "memory");
     };
     const uint32_t ones = q4_ones();
@@ -575,10 +577,10 @@ __device__ __forceinline__ void q4_matmul_workgroup(
 #pragma unroll
             for (int z = 0; z < ZT; ++z) {
                 q4_float4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.hi[z], wk, zero, 0, 0, 0);
-                if constexpr (!PACKED) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.lo[z], wk, s, 0, 0, 0);
+                if constexpr (!BOTH) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.lo[z], wk, s, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
-                    acc[r][z][i] = fmaf(BS ? d * sc[z][i] : d, PACKED ? s[i] + s[(i + NI) % 4] : s[i], acc[r][z][i]);
+                    acc[r][z][i] = fmaf(BS ? d * sc[z][i] : d, BOTH ? s[i] + s[(i + NI) % 4] : s[i], acc[r][z][i]);
                 // (here, and not further down, where the compiler would move it: a quad's products do not fit
                 // the 128 registers a wave has)
 #pragma unroll
