@@ -66,6 +66,7 @@ constexpr uint32_t kReplayTagStep = 4096;   // decode launches of one captured p
 
 // Room for the words between two matmuls of a launch (q4_link_words): four requests of 4096 columns, eight copies, take 2.2 MB.
 constexpr size_t kLinkBytes = 4u << 20;
+constexpr size_t kChainBatch = 4;   // requests, at most (q4_chain_kernel: what more cost)
 
 // Rounds that a wait for tagged words polls before it is given up (about 0.1 s).
 constexpr long kSpinLimit = 200000;
@@ -630,7 +631,7 @@ int launch_chain(Q4Form form, bool block_scales, Q4RopeArgs& b) {
     Q4RopeArgs& a = g.front.a;
     const size_t batch = b.batch;
     if (!g.opt_q4_chain || (form != kQ4Silu && form != kQ4Rope) || !block_scales || !g.front.block_scales || !b.ssq_in || b.ssq_in != a.ssq_out ||
-        batch > 4 || b.slices != 1 || q4_waves(a) != 16 || q4_waves(b) != 16 || q4_tiles(kQ4Add, a.rows, batch, a.slices) != 2)
+        batch > kChainBatch || b.slices != 1 || q4_waves(a) != 16 || q4_waves(b) != 16 || q4_tiles(kQ4Add, a.rows, batch, a.slices) != 2)
         return -1;
     const int rt = q4_tiles(form, b.rows, batch, 1);
     if (rt * ((b.nquads + 15) / 16) > 4) return -1;
@@ -672,7 +673,7 @@ int launch_chain(Q4Form form, bool block_scales, Q4RopeArgs& b) {
     const size_t bytes = q4_link_words(a.rows, b.batch) * 8 * kQ4LinkCopies;
     if (!apart || bytes > kLinkBytes || !sliced_tags_left()) return -1;
     Q4Link link;
-    link.words = meeting_words("q4_link_words", kLinkBytes);
+    link.words = meeting_words("q4_link_words", kLinkBytes);   // (there since the first one was held back)
     if (!link.words) return -1;
     link.tags = next_sliced_tags();
     g.front.active = false;

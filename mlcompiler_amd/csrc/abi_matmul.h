@@ -236,12 +236,17 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
             norm.rms_n_gamma = p.n_weight;
             g.rows.active = false;   // the two matmuls do the chain's work
             ++g.gemm_rms_fused;
-            // (nothing else is pending: settle() would launch it, and does where this matmul turns out to go out alone)
+            // It waits in front of this one, where the two may share a launch.  (Nothing else is pending.  The words' memory is taken now:
+            // what launches the two later may be a call that allocates nothing.)
             if (!settle_front()) return 0;
-            m.active = false;
-            g.front.active = true;
-            g.front.block_scales = m.block_scales;
-            static_cast<Q4Args&>(g.front.a) = m.a;
+            if (g.opt_q4_chain && batch <= kChainBatch && meeting_words("q4_link_words", kLinkBytes)) {
+                m.active = false;
+                g.front.active = true;
+                g.front.block_scales = m.block_scales;
+                static_cast<Q4Args&>(g.front.a) = m.a;
+            } else if (!settle()) {
+                return 0;
+            }
         } else if (feeds) {  // the chain that produces the input also splits it (batch <= 64: one round)
             g.rows.p.frag = frag;
             g.rows.p.inv_scale = inv;

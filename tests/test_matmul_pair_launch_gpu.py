@@ -185,3 +185,34 @@ def test_words_that_never_come(exe):
         exe.setOption("decode_spin_limit", 200000)
         exe.setOption("decode_test_flags", 0)
         c.free()
+
+
+MEMORY = """
+import ctypes as C, sys
+sys.path[:0] = ["tests", "."]
+from mlcompiler_amd import HipExecutor
+from test_matmul_pair_launch_gpu import Pair
+exe, hip = HipExecutor.Instance(), C.CDLL("libamdhip64.so")
+exe.requireAvailable()
+free, total = C.c_size_t(), C.c_size_t()
+def used():
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return total.value - free.value
+c = Pair(exe, "silu", 4, 4224, 4096 // 2, 88)
+assert exe.beginForwardPassCB() and c.encode()
+before = used()
+assert exe.flushForwardPassCB(), exe.lastError()
+print("used", before, used())
+"""
+
+
+def test_the_launch_of_a_held_back_pair_allocates_nothing():
+    """(A process of its own: the library's buffers are for good.)"""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", MEMORY], cwd=root, capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr
+    before, after = (int(v) for v in out.stdout.split("used")[1].split())
+    assert before == after
