@@ -42,6 +42,7 @@
 #include "matmul_tokens_args.h"
 #include "q4_matmul_mfma.h"
 #include "q6k_unpack.h"
+#include "wave_reduce.h"
 
 namespace mlc_hip {
 
@@ -78,8 +79,7 @@ __global__ __launch_bounds__(THREADS) void tokens_split_kernel(const float* __re
     } else if (live) {
         for (uint32_t k8 = g0; k8 < groups; k8 += PER) amax = max8(amax, xr[k8 * 2], xr[k8 * 2 + 1]);
     }
-#pragma unroll
-    for (int off = 32; off >= 4; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = wave_max_of<4>(amax);
     if (threadIdx.x % 64 < 4) red[threadIdx.x / 64][n4] = amax;
     __syncthreads();
     amax = red[0][n4];

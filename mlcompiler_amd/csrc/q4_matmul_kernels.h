@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "q4_matmul_mfma.h"
+#include "wave_reduce.h"
 
 namespace mlc_hip {
 
@@ -69,8 +70,7 @@ __global__ __launch_bounds__(THREADS) void q4_split_activations_kernel(
             }
         }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = wave_max_of(amax);
     if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = amax;
     __syncthreads();
     amax = red[0];
