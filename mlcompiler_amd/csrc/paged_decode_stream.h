@@ -789,8 +789,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             // (as a difference, which is exact where it matters: a sum would be rounded, for large scores to
             // more than the weight's 16 bits of range allow)
             if (__any(mloc - mf_m > kLazyTau + kWeightShift)) {
-                float mcol = max_nn(mloc, __shfl_xor(mloc, 16));
-                mcol = max_nn(mcol, __shfl_xor(mcol, 32));
+                const float mcol = across32(across16(mloc, OpMax()), OpMax());
                 const float m_new = max_nn(mf_m, mcol - kWeightShift);
                 const float alpha = fast_exp2(mf_m - m_new);
                 mf_m = m_new;
@@ -1016,8 +1015,7 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
             // combines the four for its own heads, in the lane layout the code below expects
             // (lane (r, c): dims c*8 + r*HPK + kk).  The sums run over the waves in a fixed
             // order in every lane, so l does not depend on the lane it is read from.
-            float lt = mf_l + __shfl_xor(mf_l, 16);
-            lt += __shfl_xor(lt, 32);
+            const float lt = across32(across16(mf_l, OpAdd()), OpAdd());
             if (n16 < G) {
 #pragma unroll
                 for (int b = 0; b < DB; ++b)
@@ -1066,8 +1064,8 @@ __global__ __launch_bounds__(64 * NW) void paged_decode_stream_kernel(const Stre
 #pragma unroll
         for (int h = 0; h < HPW; ++h) {
             float m = m_ref[h];
-#pragma unroll
-            for (int off = CPR; off < 64; off <<= 1) m = max_nn(m, __shfl_xor(m, off));
+            if constexpr (CPR == 8) m = max_nn(m, dpp_f<kDppRowRor8>(m));
+            m = across32(across16(m, OpMax()), OpMax());
             m_all[h] = m;
             const float wgt = fast_exp2(m_ref[h] - m);
             // with CPR == 16 every token's weight sits in two lanes (c and c^8): count it once

@@ -34,6 +34,7 @@
 
 #include <type_traits>
 
+#include "paged_decode_kernels.h"
 #include "paged_prefill_args.h"
 #include "store_through.h"
 
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
         float mx = s[0];
 #pragma unroll
         for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32)) * a.scale_log2e;  // scale > 0: max commutes
+        mx = across32(mx, OpMax()) * a.scale_log2e;  // scale > 0: max commutes
         if (__any(mx > m_run + 8.0f)) {
             const float m_new = fmaxf(m_run, mx);
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -354,7 +355,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_prefill_mfma_kernel(const
 
     // ---- write O: lane owns row my_row; register i of block mb is dim mb*32 + (i/4)*8 + half*4 + i%4
     if (row_ok) {
-        l_run += __shfl_xor(l_run, 32);
+        l_run = across32(l_run, OpAdd());
         if (gridDim.y > 1) {   // a part's sums, on the part's own reference, for prefill_combine_kernel
             const uint32_t part_wave = (blockIdx.y * gridDim.x + wg) * kPfWaves + wave;
             if (half == 0) store_through(&a.part_ml[part_wave * kPfRows + l32], make_float2(m_run, l_run));
@@ -968,7 +969,7 @@ __global__ __launch_bounds__(256) void paged_prefill_mfma64_kernel(const Prefill
 #pragma unroll
     for (int hb = 0; hb < HALVES; ++hb) {
         if (row_ok[hb]) {
-            const float l = l_run[hb] + __shfl_xor(l_run[hb], 32);
+            const float l = across32(l_run[hb], OpAdd());
             const float inv = l > 0.f ? 1.0f / l : 0.f;
             float* orow = a.o + out_row[hb];
 #pragma unroll

@@ -13,10 +13,7 @@ static constexpr int kDppRowRor4 = 0x124;   // row_ror:4: within 16 lanes whose 
 template <int LAST = 1, class Op>
 __device__ __forceinline__ float wave_butterfly(float v, Op op) {
     static_assert(LAST == 1 || LAST == 4, "all lanes, or lanes that are equal modulo 4");
-    const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = op(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
-    const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = op(__uint_as_float(s16[0]), __uint_as_float(s16[1]));
+    v = across16(across32(v, op), op);
     v = op(v, dpp_f<kDppRowRor8>(v));
     v = op(v, dpp_f<kDppRowRor4>(v));
     if constexpr (LAST == 1) {
