@@ -190,7 +190,9 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
 
     // MFMA path, one pass over at most 64 requests at a time.
     const size_t nblocks = cols / 32, quads = (nblocks + 3) / 4;
-    const bool rows_in = sync && g.opt_q4_int_operand && !feeds && !block_scales && aligned16(in) && q4_splits_rows(rows, cols, batch);
+    // (its workgroups read rows that others have not come to yet while the first ones store: only where the output lies apart)
+    const bool rows_in = sync && g.opt_q4_int_operand && !feeds && !block_scales && aligned16(in) && q4_splits_rows(rows, cols, batch) &&
+                         !overlap(in, batch * cols * 4, out, batch * rows * 4);
     for (size_t bo = 0; bo < batch; bo += 64) {
         const size_t bn = std::min<size_t>(64, batch - bo);
         const size_t bpad = (bn + 31) / 32 * 32;

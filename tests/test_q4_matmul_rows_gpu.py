@@ -42,6 +42,32 @@ def test_one_call_reads_its_rows_only(exe):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("batch", [1, 4, 5, 8])
+@pytest.mark.parametrize("rows,cols,at", [
+    (2048, 2048, 0), (4096, 4096, 0),       # in place
+    (2048, 2048, -1024), (2048, 2048, 1024),
+    (32768, 512, 0), (32768, 512, -32768),  # more workgroups than run at a time
+    (256, 8224, 4096),                      # K slices
+])
+def test_output_over_the_input(exe, rows, cols, batch, at):
+    """The output may lie where the input does: all of it is read first.  `at`: floats from the input's start to the output's."""
+    q, x, stride = q4.make(rows, cols, batch, rows + cols + batch)
+    start, out = max(0, -at), max(0, at)
+    room = np.full(max(start + batch * cols, out + batch * rows), np.nan, np.float32)
+    room[start:start + batch * cols] = x.reshape(-1)
+    dev = exe.allocateScratchBuffer(room.nbytes)
+    try:
+        for _ in range(3):
+            assert exe.uploadToBuffer(dev, room)
+            assert exe.encodeMatMulQ4_0Batched(f"over_{rows}_{cols}_{batch}", q, dev + start * 4, batch, rows, cols, stride, 1, dev + out * 4,
+                                               sync=True), exe.lastError()
+            after = np.empty_like(room)
+            assert exe.downloadFromBuffer(dev, after)
+            q4.check(after[out:out + batch * rows].reshape(batch, rows), q, x, batch, rows, cols, stride)
+    finally:
+        exe.releaseScratchBuffer(dev)
+
+
 @pytest.mark.parametrize("batch", [2, 7])
 def test_blocks_far_apart(exe, batch):
     """Every block has a power of two of its own: one whose elements are 2^-60 of another's keeps its 22 bits."""
