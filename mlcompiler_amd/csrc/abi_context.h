@@ -640,6 +640,10 @@ int launch_chain(Q4Form form, bool block_scales, Q4RopeArgs& b) {
     b.row_groups = (uint32_t)(b.rows / 16 / rt);
     const uint32_t blocks = (a.row_groups + 7) / 8 * 8 * a.slices, grid = blocks + (b.row_groups + 7) / 8 * 8;
     if (blocks > 0xFFFFu || grid > 2 * (uint32_t)g.n_cu) return -1;
+    // On every XCD a CU stays free of the second one's workgroups, which wait with a whole CU each (tagged_words.h: two
+    // processes).  That costs nothing: where they take all CUs, the first one's hold up as many of them.  (8 layers of hidden 2048 and
+    // FFN width 8192, 256 groups for gate/up, 1 to 4 requests, us, with gate/up in pairs -> by itself: 245, 253, 259, 268 -> 242, 246, 251, 256.)
+    if ((b.row_groups + 7) / 8 >= (uint32_t)g.n_cu / 8) return -1;
     // The second matmul's workgroups run beside the first one's: what they write must be nothing that those read or write,
     // and what they read besides the words nothing that those write.
     const size_t row = batch * a.rows * 4;

@@ -14,8 +14,13 @@
 //     lower numbers at most, which all have, and ends.
 //   * Two matmuls in one launch: the second one's workgroups, the last of the launch, wait for the first one's, which wait for
 //     each other's slices at most.  None of the second's has started on an XCD where one of the first's has yet to start.
-// That holds for one such launch at a time (scratch_follow orders them across streams), beside launches that end by
-// themselves.  The waits are bounded all the same: a pass then fails instead of hanging.
+// That holds for one such launch at a time (scratch_follow orders those of a process across streams), beside launches that
+// end by themselves.  Two processes on a GPU are not ordered.  K slices of up to 64 requests end even then: who waits has its
+// partners on its own XCD.  So do two matmuls in one launch: a workgroup that waits may have a CU to itself (1024 threads of up to
+// 128 registers), but those of one launch leave a CU of every XCD to others (launch_chain): room for the first matmuls' workgroups, and
+// for what the other process has yet to start.  With a third process they need not end, nor the decode launches
+// of two processes beside each other, nor K slices of many tokens: each may hold the place that the other waits for.  The
+// waits are bounded all the same: a pass then fails instead of hanging.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -97,6 +97,9 @@ def _same_bits(got, want):
     ("silu", 3, 5632, 192, 72, True),       # a quad and a half; the first matmul's K in slices
     ("silu", 1, 4224, 2112, 88, False),     # more than a quad per wave
     ("silu", 5, 4224, 1024, 88, False),     # more requests
+    ("silu", 1, 4224, 1024, 124, True),     # 31 of an XCD's 32 CUs
+    ("silu", 1, 4224, 1024, 125, False),    # all of them: none is left for what they wait for, if that is another process's turn
+    ("silu", 2, 4224, 1024, 128, False),
     ("rope", 1, 5632, 2048, 32, True),      # three slices, one row tile to a workgroup
     ("rope", 4, 4160, 2112, 8, True),       # a wave with a second quad, and that a part of one
     ("rope", 2, 4224, 4096, 72, True),      # two quads per wave, two row tiles
