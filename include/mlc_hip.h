@@ -434,8 +434,9 @@ long mlc_hip_decode_table_uploads(void);
  *                           the kernel with 64 rows per wave has no 2-stage build and runs 4
  *                           stages when 2 is asked for
  *   "prefill_rows64"        1 (default) = heads/kv_heads up to 4, and 8 where the keys are more than a few
- *                           tiles, run the prefill kernel with 64 chunk rows per wave; 0 = the
- *                           kernel with 32 rows per wave for every ratio
+ *                           tiles and blocks of 64 rows take no more rounds over the CUs, run the
+ *                           prefill kernel with 64 chunk rows per wave; 0 = the kernel with 32 rows
+ *                           per wave for every ratio
  * Returns 0 for an unknown name or value. */
 int mlc_hip_set_option(const char* name, long value);
 

@@ -84,7 +84,8 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
     a.part_o = splits > 1 ? static_cast<float4*>(cached_buffer("prefill_parts", kPartBytes)) : nullptr;
     if (!a.part_o) splits = 1;
     a.part_ml = reinterpret_cast<float2*>(a.part_o + (splits > 1 ? splits * wgs * kPfWaves * kPfRows * head_dim / 4 : 0));
-    const bool rows64 = g.opt_prefill_rows64 && (num_heads / kv_heads < 8 || prefill_rows64_ratio8(head_dim, max_tiles));
+    const bool rows64 = g.opt_prefill_rows64 &&
+                        (num_heads / kv_heads < 8 || prefill_rows64_ratio8(head_dim, max_tiles, chunk, batch * kv_heads, (size_t)g.n_cu));
     launch_prefill(a, head_dim, (int)g.opt_prefill_stages, rows64, splits, g.stream);
     return finish(sync);
 }

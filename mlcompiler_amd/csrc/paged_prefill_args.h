@@ -31,12 +31,20 @@ static constexpr int kPfRows = 32;   // chunk rows per wave
 static constexpr int kPfWaves = 8;   // waves per workgroup
 
 // GQA ratio 8: 64 rows of four heads per workgroup where there are enough key tiles, else 32 rows of all eight.  Both have 256
-// (row, head) pairs; the kernel with 64 rows reads an operand from LDS for two products, and takes longer until its first tile and in
-// the last row block, half of which a chunk may not fill.  (Whole calls, us, 32 -> 64 rows, by tiles of the longest
+// (row, head) pairs; the kernel with 64 rows reads an operand from LDS for two products, and takes longer until its first tile.
+// (Whole calls, us, 32 -> 64 rows, by tiles of the longest
 // row block.  head_dim 64: 2 tiles 20.3 -> 21.3, 4 23.3 -> 23.9, 8 25.9 -> 26.2, 34.1 -> 32.8 and 24.5 -> 24.5, 9 30.8 -> 31.5, 10 34.0 -> 31.5
 // and 41.9 -> 41.4, 12 37.5 -> 34.1, 25 47.1 -> 40.4, 128 124 -> 110.  128: 4 28.6 -> 30.1, 8 48.5 -> 51.4 and 30.3 -> 30.6, 10 60.8 -> 63.2,
 // 12 50.8 -> 51.7 and 52.5 -> 51.8, 16 62.5 -> 60.7 and 40.2 -> 38.5, 25 58.1 -> 53.8, 128 162 -> 146.)
-inline bool prefill_rows64_ratio8(size_t head_dim, size_t max_tiles) { return max_tiles >= (head_dim == 64 ? 10u : 16u); }
+// And it takes workgroups of its own for a last row block of at most 32 rows: only where they are no more rounds over the CUs, or
+// hardly more.  (By rounds of 32 and of 64 rows, 19 or 47 tiles, 32 -> 64 rows: equal 0.99 to 1.15 times as fast; 1 and 2 0.63
+// to 0.83, 2 and 4 0.65 to 0.75, 2 and 3 0.78 to 0.86, 3 and 4, 4 and 5 0.86 to 0.97, 5 and 6 0.93 to 1.01, 11 and 12 0.95 to 0.98.  32
+// requests of 32 rows behind 3 000 keys with 8 KV heads of 128 153 -> 201 us, 40 of 96 behind 1 000 208 -> 224: both 32 rows.)
+// pairs: requests x KV heads.
+inline bool prefill_rows64_ratio8(size_t head_dim, size_t max_tiles, size_t chunk, size_t pairs, size_t n_cu) {
+    const auto rounds = [&](size_t blocks) { return (blocks * pairs + n_cu - 1) / n_cu; };
+    return max_tiles >= (head_dim == 64 ? 10u : 16u) && rounds((chunk + 63) / 64 * 2) * 20 <= rounds((chunk + 31) / 32) * 21;
+}
 
 inline bool prefill_shape_supported(size_t head_dim, size_t page_size, size_t num_heads,
                                     size_t kv_heads) {
