@@ -30,24 +30,35 @@ Q4Slices q4_slices(size_t rows, size_t cols, size_t batch) {
     return {(quads + per_slice - 1) / per_slice, per_slice};
 }
 
-// A matmul that is a call of its own takes its rows of floats as they are and splits them itself, every workgroup all of them: that
-// takes the launch in front away, 2 us and, for long rows, its time.  (The split is of every block by itself, as the fused
-// launches have it.)  Up to four requests that pays everywhere, up to eight where a workgroup has one row tile, or two and K is long:
-// a build for four tiles spills.  Whole calls, us, split in front -> now, and with 5 and 8 tokens in brackets where the split stays in front:
-//   rows x columns | 1           | 4           | 5             | 8
-//   2560 x 2048    | 17.4 / 14.9 | 17.4 / 15.4 | 17.6 / 15.8   | 18.0 / 16.6
-//   11264 x 2048   | 19.2 / 16.9 | 19.3 / 17.6 | (19.9 / 22.0) | (20.0 / 22.6)
-//   2048 x 5632    | 18.7 / 16.0 | 18.7 / 16.8 | 19.2 / 17.6   | 19.3 / 18.2
-//   6144 x 4096    | 20.0 / 17.8 | 20.0 / 18.9 | (20.9 / 20.2) | (20.8 / 21.7)
-//   4096 x 4096    | 18.7 / 16.1 | 18.7 / 16.8 | 19.0 / 17.4   | 19.3 / 18.3
-//   28672 x 4096   | 30.2 / 27.8 | 30.4 / 29.9 | (32.0 / 44.7) | (32.1 / 48.5)
-//   4096 x 14336   | 32.7 / 22.3 | 32.1 / 23.3 | 33.9 / 26.0   | 33.7 / 27.7
+// A matmul that is a call of its own takes its rows of floats as they are and splits them itself, every workgroup all of them, where
+// that takes less than a launch in front, 1.5 to 2 us and a little for long rows.  (The split is of every block by itself, as the fused
+// launches have it.)  A wave splits 128 columns of every request in each of its turns, and what that takes, 0.15 us per turn and request with 16
+// waves on a CU, is on the way of everybody behind it.  More than four requests: a build for eight, which splits as if there were eight, and for
+// four row tiles to a workgroup would spill.  Whole calls, us, split in front / now, in brackets where the split stays in front (turns):
+//   rows x columns | 1             | 4             | 5             | 8
+//   2560 x 2048    | 16.4 / 14.3   | 16.1 / 15.0   | 17.0 / 15.6   | 16.9 / 16.2     (1)
+//   8192 x 2048    |               |               | 18.5 / 16.9   | 18.5 / 17.5     (1, two row tiles)
+//   2048 x 5632    | 17.5 / 15.7   | 17.4 / 16.3   | 19.2 / 17.7   | 19.2 / 18.4     (1)
+//   2560 x 6912    |               |               | 19.8 / 18.7   | 19.7 / 19.0     (1.1)
+//   11264 x 2048   | 17.9 / 16.2   | 17.9 / 17.0   | four tiles    |                 (1)
+//   4096 x 14336   | 24.3 / 21.7   | 24.3 / 23.3   | (26.1 / 26.3) | (25.9 / 27.7)   (3.5)
+//   28672 x 4096   | 29.2 / 27.8   | (29.5 / 29.9) | four tiles    |                 (4)
+//   8192 x 8192    | 23.6 / 22.1   | (24.0 / 24.4) | (25.5 / 27.7) | (25.6 / 30.1)   (4)
+//   5120 x 13824   | 27.8 / 26.0   | (27.0 / 29.2) |               |                 (6.8)
+//   64000 x 4096   | 42.2 / 42.1   | (42.1 / 46.1) | four tiles    |                 (8: two rounds of workgroups)
+//   128256 x 4096  | (65.4 / 69.6) | (70.2 / 78.2) | four tiles    |                 (16)
 bool q4_splits_rows(size_t rows, size_t cols, size_t batch) {
-    const int tiles = batch <= 8 ? q4_tiles(kQ4Rows, rows, batch, q4_slices(rows, cols, batch).n) : 4;
-    return batch <= 4 || (batch <= 8 && (tiles == 1 || (tiles == 2 && cols > 4096)));
+    if (batch > 8) return false;
+    const Q4Slices s = q4_slices(rows, cols, batch);
+    if (batch > 4 && q4_tiles(kQ4Rows, rows, batch, s.n) > 2) return false;
+    // (as many workgroups as CUs have 16 waves, more of them 8, two workgroups to a CU: q4_waves)
+    const size_t n_cu = (size_t)g.n_cu, wgs = rows / 64 * s.n, waves = wgs > n_cu ? 8 : 16;
+    const size_t rounds = wgs > n_cu ? (wgs + 2 * n_cu - 1) / (2 * n_cu) : 1;
+    const size_t turns16 = rounds * std::max(waves, s.quads) * 16 / waves;   // sixteenths
+    return turns16 * (batch <= 4 ? batch : 8) <= 16 * 11 + cols / 256;
 }
 
-// The split of a batch's rows into fragments: 1024 threads per row from 4096 columns on, where 256 keep no row in registers.
+// The split of a batch's rows into fragments: 1024 threads per row above 4096 columns, where 256 keep no row in registers.
 void launch_q4_split(const float* x, _Float16* frag, float* inv_scale, size_t batch, size_t cols) {
     const unsigned threads = cols > 4096 ? 1024 : 256;
     hipLaunchKernelGGL(threads == 1024 ? q4_split_activations_kernel<1024> : q4_split_activations_kernel<256>, dim3((unsigned)batch), dim3(threads),

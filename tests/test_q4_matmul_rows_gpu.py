@@ -8,13 +8,15 @@ import test_q4_matmul_gpu as q4
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("batch", [1, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("batch", [1, 3, 4, 5, 7, 8, 9])
 @pytest.mark.parametrize("rows,cols", [
     (64, 64), (192, 96),            # half a quad; three blocks
     (2048, 2080),                   # slices, the last of them with a quad of one block
+    (256, 8224),                    # five slices of long rows
     (4160, 160), (8192, 2048),      # two row tiles
+    (2048, 5632), (2560, 6912),     # ... with three slices, a quad to a wave and for some a second one
     (8256, 288), (16448, 128),      # four, of 16 and 8 waves
-    (256, 8224),                    # two tiles or one, many quads to a wave
+    (16448, 4096),                  # four quads to a wave: split in front for four requests
 ])
 def test_rows_of_floats(exe, rows, cols, batch):
     q, x, stride = q4.make(rows, cols, batch, rows + cols + batch)
