@@ -72,19 +72,30 @@ def test_output_over_the_input(exe, rows, cols, batch, at):
 
 @pytest.mark.parametrize("batch", [2, 7])
 def test_blocks_far_apart(exe, batch):
-    """Every block has a power of two of its own: one whose elements are 2^-60 of another's keeps its 22 bits."""
+    """Every block has a power of two of its own: one whose elements are 2^-60 of another's keeps its 22 bits.  (The large
+    ones' weights are zeros: one power of two for a row would leave nothing of what is summed up.)"""
     rows, cols = 256, 512
     q, x, stride = q4.make(rows, cols, batch, 5)
+    q.reshape(rows, cols // 32, 18)[:, :8, :2] = 0          # (their scales)
     x[:, :256] *= 2.0 ** 60
     x[0, 32:64] = 0.0
-    x[1, 64:96] *= 2.0 ** -130          # (denormal numbers)
-    only_small = x.copy()
-    only_small[:, :256] = 0.0
-    for v in (x, only_small):
-        got = q4.run(exe, f"rowsin_far_{batch}", q, v, batch, rows, cols, stride)
-        w = q4.dequant(q, cols)
-        scale = np.abs(v.astype(np.float64)) @ np.abs(w).T
-        assert (np.abs(got - v.astype(np.float64) @ w.T) <= 4e-6 * scale + 1e-300).all()
+    got = q4.run(exe, f"rowsin_far_{batch}", q, x, batch, rows, cols, stride)
+    q4.check(got, q, x, batch, rows, cols, stride)
     x[0, 100] = np.inf
     got = q4.run(exe, f"rowsin_far_{batch}", q, x, batch, rows, cols, stride)
     assert not np.isfinite(got[0]).any() and np.isfinite(got[1:]).all()
+
+
+@pytest.mark.parametrize("batch", [2, 7])
+@pytest.mark.parametrize("exponent", [-88, -100, -118, -130])
+def test_tiny_numbers(exe, batch, exponent):
+    """The power of two is at most 2^100: smaller elements than 2^-86 have what an fp16 number of theirs has, down to its last
+    bit, 2^-24, of which rounding leaves half."""
+    rows, cols = 256, 512
+    q, x, stride = q4.make(rows, cols, batch, 6)
+    x = (x * 2.0 ** exponent).astype(np.float32)
+    got = q4.run(exe, f"rowsin_tiny_{batch}", q, x, batch, rows, cols, stride)
+    w, x64 = q4.dequant(q, cols), x.astype(np.float64)
+    # (2^-149 per addition: sums that are denormal numbers themselves)
+    bound = 4e-6 * (np.abs(x64) @ np.abs(w).T) + 2.0 ** -125 * np.abs(w).sum(1) + cols * 2.0 ** -149
+    assert (np.abs(got - x64 @ w.T) <= bound).all()
