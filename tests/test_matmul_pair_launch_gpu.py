@@ -14,7 +14,9 @@ def _weights(rng, rows, cols):
 
 
 class Pair:
-    """h = r + W0 mix, where mix = silu(gate) * up of Wg x0; n = norm(h); then W1 n and its split + SiLU or its split + RoPE + cast"""
+    """h = r + W0 mix, where mix = silu(gate) * up of Wg x0; n = norm(h); then W1 n and its split + SiLU ("silu"), its split + RoPE +
+    cast ("rope"), that and the scatters of K and V ("scatters") or the call that does all of it ("pages")"""
+    PAGE, PAGES = 16, 9
 
     def __init__(self, exe, reader, batch, mid, hid, heads, same=()):
         rng = np.random.default_rng(batch * 1000 + hid)
@@ -28,9 +30,12 @@ class Pair:
         shapes = {"x0": 64, "gu": 2 * mid, "g0": mid, "u0": mid, "mix": mid, "p": hid, "r": hid, "h": hid, "n": hid, "y": self.rows}
         shapes |= {"g": half, "u": half, "m": half} if reader == "silu" else {"q": heads * self.d, "k": kvd, "v": kvd}
         self.init = {m: rng.standard_normal((batch, n)).astype(np.float32) for m, n in shapes.items()}
-        if reader == "rope":
+        if reader != "silu":
             self.init |= {m: rng.uniform(-1, 1, (batch, self.d // 2)).astype(np.float32) for m in ("cos", "sin")}
             self.init |= {m: np.zeros((batch, kvd), np.uint16) for m in ("k16", "v16")}
+        if reader in ("scatters", "pages"):
+            self.init |= {m: np.zeros((self.PAGES, self.PAGE, kvd), np.uint16) for m in ("kp", "vp")}
+            self.ids, self.slots = rng.permutation(self.PAGES)[:batch].astype(np.uint32), rng.integers(0, self.PAGE, batch).astype(np.uint32)
         most = max(a.nbytes for a in self.init.values())       # (any of them can be another)
         self.dev = {m: exe.allocateScratchBuffer(most) for m in self.init}
         self.reset()
@@ -60,21 +65,30 @@ class Pair:
         if self.reader == "silu":
             return ok and exe.encodeGateUpSplitSiluMul(at("y"), at("g"), at("u"), at("m"), b, self.rows // 2, self.rows)
         kvd = self.kv * self.d
-        return ok and exe.encodeQkvSplitRopeCast(at("y"), at("q"), at("k"), at("v"), at("k16"), at("v16"), at("cos"), at("sin"), b,
-                                                 self.heads, self.kv, self.d, self.rows, self.heads * self.d, kvd, kvd, self.d)
+        sizes = b, self.heads, self.kv, self.d, self.rows, self.heads * self.d, kvd, kvd, self.d
+        if self.reader == "pages":
+            return ok and exe.encodeQkvSplitRopeScatter(at("y"), at("q"), at("kp"), at("vp"), at("cos"), at("sin"), self.ids, self.slots,
+                                                        self.PAGE, *sizes, at("k"), at("v"))
+        ok = ok and exe.encodeQkvSplitRopeCast(at("y"), at("q"), at("k"), at("v"), at("k16"), at("v16"), at("cos"), at("sin"), *sizes)
+        for pages, src in (("kp", "k16"), ("vp", "v16")) if self.reader == "scatters" else ():
+            ok = ok and exe.encodeScatterKVPagedBatched(at(pages), self.ids, self.slots, self.PAGE, self.kv, self.d, b, at(src))
+        return ok
 
     def once(self):
         return self.exe.beginForwardPassCB() and self.encode() and self.exe.flushForwardPassCB()
 
-    def captured(self, replays):
-        """(launches of the pass, the buffers after every replay)"""
+    def captured(self, replays, places=()):
+        """(launches of the pass, the buffers after every replay); places: pages and slots for each replay"""
         exe = self.exe
         assert exe.beginForwardPassCB() and exe.captureBegin() and self.encode()
         handle = exe.captureEnd()
         assert handle > 0 and exe.flushForwardPassCB(), exe.lastError()
         out = []
-        for _ in range(replays):
+        none = np.zeros(0, np.uint32)
+        for i in range(replays):
             self.reset()
+            if places:
+                assert exe.replayUpdate(handle, none, np.zeros(1, np.uint32), np.zeros(self.batch, np.uint32), none, *places[i]), exe.lastError()
             assert exe.beginForwardPassCB() and exe.replay(handle) and exe.flushForwardPassCB(), exe.lastError()
             out.append(self.read())
         n = exe.capturedLaunches(handle)
@@ -125,14 +139,49 @@ def test_two_matmuls_in_a_launch(exe, reader, batch, mid, hid, heads, pair):
         c.free()
 
 
-@pytest.mark.parametrize("same,pair", [
-    ({"h": "r"}, True), ({"h": "p"}, True),           # the first matmul's own buffers
-    ({"n": "h"}, False), ({"y": "r"}, False), ({"m": "p"}, False), ({"u": "r", "g": "p"}, False),
-    ({"m": "mix"}, True), ({"m": "x0"}, True),        # what the launch in front has read
+@pytest.mark.parametrize("reader,batch,mid,hid,heads", [
+    ("pages", 1, 5632, 2048, 32), ("pages", 4, 4224, 1984, 4), ("pages", 3, 4224, 4096, 72), ("scatters", 2, 5632, 2048, 32), ("scatters", 4, 4224, 4096, 72)])
+def test_rows_of_keys_and_values_in_pages(exe, reader, batch, mid, hid, heads):
+    """Page rows inside the arguments and, in a captured pass, on the device, where they change from replay to replay."""
+    c = Pair(exe, reader, batch, mid, hid, heads)
+    rng = np.random.default_rng(batch)
+    places = [(rng.permutation(c.PAGES)[:batch].astype(np.uint32), rng.integers(0, c.PAGE, batch).astype(np.uint32)) for _ in range(2)]
+    places = [(c.ids, c.slots), *places, (c.ids, c.slots)]
+    try:
+        got = {}
+        for on in (0, 1):
+            assert exe.setOption("q4_chain", on)
+            c.reset()
+            assert c.once(), exe.lastError()
+            got[on] = c.read(), *c.captured(4, places)
+        _same_bits(got[1][0], got[0][0])
+        _same_bits(got[1][2][0], got[0][0])
+        for i, (ids, slots) in enumerate(places):
+            _same_bits(got[1][2][i], got[0][2][i])
+            for pages, rows in (("kp", "k"), ("vp", "v")):
+                want = np.zeros_like(c.init[pages])
+                want[ids, slots] = got[1][2][i][rows].astype(np.float16).view(np.uint16)
+                assert np.array_equal(got[1][2][i][pages], want), (pages, i)
+        assert got[0][1] - got[1][1] == 1
+    finally:
+        exe.setOption("q4_chain", 1)
+        c.free()
+
+
+@pytest.mark.parametrize("reader,same,pair", [
+    ("silu", {"h": "r"}, True), ("silu", {"h": "p"}, True),           # the first matmul's own buffers
+    ("silu", {"n": "h"}, False), ("silu", {"y": "r"}, False), ("silu", {"m": "p"}, False), ("silu", {"u": "r", "g": "p"}, False),
+    ("silu", {"m": "mix"}, True), ("silu", {"m": "x0"}, True),        # what the launch in front has read
+    ("rope", {"q": "r"}, False), ("rope", {"k": "p"}, False), ("rope", {"v": "r"}, False), ("rope", {"k16": "p"}, False),
+    ("rope", {"v16": "r"}, False), ("rope", {"q": "h"}, False), ("rope", {"cos": "h"}, False), ("rope", {"sin": "p"}, False),
+    ("rope", {"cos": "r"}, True),                                     # both read it
+    ("rope", {"q": "mix", "k16": "x0"}, True),
+    ("pages", {"kp": "r"}, False), ("pages", {"vp": "p"}, False), ("pages", {"kp": "mix"}, True), ("scatters", {"vp": "r"}, False),
 ])
-def test_buffers_that_meet(exe, same, pair):
-    """Where the second matmul writes what the first one reads or writes the two are launched one after the other."""
-    c = Pair(exe, "silu", 2, 5632, 512, 88, same)
+def test_buffers_that_meet(exe, reader, same, pair):
+    """Where the second matmul writes what the first one reads or writes, or reads what it writes, the two are launched one after the
+    other."""
+    c = Pair(exe, reader, 2, 5632, 512, 88 if reader == "silu" else 32, same)
     try:
         got = {}
         for on in (0, 1):
