@@ -269,10 +269,12 @@ int mlc_hip_paged_attn_prefill(const void* q_f16, const void* k_pages, const voi
  * library's stream and looks up the scratch array's device address).  The call returns when the
  * kernel is enqueued (no synchronisation).  Every decode launch of this library on one GPU
  * uses the same scratch array, so they must follow each other, and so must they and matmuls whose
- * K slices meet inside the launch (both wait for workgroups of their own): the library remembers the
- * stream of the last one and puts a launch on another stream behind what that stream held at the time
- * (events created at set-up); what the caller enqueues on its own streams by other means is the
- * caller's to order.  A caller that records the call into a graph of its own may replay it: the launch
+ * K slices meet inside the launch, or two of which go out in one launch (all wait for workgroups of
+ * their own): the library remembers the stream of the last one and puts a launch on another stream
+ * behind what that stream held at the time (events created at set-up); what the caller enqueues on its
+ * own streams by other means is the caller's to order.  Another process on the same GPU is not ordered
+ * with them: the decode launches of two processes may hold each other up, and so may launches of two
+ * matmuls of three processes (option "q4_chain" = 0: none), until the wait is given up and both passes fail.  A caller that records the call into a graph of its own may replay it: the launch
  * keeps this call's lengths and reads everything else anew, and one small launch in front of it tells
  * the replay's partials from those of the replay before.  Operators that earlier encode calls held back are launched first, on the
  * library's stream, and a caller's stream is put behind them.  Not possible while a pass is
@@ -307,10 +309,11 @@ int mlc_hip_paged_attn_decode_noalloc(const void* q, const void* k_pages, const 
  * 128, page sizes and GQA ratios as in the call above, 16-byte aligned buffers).  mlc_hip_capture_end returns a
  * handle > 0, or 0 (then nothing was kept; encode the pass uncaptured).  mlc_hip_captured_launches
  * counts the launches of the encode calls; the pass holds one more, the library's own first launch,
- * which moves a device word on by which the decode launches of one replay, and its matmuls whose K
- * slices meet inside the launch, tell their partials from those of the replay before.  A pass holds at
- * most 4096 decode launches; matmuls beyond 4096 such ones, and ones that find no buffer to meet in from
- * an uncaptured call, take K whole.
+ * which moves a device word on by which the decode launches of one replay, its matmuls whose K slices
+ * meet inside the launch and its launches of two matmuls tell their words from those of the replay
+ * before.  A pass holds at most 4096 decode launches, and 4096 times slices or second matmuls in a
+ * launch; matmuls beyond, and ones that find no buffer to meet in from an uncaptured call, take K whole
+ * and a launch each.
  *
  * mlc_hip_replay_update copies the step's tables (seq_lens [batch], q_positions [batch],
  * page_table_offsets [batch + 1], the flat table; page_ids / slots_in_page [batch]) over the
@@ -420,7 +423,11 @@ long mlc_hip_decode_table_uploads(void);
  *                           see the mlc_hip_fused_* counters above.
  *                           0 = each operator is launched when it is encoded
  *   "q4_chain"              1 (default) = for up to four requests, a Q4_0 matmul with its residual add and the
- *                           matmul that reads the RMSNorm behind it go out in one launch; 0 = always two
+ *                           matmul that reads the RMSNorm behind it go out in one launch, if that is
+ *                           followed by the gate/up split (up to 2048 columns and 15872 rows) or by
+ *                           the split of a qkv row (up to 4096 columns); 0 = always two.  The second
+ *                           matmul's workgroups wait for the first one's: with three or more processes
+ *                           on one GPU set it to 0
  *   "decode_pair_cost"      0..64: the tile-balanced decode kernel gives every workgroup the same
  *                           number of units, a KV tile counting one and the end of a (request,
  *                           KV head) pair this many; 0 = the same number of tiles; -1 (default) =

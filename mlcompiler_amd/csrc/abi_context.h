@@ -626,7 +626,9 @@ bool overlap(const void* a, size_t na, const void* b, size_t nb) {
     return x < y + nb && y < x + na;
 }
 
-// The matmul in front and the held-back one in one launch (q4_chain_kernel): 1, 0 on failure, -1 where they cannot be.
+// The matmul in front and the held-back one in one launch (q4_chain_kernel): 1, 0 on failure, -1 where they cannot be.  A wave
+// of the second one holds its weights unpacked, 16 registers per row tile and quad of K, 64 of them at most: gate/up projections (four
+// tiles) of up to 2048 columns, qkv projections (one or two) of up to 4096, which are as many as a norm in between has.
 int launch_chain(Q4Form form, bool block_scales, Q4RopeArgs& b) {
     Q4RopeArgs& a = g.front.a;
     const size_t batch = b.batch;

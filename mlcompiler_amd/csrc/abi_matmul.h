@@ -268,8 +268,9 @@ int mlc_hip_matmul_q4_0_batched(const char* weight_name, const void* weights, si
         } else if (!rows_in) {
             launch_q4_split(xin, frag, inv, bn, cols);
         }
-        // The slices' sums meet in the launch; a matmul that has no tag or no memory for that takes all of K.  (Everything
-        // held back has been launched: buffers that it reads may be replaced now.)
+        // The slices' sums meet in the launch; a matmul that has no tag or no memory for that takes all of K.  (What was held
+        // back has been launched, but for a matmul that waits in front of this one: that one takes no slices here, and
+        // cached_buffer launches the other before it gives up a buffer.)
         Q4Slices split = feeds_rms ? Q4Slices{1, quads} : q4_slices(rows, cols, std::min<size_t>(batch, 64));
         uint64_t* words = nullptr;
         if (split.n > 1 && g.opt_q4_int_operand) {

@@ -309,7 +309,7 @@ enum Q4Form { kQ4Plain = 0, kQ4Silu = 1, kQ4Rope = 2, kQ4Add = 3, kQ4Rows = 4 };
 // a wave's last blocks) -> now.  One request of the 1 B shape: qkv (2560 x 2048) 7.0 -> 4.5, out-projection with the
 // residual add 8.4 -> 4.6, gate/up with SiLU (11264 x 2048) 11.2 -> 7.0, down (2048 x 5632) 8.1 and 5.0 for the sum of
 // its K slices -> 5.5 with the residual add, three slices that meet in here; a step of 22 layers 1 145 -> 801 (845 with the
-// fragments of 32 requests as they are for larger batches; 703 with everything since).  32 requests: qkv 7.5 -> 6.9,
+// fragments of 32 requests as they are for larger batches; 670 with everything since but q4_chain_kernel, 609 with that).  32 requests: qkv 7.5 -> 6.9,
 // gate/up 13.3 -> 13.3, a step 1 330 -> 1 199 (1 108).  16 requests of the 8 B shape: gate/up (28672 x 4096) 28.9 -> 23,
 // a layer 140 -> 112 (106).  2-norm error against float64 of rows of 2048 to 14336: 0.95e-7 .. 1.17e-7, before 1.03e-7 .. 1.62e-7.
 //
@@ -342,8 +342,8 @@ __global__ __launch_bounds__(WAVES * 64, ZT > 1 ? 2 : 4) void q4_matmul_kernel(
     const uint4* const w_q, const uint2* const w_d, const _Float16* const xfrag, const float* const blk_scale, const float* const ssq_in,
     const uint32_t nblocks, const uint32_t quads_per_slice, const uint32_t row_groups, const uint32_t batch_z,
     const std::conditional_t<FORM == kQ4Rope, Q4RopeArgs, Q4Args> a) {
-    // (The body itself and LDS arrays of their own, not a call of q4_matmul_workgroup: behind one the compiler takes 174 registers
-    // instead of 156 for gate/up at 32 requests, and the launch 12.74 us instead of 12.60.)
+    // (The body itself and LDS arrays of their own, not a call of q4_matmul_workgroup: behind one, given the arrays in a struct or as
+    // pointers, the compiler takes 174 registers instead of 156 for gate/up at 32 requests, and the launch 12.74 us instead of 12.60.)
     constexpr int LINK = kQ4LinkNone, QUADS = 1;
     typedef Q4Lds<NI, RT, WAVES, BS, ZT> Lds;
     __shared__ decltype(Lds::red) red;
@@ -375,11 +375,13 @@ __device__ __forceinline__ void q4_matmul_workgroup(
 // one's way to its first weights off the chain of launches that a step is, and its unpacking, 0.7 us of the vector pipe per four
 // row tiles: while it waits a wave holds its weights as halves in up to 64 registers.
 //
-// Measured: out-projection and gate/up of the 1 B shape at one request 12.0 us in two launches, 8.0 in one, of which, from the
-// start: the first one's weights back 1.5, its sums published 3.5 (vector pipe, 16 waves), seen 4.3, all words in LDS 4.9, products
-// 5.9, waves' sums met 6.3, stored 7.4.  With one copy of the words, a quad's scales in the lines of all the others' they were seen at
-// 5.5.  Steps of 22 layers, us, two launches -> one: 1, 2, 3, 4 requests 683, 696, 702, 705 -> 618, 643, 654, 673; a
-// build for 5 and 8 requests 771, 778 -> 763, 784 (every workgroup fetches 8 bytes per request and column): two launches there.
+// Measured: out-projection and gate/up of the 1 B shape at one request, in a kernel trace, 4.6 and 6.9 us and a launch's 2.3 in
+// between, 9.1 in one launch; down-projection and qkv 6.2 and 4.0, 9.2.  From the start, by the time stamps of a probe build (out-projection
+// and gate/up): the first one's weights back 1.5, its sums published 3.5 (vector pipe, 16 waves), seen 4.3, all words in LDS 4.9,
+// products 5.9, waves' sums met 6.3, stored 7.4.  With one copy of the words, a quad's scales in the lines of all the others', they were
+// seen at 5.5.  Steps of 22 layers and the lm_head, us, option q4_chain 0 -> 1, 600 cached tokens: 1, 2, 3, 4 requests 670, 678, 686, 695 ->
+// 609, 638, 649, 668; a build for 5 and 8 requests 771, 778 -> 763, 784 (every workgroup fetches 8 bytes per request and column): two
+// launches there.
 template <int FORM>
 struct Q4ChainArgs {
     Q4Args first;
